@@ -4,6 +4,18 @@
 
 namespace kascade {
 
+// Raw scores travel from the anchor pass to the pooling kernel in a compact form: per head a row of
+// scores_stride floats holds, in its first half, one 16-bit code per token and, behind them, one
+// fp32 reference per granule of 64 tokens (the granule's largest scaled score, log2 domain).
+// code = round((reference - score*scale) * 2048), i.e. steps of 2^-11 in the exponent: the
+// probability recovered from it is within 1.7e-4 (a third of an fp16 step) of the exact one, and
+// a code of 65534 steps (2^-32 of the granule's maximum, itself at most the row's log-sum) is far
+// below what survives the pooled sum's fp16 rounding.  65535 marks a masked position.  Splits
+// start at multiples of 64 tokens, so a granule belongs to one workgroup.  Half the bytes of fp32
+// scores: their write-back to HBM, interleaved with the K stream, costs several times its size.
+constexpr float kScoreSteps = 2048.f;
+constexpr uint32_t kScoreNone = 65535u;
+
 struct DecodeParams {
     // Q, K, V, the new rows and the output hold elements of kind `elem` (fp16 or bf16); G KV heads,
     // H = gs G query heads, head dimension head_dim (64 or 128).
@@ -44,6 +56,9 @@ struct DecodeParams {
     int scores_stride;
     int num_split;
     int rows_per_split;     // multiple of 64; num_split*rows_per_split >= longest row list
+    // set by launch_decode_split
+    int strip_shift;        // log2 of a wavefront's strip (token ranges)
+    int number_splits;      // number the non-empty splits of a ragged batch consecutively
     int B;
     int G;                  // KV heads
     int head_dim;           // 64 or 128

@@ -27,20 +27,9 @@ constexpr int kThreads = 256;
 // The instruction scheduler otherwise sinks every prefetch load down to its first use (to save
 // registers), which serialises load -> wait -> use and removes all memory-level parallelism.
 #define KASCADE_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
-constexpr int kStripRows = 256;               // consecutive tokens a wavefront owns per 1024
+constexpr int kStripRows = 256;               // consecutive tokens a wavefront owns, at most (p.strip_shift)
+constexpr int kMaxNumbered = 256;             // sequences whose splits one wavefront numbers
 constexpr int kSubChunk = 2048;               // rows whose physical ids are staged in LDS at once
-// Raw scores travel from the anchor pass to the pooling kernel in a compact form: per head a row of
-// scores_stride floats holds, in its first half, one 16-bit code per token and, behind them, one
-// fp32 reference per granule of 64 tokens (the granule's largest scaled score, log2 domain).
-// code = round((reference - score*scale) * 2048), i.e. steps of 2^-11 in the exponent: the
-// probability recovered from it is within 1.7e-4 (a third of an fp16 step) of the exact one, and
-// a code of 65534 steps (2^-32 of the granule's maximum, itself at most the row's log-sum) is far
-// below what survives the pooled sum's fp16 rounding.  65535 marks a masked position.  Splits
-// start at multiples of 64 tokens, so a granule belongs to one workgroup.  Half the bytes of fp32
-// scores: their write-back to HBM, interleaved with the K stream, costs several times its size.
-constexpr float kScoreSteps = 2048.f;
-constexpr uint32_t kScoreNone = 65535u;
-
 // Device-coherent accesses (relaxed atomics at agent scope) for data that one workgroup writes
 // and another workgroup of the same launch reads.
 __device__ __forceinline__ void store_device(float* p, float v) {
@@ -116,6 +105,10 @@ void decode_split_kernel(DecodeParams p) {
     const int wave = tid >> 6;
     const int lane = tid & 63;
 
+    // Gather mode: requested at once, together with the lengths (it decides where the list is, the next
+    // trip to memory).  A map built for another KV-head count must not leave the index tensor.
+    const int map_g = GATHER ? max(0, min(p.head_map[g], kvh - 1)) : 0;
+
     // The longest context memory allows a sequence that claims `len` tokens: lengths live in device
     // memory, the host sized every buffer from its own arguments, so each length is cut down to
     // what the block table covers (or the cache holds) and, on an anchor pass, to the row width of
@@ -152,15 +145,13 @@ void decode_split_kernel(DecodeParams p) {
     // ragged batch has many -- come last in dispatch order and exit at once, instead of being
     // scattered among the working ones, which left some compute units with several streams and
     // others with none (four sequences of 131072..524288 tokens, 512 working workgroups: gather
-    // 101 -> 86 us).  One sequence needs none of this; beyond 64 * kMapRounds sequences the
-    // workgroups keep their grid position.  Neither do gather launches whose lists all have the
-    // same length (no per-sequence budget): every split of the grid has work, and leaving the
-    // numbering out takes one dependent trip to memory off the start of every workgroup.
-    constexpr int kMapRounds = 4;
+    // 101 -> 86 us).  One sequence needs none of this, and neither do launches that are resident
+    // at once or whose lists all have the same length (launch_decode_split decides); beyond
+    // kMaxNumbered sequences the workgroups keep their grid position.
+    constexpr int kMapRounds = kMaxNumbered / 64;
     int b, split, nsplit_b, seqlen;
     bool len_cut;
-    const bool ragged_rows = !GATHER || p.topk_percent > 0.f;
-    if (p.seqlens != nullptr && p.B > 1 && p.B <= 64 * kMapRounds && ragged_rows) {
+    if (p.number_splits) {
         // every wavefront works it out for itself: lane l holds sequences l, l + 64, ...; no LDS,
         // no barrier, and the sequence's length comes out of the same loads (all issued first)
         const int w = blockIdx.y + gridDim.y * blockIdx.z;
@@ -207,6 +198,10 @@ void decode_split_kernel(DecodeParams p) {
         const int raw = p.seqlens ? p.seqlens[b] : p.kv_stride_tokens;
         seqlen = safe_len(raw);
         len_cut = seqlen != raw;
+        if (p.seqlens != nullptr) {
+            nsplit_b = split_count(rows_for(seqlen));
+            if (split >= nsplit_b) return;   // the first split marks the missing ones as empty
+        }
     }
     const int n = rows_for(seqlen);  // rows this (b, g) pair attends to
     // contiguous range of this split; every split covers rows_per_split rows, sequences
@@ -290,8 +285,7 @@ void decode_split_kernel(DecodeParams p) {
     for (int blk = 0; blk < (WITH_V ? kOBlocks : 1); ++blk) oacc[blk] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     const int* idx_row = nullptr;
-    // a map built for another KV-head count must not leave the index tensor
-    if (GATHER) idx_row = p.idx + ((size_t)b * kvh + max(0, min(p.head_map[g], kvh - 1))) * p.topk;
+    if (GATHER) idx_row = p.idx + ((size_t)b * kvh + map_g) * p.topk;
     const int page_mask = (1 << p.page_shift) - 1;
     const unsigned stride_l = p.kv_stride_l;
     T* kt = &s_kt[wave][0];
@@ -532,19 +526,22 @@ void decode_split_kernel(DecodeParams p) {
         };
         if (p.block_table) run(std::true_type{}); else run(std::false_type{});
     } else {
-        // Token range [r0, r1) (dense baseline, anchor passes): no staging.  A wavefront owns 256
-        // consecutive tokens of every 1024 and walks them in tiles of 16, four consecutive tiles
+        // Token range [r0, r1) (dense baseline, anchor passes): no staging.  A wavefront owns one strip
+        // of consecutive tokens out of every four and walks it in tiles of 16, four consecutive tiles
         // (one 64-token granule of the score codes) per loop iteration: 16 KB in flight per
         // wavefront (two tiles of K and V, or four of K alone), block table entries one round
-        // further ahead so that no row address waits for its page number.
+        // further ahead so that no row address waits for its page number.  Strips are 256 tokens in
+        // long splits; shorter in splits of up to 2048 tokens, which 256-token strips leave to some of
+        // the wavefronts (a split of 192 tokens ran on one, in 16 serial tiles: 700 tokens, batch 1,
+        // 11.1 us for K alone and 17.1 with V; 6.7 and 8.2 with 64-token strips).
         const int cn = r1 - r0;
         const int* bt_row = p.block_table ? p.block_table + (size_t)b * p.max_pages : nullptr;
         constexpr int kDepth = WITH_V ? 2 : 4;
-        constexpr int kTilesPerStrip = kStripRows / 16;
+        const int strip_shift = p.strip_shift, strip = 1 << strip_shift, tps = strip >> 4;   // tiles per strip: 4, 8 or 16
         auto run = [&](auto paged_tag) {
         constexpr bool PAGED = decltype(paged_tag)::value;
-        // tile k of this wavefront: 16 keys from row (k / 16) * 1024 + wave * 256 + (k % 16) * 16
-        auto tile_row = [&](int k) { return (k / kTilesPerStrip) * (4 * kStripRows) + wave * kStripRows + (k % kTilesPerStrip) * 16; };
+        // tile k of this wavefront: 16 keys from row (k / tps) * 4 strips + wave * strip + (k % tps) * 16
+        auto tile_row = [&](int k) { return ((k >> (strip_shift - 4)) << (strip_shift + 2)) + (wave << strip_shift) + ((k & (tps - 1)) << 4); };
         auto tok_of = [&](int k, int i) { return min(r0 + tile_row(k) + kRowsPerLoad * i + lr, r1 - 1); };   // past the end: clamped, masked later
         auto fetch_pages = [&](int k, int (&pg)[kLoads]) {
 #pragma unroll
@@ -558,17 +555,23 @@ void decode_split_kernel(DecodeParams p) {
             }
         };
         if (cn > 0) {
-            const int nsup = (cn + 4 * kStripRows - 1) / (4 * kStripRows);
-            const int ntile = nsup * kTilesPerStrip;   // the same for every wavefront
+            const int nsup = (cn + 4 * strip - 1) >> (strip_shift + 2);
+            // every strip of this wavefront but its last is full; of that one only the granules that hold tokens
+            const int tail = cn - ((nsup - 1) << (strip_shift + 2)) - (wave << strip_shift);
+            const int ntile = (nsup - 1) * tps + max(0, min(tps, (tail + 63) / 64 * 4));
+            const int phase_sups = kPhaseRows >> (strip_shift + 2);   // rounds of four strips whose codes fit in LDS
+            int phase = 0, in_phase = 0;
             Tile buf[kDepth];
             int pgn[kDepth][kLoads];
+            if (ntile > 0) {   // uniform over the wavefront
 #pragma unroll
-            for (int j = 0; j < kDepth; ++j) {
-                fetch_pages(j, pgn[j]);
-                issue(j, pgn[j], buf[j]);
+                for (int j = 0; j < kDepth; ++j) {
+                    fetch_pages(j, pgn[j]);
+                    issue(j, pgn[j], buf[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < kDepth; ++j) fetch_pages(kDepth + j, pgn[j]);
             }
-#pragma unroll
-            for (int j = 0; j < kDepth; ++j) fetch_pages(kDepth + j, pgn[j]);
             for (int k = 0; k < ntile; k += 4) {   // four consecutive tiles: one granule of 64 tokens
                 float4_t sc[4];
 #pragma unroll
@@ -581,12 +584,18 @@ void decode_split_kernel(DecodeParams p) {
                     KASCADE_SCHED_FENCE();
                 }
                 if (WRITE_SCORES) {
-                    const int sup = k / kTilesPerStrip;
-                    encode_granule(sc, (sup % kCodePhase) * (4 * kStripRows) + wave * kStripRows + (k % kTilesPerStrip) * 16);
-                    if ((k + 4) % (kTilesPerStrip * kCodePhase) == 0) flush_phase(sup / kCodePhase);
+                    const int sup = k >> (strip_shift - 4);
+                    encode_granule(sc, (in_phase << (strip_shift + 2)) + (wave << strip_shift) + ((k & (tps - 1)) << 4));
+                    if (((k + 4) & (tps - 1)) == 0) {   // end of a strip
+                        // the last phase leaves after the loop: there the wavefronts' tile counts may differ
+                        if (++in_phase == phase_sups && sup + 1 < nsup) {
+                            flush_phase(phase++);
+                            in_phase = 0;
+                        }
+                    }
                 }
             }
-            if (WRITE_SCORES && nsup % kCodePhase != 0) flush_phase(nsup / kCodePhase);
+            if (WRITE_SCORES) flush_phase((nsup - 1) / phase_sups);
         }
         };
         if (bt_row) run(std::true_type{}); else run(std::false_type{});
@@ -641,7 +650,12 @@ void decode_split_kernel(DecodeParams p) {
         const size_t ph = ((size_t)b * nheads + g * gs + h) * p.num_split + split;
         const float lse_part = (L > 0.f) ? (fast_log2(L) + mref) : -INFINITY;
         const float inv = (L > 0.f) ? 1.f / L : 0.f;
-        if (p.counters == nullptr) {
+        if (p.counters != nullptr && nsplit_b == 1) {
+            // the only split of its sequence: nothing to merge, no counter and no second trip
+            const size_t hd = (size_t)b * nheads + g * gs + h;
+            if (p.row_sums && (tid & 63) == 0) p.row_sums[hd] = lse_part;
+            if (WITH_V && has_d) *reinterpret_cast<x2_t*>((T*)p.out + hd * D + d0) = x2_t{(T)(o0 * inv), (T)(o1 * inv)};
+        } else if (p.counters == nullptr) {
             if ((tid & 63) == 0) p.glse[ph] = lse_part;
             if (WITH_V && has_d) *reinterpret_cast<float2*>(p.opart + ph * D + d0) = make_float2(o0 * inv, o1 * inv);
         } else {
@@ -662,7 +676,7 @@ void decode_split_kernel(DecodeParams p) {
     // waits for those stores before thread 0 counts this workgroup in; the merging workgroup
     // reads them back with device-coherent loads.  No device-wide fence is involved: one per
     // workgroup would write back and invalidate the L2 that the K/V stream lives in.
-    if (p.counters == nullptr) return;
+    if (p.counters == nullptr || nsplit_b == 1) return;
     // Every wavefront waits until its own stores above have been acknowledged (they are
     // write-through at device scope, so an acknowledged store is in device-coherent memory) and
     // only then joins the barrier.  The barrier by itself does not do this: at workgroup scope
@@ -931,8 +945,16 @@ hipError_t launch_combine_t(const float* glse, const float* opart, void* out, fl
 }  // namespace
 
 // head_dim in {64, 128}, elem in {kElemF16, kElemBF16}: checked by the callers
-hipError_t launch_decode_split(const DecodeParams& p, bool gather, bool with_v, bool write_scores,
+hipError_t launch_decode_split(const DecodeParams& p0, bool gather, bool with_v, bool write_scores,
                                hipStream_t stream) {
+    DecodeParams p = p0;
+    // strips: what leaves no wavefront more than one granule ahead in splits of up to 1024 tokens
+    p.strip_shift = p.rows_per_split <= 1024 ? 6 : p.rows_per_split <= 2048 ? 7 : 8;
+    // Numbering the non-empty splits costs every workgroup a trip to memory and a scan; it pays where
+    // the grid is larger than what is resident at once (two workgroups on each of 256 compute units).
+    const bool ragged_rows = !gather || p.topk_percent > 0.f;
+    p.number_splits = p.seqlens != nullptr && p.B > 1 && p.B <= kMaxNumbered && ragged_rows &&
+                      (long long)p.G * p.num_split * p.B > 512;
     if (p.head_dim == 128)
         return p.elem == kElemBF16 ? launch_split_t<128, bf16_t>(p, gather, with_v, write_scores, stream)
                                    : launch_split_t<128, half_t>(p, gather, with_v, write_scores, stream);
