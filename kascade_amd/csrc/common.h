@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace kascade {
 
 constexpr int kHeads = 32;     // query heads
@@ -113,6 +115,14 @@ __device__ __forceinline__ float sum_with_other_half(float x) {
 
 __device__ __forceinline__ uint4_t ld_global_16(const void* p) {
     return *reinterpret_cast<const uint4_t*>(p);
+}
+
+// f(integral_constant<int, I>) for I in [FROM, TO): for register arrays whose indices must be constants
+template <int FROM, int TO, typename F> __device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (FROM < TO) {
+        f(std::integral_constant<int, FROM>{});
+        static_for<FROM + 1, TO>(f);
+    }
 }
 
 inline int ilog2_exact(int x) {  // host: log2 of a power of two, -1 otherwise

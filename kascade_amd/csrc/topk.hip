@@ -10,6 +10,7 @@
 
 #include <type_traits>
 
+#include "decode.h"    // score codes
 #include "prefill.h"   // launch_translate_indices
 
 namespace kascade {
@@ -19,6 +20,7 @@ namespace {
 constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
 constexpr int kChunk = kThreads * 8;
+constexpr int kComputeUnits = 256;
 constexpr int kBins1 = 2048;
 }  // namespace
 constexpr int kSplitMinLen = 65537;   // longer than a workgroup's registers hold: multi-workgroup path
@@ -37,7 +39,7 @@ struct RowsOut {
 };
 
 __device__ __forceinline__ int to_cache_row(const RowsOut& ro, long long row, int pos) {
-    const int* bt = ro.block_table + (row / ro.rows_per_seq) * ro.max_pages;
+    const int* bt = ro.block_table + (long long)((uint32_t)row / (uint32_t)ro.rows_per_seq) * ro.max_pages;   // rows fit an int (host)
     pos = max(0, min(pos, (ro.max_pages << ro.page_shift) - 1));
     return (bt[pos >> ro.page_shift] << ro.page_shift) + (pos & ((1 << ro.page_shift) - 1));
 }
@@ -249,58 +251,290 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(
 }
 
 
-// The same selection with the row held in registers: every thread loads its share of the row
-// once (MAXC 16-byte loads in flight, instead of one per pass and chunk with its latency
-// exposed), turns it into packed order keys once, and the three passes run on registers.  With
-// 16 to 64 entries per thread and eight wavefronts per SIMD the kernel is bound by the
-// instructions spent per entry, so the per-entry work is kept to a few instructions:
-//  * Real entries carry keys >= 1 (the two lowest negative NaN patterns share key 1) and the
-//    slots past the end of the row key 0, so the threshold key T is >= 1 and no count needs a
-//    validity test: a slot past the end is neither above T nor equal to it.
-//  * The coarse histogram is kept in kCopies copies selected by the lane number, which spreads
-//    the same-address conflicts of the LDS atomics (pooled softmax scores crowd into a few
+// ---- selection with the row in registers ----
+// A workgroup of THREADS threads holds one row and runs the passes on registers.  Its wavefronts own
+// contiguous parts of the row, `nch` chunks of 512 slots each: lane l of a wavefront holds slots
+// [512 c + 8 l, +8) of chunk c of its part as packed 16-bit order keys, 0 where there is no entry.
+//
+// What bounds it is instruction issue on the one compute unit the row runs on -- every entry costs
+// about ten instructions, every wavefront about three hundred on top whatever it holds -- so rows get the
+// fewest wavefronts that hold them, the work per entry is kept to a few instructions on packed halves,
+// nothing has a second copy for partial chunks, and the position order (wavefront, chunk, lane, entry)
+// needs one scan over the wavefronts instead of one over all (chunk, wavefront) pairs:
+//  * Real entries carry keys >= 1 (the two lowest negative NaN patterns share key 1) and absent
+//    slots key 0, so the threshold key T is >= 1 and no count needs a validity test.
+//  * The coarse histogram (key >> 5) is kept in four copies selected by the lane number, which
+//    spreads the same-address conflicts of the LDS atomics (pooled softmax scores crowd into a few
 //    exponent bins).  The bin of +0 and the 31 smallest subnormals, where pooled probabilities
 //    underflow to by the thousand, is not counted at all: its count is the row length minus the
-//    sum of the others.
+//    sum of the others.  NONNEG: no entry is below +0 (pooled probabilities), half the bins.
 //  * The fine histogram tests both halves of a word against the threshold bin at once; the counts
 //    above / equal to T are sums of min(sat(key - (T-1)), 2) over packed halves.
-//  * The compaction computes every (chunk, thread) offset with two barriers in all (per-chunk
-//    wavefront scans, then one scan over the chunk x wavefront totals), and stages the selected
-//    indices in LDS in their final order, so that the row's list leaves as full-width stores.
+//  * The selected positions are staged in LDS in their final order, so that the list leaves as
+//    full-width stores.
+// Causal prompt tiles (8 heads x L/32 rows, ragged): L = 4096 18.2 -> 10.2 us, 8192 34 -> 20, 16384
+// 73 -> 48, 32768 178 -> 151, 65536 905 -> 584 us; 2048 full rows of 65536: 141 us = 1.9 TB/s.
+// Sum of the entries of s_wave before `wave`, and of all of them (one per wavefront, in LDS).
+template <int THREADS>
+__device__ __forceinline__ void scan_waves(const uint32_t* s_wave, int wave, uint32_t& before, uint32_t& all) {
+    constexpr int kW = THREADS / 64;
+    const int lane = threadIdx.x & 63;
+    const uint32_t inc = wave_incl_scan(lane < kW ? s_wave[lane] : 0u);
+    all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    before = wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)inc, wave - 1) : 0u;
+}
+
+template <int THREADS, int MAXC, bool NONNEG>
+__device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch, int lead, int row_len, int n, int k,
+                                           int fill, int* __restrict__ out, long long row, const RowsOut& ro) {
+    constexpr int kW = THREADS / 64;
+    constexpr int kCopies = 4;
+    constexpr int kNB = NONNEG ? 1024 : 2048;                        // coarse bins ...
+    constexpr uint32_t kBin0 = NONNEG ? 1024 : 0;                    // ... from this one on
+    constexpr int kStage = kNB * kCopies;                            // positions staged in the histogram's LDS
+    constexpr uint32_t kOne = 0x00010001u, kTwo = 0x00020002u;
+    constexpr uint32_t kZeroKey = 0x8000u;                           // order key of +0
+    constexpr uint32_t kSkipBin = kZeroKey >> 5;                     // coarse bin of +0: counted by subtraction
+    constexpr int kBPT = kNB / THREADS > 0 ? kNB / THREADS : 1;      // bins per thread in the scan
+    static_assert(kNB % THREADS == 0 || kNB < THREADS, "whole bins per thread");
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist[kNB * kCopies];
+    __shared__ uint32_t s_hist2[32];
+    __shared__ uint32_t s_wave[kW], s_gt[kW], s_eq[kW];
+    __shared__ uint32_t s_sel[2];  // b1, cum_above
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int* dst = out + row * (long long)k;
+    int* rdst = ro.rows ? ro.rows + row * (long long)k : nullptr;
+
+    // ---- pass 1: coarse histogram ----
+    for (int i = tid * 4; i < kNB * kCopies; i += THREADS * 4) *reinterpret_cast<uint4_t*>(&s_hist[i]) = uint4_t{0, 0, 0, 0};
+    if (tid < 32) s_hist2[tid] = 0;
+    __syncthreads();
+    const uint32_t copy = tid & (kCopies - 1);
+    auto count1 = [&](uint32_t key) {   // absent entries and the bin of +0 are not counted
+        const uint32_t bin = key >> 5;
+        if (NONNEG ? bin > kSkipBin : (key != 0 && bin != kSkipBin)) atomicAdd(&s_hist[(bin - kBin0) * kCopies + copy], 1u);
+    };
+    static_for<0, MAXC>([&](auto c_c) {
+        constexpr int c = decltype(c_c)::value;
+        if (c < nch) {   // uniform
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                count1(data[c][j] & 0xFFFFu);
+                count1(data[c][j] >> 16);
+            }
+        }
+    });
+    __syncthreads();
+    {
+        // thread t owns kBPT bins, in descending order
+        uint32_t cnt[kBPT], mine = 0;
+        const int first = kNB - 1 - kBPT * tid;
+#pragma unroll
+        for (int u = 0; u < kBPT; ++u) {
+            cnt[u] = 0;
+            if (kNB >= THREADS || tid < kNB) {
+                const uint4_t h = *reinterpret_cast<const uint4_t*>(&s_hist[(first - u) * kCopies]);
+                cnt[u] = h[0] + h[1] + h[2] + h[3];
+            }
+            mine += cnt[u];
+        }
+        const uint32_t inc = wave_incl_scan(mine);
+        if (lane == 63) s_wave[wave] = inc;
+        __syncthreads();
+        uint32_t before, total;
+        scan_waves<THREADS>(s_wave, wave, before, total);
+        uint32_t above = before + inc - mine;
+        const uint32_t skipped = (uint32_t)row_len - total;
+        constexpr int kSkipAt = kNB - 1 - (int)(kSkipBin - kBin0);   // place of the uncounted bin in descending order
+        if (tid > kSkipAt / kBPT) above += skipped;
+#pragma unroll
+        for (int u = 0; u < kBPT; ++u) {
+            const uint32_t c = cnt[u] + (kBPT * tid + u == kSkipAt ? skipped : 0u);
+            if (above < (uint32_t)n && (uint32_t)n <= above + c) {
+                s_sel[0] = (uint32_t)(first - u) + kBin0;
+                s_sel[1] = above;
+            }
+            above += c;
+        }
+    }
+    __syncthreads();
+    const uint32_t b1 = s_sel[0];
+    const uint32_t cum_above = s_sel[1];
+
+    // ---- pass 2: fine histogram inside the threshold bin.  Few entries match: both halves of a word
+    // are tested at once.  +0 is left out of the atomics (that many on one address would serialise)
+    // and counted per wavefront where its bin is the threshold's ----
+    {
+        const uint32_t bb = (b1 << 5) | (b1 << 21);
+        uint32_t nonzero = 0;   // per half: slots of this thread that do not hold +0 (<= 4 MAXC)
+        static_for<0, MAXC>([&](auto c_c) {
+            constexpr int c = decltype(c_c)::value;
+            if (c < nch) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t w = data[c][j];
+                    const uint32_t x = (w ^ bb) & 0xFFE0FFE0u;   // a half is 0 iff its key lies in the bin
+                    nonzero = pk_add_u16(nonzero, pk_min_u16(w ^ 0x80008000u, kOne));
+                    if (pk_min_u16(x, kOne) != kOne) {
+                        if ((x & 0xFFFFu) == 0 && (w & 0xFFFFu) != kZeroKey) atomicAdd(&s_hist2[w & 31u], 1u);
+                        if ((x >> 16) == 0 && (w >> 16) != kZeroKey) atomicAdd(&s_hist2[(w >> 16) & 31u], 1u);
+                    }
+                }
+            }
+        });
+        if (b1 == kSkipBin) {
+            uint32_t z = 8u * (uint32_t)nch - (nonzero & 0xFFFFu) - (nonzero >> 16);
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) z += __shfl_xor(z, o);
+            if (lane == 0 && z) atomicAdd(&s_hist2[kZeroKey & 31u], z);
+        }
+    }
+    __syncthreads();
+    uint32_t T, r;   // threshold key and the number of entries equal to it to take: every wavefront for itself
+    {
+        // suffix sums of the 32 fine bins, top bin first; the threshold is the first bin whose
+        // running count reaches n
+        const uint32_t c = (lane < 32) ? s_hist2[31 - lane] : 0u;
+        const uint32_t v = wave_incl_scan(c);
+        const uint32_t above = cum_above + v - c;             // entries in finer bins above this one
+        const bool hit = lane < 32 && above < (uint32_t)n && (uint32_t)n <= above + c;
+        // bin 0 takes what is left when no finer bin reaches n (cannot happen for a consistent histogram)
+        const unsigned long long m = __ballot(hit);
+        const int first = m ? __ffsll((long long)m) - 1 : 31;
+        T = max((b1 << 5) | (uint32_t)(31 - first), 1u);
+        r = (uint32_t)n - (uint32_t)__builtin_amdgcn_readlane((int)above, first);
+    }
+    const uint32_t tm1 = (T - 1u) | ((T - 1u) << 16);   // T >= 1
+
+    // ---- pass 3: ordered compaction ----
+    // code of a half: min(sat(key - (T-1)), 2) = 0 below T, 1 equal to T, 2 above T
+    {
+        uint32_t sum = 0, ties = 0;   // per half: sum of the codes (<= 8 MAXC), number of ones (<= 4 MAXC)
+        static_for<0, MAXC>([&](auto c_c) {
+            constexpr int c = decltype(c_c)::value;
+            if (c < nch) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1), kTwo);
+                    sum = pk_add_u16(sum, code);
+                    ties = pk_add_u16(ties, code & kOne);
+                }
+            }
+        });
+        const uint32_t eq = (ties & 0xFFFFu) + (ties >> 16);
+        // above T in the low half, equal to T in the high half (a wavefront holds at most 8192 entries)
+        const uint32_t all = wave_incl_scan((((sum & 0xFFFFu) + (sum >> 16) - eq) >> 1) | (eq << 16));
+        if (lane == 63) {
+            s_gt[wave] = all & 0xFFFFu;
+            s_eq[wave] = all >> 16;
+        }
+    }
+    __syncthreads();
+    uint32_t gt_before, eq_before, unused;
+    scan_waves<THREADS>(s_gt, wave, gt_before, unused);
+    scan_waves<THREADS>(s_eq, wave, eq_before, unused);
+    // The selected positions are staged in LDS, kStage per round (one round unless n > kStage).
+    int* stage = reinterpret_cast<int*>(s_hist);
+    const int base0 = wave * nch * 512 + lane * 8 - lead;      // position of this thread's first entry
+#pragma clang loop unroll(disable)
+    for (uint32_t lo = 0; lo < (uint32_t)n; lo += kStage) {
+        // opaque copy: the codes are recomputed per round instead of being kept in registers across rounds
+        uint32_t tm1_r = tm1;
+        asm volatile("" : "+v"(tm1_r));
+        uint32_t carry = 0;   // entries of the wavefront's part before the chunk: above T / equal to T, packed
+        static_for<0, MAXC>([&](auto c_c) {
+            constexpr int c = decltype(c_c)::value;
+            if (c < nch) {
+                uint32_t above = 0, equal = 0;   // bit e: entry e of the chunk is above / equal to T
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1_r), kTwo);
+                    above |= (((code >> 1) & 1u) | ((code >> 16) & 2u)) << (2 * j);
+                    equal |= ((code & 1u) | ((code >> 15) & 2u)) << (2 * j);
+                }
+                const uint32_t cnt = (uint32_t)__popc(above) | ((uint32_t)__popc(equal) << 16);
+                const uint32_t v = wave_incl_scan(cnt);
+                if (cnt) {
+                    const uint32_t ex = carry + v - cnt;
+                    const uint32_t my_eq = eq_before + (ex >> 16);
+                    // where the next selected entry goes: after the earlier ones above T and the
+                    // earlier ties taken
+                    uint32_t pos = gt_before + (ex & 0xFFFFu) + min(my_eq, r) - lo;
+                    const uint32_t room = r - min(my_eq, r);             // ties that still fit, the lower positions first
+#pragma clang loop unroll(disable)
+                    while ((uint32_t)__popc(equal) > room) equal &= ~(0x80000000u >> __clz(equal));
+#pragma clang loop unroll(disable)
+                    for (uint32_t m = above | equal; m != 0; m &= m - 1, ++pos)
+                        if (pos < (uint32_t)kStage) stage[pos] = base0 + c * 512 + __ffs(m) - 1;
+                }
+                carry += (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+            }
+        });
+        __syncthreads();
+        // this round's slots; the last round also fills the slots from n to k
+        const int hi = (lo + kStage >= (uint32_t)n) ? k : (int)(lo + kStage);
+        // k is a multiple of 4 for every budget the library produces; otherwise element stores
+        const bool wide = (k & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
+                          (reinterpret_cast<uintptr_t>(ro.rows) & 15) == 0;
+        if (wide) {
+#pragma clang loop unroll(disable)
+            for (int i = (int)lo + tid * 4; i < hi; i += THREADS * 4) {
+                int4_t v, w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (i + e < n) ? stage[i + e - lo] : fill;
+                *reinterpret_cast<int4_t*>(dst + i) = v;
+                if (rdst) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = to_cache_row(ro, row, v[e]);
+                    *reinterpret_cast<int4_t*>(rdst + i) = w;
+                }
+            }
+        } else {
+#pragma clang loop unroll(disable)
+            for (int i = (int)lo + tid; i < hi; i += THREADS) {
+                const int v = (i < n) ? stage[i - lo] : fill;
+                dst[i] = v;
+                if (rdst) rdst[i] = to_cache_row(ro, row, v);
+            }
+        }
+        __syncthreads();   // the stage is free for the next round
+    }
+}
+
+// A row with nothing to select from: its first n positions, then the fill value.
+template <int THREADS>
+__device__ __forceinline__ void list_head(int n, int k, int fill, int* __restrict__ out, long long row, const RowsOut& ro) {
+    int* dst = out + row * (long long)k;
+    int* rdst = ro.rows ? ro.rows + row * (long long)k : nullptr;
+#pragma clang loop unroll(disable)
+    for (int i = threadIdx.x; i < k; i += THREADS) {
+        const int pos = (i < n) ? i : fill;
+        dst[i] = pos;
+        if (rdst) rdst[i] = to_cache_row(ro, row, pos);
+    }
+}
+
 // The tensor must start 16-byte aligned (its rows need not) and a row, with the up to 7 slots
-// between the boundary before it and its start, must fit MAXC*8192 slots (MAXC = 16: 131072, 64
-// registers of row data per thread, still one workgroup of 1024 threads per CU).
-template <int MAXC>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MAXC <= 4 ? 8 : 4)))
+// between the boundary before it and its start, must fit THREADS * 8 * MAXC slots.
+template <int THREADS, int MAXC>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 void topk_select_reg_kernel(
     const uint16_t* __restrict__ scores, int* __restrict__ out, long long row_stride,
     int uniform_len, const int* __restrict__ valid_len, const int* __restrict__ n_sel, int period,
     int k, int fill, RowsOut ro) {
-    constexpr int kCopies = 4;
-    constexpr int kStage = kBins1 * kCopies;       // selected indices staged in the histogram's LDS
-    constexpr uint32_t kOne = 0x00010001u, kTwo = 0x00020002u;
-    constexpr uint32_t kZeroKey = 0x8000u;         // order key of +0
-    constexpr uint32_t kSkipBin = kZeroKey >> 5;   // coarse bin of +0: counted by subtraction
-    __shared__ __attribute__((aligned(16))) uint32_t s_hist[kBins1 * kCopies];
-    __shared__ uint32_t s_hist2[32];
-    __shared__ uint32_t s_wave[kWaves];
-    __shared__ uint32_t s_tot[MAXC * kWaves];      // pass 3: totals per (chunk, wavefront), packed
-    __shared__ uint32_t s_pgt[MAXC * kWaves];      // pass 3: exclusive prefixes of the counts above T
-    __shared__ uint32_t s_peq[MAXC * kWaves];      // ... and of the counts equal to T
-    __shared__ uint32_t s_sel[4];  // b1, cum_above, T, r
-    // pass 3: the wavefront scans of the per-thread counts; in registers up to 8 chunks, beyond
-    // that the row itself fills the register file
-    constexpr bool kExwInLds = MAXC > 8;
-    __shared__ uint32_t s_exw[kExwInLds ? MAXC * kThreads : 1];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
+    constexpr uint32_t kOne = 0x00010001u;
     const long long row = blockIdx.x;
-    const int pr = (int)(row % period);
+    const int pr = (int)(blockIdx.x % (uint32_t)period);
     const int len = valid_len ? min(valid_len[pr], uniform_len) : uniform_len;
     int n = n_sel ? n_sel[pr] : k;
     n = max(0, min(n, k));
+    if (len <= n || n == 0) {
+        list_head<THREADS>(n, k, fill, out, row, ro);
+        return;
+    }
     // A row that does not start on a 16-byte boundary (a row stride that is no multiple of 8) is
     // read from the boundary before it: `lead` slots in front of the row count as absent, like
     // the slots past its end, and every position below is taken in these shifted coordinates
@@ -308,301 +542,57 @@ void topk_select_reg_kernel(
     const uint16_t* row_src = scores + row * row_stride;
     const int lead = (int)((reinterpret_cast<uintptr_t>(row_src) & 15) >> 1);
     const uint16_t* src = row_src - lead;
-    const int row_len = len;            // entries of the row itself
-    int* dst = out + row * (long long)k;
-    int* rdst = ro.rows ? ro.rows + row * (long long)k : nullptr;
-    auto put = [&](int slot, int pos) {
-        dst[slot] = pos;
-        if (rdst) rdst[slot] = to_cache_row(ro, row, pos);
-    };
+    const int slots = len + lead;   // the row in shifted coordinates: [lead, slots)
+    const int nch = (slots + THREADS * 8 - 1) / (THREADS * 8);   // <= MAXC (host)
+    const int first = (threadIdx.x >> 6) * nch * 512 + (threadIdx.x & 63) * 8;   // slot of this thread's chunk 0
 
-    if (row_len <= n || n == 0) {
-        for (int i = tid; i < k; i += kThreads) put(i, (i < n) ? i : fill);
-        return;
-    }
-    const int slots = row_len + lead;   // the row in shifted coordinates: [lead, slots)
-    const int nchunks = (slots + kChunk - 1) / kChunk;   // <= MAXC (host)
-
-    // ---- the row: chunk c, slots [c*8192 + 8*tid, +8) as packed order keys ----
-    uint4_t data[MAXC];
-    // slots of chunk c that lie before the row's end (recomputed where needed: an array of them
-    // would cost MAXC registers), and the absent slots in front (only the first thread has any)
-    auto nv_of = [&](int c) { return max(0, min(8, slots - (c * kChunk + tid * 8))); };
-    auto lead_of = [&](int c) { return (c == 0 && tid == 0) ? lead : 0; };
     // Every thread loads 16 bytes per chunk without a branch around the load, so that the loads
-    // are in flight together: where the chunk's share lies past the end of the row the address
-    // is pulled back inside it and the data replaced below.
+    // are in flight together: where the chunk's share is not wholly inside the row the address is
+    // pulled back inside it and the data replaced below.
+    uint4_t data[MAXC];
     const int last_full = max(slots - 8, 0) & ~7;
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
+    static_for<0, MAXC>([&](auto c_c) {
+        constexpr int c = decltype(c_c)::value;
         data[c] = uint4_t{0, 0, 0, 0};
-        if (slots >= 8)   // uniform
-            data[c] = *reinterpret_cast<const uint4_t*>(src + min(c * kChunk + tid * 8, last_full));
-    }
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-        const int base = c * kChunk + tid * 8;
-        const int nvc = nv_of(c);
-        const int ldc = lead_of(c);
-        uint4_t raw = data[c];
-        if (nvc == 8 && ldc == 0) {
-            // order_key on both halves at once: negative values flip every bit, others the sign
-            // bit; then at least 1
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                raw[j] = pk_max_u16(raw[j] ^ (pk_sign_mask_i16(raw[j]) | 0x80008000u), kOne);
-        } else {   // the thread at the end of the row, and every thread beyond it
-            uint32_t w[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t lo = (2 * e < nvc && 2 * e >= ldc) ? max(order_key(src[base + 2 * e]), 1u) : 0u;
-                const uint32_t hi = (2 * e + 1 < nvc && 2 * e + 1 >= ldc) ? max(order_key(src[base + 2 * e + 1]), 1u) : 0u;
-                w[e] = lo | (hi << 16);
-            }
-            raw = uint4_t{w[0], w[1], w[2], w[3]};
+        if (c < nch && slots >= 8)   // uniform
+            data[c] = *reinterpret_cast<const uint4_t*>(src + min(first + c * 512, last_full));
+    });
+    // the pieces at the row's two ends, one thread each, entry by entry (0: no entry)
+    const int tail = slots & ~7;    // first slot of the partial piece at the end
+    auto piece = [&](int s0) {
+        unsigned long long w[2] = {0, 0};
+#pragma clang loop unroll(disable)
+        for (int e = 0; e < 8; ++e) {
+            const int s = s0 + e;
+            const unsigned long long key = (s >= lead && s < slots) ? max(order_key(src[s]), 1u) : 0u;
+            if (e < 4) w[0] |= key << (16 * e); else w[1] |= key << (16 * (e - 4));
         }
-        data[c] = raw;
-    }
-
-    // ---- pass 1: coarse histogram ----
-    {
-        const uint4_t z = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < kBins1 * kCopies / (4 * kThreads); ++i)
-            *reinterpret_cast<uint4_t*>(&s_hist[(i * kThreads + tid) * 4]) = z;
-    }
-    if (tid < 32) s_hist2[tid] = 0;
-    __syncthreads();
-    const uint32_t copy = tid & (kCopies - 1);
-    auto count1 = [&](uint32_t key) {
-        const uint32_t bin = key >> 5;
-        if (bin != kSkipBin) atomicAdd(&s_hist[bin * kCopies + copy], 1u);
+        return uint4_t{(uint32_t)w[0], (uint32_t)(w[0] >> 32), (uint32_t)w[1], (uint32_t)(w[1] >> 32)};
     };
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-        if (c < nchunks) {
-            const int nvc = nv_of(c);
-            const int ldc = lead_of(c);
-            if (nvc == 8 && ldc == 0) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    count1(data[c][j] & 0xFFFFu);
-                    count1(data[c][j] >> 16);
-                }
-            } else if (nvc > 0) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (e < nvc && e >= ldc) count1((e & 1) ? (data[c][e >> 1] >> 16) : (data[c][e >> 1] & 0xFFFFu));
-            }
-        }
-    }
-    __syncthreads();
-    {
-        // thread t owns bins 2047-2t and 2046-2t (descending order); the uncounted bin is the
-        // lower bin of its owner
-        const int rb0 = kBins1 - 1 - 2 * tid;
-        constexpr int kSkipOwner = (kBins1 - 2 - (int)kSkipBin) / 2;
-        static_assert(kBins1 - 2 - 2 * kSkipOwner == (int)kSkipBin, "the uncounted bin must be a lower bin");
-        const uint4_t h0 = *reinterpret_cast<const uint4_t*>(&s_hist[rb0 * kCopies]);
-        const uint4_t h1 = *reinterpret_cast<const uint4_t*>(&s_hist[(rb0 - 1) * kCopies]);
-        const uint32_t c0 = h0[0] + h0[1] + h0[2] + h0[3];
-        uint32_t c1 = h1[0] + h1[1] + h1[2] + h1[3];
-        uint32_t total;
-        uint32_t above0 = block_excl_scan(c0 + c1, s_wave, &total);
-        const uint32_t skipped = (uint32_t)row_len - total;
-        if (tid == kSkipOwner) c1 += skipped;
-        if (tid > kSkipOwner) above0 += skipped;
-        const uint32_t above1 = above0 + c0;
-        const uint32_t un = (uint32_t)n;
-        if (above0 < un && un <= above0 + c0) {
-            s_sel[0] = rb0;
-            s_sel[1] = above0;
-        } else if (above1 < un && un <= above1 + c1) {
-            s_sel[0] = rb0 - 1;
-            s_sel[1] = above1;
-        }
-    }
-    __syncthreads();
-    const uint32_t b1 = s_sel[0];
-    const uint32_t cum_above = s_sel[1];
-
-    // ---- pass 2: fine histogram inside the threshold bin ----
-    if (b1 != kSkipBin) {
-        // few entries match: test both halves of a word at once, then a branch
-        const uint32_t bb = (b1 << 5) | (b1 << 21);
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            if (c < nchunks) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t w = data[c][j];
-                    const uint32_t x = (w ^ bb) & 0xFFE0FFE0u;   // a half is 0 iff its key lies in the bin
-                    if (pk_min_u16(x, kOne) != kOne) {
-                        if ((x & 0xFFFFu) == 0) atomicAdd(&s_hist2[w & 31u], 1u);
-                        if ((x >> 16) == 0) atomicAdd(&s_hist2[(w >> 16) & 31u], 1u);
-                    }
-                }
-            }
-        }
-    } else {
-        // The threshold lies among +0 and the smallest subnormals: that many atomics on one
-        // address would serialise, so each wavefront counts its zeros with a ballot.
-        uint32_t zeros = 0;                        // wavefront-uniform
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            if (c < nchunks) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const uint32_t w = data[c][e >> 1];
-                    const uint32_t key = (e & 1) ? (w >> 16) : (w & 0xFFFFu);
-                    const bool zero = key == kZeroKey;
-                    zeros += (uint32_t)__popcll(__ballot(zero));
-                    if ((key >> 5) == b1 && !zero) atomicAdd(&s_hist2[key & 31u], 1u);
-                }
-            }
-        }
-        if (lane == 0 && zeros) atomicAdd(&s_hist2[kZeroKey & 31u], zeros);
-    }
-    __syncthreads();
-    if (tid < 64) {
-        // suffix sums of the 32 fine bins, top bin first; the threshold is the first bin whose
-        // running count reaches n
-        const uint32_t c = (lane < 32) ? s_hist2[31 - lane] : 0u;
-        const uint32_t v = wave_incl_scan(c);
-        const uint32_t above = cum_above + v - c;             // entries in finer bins above this one
-        const bool hit = lane < 32 && above < (uint32_t)n && (uint32_t)n <= above + c;
-        // bin 0 takes what is left when no finer bin reaches n (cannot happen for a consistent
-        // histogram; kept so that s_sel is always written)
-        const unsigned long long m = __ballot(hit);
-        const int first = m ? __ffsll((long long)m) - 1 : 31;
-        if (lane == first) {
-            s_sel[2] = max((b1 << 5) | (uint32_t)(31 - first), 1u);
-            s_sel[3] = (uint32_t)n - above;  // entries equal to T to take
-        }
-    }
-    __syncthreads();
-    const uint32_t T = s_sel[2];
-    const uint32_t r = s_sel[3];
-    const uint32_t tm1 = (T - 1u) | ((T - 1u) << 16);   // T >= 1
-
-    // ---- pass 3: ordered compaction (index order = chunk, then thread, then element) ----
-    // code of a half: min(sat(key - (T-1)), 2) = 0 below T, 1 equal to T, 2 above T
-    // counts of one (chunk, thread): entries above T in the low half, equal to T in the high half
-    uint32_t exw[kExwInLds ? 1 : MAXC];   // exclusive scan of the counts over the wavefront
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-        uint32_t cnt = 0;
-        if (c < nchunks) {
-            uint32_t sum = 0, ties = 0;   // per half: sum of the codes (<= 8), number of ones (<= 4)
+    const bool at_front = first == 0 && (lead > 0 || tail == 0);
+    const int d_tail = tail - first;   // chunk d_tail / 512 of this thread is the partial one, if it is a whole chunk away
+    const bool at_tail = tail < slots && d_tail >= 0 && (d_tail & 511) == 0 && d_tail < nch * 512 && !(at_front && tail == 0);
+    uint4_t end_w[2] = {};
+    if (at_front) end_w[0] = piece(0);
+    if (at_tail) end_w[1] = piece(tail);
+    static_for<0, MAXC>([&](auto c_c) {
+        constexpr int c = decltype(c_c)::value;
+        if (c < nch) {
+            const int s0 = first + c * 512;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1), kTwo);
-                sum = pk_add_u16(sum, code);
-                ties = pk_add_u16(ties, code & kOne);
-            }
-            const uint32_t s2 = (sum & 0xFFFFu) + (sum >> 16);     // ties + 2 * above
-            const uint32_t eq = (ties & 0xFFFFu) + (ties >> 16);
-            cnt = ((s2 - eq) >> 1) | (eq << 16);
-        }
-        const uint32_t v = wave_incl_scan(cnt);
-        if (kExwInLds) s_exw[c * kThreads + tid] = v - cnt;
-        else exw[c] = v - cnt;
-        if (lane == 63) s_tot[c * kWaves + wave] = v;
-    }
-    __syncthreads();
-    if (wave == 0) {
-        // exclusive prefixes over the MAXC*16 (chunk, wavefront) totals, chunk-major, 64 per step.
-        // A wavefront's totals fit the packed halves (at most 512 entries each); the prefixes over
-        // a row of more than 65536 entries do not, so they are kept apart.
-        uint32_t carry_gt = 0, carry_eq = 0;
-#pragma unroll
-        for (int i0 = 0; i0 < MAXC * kWaves; i0 += 64) {
-            const uint32_t x = s_tot[i0 + lane];
-            const uint32_t xg = x & 0xFFFFu, xe = x >> 16;
-            const uint32_t vg = wave_incl_scan(xg), ve = wave_incl_scan(xe);
-            s_pgt[i0 + lane] = carry_gt + vg - xg;
-            s_peq[i0 + lane] = carry_eq + ve - xe;
-            carry_gt += (uint32_t)__builtin_amdgcn_readlane((int)vg, 63);
-            carry_eq += (uint32_t)__builtin_amdgcn_readlane((int)ve, 63);
-        }
-    }
-    __syncthreads();
-    // The selected indices are staged in LDS in their final order, kStage positions per round (one
-    // round unless n > kStage), and leave as full-width stores.
-    int* stage = reinterpret_cast<int*>(s_hist);
-    for (uint32_t lo = 0; lo < (uint32_t)n; lo += kStage) {
-        auto emit = [&](uint32_t pos, int idx) {
-            if (pos - lo < (uint32_t)kStage) stage[pos - lo] = idx;
-        };
-        // opaque copy: the codes are recomputed per round instead of being kept in registers
-        // across rounds (a second workgroup per CU needs the kernel within 64 registers)
-        uint32_t tm1_r = tm1;
-        asm volatile("" : "+v"(tm1_r));
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            // with 16 chunks the row fills the registers: keep the chunks' LDS reads from
-            // being moved ahead of the earlier chunks' work
-            if (kExwInLds) __builtin_amdgcn_sched_barrier(0);
-            if (c < nchunks) {
-                const uint32_t ex = kExwInLds ? s_exw[c * kThreads + tid] : exw[c];
-                uint32_t my_eq = s_peq[c * kWaves + wave] + (ex >> 16);
-                // where the next selected entry goes: after the earlier ones above T and the
-                // earlier ties taken
-                uint32_t pos = s_pgt[c * kWaves + wave] + (ex & 0xFFFFu) + min(my_eq, r);
-                const int base = c * kChunk + tid * 8 - lead;   // back to positions of the row
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1_r), kTwo);
-                    if ((code & kOne) == 0) {           // no tie in this word: the common case
-                        if (code & 0xFFFFu) emit(pos++, base + 2 * j);
-                        if (code >> 16) emit(pos++, base + 2 * j + 1);
-                    } else {
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const uint32_t ch = h ? (code >> 16) : (code & 0xFFFFu);
-                            if (ch == 2u) {
-                                emit(pos++, base + 2 * j + h);
-                            } else if (ch == 1u) {
-                                if (my_eq < r) emit(pos++, base + 2 * j + h);
-                                ++my_eq;
-                            }
-                        }
-                    }
-                }
+                // order_key on both halves at once: negative values flip every bit, others the sign
+                // bit; then at least 1
+                const uint32_t raw = data[c][j];
+                uint32_t key = pk_max_u16(raw ^ (pk_sign_mask_i16(raw) | 0x80008000u), kOne);
+                key = s0 < tail ? key : (at_tail && s0 == tail) ? end_w[1][j] : 0u;
+                if (c == 0) key = at_front ? end_w[0][j] : key;
+                data[c][j] = key;
             }
         }
-        __syncthreads();
-        // this round's slots; the last round also fills the slots from n to k
-        const int hi = (lo + kStage >= (uint32_t)n) ? k : (int)(lo + kStage);
-        // k is a multiple of 4 for every budget the library produces; otherwise element stores
-        if ((k & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-            for (int i = (int)lo + tid * 4; i < hi; i += kThreads * 4) {
-                int4 v;
-                v.x = (i + 0 < n) ? stage[i + 0 - lo] : fill;
-                v.y = (i + 1 < n) ? stage[i + 1 - lo] : fill;
-                v.z = (i + 2 < n) ? stage[i + 2 - lo] : fill;
-                v.w = (i + 3 < n) ? stage[i + 3 - lo] : fill;
-                *reinterpret_cast<int4*>(dst + i) = v;
-                if (rdst) {   // k % 4 == 0 here; the rows tensor has the layout of the index tensor
-                    int4 w;
-                    w.x = to_cache_row(ro, row, v.x);
-                    w.y = to_cache_row(ro, row, v.y);
-                    w.z = to_cache_row(ro, row, v.z);
-                    w.w = to_cache_row(ro, row, v.w);
-                    if ((reinterpret_cast<uintptr_t>(ro.rows) & 15) == 0) {
-                        *reinterpret_cast<int4*>(rdst + i) = w;
-                    } else {
-                        rdst[i] = w.x; rdst[i + 1] = w.y; rdst[i + 2] = w.z; rdst[i + 3] = w.w;
-                    }
-                }
-            }
-        } else {
-            for (int i = (int)lo + tid; i < hi; i += kThreads) put(i, (i < n) ? stage[i - lo] : fill);
-        }
-        __syncthreads();   // the stage is free for the next round
-    }
+    });
+    select_row<THREADS, MAXC, false>(data, nch, lead, len, n, k, fill, out, row, ro);
 }
-
 
 // --------------------------------------------------------------------------
 // Long rows: the same radix select spread over several workgroups per row.
@@ -1199,15 +1189,32 @@ hipError_t launch_topk(const half_t* scores, int* out_idx, int rows, long long r
     // anything else streams the row three times
     const bool aligned_rows = (reinterpret_cast<uintptr_t>(scores) & 15) == 0;
     const int slots = uniform_len + (row_stride % 8 != 0 ? 7 : 0);
-    if (aligned_rows && slots <= 4 * kChunk)
-        hipLaunchKernelGGL(topk_select_reg_kernel<4>, dim3(rows), dim3(kThreads), 0, stream, src, out_idx,
-                           row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);
-    else if (aligned_rows && slots <= 8 * kChunk)
-        hipLaunchKernelGGL(topk_select_reg_kernel<8>, dim3(rows), dim3(kThreads), 0, stream, src, out_idx,
-                           row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);
-    else if (aligned_rows && slots <= 16 * kChunk)
-        hipLaunchKernelGGL(topk_select_reg_kernel<16>, dim3(rows), dim3(kThreads), 0, stream, src, out_idx,
-                           row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);
+    auto go = [&](auto threads, auto chunks) {
+        constexpr int kT = decltype(threads)::value;
+        hipLaunchKernelGGL((topk_select_reg_kernel<kT, decltype(chunks)::value>), dim3(rows), dim3(kT), 0, stream, src,
+                           out_idx, row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);
+    };
+    // The fewest chunks per wavefront in workgroups of up to 512 threads; long rows take 1024 threads
+    // while all their workgroups are resident at once (two per compute unit at four chunks, one at
+    // eight), where a row's latency is the time (64 rows: 32768 entries 13.7 -> 11.5 us, 65536
+    // 24 -> 19): with more rows the scans over more wavefronts cost throughput (2048 rows: 61 -> 65 us
+    // and 141 -> 172).
+    const bool few32k = rows <= 2 * kComputeUnits, few64k = rows <= kComputeUnits;
+    std::integral_constant<int, 256> t256{};
+    std::integral_constant<int, 512> t512{};
+    std::integral_constant<int, 1024> t1024{};
+    std::integral_constant<int, 1> c1{};
+    std::integral_constant<int, 2> c2{};
+    std::integral_constant<int, 4> c4{};
+    std::integral_constant<int, 8> c8{};
+    std::integral_constant<int, 16> c16{};
+    if (aligned_rows && slots <= 2048) go(t256, c1);
+    else if (aligned_rows && slots <= 4096) go(t512, c1);
+    else if (aligned_rows && slots <= 8192) go(t512, c2);
+    else if (aligned_rows && slots <= 16384) go(t512, c4);
+    else if (aligned_rows && slots <= 32768) few32k ? go(t1024, c4) : go(t512, c8);
+    else if (aligned_rows && slots <= 65536) few64k ? go(t1024, c8) : go(t512, c16);
+    else if (aligned_rows && slots <= 131072) go(t1024, c16);
     else
         hipLaunchKernelGGL(topk_select_kernel, dim3(rows), dim3(kThreads), 0, stream, src, out_idx,
                            row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);

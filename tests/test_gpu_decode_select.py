@@ -1,4 +1,6 @@
 """The selection's and the decode split's dispatch lines: sizes at the edges of each variant."""
+import math
+
 import pytest
 import torch
 
@@ -6,6 +8,32 @@ from oracle import kascade_oracle as orc
 from tests.helpers import assert_close
 
 pytestmark = pytest.mark.gpu
+
+
+def _check_rows(scores, idx, n_of, valid_of, what):
+    for r in range(scores.shape[0]):
+        n, valid = n_of(r), valid_of(r)
+        if valid <= n:      # every token, then the positions behind them
+            assert torch.equal(idx[r, :n], torch.arange(n, dtype=torch.int32)), f"{what} row {r}"
+            continue
+        ok, _, msg = orc.topk_agreement(scores[r], idx[r], n, valid, ulps=0.0)
+        assert ok, f"{what} row {r}: {msg}"
+        assert bool((idx[r, 1:n] > idx[r, :n - 1]).all()), f"{what} row {r}: not ascending"
+
+
+@pytest.mark.parametrize("L", [1, 8, 511, 513, 2048, 2049, 4096, 4097, 8193, 16384, 16385, 32768, 32769, 65536])
+@pytest.mark.parametrize("rows", [3, 257])
+def test_register_selection_edges(cuda, L, rows):
+    """Longest row of every workgroup size and chunk count, one more entry, and both sides of the
+    row count at which long rows change the workgroup size.  The selection is exact: no tolerance."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(L)
+    base = (torch.rand(3, L, generator=gen) ** 4 * 512).round().half() / 512      # many ties
+    k = max(1, L // 10)
+    sc = base.to(cuda).repeat(math.ceil(rows / 3), 1)[:rows].contiguous()
+    idx = kernels.topk_indices(sc, k).cpu()
+    assert all(torch.equal(idx[r], idx[r % 3]) for r in range(rows))
+    _check_rows(base, idx[:3], lambda r: k, lambda r: L, f"L={L}")
 
 
 @pytest.mark.parametrize("seqlens,ns", [([1024], 1), ([1025], 1), ([2048, 1], 1), ([2049, 64], 1), ([255, 257, 4096], 2),
