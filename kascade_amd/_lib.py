@@ -45,6 +45,8 @@ SIGNATURES = {
                                              _P, _P, _P, _P]),
     "kascade_decode_recompute_paged_call": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I,
                                                  _I, _I, _P, _I, _I, _SP, _P, _P, _P, _P]),
+    "kascade_decode_anchor_topk_call": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
+                                             _I, _I, _I, _F, _P, _P, _P, _P, _I, _I, _SP, _P, _P, _P, _P]),
     "kascade_topk_workspace_bytes": (_L, [_I, _L]),
     "kascade_topk_call": (_I, [_P, _P, _I, _L, _I, _P, _P, _I, _I, _I, _P, _P]),
     "kascade_topk_sorted_workspace_bytes": (_L, [_I, _L, _I]),
@@ -128,3 +130,20 @@ def init() -> C.CDLL:
         check(lib.kascade_init())
         _initialised = True
     return lib
+
+
+_native = None
+
+
+def native():
+    """The host extension module ``_native`` (per-layer calls in one step), after ``init()``."""
+    global _native
+    if _native is None:
+        init()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise KascadeError(f"{LIB_PATH.with_name('_native.so')} is missing or does not load ({e}): build it with "
+                               "`python -m kascade_amd.build` (there is no fallback path)") from e
+        _native = module
+    return _native

@@ -170,7 +170,7 @@ int set_append(DecodeParams& p, const kascade_half* k_new, const kascade_half* v
 
 extern "C" {
 
-int kascade_abi_version(void) { return 10; }
+int kascade_abi_version(void) { return 11; }
 
 const char* kascade_get_last_error(void) { return g_err; }
 
@@ -416,6 +416,37 @@ int kascade_decode_dense_paged_shaped_call(const kascade_shape* shape, const kas
 
 }  // extern "C"
 namespace {
+// The selection that follows an anchor pass in the same call.
+struct AnchorSelect {
+    int32_t* out_idx;
+    const TopkRows* rows;      // or null
+    int row_len, k, fill;
+    float topk_percent;
+    const int32_t *valid_len, *n_sel;   // long rows only
+    void* workspace;
+};
+
+static_assert(KASCADE_POOL_SELECT_ROW == kPoolSelectRow, "the header's limit is the kernel's");
+
+// rows that start 16-byte aligned and fit one workgroup's registers
+bool one_workgroup_rows(int len) { return len <= topk_max_register_row(); }
+
+// Selection over a tensor of scores, as kascade_topk_rows_call describes it (arguments checked).
+int select_rows(const half_t* scores, int32_t* out_idx, int rows, int64_t row_stride, int uniform_len,
+                const int32_t* valid_len, const int32_t* n_sel, int period, int k, int fill_value,
+                void* workspace, const TopkRows& tr, hipStream_t s) {
+    // rows of up to 131072 entries fit one workgroup's registers: one launch; longer (or unaligned
+    // long) rows go to several workgroups per row, four launches
+    const bool one_workgroup = one_workgroup_rows(uniform_len + (row_stride % 8 != 0 ? 7 : 0)) &&
+                               (reinterpret_cast<uintptr_t>(scores) & 15) == 0;
+    if (!one_workgroup && workspace && topk_split_workspace_bytes(rows, uniform_len) > 0)
+        return check_hip(launch_topk_split(scores, out_idx, rows, row_stride, uniform_len,
+                                           uniform_len, valid_len, n_sel, period, k, fill_value,
+                                           workspace, &tr, s), "topk (split)");
+    return check_hip(launch_topk(scores, out_idx, rows, row_stride, uniform_len, valid_len, n_sel,
+                                 period, k, fill_value, &tr, s), "topk");
+}
+
 int decode_recompute_paged_impl(const Shape& sh, const kascade_half* Q, const kascade_half* K,
                                         const kascade_half* V, const int32_t* cache_seqlens,
                                         float* glse, float* Output_partial, float* row_sums,
@@ -426,8 +457,8 @@ int decode_recompute_paged_impl(const Shape& sh, const kascade_half* Q, const ka
                                         int max_pages, int page_size,
                                         const kascade_strides* kv_strides,
                                         const kascade_half* k_new, const kascade_half* v_new,
-                                        int32_t* sync_counters, void* stream) {
-    REQUIRE(Q && K && glse && row_sums && scores && aggregated_scores,
+                                        int32_t* sync_counters, const AnchorSelect* sel, void* stream) {
+    REQUIRE(Q && K && glse && row_sums && scores && (aggregated_scores || (sel && sel->row_len <= KASCADE_POOL_SELECT_ROW)),
             "decode_recompute: null pointer argument");
     REQUIRE(!with_output || (V && Output && Output_partial),
             "decode_recompute: with_output needs V, Output and Output_partial");
@@ -457,22 +488,35 @@ int decode_recompute_paged_impl(const Shape& sh, const kascade_half* Q, const ka
     p.rows_per_split = rows_per_split(max_rows, num_split);
     p.counters = sync_counters; p.out = H(Output); p.row_sums = row_sums;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // Without an output the only thing left to merge is the log-sums, which the pooling launch does
+    // for itself: no combine launch, no counters.
+    if (!with_output) p.counters = nullptr;
     if (check_hip(launch_decode_split(p, false, with_output != 0, true, s), "decode_recompute split"))
         return -1;
     // the kernels cut every sequence length down to this (decode_split_kernel's safe_len)
     long long len_cap = block_table ? (long long)max_pages * page_size : (long long)kv_stride_tokens;
     if (len_cap > scores_stride) len_cap = scores_stride;
-    // Without an output the only thing left to merge is the log-sums, which the aggregate
-    // launch does for itself: no combine launch.
-    const bool merge_in_aggregate = !sync_counters && !with_output;
     if (!sync_counters && with_output &&
         check_hip(launch_decode_combine(glse, Output_partial, E(Output), row_sums, batch, sh.H(), num_split, true, sh.D, sh.elem, s), "decode_recompute combine"))
         return -1;
-    return check_hip(launch_decode_aggregate(scores, merge_in_aggregate ? nullptr : row_sums,
-                                             merge_in_aggregate ? glse : nullptr, num_split, row_sums,
-                                             cache_seqlens, H(aggregated_scores), batch, sh.G, sh.gs, scores_stride,
-                                             kv_stride_tokens, (int)len_cap, s),
-                     "decode_recompute aggregate");
+    const float* parts = with_output ? nullptr : glse;   // log-sums still to be merged
+    const TopkRows no_rows{};
+    if (sel && sel->row_len <= KASCADE_POOL_SELECT_ROW) {
+        DecodePoolParams pp{};
+        pp.scores = scores; pp.glse = parts; pp.row_sums = row_sums; pp.seqlens = cache_seqlens;
+        pp.num_split = num_split; pp.groups = sh.G; pp.group_size = sh.gs; pp.scores_stride = scores_stride;
+        pp.uniform_len = sel->row_len; pp.len_cap = (int)len_cap; pp.topk_percent = sel->topk_percent;
+        return check_hip(launch_decode_pool_select(pp, batch * sh.G, sel->k, sel->fill, sel->out_idx,
+                                                   sel->rows ? sel->rows : &no_rows, s), "decode_anchor pool+topk");
+    }
+    if (check_hip(launch_decode_aggregate(scores, with_output ? row_sums : nullptr, parts, num_split, row_sums,
+                                          cache_seqlens, H(aggregated_scores), batch, sh.G, sh.gs, scores_stride,
+                                          kv_stride_tokens, (int)len_cap, s),
+                  "decode_recompute aggregate"))
+        return -1;
+    if (!sel) return 0;
+    return select_rows(H(aggregated_scores), sel->out_idx, batch * sh.G, scores_stride, sel->row_len, sel->valid_len,
+                       sel->n_sel, batch * sh.G, sel->k, sel->fill, sel->workspace, sel->rows ? *sel->rows : no_rows, s);
 }
 }  // namespace
 extern "C" {
@@ -488,7 +532,7 @@ int kascade_decode_recompute_paged_call(const kascade_half* Q, const kascade_hal
                                         const kascade_strides* kv_strides,
                                         const kascade_half* k_new, const kascade_half* v_new,
                                         int32_t* sync_counters, void* stream) {
-    return decode_recompute_paged_impl(kRefShape, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, stream);
+    return decode_recompute_paged_impl(kRefShape, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, nullptr, stream);
 }
 
 int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K,
@@ -504,7 +548,44 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
                                         int32_t* sync_counters, void* stream) {
     Shape sh;
     if (get_shape(shape, &sh)) return -1;
-    return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, stream);
+    return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, nullptr, stream);
+}
+
+int kascade_decode_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K,
+                                    const kascade_half* V, const int32_t* cache_seqlens, float* glse,
+                                    float* Output_partial, float* row_sums, float* scores, kascade_half* Output,
+                                    kascade_half* aggregated_scores, int32_t* out_idx, int32_t* out_rows, int batch,
+                                    int kv_stride_tokens, int scores_stride, int num_split, int with_output,
+                                    int row_len, int k, int fill_value, float topk_percent, const int32_t* valid_len,
+                                    const int32_t* n_sel, void* workspace, const int32_t* block_table, int max_pages,
+                                    int page_size, const kascade_strides* kv_strides, const kascade_half* k_new,
+                                    const kascade_half* v_new, int32_t* sync_counters, void* stream) {
+    Shape sh = kRefShape;
+    if (shape && get_shape(shape, &sh)) return -1;
+    REQUIRE(out_idx, "decode_anchor_topk: null pointer argument");
+    REQUIRE(k > 0 && row_len > 0 && row_len <= scores_stride, "decode_anchor_topk: k > 0 and 0 < row_len <= scores_stride required");
+    REQUIRE(!(topk_percent > 0.f) || cache_seqlens, "decode_anchor_topk: topk_percent needs cache_seqlens");
+    REQUIRE((long long)batch * sh.G < (1LL << 31), "decode_anchor_topk: too many rows");
+    const bool one = row_len <= KASCADE_POOL_SELECT_ROW;
+    REQUIRE(one || aggregated_scores, "decode_anchor_topk: rows of more than %d tokens need aggregated_scores", KASCADE_POOL_SELECT_ROW);
+    REQUIRE(one || !(topk_percent > 0.f) || (valid_len && n_sel),
+            "decode_anchor_topk: rows of more than %d tokens need valid_len and n_sel", KASCADE_POOL_SELECT_ROW);
+    TopkRows tr{};
+    if (out_rows) {
+        REQUIRE(block_table, "decode_anchor_topk: out_rows needs a block table");
+        int shift;
+        if (check_paging(block_table, max_pages, page_size, &shift)) return -1;
+        REQUIRE((long long)max_pages * page_size >= row_len, "decode_anchor_topk: block table shorter than the rows it is to translate");
+        tr.out_rows = out_rows; tr.block_table = block_table; tr.max_pages = max_pages;
+        tr.page_shift = shift; tr.rows_per_seq = sh.G;
+    }
+    AnchorSelect sel{};
+    sel.out_idx = out_idx; sel.rows = &tr; sel.row_len = row_len; sel.k = k; sel.fill = fill_value;
+    sel.topk_percent = topk_percent; sel.valid_len = valid_len; sel.n_sel = n_sel; sel.workspace = workspace;
+    return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output,
+                                       aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output,
+                                       block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, &sel,
+                                       stream);
 }
 
 int64_t kascade_topk_workspace_bytes(int rows, int64_t row_len) {
@@ -540,16 +621,8 @@ int kascade_topk_rows_call(const kascade_half* scores, int32_t* out_idx, int row
     REQUIRE(!(valid_len || n_sel) || period > 0, "topk: period must be > 0 with per-row arrays");
     if (period <= 0) period = 1;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // rows of up to 131072 entries that start 16-byte aligned fit one workgroup's registers: one
-    // launch; longer (or unaligned long) rows go to several workgroups per row, four launches
-    const bool one_workgroup = uniform_len + (row_stride % 8 != 0 ? 7 : 0) <= topk_max_register_row() &&
-                               (reinterpret_cast<uintptr_t>(scores) & 15) == 0;
-    if (!one_workgroup && workspace && topk_split_workspace_bytes(rows, uniform_len) > 0)
-        return check_hip(launch_topk_split(H(scores), out_idx, rows, row_stride, uniform_len,
-                                           uniform_len, valid_len, n_sel, period, k, fill_value,
-                                           workspace, &tr, s), "topk (split)");
-    return check_hip(launch_topk(H(scores), out_idx, rows, row_stride, uniform_len, valid_len, n_sel,
-                                 period, k, fill_value, &tr, s), "topk");
+    return select_rows(H(scores), out_idx, rows, row_stride, uniform_len, valid_len, n_sel, period, k, fill_value, workspace,
+                       tr, s);
 }
 
 namespace {

@@ -17,6 +17,23 @@ hipError_t launch_topk(const half_t* scores, int* out_idx, int rows, long long r
                        int uniform_len, const int* valid_len, const int* n_sel, int period, int k,
                        int fill, const TopkRows* tr, hipStream_t stream);
 
+// Pooling and selection of decode anchors in one launch, one workgroup per (sequence, KV head) row
+// of up to kPoolSelectRow tokens (longer rows: pooling spread over the chip, then a selection, is faster --
+// one sequence of 32768 tokens 34.1 -> 32.0 us with its scores pass, of 65536 57 -> 63.5).
+constexpr int kPoolSelectRow = 32768;
+struct DecodePoolParams {
+    const float* scores;      // [rows, group_size, scores_stride]: score codes and references (decode.h)
+    const float* glse;        // [rows, group_size, num_split] log-sums of the splits, or null: row_sums holds them merged
+    float* row_sums;          // [rows, group_size]: written when glse is given
+    const int* seqlens;       // [sequences] or null (uniform_len tokens each)
+    int num_split, groups, group_size, scores_stride;
+    int uniform_len;          // longest row
+    int len_cap;              // bound the scores pass put on every length
+    float topk_percent;       // > 0: a row selects 128*ceil(floor(percent*len/100)/128) of its len tokens; else k of uniform_len
+};
+hipError_t launch_decode_pool_select(const DecodePoolParams& p, int rows, int k, int fill, int* out_idx,
+                                     const TopkRows* tr, hipStream_t stream);
+
 // Multi-workgroup variant for long rows.  Returns 0 bytes when the single-workgroup kernel
 // is the right choice (short rows, or too many rows for the 8 KB/row workspace).
 long long topk_split_workspace_bytes(int rows, long long row_len);

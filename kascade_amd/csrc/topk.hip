@@ -594,6 +594,136 @@ void topk_select_reg_kernel(
     select_row<THREADS, MAXC, false>(data, nch, lead, len, n, k, fill, out, row, ro);
 }
 
+// Decode anchors: pooling and selection of a (sequence, KV head) row in one workgroup.  What the
+// scores pass left -- per query head a row of 16-bit score codes with one fp32 reference per 64 tokens
+// (decode.h), and the log-sums of its splits -- becomes the row of pooled probabilities
+// sum_h exp2(score - lse_h), rounded to fp16 as decode_aggregate_kernel rounds it, and goes straight
+// into the selection's registers: no pooled row in memory, one launch instead of two (merge of the
+// log-sums included).  Bound by the latency of one workgroup: its exponentials (8 per head and lane and
+// chunk) and the selection's scans; the launch pays for the few compute units it uses up to about
+// 32768 tokens.  With the scores pass, K only, one sequence of 32 / 8 heads: 2000 tokens 14.9 -> 11.9 us,
+// 8192 20.6 -> 14.9, 16384 27.3 -> 21.0, 32768 34.1 -> 32.0; 16 sequences of 4096: 38.0 -> 33.4.
+template <int THREADS, int MAXC>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS > 512 ? 4 : THREADS > 256 ? 2 : 1, 4)))
+void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restrict__ out, RowsOut ro) {
+    constexpr int kMaxGroup = 16;
+    __shared__ float s_lse[kMaxGroup];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = blockIdx.x, b = row / p.groups;
+    const int raw = p.seqlens ? p.seqlens[b] : p.uniform_len;
+    const float* base = p.scores + (long long)row * p.group_size * p.scores_stride;   // heads of a KV head are adjacent
+    const int len = max(0, min(raw, p.len_cap));           // tokens whose scores were written
+    int row_len = min(raw, p.uniform_len), n = k;
+    if (p.topk_percent > 0.f) {
+        const long long fl = (long long)floor((double)p.topk_percent * (double)raw / 100.0);
+        n = (int)min((long long)k, (fl + 127) / 128 * 128);
+    } else {
+        row_len = p.uniform_len;                           // every row the same: positions past a sequence pool to 0
+    }
+    n = max(0, n);
+    if (row_len <= n || n == 0) {
+        if (p.glse == nullptr) {
+            list_head<THREADS>(n, k, fill, out, row, ro);
+            return;
+        }
+    }
+    // the heads' log-sums: merged from the splits' parts by a wavefront per head, or ready
+    for (int h = wave; h < p.group_size; h += THREADS / 64) {
+        const long long head = (long long)row * p.group_size + h;
+        if (p.glse) {
+            const float* gl = p.glse + head * p.num_split;
+            const float g0 = lane < p.num_split ? gl[lane] : -INFINITY;
+            float mx = g0;
+            for (int s = lane + 64; s < p.num_split; s += 64) mx = fmaxf(mx, gl[s]);
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            const float mref = (mx == -INFINITY) ? 0.f : mx;
+            float sum = fast_exp2(g0 - mref);
+            for (int s = lane + 64; s < p.num_split; s += 64) sum += fast_exp2(gl[s] - mref);
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+            const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
+            if (lane == 0) {
+                s_lse[h] = v;
+                p.row_sums[head] = v;
+            }
+        } else if (lane == 0) {
+            s_lse[h] = p.row_sums[head];
+        }
+    }
+    if (row_len <= n || n == 0) {
+        list_head<THREADS>(n, k, fill, out, row, ro);
+        return;
+    }
+    // Scores four heads at a time (a batch), two batches ahead on their way.
+    const int nch = (row_len + THREADS * 8 - 1) / (THREADS * 8);   // <= MAXC (host)
+    const int first = wave * nch * 512 + lane * 8;
+    const int last_piece = max(0, len - 1) & ~7;
+    struct Batch {
+        uint4_t q[4];
+        float ref[4];
+    };
+    const int nb = (p.group_size + 3) / 4;                 // batches per chunk
+    auto load_batch = [&](int i, Batch& bt) {              // batch i: heads 4 (i % nb) .. +3 of chunk i / nb
+        const int c = min(i / nb, nch - 1), h0 = 4 * (i - i / nb * nb);
+        const int jc = min(first + c * 512, last_piece);   // past the tokens: entries that exist, dropped below
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float* hr = base + (long long)min(h0 + u, p.group_size - 1) * p.scores_stride;
+            bt.q[u] = *reinterpret_cast<const uint4_t*>(reinterpret_cast<const uint16_t*>(hr) + jc);
+            bt.ref[u] = hr[p.scores_stride / 2 + (jc >> 6)];
+        }
+    };
+    uint4_t data[MAXC];
+    Batch cur, n1, n2;
+    load_batch(0, n1);
+    load_batch(1, n2);
+    __syncthreads();   // s_lse
+    static_for<0, MAXC>([&](auto c_c) {
+        constexpr int c = decltype(c_c)::value;
+        data[c] = uint4_t{0, 0, 0, 0};
+        const int j0 = first + c * 512;
+        if (c < nch && wave * nch * 512 + c * 512 < row_len) {     // uniform over the wavefront
+            float sum[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma clang loop unroll(disable)
+            for (int hb = 0; hb < nb; ++hb) {
+                cur = n1;
+                n1 = n2;
+                load_batch(c * nb + hb + 2, n2);
+                __builtin_amdgcn_sched_barrier(0);
+                const int h0 = 4 * hb;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    // a slot past the last head adds exp2(-inf) = 0
+                    const float ref = h0 + u < p.group_size ? cur.ref[u] - s_lse[h0 + u] : -INFINITY;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const uint32_t q = (e & 1) ? cur.q[u][e >> 1] >> 16 : cur.q[u][e >> 1] & 0xFFFFu;
+                        sum[e] += fast_exp2(__builtin_fmaf((float)q, -1.f / kScoreSteps, ref));
+                    }
+                }
+            }
+            // packed order keys: no entry is negative, so the key is the value with the top bit set
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const half2_t x = {(half_t)sum[e], (half_t)sum[e + 1]};
+                data[c][e >> 1] = __builtin_bit_cast(uint32_t, x) | 0x80008000u;
+            }
+            if (j0 + 8 > len) {   // the piece at the tokens' end and those behind it: probability 0, or no entry
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int sh = 16 * (e & 1);
+                    const uint32_t key = j0 + e < len ? (data[c][e >> 1] >> sh) & 0xFFFFu : j0 + e < row_len ? 0x8000u : 0u;
+                    data[c][e >> 1] = (data[c][e >> 1] & (0xFFFF0000u >> sh)) | (key << sh);
+                }
+            }
+        }
+    });
+    select_row<THREADS, MAXC, true>(data, nch, 0, row_len, n, k, fill, out, row, ro);
+}
+
 // --------------------------------------------------------------------------
 // Long rows: the same radix select spread over several workgroups per row.
 // Every workgroup owns one chunk of kSplitChunk entries of one row and holds it in registers
@@ -1218,6 +1348,31 @@ hipError_t launch_topk(const half_t* scores, int* out_idx, int rows, long long r
     else
         hipLaunchKernelGGL(topk_select_kernel, dim3(rows), dim3(kThreads), 0, stream, src, out_idx,
                            row_stride, uniform_len, valid_len, n_sel, period, k, fill, ro);
+    return hipGetLastError();
+}
+
+hipError_t launch_decode_pool_select(const DecodePoolParams& p, int rows, int k, int fill, int* out_idx, const TopkRows* tr,
+                                     hipStream_t stream) {
+    if (rows == 0) return hipSuccess;
+    const RowsOut ro = rows_out(tr);
+    auto go = [&](auto threads, auto chunks) {
+        constexpr int kT = decltype(threads)::value;
+        hipLaunchKernelGGL((decode_pool_select_kernel<kT, decltype(chunks)::value>), dim3(rows), dim3(kT), 0, stream, p, k,
+                           fill, out_idx, ro);
+    };
+    std::integral_constant<int, 256> t256{};
+    std::integral_constant<int, 512> t512{};
+    std::integral_constant<int, 1024> t1024{};
+    std::integral_constant<int, 1> c1{};
+    std::integral_constant<int, 2> c2{};
+    std::integral_constant<int, 4> c4{};
+    const int len = p.uniform_len;
+    if (len > kPoolSelectRow) return hipErrorInvalidValue;
+    if (len <= 2048) go(t256, c1);
+    else if (len <= 4096) go(t256, c2);
+    else if (len <= 8192) go(t512, c2);
+    else if (len <= 16384) go(t512, c4);
+    else go(t1024, c4);
     return hipGetLastError();
 }
 

@@ -1,4 +1,5 @@
 """The selection's and the decode split's dispatch lines: sizes at the edges of each variant."""
+import ctypes
 import math
 
 import pytest
@@ -34,6 +35,56 @@ def test_register_selection_edges(cuda, L, rows):
     idx = kernels.topk_indices(sc, k).cpu()
     assert all(torch.equal(idx[r], idx[r % 3]) for r in range(rows))
     _check_rows(base, idx[:3], lambda r: k, lambda r: L, f"L={L}")
+
+
+@pytest.mark.parametrize("H,G,L", [(32, 8, 1), (32, 8, 2047), (8, 8, 2049), (28, 4, 4096), (40, 8, 4097), (64, 4, 8192),
+                                   (32, 8, 8193), (28, 4, 16384), (16, 2, 16385), (32, 8, 32768), (32, 8, 32769)])
+@pytest.mark.parametrize("ragged", [False, True])
+def test_anchor_selection_in_one_call(cuda, H, G, L, ragged):
+    """kascade_decode_anchor_topk_call selects exactly the largest of the scores that the anchor pass
+    pools by itself (checked against the oracle in test_gpu_decode): the two share the arithmetic, so
+    there is no tolerance.  Row lengths at the edges of each pooling variant, groups of 1 to 16 heads."""
+    from kascade_amd import _lib, kernels
+    D, page, p = 128, 16, 10.0
+    gen = torch.Generator().manual_seed(L + H)
+    lens = [L, max(1, L // 3), max(1, L - 1)] if ragged else [L, L]
+    B, pages = len(lens), math.ceil(L / page)
+    q = torch.randn(B, H, D, generator=gen).half().to(cuda)
+    kp = torch.randn(B * pages, page, G, D, generator=gen).half().to(cuda)
+    bt = torch.randperm(B * pages, generator=gen).to(torch.int32).view(B, pages).to(cuda)
+    seq = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    ns, stride = min(4, math.ceil(L / 64)), (L + 7) // 8 * 8
+    glse = torch.empty(B, H, ns, device=cuda)
+    sums, scores = torch.empty(B, H, device=cuda), torch.empty(B, H, stride, device=cuda)
+    _, agg = kernels.decode_recompute(q, kp, kp, glse, None, sums, scores, 1, cache_seqlens=seq, block_table=bt,
+                                      page_size=page, kv_len=L)
+    want_sums = sums.clone()
+    nsel = [math.ceil(int(p * n / 100) / 128) * 128 for n in lens] if ragged else [max(1, L // 10)] * B
+    k = max(1, max(nsel))
+    lib, ptr = _lib.init(), lambda t: None if t is None else t.data_ptr()
+    idx = torch.full((B, G, k), -7, dtype=torch.int32, device=cuda)
+    rows = torch.full_like(idx, -7)
+    big = L > 32768
+    per_row = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda).repeat_interleave(G) if big and ragged else None
+    valid_d, nsel_d = per_row(lens), per_row(nsel)
+    agg2 = torch.empty(B, G, stride, device=cuda, dtype=torch.float16) if big else None
+    shape = ctypes.byref(_lib.Shape(G, D, kernels._ELEM[torch.float16], H // G))
+    _lib.check(lib.kascade_decode_anchor_topk_call(
+        shape, ptr(q), ptr(kp), None, ptr(seq), ptr(glse), None, ptr(sums), ptr(scores), None, ptr(agg2), ptr(idx), ptr(rows),
+        B, L, stride, ns, 0, L, k, 5, p if ragged else 0.0, ptr(valid_d), ptr(nsel_d), None, ptr(bt), pages, page, None, None,
+        None, None, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(sums, want_sums)
+    idx, pooled = idx.cpu(), agg.cpu()
+    table = bt.cpu().long()
+    for b in range(B):
+        n, valid = nsel[b], lens[b]
+        _check_rows(pooled[b], idx[b], lambda r: n, lambda r: valid, f"sequence {b}")
+        assert bool((idx[b, :, n:] == 5).all())
+        t = idx[b].long()
+        inside = t < L
+        want = table[b][(t.clamp(max=L - 1)) // page] * page + t % page
+        assert torch.equal(rows[b].cpu().long()[inside], want[inside])
 
 
 @pytest.mark.parametrize("seqlens,ns", [([1024], 1), ([1025], 1), ([2048, 1], 1), ([2049, 64], 1), ([255, 257, 4096], 2),
