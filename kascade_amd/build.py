@@ -1,6 +1,7 @@
-"""Builds libkascade_hip.so (gfx950) from kascade_amd/csrc with hipcc.
+"""Builds libkascade_hip.so (gfx950) from kascade_amd/csrc with hipcc, and the extension module
+_native (host code against torch's C++ interface, linked to that library) with g++.
 
-The library is built in-tree (kascade_amd/libkascade_hip.so).  ``build()``
+Both are built in-tree (kascade_amd/libkascade_hip.so, kascade_amd/_native.so).  ``build()``
 always recompiles; ``ensure_built()`` compiles only when no library exists.
 Run ``python -m kascade_amd.build`` to build from a shell.
 """
@@ -10,12 +11,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libkascade_hip.so"
+NATIVE_PATH = PKG_DIR / "_native.so"
 SOURCES = ["capi.hip", "decode.hip", "topk.hip", "prefill.hip", "paged.hip", "diag.hip"]
 ARCH = "gfx950"
 
@@ -64,11 +67,24 @@ def build(verbose: bool = False, extra_flags=()) -> Path:
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wno-unused-command-line-argument",
           *map(str, objs), "-o", str(tmp)])
     os.replace(tmp, LIB_PATH)
+    build_native()
     return LIB_PATH
 
 
+def build_native() -> Path:
+    """The host extension: plain C++ (no device code), so g++ builds it."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{root / 'include'}",
+          f"-I{sysconfig.get_paths()['include']}", str(CSRC / "native.cpp"), f"-L{PKG_DIR}", "-l:libkascade_hip.so",
+          f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN", "-o", str(tmp)])
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def ensure_built() -> Path:
-    if not LIB_PATH.exists():
+    if not (LIB_PATH.exists() and NATIVE_PATH.exists()):
         build()
     return LIB_PATH
 

@@ -30,12 +30,13 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
-from . import budgets, kernels
+from . import _lib, budgets, kernels
 from ._lib import KascadeError
 
 H, G, D, TILE = 32, 8, 128, 32
 FUSED_MERGE_MAX_SPLITS = 32
 ANCHOR_ROWS_PER_SPLIT = 8192
+POOL_SELECT_ROW = 32768   # tokens of a decode row that one workgroup pools and selects
 
 
 def get_head_mapping(model_name: str, recompute_layers: Sequence[int],
@@ -93,19 +94,31 @@ class EfficientKascadeStrategy:
         self._topk_to_reuse = None
         self._hm_cache = {}
         self._budget_cache = {}
+        self._merge_counters = None
+        cls = type(self)   # a subclass that replaces a seam gets its layers through it
+        self._own_seams = all(getattr(cls, name) is getattr(EfficientKascadeStrategy, name)
+                              for name in ("_prefill_recomp_forward", "_prefill_reuse_forward",
+                                           "_decode_recomp_forward", "_decode_reuse_forward"))
         if register:
             self.register_attention()
 
     # ------------------------------------------------------------------ helpers
     def _hm(self, layer, device, groups: int = G) -> torch.Tensor:
-        key = (layer, str(device), groups)
-        if key not in self._hm_cache:
+        key = (layer, device, groups)
+        hm = self._hm_cache.get(key)
+        if hm is None:
             row = list(range(groups)) if layer is None else self._head_mapping[layer]
-            self._hm_cache[key] = _head_map_tensor(row, groups, layer, device)
-        return self._hm_cache[key]
+            hm = self._hm_cache[key] = _head_map_tensor(row, groups, layer, device)
+        return hm
+
+    def _counters(self):
+        """Arrival counters of the decode launches' split merge, one array per stream."""
+        if self._merge_counters is None:
+            self._merge_counters = _lib.native().Counters()
+        return self._merge_counters
 
     def _tile_budgets(self, L, width, device):
-        key = (L, width, self.rolling_prefill, float(self.k), str(device))
+        key = (L, width, self.rolling_prefill, float(self.k), device)
         if key not in self._budget_cache:
             valid, nsel = budgets.prefill_tile_budgets(L, self.tile_size, self.k, self.rolling_prefill, width)
             self._budget_cache[key] = (torch.tensor(valid, device=device, dtype=torch.int32),
@@ -113,125 +126,135 @@ class EfficientKascadeStrategy:
         return self._budget_cache[key]
 
     # ------------------------------------------------------------------ prefill
-    def _prefill_recomp_forward(self, Q, K, V, topk, tile_size, layer, topk_percent):
+    # The layer calls below take query [B,H,Lq,D] and key/value [B,G,Lk,D]; the seams of the same names
+    # without "_hf" take the reference's [B,L,heads,D] order, as views of the same memory.
+    def _hf_prefill_recomp(self, query, key, value, topk, layer, topk_percent):
         """Anchor prefill (EfficientKascadeStrategy.py:72-93): log-sum pass (+ dense output on
         layer 0), pooled tile scores, per-tile selection, and on layers > 0 the sparse pass with
         the fresh indices and the identity head map."""
-        B, L = Q.shape[:2]
-        G = K.shape[2]                      # KV heads of this model (8 for the reference's shape)
-        T = math.ceil(L / tile_size)
+        B, G, L = key.shape[:3]             # KV heads of this model (8 for the reference's shape)
+        device = query.device
+        valid, nsel = self._tile_budgets(L, topk, device)
+        if L <= self.WHOLE_PROMPT_SCORES:
+            o, self._topk_to_reuse = _lib.native().hf_prefill_anchor(
+                query, key, value, layer == 0, topk, valid, nsel, self._hm(None, device, G), topk_percent,
+                self.rolling_prefill)
+            return o
+        # Long prompts: pool and select SCORE_CHUNK_TILES tiles at a time.  The whole score
+        # tensor would take L^2/4 bytes (8 GiB at 131072 tokens), and rows beyond 65536 entries
+        # go to the multi-workgroup selection, which takes a few thousand rows per call.  The
+        # reference keeps the whole tensor and chunks its torch.topk by rows above 131072
+        # tokens (EfficientKascadeStrategy.py:83-90); the indices are the same.
+        Q, K, V = query.transpose(1, 2), key.transpose(1, 2), value.transpose(1, 2)
+        tile = self.tile_size
+        T = math.ceil(L / tile)
         if layer == 0:
             log_sum, o = kernels.prefill_recompute0(Q, K, V)
         else:
             log_sum = kernels.prefill_recompute1(Q, K)
-        valid, nsel = self._tile_budgets(L, topk, Q.device)
-        if L <= self.WHOLE_PROMPT_SCORES:
-            scores = torch.empty((B, G, T, L), device=Q.device, dtype=torch.float16)
-            kernels.prefill_aggregate(Q, K, log_sum, scores)
-            self._topk_to_reuse = kernels.topk_indices(scores, topk, valid_len=valid, n_sel=nsel)
-        else:
-            # Long prompts: pool and select SCORE_CHUNK_TILES tiles at a time.  The whole score
-            # tensor would take L^2/4 bytes (8 GiB at 131072 tokens), and rows beyond 65536 entries
-            # go to the multi-workgroup selection, which takes a few thousand rows per call.  The
-            # reference keeps the whole tensor and chunks its torch.topk by rows above 131072
-            # tokens (EfficientKascadeStrategy.py:83-90); the indices are the same.
-            idx = torch.empty((B, G, T, topk), device=Q.device, dtype=torch.int32)
-            step = max(32, self.SCORE_CHUNK_TILES // B)
-            buf = torch.empty(B * G * step * L, device=Q.device, dtype=torch.float16)
-            for t0 in range(0, T, step):
-                t1 = min(t0 + step, T)
-                s, e = t0 * tile_size, min(t1 * tile_size, L)
-                scores = buf[:B * G * (t1 - t0) * e].view(B, G, t1 - t0, e)
-                kernels.prefill_aggregate_range(Q, K, log_sum, scores, s, e - s)
-                idx[:, :, t0:t1] = kernels.topk_indices(scores, topk, valid_len=valid[t0:t1].contiguous(),
-                                                        n_sel=nsel[t0:t1].contiguous(), fill_value=L - 1)
-            self._topk_to_reuse = idx
+        idx = torch.empty((B, G, T, topk), device=device, dtype=torch.int32)
+        step = max(32, self.SCORE_CHUNK_TILES // B)
+        buf = torch.empty(B * G * step * L, device=device, dtype=torch.float16)
+        for t0 in range(0, T, step):
+            t1 = min(t0 + step, T)
+            s, e = t0 * tile, min(t1 * tile, L)
+            scores = buf[:B * G * (t1 - t0) * e].view(B, G, t1 - t0, e)
+            kernels.prefill_aggregate_range(Q, K, log_sum, scores, s, e - s)
+            idx[:, :, t0:t1] = kernels.topk_indices(scores, topk, valid_len=valid[t0:t1].contiguous(),
+                                                    n_sel=nsel[t0:t1].contiguous(), fill_value=L - 1)
+        self._topk_to_reuse = idx
         if layer != 0:
-            o = kernels.prefill_reuse(Q, K, V, self._topk_to_reuse, self._hm(None, Q.device, G), topk_percent,
-                                      self.rolling_prefill)
+            o = kernels.prefill_reuse(Q, K, V, idx, self._hm(None, device, G), topk_percent, self.rolling_prefill)
         return o
 
-    def _prefill_reuse_forward(self, Q, K, V, topk_percent, layer):
+    def _hf_prefill_reuse(self, query, key, value, topk_percent, layer):
         """Reuse prefill (EfficientKascadeStrategy.py:95-98)."""
         if self._topk_to_reuse is None:
             raise KascadeError("reuse layer called before any anchor layer")
-        return kernels.prefill_reuse(Q, K, V, self._topk_to_reuse, self._hm(layer, Q.device, K.shape[2]), topk_percent,
-                                     self.rolling_prefill)
+        return _lib.native().hf_prefill_reuse(query, key, value, self._topk_to_reuse,
+                                              self._hm(layer, query.device, key.shape[1]), topk_percent,
+                                              self.rolling_prefill)
+
+    def _prefill_recomp_forward(self, Q, K, V, topk, tile_size, layer, topk_percent):
+        return self._hf_prefill_recomp(Q.transpose(1, 2), K.transpose(1, 2), V.transpose(1, 2), topk, layer, topk_percent)
+
+    def _prefill_reuse_forward(self, Q, K, V, topk_percent, layer):
+        return self._hf_prefill_reuse(Q.transpose(1, 2), K.transpose(1, 2), V.transpose(1, 2), topk_percent, layer)
 
     # ------------------------------------------------------------------- decode
-    def _decode_scratch(self, Q, ns):
-        B, heads, dim = Q.shape
-        return (torch.empty(B, heads, ns, device=Q.device, dtype=torch.float32),
-                torch.empty(B, heads, ns, dim, device=Q.device, dtype=torch.float32))
-
-    def _decode_recomp_forward(self, Q, K, V, topk, layer):
-        """Anchor decode (EfficientKascadeStrategy.py:100-115) over a contiguous [B,L,G,D] cache."""
-        B, L, G = K.shape[:3]
-        H = Q.shape[1]
-        ns = kernels.default_num_split(B * G * L, L, heads=G)
-        glse, part = self._decode_scratch(Q, ns)
-        row_sums = torch.empty(B, H, device=Q.device, dtype=torch.float32)
-        stride = ((L + 7) // 8) * 8
-        scores = torch.empty(B, H, stride, device=Q.device, dtype=torch.float32)
-        o, agg = kernels.decode_recompute(Q, K, V, glse, part, row_sums, scores, layer)
-        self._topk_to_reuse = kernels.topk_indices(agg[:, :, :L], topk, fill_value=0)
-        if layer != 0:
-            ns = kernels.default_num_split(B * G * topk, topk, cap_rows=kernels.GATHER_ROWS_PER_SPLIT, heads=G)
-            glse, part = self._decode_scratch(Q, ns)
-            o = kernels.decode_reuse(Q, K, V, self._topk_to_reuse, self._hm(None, Q.device, G), glse, part)
+    def _hf_decode_recomp(self, query, key, value, topk, layer):
+        """Anchor decode (EfficientKascadeStrategy.py:100-115): scores pass (+ dense output on
+        layer 0), pooling and selection, and on layers > 0 the gather with the fresh indices."""
+        native = _lib.native()
+        o, self._topk_to_reuse = native.hf_decode_anchor(self._counters(), query, key, value, layer == 0, topk,
+                                                         self._hm(None, query.device, key.shape[1]))
         return o
 
-    def _decode_reuse_forward(self, Q, K, V, layer):
+    def _hf_decode_reuse(self, query, key, value, layer):
         """Reuse decode (EfficientKascadeStrategy.py:117-123)."""
         if self._topk_to_reuse is None:
             raise KascadeError("reuse layer called before any anchor layer")
-        B, G = Q.shape[0], K.shape[2]
-        topk = self._topk_to_reuse.shape[-1]
-        ns = kernels.default_num_split(B * G * topk, topk, cap_rows=kernels.GATHER_ROWS_PER_SPLIT, heads=G)
-        glse, part = self._decode_scratch(Q, ns)
-        return kernels.decode_reuse(Q, K, V, self._topk_to_reuse, self._hm(layer, Q.device, G), glse, part)
+        native = _lib.native()
+        return native.hf_decode_reuse(self._counters(), query, key, value, self._topk_to_reuse,
+                                      self._hm(layer, query.device, key.shape[1]))
+
+    def _decode_recomp_forward(self, Q, K, V, topk, layer):
+        return self._hf_decode_recomp(Q.unsqueeze(2), K.transpose(1, 2), V.transpose(1, 2), topk, layer).squeeze(1)
+
+    def _decode_reuse_forward(self, Q, K, V, layer):
+        return self._hf_decode_reuse(Q.unsqueeze(2), K.transpose(1, 2), V.transpose(1, 2), layer).squeeze(1)
 
     # --------------------------------------------------------------- HF boundary
     def attention_forward(self, module, query, key, value, attention_mask, scaling, dropout=0.0, **kwargs):
         """EfficientKascadeStrategy.py:126-161.  query [B,H,Lq,D], key/value [B,G,Lk,D]."""
-        if key.shape[-2] <= 128:
+        _, G, Lk, _ = key.shape
+        if Lk <= 128:
             from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
             return ALL_ATTENTION_FUNCTIONS["sdpa"](module, query, key, value, attention_mask,
                                                    scaling=scaling, dropout=dropout, **kwargs)
         # the reference's kernels exist for fp16, 32 query / 8 KV heads, head_dim 128 only
         # (EfficientKascadeStrategy.py:19-21); here any model with 1 to 16 query heads per KV head,
         # head_dim 64 or 128, in fp16 or bf16
-        if query.shape[1] % key.shape[1] or query.shape[1] // key.shape[1] not in kernels.GROUPS_OK \
-                or query.shape[-1] not in (64, 128) or query.dtype not in (torch.float16, torch.bfloat16):
+        _, H, Lq, D = query.shape
+        if H % G or H // G not in kernels.GROUPS_OK \
+                or D not in (64, 128) or query.dtype not in (torch.float16, torch.bfloat16):
             raise KascadeError("efficient_kascade needs fp16 or bf16, 1 to 16 query heads per KV head, "
                                "head_dim 64 or 128")
-        is_decode = (query.shape[2] == 1)
-        Lk = key.shape[-2]
-        rounded_k = budgets.topk_width(Lk, self.k)
-        query = query.transpose(1, 2)   # B, L, H, D (strided view)
-        key = key.transpose(1, 2)
-        value = value.transpose(1, 2)
         layer = module.layer_idx
-        if is_decode:
-            query = query.squeeze(1).contiguous()
-            # The reference copies the whole cache to [B,L,G,D] here on every step
-            # (EfficientKascadeStrategy.py:149-150); the decode kernels take the strided view of
-            # HF's head-major cache instead and read it in place.
-            if key.stride(-1) != 1 or value.stride() != key.stride():
-                key, value = key.contiguous(), value.contiguous()
-            if layer in self.recompute_layers:
-                o = self._decode_recomp_forward(query, key, value, rounded_k, layer)
+        anchor = layer in self.recompute_layers
+        if Lq != 1 and Lq != Lk:
+            raise KascadeError("prefill needs Lq == Lk (no cached prefix), as in the reference kernels")
+        if not self._own_seams:
+            return self._through_seams(query, key, value, layer, anchor), None
+        # The reference copies the whole cache to [B,L,G,D] here on every decode step
+        # (EfficientKascadeStrategy.py:149-150); the kernels take strided views of HF's head-major
+        # tensors instead and read them in place.
+        if Lq == 1:
+            if anchor:
+                o = self._hf_decode_recomp(query, key, value, budgets.topk_width(Lk, self.k), layer)
             else:
-                o = self._decode_reuse_forward(query, key, value, layer)
-            o = o.unsqueeze(1)
+                o = self._hf_decode_reuse(query, key, value, layer)
+        elif anchor:
+            o = self._hf_prefill_recomp(query, key, value, budgets.topk_width(Lk, self.k), layer, self.k)
         else:
-            if query.shape[1] != Lk:
-                raise KascadeError("prefill needs Lq == Lk (no cached prefix), as in the reference kernels")
-            if layer in self.recompute_layers:
-                o = self._prefill_recomp_forward(query, key, value, rounded_k, self.tile_size, layer, self.k)
-            else:
-                o = self._prefill_reuse_forward(query, key, value, self.k, layer)
+            o = self._hf_prefill_reuse(query, key, value, self.k, layer)
         return o, None
+
+    def _through_seams(self, query, key, value, layer, anchor):
+        """A layer of a subclass with seams of its own, which take [B,L,heads,D] views (decode: Q [B,H,D])."""
+        rounded_k = budgets.topk_width(key.shape[2], self.k)
+        K, V = key.transpose(1, 2), value.transpose(1, 2)
+        if query.shape[2] == 1:
+            Q = query.squeeze(2).contiguous()
+            if K.stride(-1) != 1 or V.stride() != K.stride():
+                K, V = K.contiguous(), V.contiguous()
+            o = self._decode_recomp_forward(Q, K, V, rounded_k, layer) if anchor else \
+                self._decode_reuse_forward(Q, K, V, layer)
+            return o.unsqueeze(1)
+        Q = query.transpose(1, 2)
+        if anchor:
+            return self._prefill_recomp_forward(Q, K, V, rounded_k, self.tile_size, layer, self.k)
+        return self._prefill_reuse_forward(Q, K, V, self.k, layer)
 
     def register_attention(self):
         """EfficientKascadeStrategy.py:163-168."""
@@ -269,6 +292,7 @@ class PagedKascadeDecoder:
         workgroups, not the grid, cover the device about twice.
         seqlens_hint: the (approximate) lengths themselves, as a serving engine's scheduler knows
         them; then the workgroups of a ragged batch are counted exactly."""
+        self._native = _lib.native()
         self.k = k
         self.page_size = page_size
         self.recompute_layers = list(recompute_layers)
@@ -338,11 +362,8 @@ class PagedKascadeDecoder:
 
     def dense(self, q, k_pages, v_pages, block_table, seqlens, max_len: int, out=None,
               k_new=None, v_new=None):
-        B = q.shape[0]
-        glse, part = self._scratch(B, self.ns_dense)
-        return kernels.decode_dense_paged(q, k_pages, v_pages, seqlens, glse, part, block_table,
-                                          self.page_size, kv_len=max_len, out=out, sync=self._sync_dense,
-                                          k_new=k_new, v_new=v_new)
+        return self._native.paged_dense(q, k_pages, v_pages, seqlens, self._glse, self._part, self.ns_dense, max_len,
+                                        block_table, self.page_size, out, self._sync_dense, k_new, v_new)
 
     def begin_step(self, seqlens: torch.Tensor, advance: int = 1):
         """One launch at the start of a decode step: the lengths grow by ``advance`` in place
@@ -361,29 +382,22 @@ class PagedKascadeDecoder:
         """Anchor layer: returns the attention output [B,H,D] (written to ``out`` when given);
         keeps indices for reuse layers.  ``k_new``/``v_new`` [B,G,D]: rows of the newest token
         (position seqlens-1), appended to the cache by the anchor launch itself."""
-        B = q.shape[0]
-        G, H = self.G, self.H
-        stride = ((max_len + 7) // 8) * 8
-        glse, part = self._scratch(B, self.ns_anchor)
-        scores = self._scores[:B * H * stride].view(B, H, stride)
-        o, agg = kernels.decode_recompute(q, k_pages, v_pages, glse, part, self._row_sums[:B], scores, layer,
-                                          cache_seqlens=seqlens, block_table=block_table,
-                                          page_size=self.page_size, kv_len=max_len, out=out, sync=self._sync_anchor,
-                                          k_new=k_new, v_new=v_new)
+        B, G = q.shape[0], self.G
+        valid = nsel = None
         if ragged:
-            width = budgets.decode_budget(max_len, self.k)
-            lens_rows, counts = self._row_budgets(seqlens)
+            width, pct = budgets.decode_budget(max_len, self.k), float(self.k)
+            if max_len > POOL_SELECT_ROW:
+                valid, nsel = self._row_budgets(seqlens)
         else:
-            width = budgets.topk_width(max_len, self.k)
-            lens_rows = counts = None
+            width, pct = budgets.topk_width(max_len, self.k), 0.0
         # One translation per anchor, inside the selection launch: every reuse launch up to the
         # next anchor reads the same block table, so the selection also leaves its lists as cache
         # rows and the gathers skip the table.
-        self._topk_to_reuse, self._rows_to_reuse = kernels.topk_indices(
-            agg[:, :, :max_len], width, valid_len=lens_rows, n_sel=counts, fill_value=0,
-            block_table=block_table, page_size=self.page_size,
-            rows_out=self._rows_buf[:B * G * width].view(B, G, width))
-        self._pct = float(self.k) if ragged else 0.0
+        rows = self._rows_buf[:B * G * width].view(B, G, width)
+        o, self._topk_to_reuse = self._native.paged_anchor(
+            q, k_pages, v_pages, seqlens, layer == 0, self._glse, self._part, self.ns_anchor, self._row_sums, self._scores,
+            max_len, width, pct, valid, nsel, block_table, self.page_size, out, self._sync_anchor, k_new, v_new, rows)
+        self._rows_to_reuse, self._pct = rows, pct
         if layer != 0:
             o = self._reuse(q, k_pages, v_pages, block_table, seqlens, self._hm[None], out)
         return o
@@ -399,11 +413,9 @@ class PagedKascadeDecoder:
         return self._counts[1], self._counts[2]
 
     def _reuse(self, q, k_pages, v_pages, block_table, seqlens, hm, out=None, k_new=None, v_new=None):
-        B = q.shape[0]
-        glse, part = self._scratch(B, self.ns_reuse)
-        return kernels.decode_reuse_rows(q, k_pages, v_pages, seqlens, self._rows_to_reuse, hm, self._pct,
-                                         glse, part, block_table, page_size=self.page_size, out=out,
-                                         sync=self._sync_reuse, k_new=k_new, v_new=v_new)
+        return self._native.paged_reuse(q, k_pages, v_pages, seqlens, self._rows_to_reuse, hm, self._pct, self._glse,
+                                        self._part, self.ns_reuse, block_table, self.page_size, out, self._sync_reuse,
+                                        k_new, v_new)
 
     def reuse(self, layer, q, k_pages, v_pages, block_table, seqlens, out=None, k_new=None, v_new=None):
         """Reuse layer: attends to rows head_mapping[layer] of the last anchor's indices."""
