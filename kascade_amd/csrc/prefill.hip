@@ -721,8 +721,9 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
             hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, true, D, T>), grid, block, 0, stream, p);
     } else if (reuse) {
         hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, false, D, T>), grid, block, 0, stream, p);
-    } else if (nqb == 2) {   // K-only log-sum pass
-        hipLaunchKernelGGL((prefill_attn_kernel_q64<D, T>), grid, block, 0, stream, p);
+    } else if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
+        if constexpr (D == 128) hipLaunchKernelGGL((prefill_attn_kernel_q64<D, T>), grid, block, 0, stream, p);
+        else return hipErrorInvalidValue;
     } else {
         if (with_v)
             hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, false, D, T>), grid, block, 0, stream, p);
