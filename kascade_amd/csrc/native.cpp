@@ -133,19 +133,19 @@ PyTypeObject CountersType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 at::Tensor counters_for(PyObject* o, void* stream, int64_t n, const at::Tensor& like) {
     if (Py_TYPE(o) != &CountersType) fail("expected a _native.Counters object");
-    auto& map = *reinterpret_cast<Counters*>(o)->by_stream;
-    auto it = map.find(stream);
-    if (it != map.end() && it->second.numel() >= n && it->second.device() == like.device()) return it->second;
-    at::Tensor t = at::zeros({std::max<int64_t>(n, 1024)}, like.options().dtype(at::kInt));
-    // zeros made while a graph is being captured are filled when the graph runs: good for it, not to be kept
     PyObject* c = PyObject_CallNoArgs(g_capturing);
     if (!c) throw Fail{};
     const bool capturing = PyObject_IsTrue(c) == 1;
     Py_DECREF(c);
-    if (!capturing) {
-        if (map.size() >= 16) map.clear();   // a program that keeps making streams
-        map[stream] = t;
-    }
+    const auto options = like.options().dtype(at::kInt);
+    // A graph replays on any stream and outlives this object: counters of its own, from its memory pool.
+    if (capturing) return at::zeros({n}, options);
+    auto& map = *reinterpret_cast<Counters*>(o)->by_stream;
+    auto it = map.find(stream);
+    if (it != map.end() && it->second.numel() >= n && it->second.device() == like.device()) return it->second;
+    const at::Tensor t = at::zeros({std::max<int64_t>(n, 1024)}, options);
+    if (map.size() >= 16) map.clear();   // a program that keeps making streams
+    map[stream] = t;
     return t;
 }
 
@@ -509,7 +509,7 @@ PyObject* attribute(const char* module, const char* name) {
 PyMODINIT_FUNC PyInit__native(void) {
     g_error = attribute("kascade_amd._lib", "KascadeError");
     g_raw_stream = attribute("torch", "_C._cuda_getCurrentRawStream");
-    g_capturing = attribute("torch.cuda", "is_current_stream_capturing");
+    g_capturing = attribute("torch", "_C._cuda_isCurrentStreamCapturing");
     if (!g_error || !g_raw_stream || !g_capturing) return nullptr;
     CountersType.tp_name = "_native.Counters";
     CountersType.tp_basicsize = sizeof(Counters);

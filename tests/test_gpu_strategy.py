@@ -216,3 +216,31 @@ def test_anchor_prefill_in_tile_chunks_equals_whole_prompt(cuda, L, B):
             assert torch.equal(torch.where(live.to(a.device), a, 0), torch.where(live.to(a.device), b, 0))
         else:
             assert torch.equal(a, b)
+
+
+def test_captured_decode_keeps_its_own_merge_counters(cuda):
+    """A captured layer replays right after the strategy that recorded it, whose eager calls on the same
+    stream came first, is gone and its memory holds something else."""
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    L = 3000
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    q = torch.randn(1, H, 1, D, device=cuda, generator=gen, dtype=torch.float32).half()
+    k, v = (torch.randn(1, G, L, D, device=cuda, generator=gen, dtype=torch.float32).half() for _ in range(2))
+    s = EfficientKascadeStrategy([0], None, k=10, tile_size=TILE, head_mapping=[list(range(G))] * 2, register=False)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        want = [s.attention_forward(_Module(l), q, k, v, None, D ** -0.5)[0].clone() for l in (0, 1)]
+    stream.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        got = [s.attention_forward(_Module(l), q, k, v, None, D ** -0.5)[0] for l in (0, 1)]
+    s._merge_counters = None
+    with torch.cuda.stream(stream):   # what the freed counters' memory is given to next
+        held = [torch.full((1024,), 5, device=cuda, dtype=torch.int32) for _ in range(8)]
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert all(bool((t == 5).all()) for t in held)
