@@ -43,6 +43,7 @@ struct PrefillParams {
     int head_dim;             // 64 or 128
     int elem;                 // kElemF16 or kElemBF16
     int gs;                   // query heads per KV head: 1 to 16 (0 = 4)
+    int key_parts, part_tiles;   // pooling kernel: parts of part_tiles key tiles a query tile's keys are cut into
     int vsub, accumulate;     // pooling kernel: sub-group of this launch; add to what agg holds
 };
 

@@ -554,7 +554,9 @@ void prefill_aggregate_kernel(PrefillParams p) {
     const int Ls = p.L;                  // width of a row of pooled scores
     const int Lq = p.Lq;
     int blk, g, b;
-    unit_of_workgroup(p.B, p.G, p.T, blk, g, b);
+    unit_of_workgroup(p.B, p.G, p.T * p.key_parts, blk, g, b);
+    const int part = blk / p.T;          // part 0 of every tile first, long tiles first within a part
+    blk -= part * p.T;
     int q_start, Lqv;                    // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
     const int L = q_start + Lqv;         // keys of this sequence
@@ -570,24 +572,9 @@ void prefill_aggregate_kernel(PrefillParams p) {
     const half_t neg_inf = (half_t)(-INFINITY);
 
     const int ntiles = tl < Lqv ? (ts + kAggKT - 1) / kAggKT : 0;   // a tile past the sequence's rows pools nothing
-    if (ntiles > 0) {
-        // A operands: row block rb = head slot rb of this launch's sub-group, row li = query tl+li
+    const int ti0 = part * p.part_tiles, ti1 = min(ntiles, ti0 + p.part_tiles);   // this workgroup's key tiles
+    if (ti0 < ti1) {
         const int head0 = g * hs.gs + 4 * p.vsub;
-        x8_t qa[kGroupSize][kKS];
-#pragma unroll
-        for (int rb = 0; rb < kGroupSize; ++rb) {
-            const int q = tl + li;
-            const bool ok = q < Lqv;
-            const T* qp = Qp + (long long)b * p.q_sb + (long long)min(q, Lqv - 1) * p.q_sl +
-                          (long long)min(head0 + rb, g * hs.gs + hs.gs - 1) * p.q_sh + lg * 8;
-#pragma unroll
-            for (int ks = 0; ks < kKS; ++ks) {
-                PackT<T> x;
-                x.u = ld_global_16(qp + ks * 16);
-                if (!ok) x.u = uint4_t{0, 0, 0, 0};
-                qa[rb][ks] = x.v8;
-            }
-        }
         if (tid < 128) {
             const int q = tl + (tid & 31);
             // a query row past the chunk, or a slot past the KV head's last query head, adds exp2(-inf) = 0
@@ -624,22 +611,47 @@ void prefill_aggregate_kernel(PrefillParams p) {
                           (lchunk ^ swz<D>(row)) * 8;
             load_to_lds_16(gp, lds_w + buf * (4 * kWaveElems * 2) + j * 1024);
         };
-        fetch_page(0);
+        // The tile's Q rows, head slot `wave` of the sub-group by this wavefront: whole rows into the
+        // other buffer, chunks permuted like the keys' (fragments read from memory directly, every
+        // wavefront all four heads, 16 bytes of 32 rows per instruction, held every workgroup up at its start:
+        // 32/8 heads, 512 tokens 13.1 -> 10.4 us, 1024 18.9 -> 16.2, 2048 35.5 -> 28.9, 4096 87 -> 84).
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int row = j * kRPL + lrow;
+            const T* qp = Qp + (long long)b * p.q_sb + (long long)min(tl + row, Lqv - 1) * p.q_sl +
+                          (long long)min(head0 + wave_u, g * hs.gs + hs.gs - 1) * p.q_sh;
+            load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_w + ((ti0 + 1) & 1) * (4 * kWaveElems * 2) + j * 1024);
+        }
+        fetch_page(ti0);
         pg_cur = pg_next;
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) issue_load(0, j, 0);
-        if (ntiles > 1) fetch_page(1);
+        for (int j = 0; j < kLoads; ++j) issue_load(ti0, j, ti0 & 1);
+        if (ti0 + 1 < ti1) fetch_page(ti0 + 1);
         const int kx = lg ^ swz<D>(li);
-        __syncthreads();   // s_lse
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // own rows have landed
+        __syncthreads();                                   // everybody's, and s_lse
+        // A operands: row block rb = head slot rb, row li = query tl + li
+        x8_t qa[kGroupSize][kKS];
+        const T* sQ = sK + ((ti0 + 1) & 1) * (4 * kWaveElems);
+#pragma unroll
+        for (int rb = 0; rb < kGroupSize; ++rb)
+#pragma unroll
+            for (int ks = 0; ks < kKS; ++ks) {
+                PackT<T> x;
+                x.v8 = *reinterpret_cast<const x8_t*>(&sQ[rb * kWaveElems + li * D + ((2 * ks) ^ kx) * 8]);
+                if (tl + li >= Lqv) x.u = uint4_t{0, 0, 0, 0};
+                qa[rb][ks] = x.v8;
+            }
+        __syncthreads();   // the other buffer takes the next tile's keys from here on
 
-        for (int ti = 0; ti < ntiles; ++ti) {
+        for (int ti = ti0; ti < ti1; ++ti) {
             // this tile's rows have landed (and the next tile's block-table entries arrived)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             const T* bK = my_k + (ti & 1) * (4 * kWaveElems);
-            const int tn = min(ti + 1, ntiles - 1);   // after the last tile: its rows once more, unused
+            const int tn = min(ti + 1, ti1 - 1);   // after the last tile: its rows once more, unused
             const int nbuf = (ti + 1) & 1;
             pg_cur = pg_next;
-            if (ti + 2 < ntiles) fetch_page(ti + 2);
+            if (ti + 2 < ti1) fetch_page(ti + 2);
 
             float16_t acc[kGroupSize];
             float16_t zero16;   // the first product of a tile starts from a constant zero
@@ -687,7 +699,8 @@ void prefill_aggregate_kernel(PrefillParams p) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
     }
     if (p.fill_invalid) {
-        for (int key = ntiles * kAggKT + tid; key < Ls; key += kThreads) out[key] = neg_inf;
+        const int end = part == p.key_parts - 1 ? Ls : min(Ls, (ti0 + p.part_tiles) * kAggKT);
+        for (int key = max(ntiles, ti0) * kAggKT + tid; key < end; key += kThreads) out[key] = neg_inf;
     }
 }
 
@@ -735,9 +748,9 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
 
 template <int D, typename T>
 hipError_t launch_aggregate_t(const PrefillParams& p, hipStream_t stream) {
-    dim3 grid(p.T, p.G, p.B), block(kThreads);
+    dim3 grid(p.T * p.key_parts, p.G, p.B), block(kThreads);
     if (pairs_fill_xcds(p.B, p.G)) {
-        const long long total = (long long)p.T * p.G * p.B;
+        const long long total = (long long)p.T * p.key_parts * p.G * p.B;
         if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
         grid = dim3((unsigned)total);
     }
@@ -765,6 +778,17 @@ hipError_t launch_prefill_aggregate(const PrefillParams& p0, hipStream_t stream)
     // pooled scores (launches on a stream run in order)
     PrefillParams p = p0;
     const int subs = head_slots(p.gs).subs;
+    // A key's pooled score needs no other key, so a query tile's keys can be cut into parts for
+    // workgroups of their own.  They are where the tiles' workgroups are all resident at once (two on
+    // each of 256 compute units): then the longest is the time, and small calls leave units idle.  Parts
+    // for about four workgroups per unit, of at least four key tiles: a workgroup's start (Q through
+    // LDS, first rows) costs as much as two or three.  32/8 heads: 1024 tokens 16.2 -> 11.9 us,
+    // 2048 28.9 -> 26.0; with 752 units (3001 tokens) two parts 48.6 -> 50.2.
+    const long long units = (long long)p.B * p.G * p.T;
+    const int max_tiles = std::max(1, (p.q_start + kTile * (p.T - 1) + kAggKT - 1) / kAggKT);
+    const int want = units <= 512 ? (int)((1024 + units - 1) / units) : 1;
+    p.part_tiles = std::max((max_tiles + want - 1) / want, std::min(4, max_tiles));
+    p.key_parts = (max_tiles + p.part_tiles - 1) / p.part_tiles;
     for (int v = 0; v < subs; ++v) {
         p.vsub = v;
         p.accumulate = v > 0;

@@ -19,3 +19,31 @@ def test_log_sums_on_both_sides_of_the_unit_size(cuda, B, L):
     _, want = orc.dense_prefill(q, k, k)
     got = kernels.prefill_recompute1(q.to(cuda).repeat(B, 1, 1, 1), k.to(cuda).repeat(B, 1, 1, 1))
     assert_close(got, want.repeat(B, 1, 1), f"log_sum {B}x{L}", atol=2e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("L", [33, 129, 517, 897, 1300, 2048, 2049])
+@pytest.mark.parametrize("heads,G,D", [(32, 8, 128), (28, 4, 64)])
+def test_pooled_scores_do_not_depend_on_the_key_parts(cuda, L, heads, G, D):
+    """Small calls cut a tile's keys into parts, a batch of copies of the same prompt does not: the same
+    bits, the invalid positions' fill included, and the oracle's scores to fp16 rounding."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(L + D)
+    q = torch.randn(1, L, heads, D, generator=gen).half()
+    k = torch.randn(1, L, G, D, generator=gen).half()
+    T, B = (L + 31) // 32, 512 // (G * ((L + 31) // 32)) + 1
+    log_sum = kernels.prefill_recompute1(q.to(cuda), k.to(cuda))
+
+    def pooled(n):
+        qd, kd = q.to(cuda).repeat(n, 1, 1, 1), k.to(cuda).repeat(n, 1, 1, 1)
+        out = torch.full((n, G, T, L), 7.0, device=cuda, dtype=torch.float16)
+        kernels.prefill_aggregate(qd, kd, log_sum.repeat(n, 1, 1), out, fill_invalid=True)
+        return out
+    one, many = pooled(1), pooled(B)
+    assert all(torch.equal(one[0], m) for m in many)
+    if L <= 1300:
+        want = orc.pooled_prefill_scores(q, k, 32).reshape(G, T, L).float()
+        keys = torch.arange(L).view(1, 1, L) < 32 * torch.arange(T).view(1, T, 1)
+        got = one[0].float().cpu()
+        assert bool((got[~keys.expand_as(got)] == -float("inf")).all())
+        # an fp16 rounding of the sum plus the fp32 noise of 128 exponentials
+        assert_close(got[keys.expand_as(got)], want[keys.expand_as(want)], "pooled scores", atol=1e-4, rtol=2e-3)
