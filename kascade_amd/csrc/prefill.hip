@@ -88,7 +88,9 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
-    unit_of_workgroup(p.B, p.G * hs.subs, nqt, blk, g, b);   // g: KV head and sub-group
+    // resident per compute unit: two with V (64 KB of LDS, 256 registers), K only by the registers
+    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : PAGED ? 3 : 4;
+    unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
     const int L = q_start + Lqv;    // keys of this sequence
@@ -554,7 +556,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
     const int Ls = p.L;                  // width of a row of pooled scores
     const int Lq = p.Lq;
     int blk, g, b;
-    unit_of_workgroup(p.B, p.G, p.T * p.key_parts, blk, g, b);
+    unit_of_workgroup(p.B, p.G, p.T * p.key_parts, 2, blk, g, b);
     const int part = blk / p.T;          // part 0 of every tile first, long tiles first within a part
     blk -= part * p.T;
     int q_start, Lqv;                    // this sequence's first position and how many of the rows are its own
