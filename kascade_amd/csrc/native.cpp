@@ -111,6 +111,8 @@ int num_split(double total_rows, double max_rows, double cap_rows, double min_ro
     return (int)std::max(1.0, std::min(256.0, std::nearbyint(max_rows / per)));
 }
 constexpr double kGatherRowsPerSplit = 1664;
+// kernels.gather_lone_rows (see there)
+int64_t gather_lone_rows(const kascade_shape& s) { return s.group_size <= 4 ? 384 : 512; }
 constexpr int kFusedMergeMaxSplits = 32;
 
 // Arrival counters of the fused split merge: zero when made, and zero again after every launch, so
@@ -194,7 +196,7 @@ const at::Tensor& head_map(PyObject* o, int64_t groups) {
 void hf_reuse(const HfTensors& h, const at::Tensor& idx, const at::Tensor& hm, PyObject* counters, const at::Tensor& out,
               int device, void* stream) {
     const int64_t topk = idx.size(-1);
-    const int ns = num_split((double)h.B * h.G * topk, (double)topk, kGatherRowsPerSplit);
+    const int ns = topk <= gather_lone_rows(h.shape) ? 1 : num_split((double)h.B * h.G * topk, (double)topk, kGatherRowsPerSplit);
     const int64_t parts = (h.B * h.H * ns + 63) / 64 * 64;
     const at::Tensor scratch = empty_like_type({parts + h.B * h.H * ns * h.D}, h.q, at::kFloat);
     at::Tensor sync;

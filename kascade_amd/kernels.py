@@ -93,8 +93,20 @@ def _blhd_strides(t: torch.Tensor, name: str) -> Strides:
 GATHER_ROWS_PER_SPLIT = 1664
 
 
+def gather_lone_rows(group_size: int) -> int:
+    """Longest list a gather launch takes in one split per (sequence, KV head).  A lone split writes its
+    result itself; merging several costs about 3 us (partial results through device-coherent memory,
+    a counter, the way back), as much as 256 rows more in one workgroup, and more with more query
+    heads.  Us per launch, one split against the best of several: 32/8 heads, batch 1, 256 rows
+    6.9 / 8.0, 384 rows 8.2 / 8.4, 512 rows 9.5 / 8.5; batch 8, 384 rows 9.4 / 9.8, 512 rows 11.0 / 10.5;
+    batch 16, 384 rows 10.8 / 12.0.  64/8 heads, batch 8: 384 rows 9.9 / 11.6, 512 rows 11.5 / 12.3, 640 rows
+    13.3 / 13.2."""
+    return 384 if group_size <= 4 else 512
+
+
 def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_rows: int = 512,
-                      cap_rows: Optional[int] = None, row_counts=None, heads: int = G) -> int:
+                      cap_rows: Optional[int] = None, row_counts=None, heads: int = G,
+                      lone_rows: int = 0) -> int:
     """Split count for a decode launch.  Every split covers the same number of rows
     (ceil(max_rows/num_split)), so the number of non-empty workgroups is about
     total_rows / rows_per_split; aim at wgs_per_cu of them per compute unit without
@@ -104,7 +116,10 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
     GATHER_ROWS_PER_SPLIT rows: twice that is 1-3 % faster on uniform batches (batch 16 x 26240
     rows: 307 us against 316 us) but 6 % slower on the ragged batch of four long sequences
     (109 us against 103 us); the streaming kernels do not care.
-    row_counts: the rows of every sequence (per KV head), when the caller knows them."""
+    row_counts: the rows of every sequence (per KV head), when the caller knows them.
+    lone_rows: lists of up to that many rows are one split (gather launches: gather_lone_rows)."""
+    if max_rows <= lone_rows:
+        return 1
     cus = _lib.init().kascade_device_cu_count() or 256
     target_wgs = wgs_per_cu * cus
     if row_counts is not None and len(row_counts) > 1 and total_rows / max(min_rows, 1) >= cus:

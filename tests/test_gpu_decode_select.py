@@ -116,3 +116,22 @@ def test_split_strips_and_direct_output(cuda, seqlens, ns):
                 assert_close(o, want, "anchor-0 output")
         if sync is not None:
             assert int(sync.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("heads,tokens", [(32, 3849), (32, 3850), (64, 5129), (64, 5130)])
+def test_lists_on_both_sides_of_the_lone_split(cuda, heads, tokens):
+    """Lists of 384 (512 from five query heads per KV head on) rows are gathered by one workgroup per
+    KV head, longer ones by several: a reuse layer against the oracle on the anchor's own lists."""
+    from types import SimpleNamespace
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    G, D = 8, 128
+    gen = torch.Generator().manual_seed(tokens)
+    q = torch.randn(2, heads, 1, D, generator=gen).half()
+    k, v = (torch.randn(2, G, tokens, D, generator=gen).half() for _ in range(2))
+    s = EfficientKascadeStrategy([0], None, k=10, tile_size=32, head_mapping=[list(range(G)), [3] * G], register=False)
+    for layer in (0, 1):
+        o, _ = s.attention_forward(SimpleNamespace(layer_idx=layer), q.to(cuda), k.to(cuda), v.to(cuda), None, D ** -0.5)
+    idx = s._topk_to_reuse.cpu()
+    assert idx.shape[-1] == (384 if heads == 32 else 512) + (0 if tokens % 2 else 128)
+    want = orc.reuse_decode(q[:, :, 0], k.transpose(1, 2), v.transpose(1, 2), idx, [3] * G, [idx.shape[-1]] * 2)
+    assert_close(o[:, 0], want, "reuse output")

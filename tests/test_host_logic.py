@@ -187,3 +187,13 @@ def test_workloads_are_seeded_and_shaped():
     assert sorted(used) == list(range(10))
     kc = orc.paged_to_contiguous(p.k_pages, p.block_table, [100, 37])
     assert torch.equal(kc[1, 5], p.k_pages[p.block_table[1, 0], 5])
+
+
+@pytest.mark.parametrize("group,limit", [(1, 384), (4, 384), (5, 512), (16, 512)])
+def test_short_gather_lists_are_one_split(group, limit):
+    from kascade_amd import kernels
+    lone = kernels.gather_lone_rows(group)
+    assert lone == limit
+    # no device query below the limit; the general rule has the say above it
+    assert kernels.default_num_split(8 * limit, limit, lone_rows=lone) == 1
+    assert kernels.default_num_split(8 * 16 * 128, 128, row_counts=[128] * 16, lone_rows=lone) == 1
