@@ -1012,7 +1012,13 @@ int prefill_chunk_dense_impl(const Shape& sh, const kascade_half* Q, const kasca
         return -1;
     p.K = E(K_pages); p.V = with_output ? E(V_pages) : E(K_pages);
     p.log_sum = log_sum; p.O = E(Output);
-    return check_hip(launch_prefill_attn(p, false, with_output != 0, 1,
+    // 64 queries per wavefront in the K-only pass as for whole prompts, and from 512 units on (two per
+    // compute unit) where the chunk's units are about equally long: 4096 queries of 32/8 heads at
+    // position 12288 567 -> 489 us, 6144 334 -> 294; at position 0 87 -> 98, and 2048 queries (256 units)
+    // at 12288 261 -> 293, so those keep 32.
+    const long long units64 = (long long)((q_len + 63) / 64) * sh.G * ((sh.gs + 3) / 4) * batch;
+    const int nqb = (with_output || sh.D != 128 || units64 < 512 || (units64 == 512 && q_start < q_len)) ? 1 : 2;
+    return check_hip(launch_prefill_attn(p, false, with_output != 0, nqb,
                                          static_cast<hipStream_t>(stream)), "prefill_chunk_dense");
 }
 

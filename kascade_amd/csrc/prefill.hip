@@ -517,11 +517,11 @@ void prefill_attn_kernel_q32(PrefillParams p) {
 // workgroups per compute unit, and the MFMA results stay in ordinary registers (with the full
 // 512-register budget the compiler parks them in accumulation registers and copies each one out
 // before the softmax).
-template <int D, typename T>
+template <bool PAGED, int D, typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_attn_kernel_q64(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
-    prefill_attn_body<2, false, false, false, D, T>(p, sK, static_cast<T*>(nullptr));
+    prefill_attn_body<2, false, false, PAGED, D, T>(p, sK, static_cast<T*>(nullptr));
 }
 
 // Pooled tile scores: out[b,g,t,key] = sum over the 32 queries of tile t and the 4 q-heads of g
@@ -727,6 +727,13 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, true, D, T, true>), grid, block, 0, stream, p);
         else
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, false, D, T, true>), grid, block, 0, stream, p);
+    } else if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
+        if constexpr (D == 128) {
+            if (paged) hipLaunchKernelGGL((prefill_attn_kernel_q64<true, D, T>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((prefill_attn_kernel_q64<false, D, T>), grid, block, 0, stream, p);
+        } else {
+            return hipErrorInvalidValue;
+        }
     } else if (paged) {
         if (reuse)
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, true, D, T>), grid, block, 0, stream, p);
@@ -736,9 +743,6 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
             hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, true, D, T>), grid, block, 0, stream, p);
     } else if (reuse) {
         hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, false, D, T>), grid, block, 0, stream, p);
-    } else if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
-        if constexpr (D == 128) hipLaunchKernelGGL((prefill_attn_kernel_q64<D, T>), grid, block, 0, stream, p);
-        else return hipErrorInvalidValue;
     } else {
         if (with_v)
             hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, false, D, T>), grid, block, 0, stream, p);
@@ -785,7 +789,8 @@ hipError_t launch_prefill_aggregate(const PrefillParams& p0, hipStream_t stream)
     // each of 256 compute units): then the longest is the time, and small calls leave units idle.  Parts
     // for about four workgroups per unit, of at least four key tiles: a workgroup's start (Q through
     // LDS, first rows) costs as much as two or three.  32/8 heads: 1024 tokens 16.2 -> 11.9 us,
-    // 2048 28.9 -> 26.0; with 752 units (3001 tokens) two parts 48.6 -> 50.2.
+    // 2048 28.9 -> 26.0, chunks at position 12288 of 512 queries 159 -> 70, of 1024 168 -> 127, of 2048
+    // 250 -> 251; with 752 units (3001 tokens) two parts 48.6 -> 50.2.
     const long long units = (long long)p.B * p.G * p.T;
     const int max_tiles = std::max(1, (p.q_start + kTile * (p.T - 1) + kAggKT - 1) / kAggKT);
     const int want = units <= 512 ? (int)((1024 + units - 1) / units) : 1;

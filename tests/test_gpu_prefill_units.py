@@ -47,3 +47,30 @@ def test_pooled_scores_do_not_depend_on_the_key_parts(cuda, L, heads, G, D):
         assert bool((got[~keys.expand_as(got)] == -float("inf")).all())
         # an fp16 rounding of the sum plus the fp32 noise of 128 exponentials
         assert_close(got[keys.expand_as(got)], want[keys.expand_as(want)], "pooled scores", atol=1e-4, rtol=2e-3)
+
+
+@pytest.mark.parametrize("B,n,start", [(16, 256, 256), (16, 250, 256), (16, 256, 0), (17, 225, 96)])
+def test_chunk_log_sums_do_not_depend_on_the_unit_size(cuda, B, n, start):
+    """A chunk's log-sums over the paged cache, in a batch large enough for 64 queries per wavefront
+    and alone (32 per wavefront): the same bits, and the oracle's values."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(n)
+    L, page = start + n, 16
+    q = torch.randn(1, L, 32, 128, generator=gen).half()
+    k = torch.randn(1, L, 8, 128, generator=gen).half()
+    per = (L + page - 1) // page
+    pages = torch.zeros(per * page, 8, 128, dtype=torch.float16)
+    pages[:L] = k[0]
+    order = torch.randperm(per, generator=gen)
+    kp = torch.empty(per, page, 8, 128, dtype=torch.float16)
+    kp[order] = pages.view(per, page, 8, 128)
+    kp = kp.to(cuda)
+
+    def log_sum(b):
+        table = order.to(torch.int32).repeat(b, 1).to(cuda)
+        return kernels.prefill_chunk_dense(q[:, start:].repeat(b, 1, 1, 1).to(cuda), kp, kp, table, start,
+                                           page_size=page, with_output=False)[0]
+    one, many = log_sum(1), log_sum(B)
+    assert all(torch.equal(one[0], m) for m in many)
+    _, want = orc.dense_prefill(q, k, k)
+    assert_close(one, want[:, start:], "chunk log_sum", atol=2e-3, rtol=1e-4)
