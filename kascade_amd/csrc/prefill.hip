@@ -655,39 +655,45 @@ void prefill_aggregate_kernel(PrefillParams p) {
             pg_cur = pg_next;
             if (ti + 2 < ti1) fetch_page(ti + 2);
 
-            float16_t acc[kGroupSize];
-            float16_t zero16;   // the first product of a tile starts from a constant zero
+            // Head by head, the exponentials of one head's scores between the matrix instructions of the
+            // next head's: a wavefront's vector and matrix work overlap within itself, which counts where
+            // few wavefronts share a SIMD (512 tokens 10.1 -> 9.1 us, 1024 12.0 -> 10.7; 32768 4.56 -> 4.44
+            // ms, where the clock follows the power limit).  Two heads' scores are live instead of four,
+            // which makes room for the tile's eight key operands.
+            float16_t acc[2];
+            float16_t zero16;   // the first product of a head starts from a constant zero
 #pragma unroll
             for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
-            auto read_b = [&](int ks) {
-                return *reinterpret_cast<const x8_t*>(&bK[li * D + ((2 * ks) ^ kx) * 8]);
+            x8_t kb[kKS];
+#pragma unroll
+            for (int ks = 0; ks < kKS; ++ks) kb[ks] = *reinterpret_cast<const x8_t*>(&bK[li * D + ((2 * ks) ^ kx) * 8]);
+            float4_t ls[4];   // log-sums of the rows of the head whose exponentials are next
+            float sum = 0.f;
+            // accumulator v of head rb is query row 8(v/4) + 4lg + v%4, column = key li
+            auto exponentials = [&](const float16_t& s, int v0, int v1) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (v >= v0 && v < v1) sum += fast_exp2(s[v] * kScaleLog2 - ls[v >> 2][v & 3]);
             };
-            x8_t kb[3];
-            kb[0] = read_b(0);
-            if (kKS > 1) kb[1] = read_b(1);
 #pragma unroll
-            for (int ks = 0; ks < kKS; ++ks) {
-                if (ks + 2 < kKS) kb[(ks + 2) % 3] = read_b(ks + 2);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int rb = 0; rb < kGroupSize; ++rb) {
 #pragma unroll
-                for (int rb = 0; rb < kGroupSize; ++rb)
-                    acc[rb] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks % 3], ks == 0 ? zero16 : acc[rb]);
-                if (ks < kLoads) issue_load(tn, ks, nbuf);
+                for (int ks = 0; ks < kKS; ++ks) {
+                    acc[rb & 1] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks], ks == 0 ? zero16 : acc[rb & 1]);
+                    if (rb == 0 && ks < kLoads) issue_load(tn, ks, nbuf);
+                    if (rb > 0 && ks > 0) exponentials(acc[(rb - 1) & 1], 16 * (ks - 1) / (kKS - 1), 16 * ks / (kKS - 1));
+                    if (ks == kKS - 1) {
+#pragma unroll
+                        for (int v4 = 0; v4 < 4; ++v4)
+                            ls[v4] = *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 8 * v4 + 4 * lg]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
 #pragma unroll
             for (int j = kKS; j < kLoads; ++j) issue_load(tn, j, nbuf);
-            // accumulator v of row block rb is query row 8(v/4) + 4lg + v%4, column = key li
             tile_phase<KASCADE_PRIO_AGG>(1);
-            float sum = 0.f;
-#pragma unroll
-            for (int rb = 0; rb < kGroupSize; ++rb)
-#pragma unroll
-                for (int v4 = 0; v4 < 4; ++v4) {
-                    const float4_t ls = *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 8 * v4 + 4 * lg]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        sum += fast_exp2(acc[rb][4 * v4 + e] * kScaleLog2 - ls[e]);
-                }
+            exponentials(acc[(kGroupSize - 1) & 1], 0, 16);
             sum = sum_with_other_half(sum);
             tile_phase<KASCADE_PRIO_AGG>(2);
             const int key = ti * kAggKT + 32 * wave + li;
