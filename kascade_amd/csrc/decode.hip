@@ -388,7 +388,7 @@ void decode_split_kernel(DecodeParams p) {
                 *reinterpret_cast<uint2*>(&s_code[col][prow + 16 * j + 4 * dq]) =
                     make_uint2(q[0] | (q[1] << 16), q[2] | (q[3] << 16));
             }
-            if (dq == 0) s_ref[col][prow >> 6] = base * kScaleLog2;
+            if (dq == 0) s_ref[col][prow >> 6] = mx * kScaleLog2;   // -inf where the whole granule is masked
         }
     };
     // The codes of phase `ph` (tokens [ph * kPhaseRows, +kPhaseRows) of the range) leave in one

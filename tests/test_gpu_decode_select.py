@@ -135,3 +135,36 @@ def test_lists_on_both_sides_of_the_lone_split(cuda, heads, tokens):
     assert idx.shape[-1] == (384 if heads == 32 else 512) + (0 if tokens % 2 else 128)
     want = orc.reuse_decode(q[:, :, 0], k.transpose(1, 2), v.transpose(1, 2), idx, [3] * G, [idx.shape[-1]] * 2)
     assert_close(o[:, 0], want, "reuse output")
+
+
+@pytest.mark.parametrize("H,G,L", [(32, 8, 2100), (8, 8, 700), (16, 1, 4200)])
+@pytest.mark.parametrize("level", [0.0, -30.0, -45.0, -55.0])
+def test_masked_scores_pool_to_nothing_in_one_call(cuda, H, G, L, level):
+    """Tokens whose score is -inf for every head (a key with an infinite component): whole granules of 64,
+    parts of some, a whole sequence -- while the other scores lie near ``level`` (log2 domain), so that a
+    masked token's share must be 0 and not the least the score codes express.  Exactly the selection
+    over the scores that the two-launch route pools; a masked token goes after every token above 0."""
+    from kascade_amd import _lib, budgets, kernels
+    D, B = 128, 2
+    gen = torch.Generator().manual_seed(L)
+    q = 1 + 0.1 * torch.randn(B, H, 1, D, generator=gen)
+    k = level / (D ** 0.5 * orc.LOG2E) + 0.2 * torch.randn(B, G, L, D, generator=gen)
+    masked = torch.zeros(B, L, dtype=torch.bool)
+    masked[0, 64:192] = masked[0, 300:500] = masked[0, L - 70:] = True
+    masked[1] = True
+    k[..., 5][masked[:, None].expand(B, G, L)] = -float("inf")
+    q, k = q.half().to(cuda), k.half().to(cuda)
+    v = torch.randn(B, G, L, D, generator=gen).half().to(cuda)
+    width = budgets.topk_width(L, 10)
+    same = torch.arange(G, device=cuda, dtype=torch.int32)
+    ns, stride = 3, (L + 7) // 8 * 8
+    glse, part = torch.empty(B, H, ns, device=cuda), torch.empty(B, H, ns, D, device=cuda)
+    sums, scores = torch.empty(B, H, device=cuda), torch.empty(B, H, stride, device=cuda)
+    native = _lib.native()
+    for layer in (0, 1):
+        _, agg = kernels.decode_recompute(q[:, :, 0], k.transpose(1, 2), v.transpose(1, 2), glse, part, sums, scores, layer)
+        assert bool((agg[:, :, :L][masked[:, None].expand(B, G, L).to(cuda)] == 0).all())
+        want = kernels.topk_indices(agg[:, :, :L], width, fill_value=0)
+        _, idx = native.hf_decode_anchor(native.Counters(), q, k, v, layer == 0, width, same)
+        assert torch.equal(idx, want), f"layer {layer}"
+        assert not bool(masked[0][idx[0].cpu().long()].any())
