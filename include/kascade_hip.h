@@ -254,15 +254,18 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
 /* An anchor pass and the selection over its pooled scores in one call: what
  * kascade_decode_recompute_paged_shaped_call followed by kascade_topk_rows_call gives, without the
  * pooled scores as a result.  shape == NULL: the reference's.  Rows of up to
- * KASCADE_POOL_SELECT_ROW tokens are pooled and selected in one launch and need neither
+ * KASCADE_POOL_SELECT_ROW tokens can be pooled and selected in one launch and need neither
  * aggregated_scores, valid_len, n_sel nor workspace (all may be NULL); longer rows need
  * aggregated_scores [B,G,scores_stride] f16, with topk_percent > 0 also valid_len and n_sel [B*G]
  * (kascade_decode_budgets_call), and take the workspace of kascade_topk_workspace_bytes(B*G, row_len).
+ * kascade_pool_select_row(group_size, B*G): the longest row for which one launch is also the faster
+ * way.  Beyond it a caller that gives these buffers gets two launches; the results are the same.
  *   out_idx  [B,G,k] i32 token positions; out_rows [B,G,k] i32 the same as cache rows, or NULL
  *   row_len  longest row, in tokens
  *   topk_percent > 0: sequence b selects 128*ceil(floor(percent*len_b/100)/128) of its len_b tokens
  *   (at most k; slots beyond hold fill_value); 0: k of row_len everywhere */
 #define KASCADE_POOL_SELECT_ROW 32768
+int kascade_pool_select_row(int group_size, int rows);
 int kascade_decode_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K,
                                     const kascade_half* V, const int32_t* cache_seqlens, float* glse,
                                     float* Output_partial, float* row_sums, float* scores, kascade_half* Output,

@@ -170,7 +170,7 @@ int set_append(DecodeParams& p, const kascade_half* k_new, const kascade_half* v
 
 extern "C" {
 
-int kascade_abi_version(void) { return 11; }
+int kascade_abi_version(void) { return 12; }
 
 const char* kascade_get_last_error(void) { return g_err; }
 
@@ -418,6 +418,7 @@ int kascade_decode_dense_paged_shaped_call(const kascade_shape* shape, const kas
 namespace {
 // The selection that follows an anchor pass in the same call.
 struct AnchorSelect {
+    bool one_launch;           // pooling and selection together
     int32_t* out_idx;
     const TopkRows* rows;      // or null
     int row_len, k, fill;
@@ -458,7 +459,7 @@ int decode_recompute_paged_impl(const Shape& sh, const kascade_half* Q, const ka
                                         const kascade_strides* kv_strides,
                                         const kascade_half* k_new, const kascade_half* v_new,
                                         int32_t* sync_counters, const AnchorSelect* sel, void* stream) {
-    REQUIRE(Q && K && glse && row_sums && scores && (aggregated_scores || (sel && sel->row_len <= KASCADE_POOL_SELECT_ROW)),
+    REQUIRE(Q && K && glse && row_sums && scores && (aggregated_scores || (sel && sel->one_launch)),
             "decode_recompute: null pointer argument");
     REQUIRE(!with_output || (V && Output && Output_partial),
             "decode_recompute: with_output needs V, Output and Output_partial");
@@ -501,7 +502,7 @@ int decode_recompute_paged_impl(const Shape& sh, const kascade_half* Q, const ka
         return -1;
     const float* parts = with_output ? nullptr : glse;   // log-sums still to be merged
     const TopkRows no_rows{};
-    if (sel && sel->row_len <= KASCADE_POOL_SELECT_ROW) {
+    if (sel && sel->one_launch) {
         DecodePoolParams pp{};
         pp.scores = scores; pp.glse = parts; pp.row_sums = row_sums; pp.seqlens = cache_seqlens;
         pp.num_split = num_split; pp.groups = sh.G; pp.group_size = sh.gs; pp.scores_stride = scores_stride;
@@ -551,6 +552,22 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
     return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, nullptr, stream);
 }
 
+// One workgroup pools a row's tokens for all query heads of its KV head, four heads at a time, where a
+// launch of its own spreads them over the chip: the saved launch (2 to 4 us) stops paying as tokens
+// and heads grow, sooner for groups that fill no whole four heads.  Us of an anchor pass without
+// output, one launch / two, 8 KV heads, batch 1:
+//   tokens   1 head    2          4          5          8          12         16 heads per KV head
+//   8192     13.6/15.3 14.3/16.7  15.0/18.6  17.5/20.6  18.0/23.5  21.0/27.4  23.5/31.8
+//   18432    23.4/24.9 23.4/25.6  24.4/27.8  29.2/29.3  29.3/32.3  34.4/36.2  39.3/40.6
+//   20480    25.7/25.5 25.4/26.6  26.5/28.4  32.3/29.4  32.6/33.1  38.4/37.0  44.2/42.1
+//   24576    26.0/26.3 27.4/27.5  27.4/29.5  33.0/31.4  33.7/34.2  39.0/38.0  45.0/42.4
+//   32768    31.0/28.8 32.6/30.7  32.7/32.4  39.4/35.0  40.5/37.8  47.2/40.9  55.0/46.1
+// With many rows the selections fill the chip by themselves: batch 8, 24576 tokens 81.9/85.8 with 2
+// heads, 95.7/98.4 with 8, 118.5/120.6 with 16; 32768 110.6/109.0, 132.3/132.8, 166.3/165.4.
+int kascade_pool_select_row(int group_size, int rows) {
+    return group_size == 3 || group_size == 4 || rows >= 64 ? 24576 : 18432;
+}
+
 int kascade_decode_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K,
                                     const kascade_half* V, const int32_t* cache_seqlens, float* glse,
                                     float* Output_partial, float* row_sums, float* scores, kascade_half* Output,
@@ -566,9 +583,10 @@ int kascade_decode_anchor_topk_call(const kascade_shape* shape, const kascade_ha
     REQUIRE(k > 0 && row_len > 0 && row_len <= scores_stride, "decode_anchor_topk: k > 0 and 0 < row_len <= scores_stride required");
     REQUIRE(!(topk_percent > 0.f) || cache_seqlens, "decode_anchor_topk: topk_percent needs cache_seqlens");
     REQUIRE((long long)batch * sh.G < (1LL << 31), "decode_anchor_topk: too many rows");
-    const bool one = row_len <= KASCADE_POOL_SELECT_ROW;
-    REQUIRE(one || aggregated_scores, "decode_anchor_topk: rows of more than %d tokens need aggregated_scores", KASCADE_POOL_SELECT_ROW);
-    REQUIRE(one || !(topk_percent > 0.f) || (valid_len && n_sel),
+    const bool fits = row_len <= KASCADE_POOL_SELECT_ROW;
+    REQUIRE(fits || aggregated_scores, "decode_anchor_topk: rows of more than %d tokens need aggregated_scores", KASCADE_POOL_SELECT_ROW);
+    const bool counted = !(topk_percent > 0.f) || (valid_len && n_sel);   // what a selection of its own needs is there
+    REQUIRE(fits || counted,
             "decode_anchor_topk: rows of more than %d tokens need valid_len and n_sel", KASCADE_POOL_SELECT_ROW);
     TopkRows tr{};
     if (out_rows) {
@@ -580,6 +598,7 @@ int kascade_decode_anchor_topk_call(const kascade_shape* shape, const kascade_ha
         tr.page_shift = shift; tr.rows_per_seq = sh.G;
     }
     AnchorSelect sel{};
+    sel.one_launch = fits && (row_len <= kascade_pool_select_row(sh.gs, batch * sh.G) || !aggregated_scores || !counted);
     sel.out_idx = out_idx; sel.rows = &tr; sel.row_len = row_len; sel.k = k; sel.fill = fill_value;
     sel.topk_percent = topk_percent; sel.valid_len = valid_len; sel.n_sel = n_sel; sel.workspace = workspace;
     return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output,

@@ -249,7 +249,7 @@ PyObject* hf_decode_anchor(PyObject* const* a) {
     float *part = lse + n_lse, *sums = part + n_part, *scores = sums + n_sums;
     const int64_t ws_bytes = kascade_topk_workspace_bytes((int)(h.B * h.G), h.L);
     at::Tensor agg, ws, sync;
-    if (h.L > KASCADE_POOL_SELECT_ROW) {   // rows that more than one workgroup selects
+    if (h.L > kascade_pool_select_row(h.shape.group_size, (int)(h.B * h.G))) {   // pooled and selected in two launches
         agg = empty_like_type({h.B, h.G, stride}, h.q, at::kHalf);
         if (ws_bytes > 0) ws = empty_like_type({ws_bytes}, h.q, at::kByte);
     }
@@ -428,7 +428,7 @@ PyObject* paged_anchor(PyObject* const* a) {
     void* stream = stream_of(device_of_caller());
     at::Tensor out, agg, ws;
     if (with_output) out = out_buffer(a[17], t);
-    if (max_len > KASCADE_POOL_SELECT_ROW) {
+    if (max_len > kascade_pool_select_row(t.shape.group_size, (int)(t.B * t.G))) {
         agg = empty_like_type({t.B, t.G, stride}, t.q, at::kHalf);
         const int64_t bytes = kascade_topk_workspace_bytes((int)(t.B * t.G), max_len);
         if (bytes > 0) ws = empty_like_type({bytes}, t.q, at::kByte);
@@ -467,6 +467,11 @@ PyObject* paged_dense(PyObject* const* a) {
     return THPVariable_Wrap(out);
 }
 
+// pool_select_row(group_size, rows): kascade_pool_select_row
+PyObject* pool_select_row(PyObject* const* a) {
+    return PyLong_FromLong(kascade_pool_select_row((int)integer(a[0]), (int)integer(a[1])));
+}
+
 // ------------------------------------------------------------------------------- module
 template <PyObject* (*F)(PyObject* const*), int N>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -486,7 +491,8 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define ENTRY(f, n) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&entry<f, n>)), METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {
     ENTRY(hf_decode_reuse, 6), ENTRY(hf_decode_anchor, 7), ENTRY(hf_prefill_reuse, 7), ENTRY(hf_prefill_anchor, 10),
-    ENTRY(paged_reuse, 16), ENTRY(paged_anchor, 22), ENTRY(paged_dense, 14), {nullptr, nullptr, 0, nullptr}};
+    ENTRY(paged_reuse, 16), ENTRY(paged_anchor, 22), ENTRY(paged_dense, 14),
+    ENTRY(pool_select_row, 2), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Per-layer host calls of the Kascade kernels.", -1, kMethods};
 

@@ -18,8 +18,7 @@ hipError_t launch_topk(const half_t* scores, int* out_idx, int rows, long long r
                        int fill, const TopkRows* tr, hipStream_t stream);
 
 // Pooling and selection of decode anchors in one launch, one workgroup per (sequence, KV head) row
-// of up to kPoolSelectRow tokens (longer rows: pooling spread over the chip, then a selection, is faster --
-// one sequence of 32768 tokens 34.1 -> 32.0 us with its scores pass, of 65536 57 -> 63.5).
+// of up to kPoolSelectRow tokens, what its registers hold (kascade_pool_select_row: where it pays).
 constexpr int kPoolSelectRow = 32768;
 struct DecodePoolParams {
     const float* scores;      // [rows, group_size, scores_stride]: score codes and references (decode.h)

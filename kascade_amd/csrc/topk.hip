@@ -601,9 +601,8 @@ void topk_select_reg_kernel(
 // into the selection's registers: no pooled row in memory, one launch instead of two (merge of the
 // log-sums included).  Masked tokens need no test of their own (one per code costs a quarter of the
 // pooling, 1.1 us at 16384 tokens of 4 heads, 3.3 of 8): see kScoreNone in decode.h.  Bound by the latency of one workgroup: its exponentials (8 per head and lane and
-// chunk) and the selection's scans; the launch pays for the few compute units it uses up to about
-// 32768 tokens.  With the scores pass, K only, one sequence of 32 / 8 heads: 2000 tokens 14.9 -> 11.9 us,
-// 8192 20.6 -> 14.9, 16384 27.3 -> 21.0, 32768 34.1 -> 32.0; 16 sequences of 4096: 38.0 -> 33.4.
+// chunk) and the selection's scans; kascade_pool_select_row has the line up to which the saved launch
+// pays for the few compute units it uses, with both sides measured.
 template <int THREADS, int MAXC>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS > 512 ? 4 : THREADS > 256 ? 2 : 1, 4)))
 void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restrict__ out, RowsOut ro) {

@@ -36,7 +36,6 @@ from ._lib import KascadeError
 H, G, D, TILE = 32, 8, 128, 32
 FUSED_MERGE_MAX_SPLITS = 32
 ANCHOR_ROWS_PER_SPLIT = 8192
-POOL_SELECT_ROW = 32768   # tokens of a decode row that one workgroup pools and selects
 
 
 def get_head_mapping(model_name: str, recompute_layers: Sequence[int],
@@ -387,7 +386,7 @@ class PagedKascadeDecoder:
         valid = nsel = None
         if ragged:
             width, pct = budgets.decode_budget(max_len, self.k), float(self.k)
-            if max_len > POOL_SELECT_ROW:
+            if max_len > self._native.pool_select_row(q.shape[1] // G, B * G):   # a selection launch of its own
                 valid, nsel = self._row_budgets(seqlens)
         else:
             width, pct = budgets.topk_width(max_len, self.k), 0.0

@@ -50,6 +50,17 @@ def test_topk_workspace_sizing(lib):
     assert n == 4 * 32 * (2048 + 2 + 8 + 16 * 36)   # 16 chunks of 32768 entries
 
 
+def test_one_launch_selection_ends_where_two_are_faster(lib):
+    """The pooling workgroup of a decode anchor takes a row's tokens for four query heads at a time: groups
+    that fill whole fours of one go further than wide or partly filled ones, at few rows."""
+    row = lib.kascade_pool_select_row
+    assert row(4, 8) == 24576
+    assert all(row(g, 8) == 18432 for g in (1, 2, 5, 7, 8, 12, 16))
+    assert all(row(g, 64) == 24576 for g in range(1, 17))
+    header = re.search(r"#define KASCADE_POOL_SELECT_ROW (\d+)", open(HEADER).read())
+    assert all(row(g, r) <= int(header.group(1)) for g in range(1, 17) for r in (1, 8, 1024))
+
+
 def _err(lib):
     return lib.kascade_get_last_error().decode()
 

@@ -168,3 +168,40 @@ def test_masked_scores_pool_to_nothing_in_one_call(cuda, H, G, L, level):
         _, idx = native.hf_decode_anchor(native.Counters(), q, k, v, layer == 0, width, same)
         assert torch.equal(idx, want), f"layer {layer}"
         assert not bool(masked[0][idx[0].cpu().long()].any())
+
+
+@pytest.mark.parametrize("H,G,L", [(64, 8, 18432), (64, 8, 18433), (28, 4, 20001), (32, 8, 24577), (4, 4, 32767), (32, 2, 32768)])
+@pytest.mark.parametrize("ragged", [False, True])
+def test_anchor_selection_with_and_without_buffers_for_two_launches(cuda, H, G, L, ragged):
+    """Rows beyond kascade_pool_select_row are pooled and selected in two launches when the caller gives the
+    buffers for it, in one otherwise: the same lists, cache rows and log-sums."""
+    from kascade_amd import _lib, kernels
+    D, page, p = 128, 16, 10.0
+    lib = _lib.init()
+    gen = torch.Generator(device=cuda).manual_seed(L)
+    lens = [L, L // 3] if ragged else [L, L]
+    B, pages = len(lens), math.ceil(L / page)
+    assert (L > lib.kascade_pool_select_row(H // G, B * G)) == (L != 18432)
+    q = torch.randn(B, H, D, generator=gen, device=cuda).half()
+    kp = torch.randn(B * pages, page, G, D, generator=gen, device=cuda).half()
+    bt = torch.arange(B * pages, dtype=torch.int32, device=cuda).view(B, pages)
+    seq = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    ns, stride = 4, (L + 7) // 8 * 8
+    nsel = [math.ceil(int(p * n / 100) / 128) * 128 for n in lens] if ragged else [L // 10] * B
+    k = max(nsel)
+    per_row = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda).repeat_interleave(G)
+    agg = torch.empty(B, G, stride, device=cuda, dtype=torch.float16)
+    shape, ptr = ctypes.byref(_lib.Shape(G, D, 0, H // G)), lambda t: None if t is None else t.data_ptr()
+    got = []
+    for buffers in ((None, None, None), (agg, per_row(lens) if ragged else None, per_row(nsel) if ragged else None)):
+        glse, sums = torch.empty(B, H, ns, device=cuda), torch.empty(B, H, device=cuda)
+        scores = torch.empty(B, H, stride, device=cuda)
+        idx = torch.full((B, G, k), -7, dtype=torch.int32, device=cuda)
+        rows = torch.full_like(idx, -7)
+        _lib.check(lib.kascade_decode_anchor_topk_call(
+            shape, ptr(q), ptr(kp), None, ptr(seq), ptr(glse), None, ptr(sums), ptr(scores), None, ptr(buffers[0]), ptr(idx),
+            ptr(rows), B, L, stride, ns, 0, L, k, 5, p if ragged else 0.0, ptr(buffers[1]), ptr(buffers[2]), None, ptr(bt),
+            pages, page, None, None, None, None, torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        got.append((idx, rows, sums))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
