@@ -251,6 +251,20 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
                                         const kascade_half* k_new, const kascade_half* v_new,
                                         int32_t* sync_counters, void* stream);
 
+/* Split counts for the decode calls (num_split), as the callers in this repository choose them.
+ * kascade_decode_num_split: for lists or caches of up to max_rows rows per (sequence, KV head),
+ *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
+ *   least min_rows rows each, at most cap_rows (0: no cap); 1 to 256.
+ * kascade_gather_lone_rows: the longest list a gather call takes in one split.
+ * KASCADE_GATHER_ROWS_PER_SPLIT: cap_rows of gather calls.
+ * KASCADE_FUSED_MERGE_MAX_SPLITS: up to this many splits the merge inside the launch (sync_counters)
+ *   is the faster one. */
+#define KASCADE_GATHER_ROWS_PER_SPLIT 1664
+#define KASCADE_FUSED_MERGE_MAX_SPLITS 32
+int kascade_decode_num_split(double total_rows, double max_rows, int compute_units, double wgs_per_cu, double min_rows,
+                             double cap_rows);
+int kascade_gather_lone_rows(int group_size);
+
 /* An anchor pass and the selection over its pooled scores in one call: what
  * kascade_decode_recompute_paged_shaped_call followed by kascade_topk_rows_call gives, without the
  * pooled scores as a result.  shape == NULL: the reference's.  Rows of up to

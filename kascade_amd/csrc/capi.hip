@@ -5,6 +5,7 @@
 #include "../../include/kascade_hip.h"
 #include "../../include/kascade_hip_diag.h"
 
+#include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
@@ -551,6 +552,26 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
     if (get_shape(shape, &sh)) return -1;
     return decode_recompute_paged_impl(sh, Q, K, V, cache_seqlens, glse, Output_partial, row_sums, scores, Output, aggregated_scores, batch, kv_stride_tokens, scores_stride, num_split, with_output, block_table, max_pages, page_size, kv_strides, k_new, v_new, sync_counters, nullptr, stream);
 }
+
+int kascade_decode_num_split(double total_rows, double max_rows, int compute_units, double wgs_per_cu, double min_rows,
+                             double cap_rows) {
+    double per = fmax(min_rows, total_rows / (wgs_per_cu * compute_units));
+    if (cap_rows > 0) per = fmin(per, cap_rows);
+    // small launch (short lists, small batch): latency, not set-up, is what counts, so spread down to
+    // 128 rows per workgroup to put one workgroup on every compute unit
+    if (total_rows / per < compute_units) per = fmax(fmin(128, min_rows), total_rows / compute_units);
+    // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
+    // of workgroups on a few units, one fewer costs nothing
+    return per > 0 ? (int)fmax(1, fmin(256, nearbyint(max_rows / per))) : 1;
+}
+
+// A lone split writes its result itself; merging several costs about 3 us (partial results through
+// device-coherent memory, a counter, the way back), as much as 256 rows more in one workgroup, and more
+// with more query heads.  Us per launch, one split against the best of several: 32/8 heads, batch 1, 256
+// rows 6.9 / 8.0, 384 rows 8.2 / 8.4, 512 rows 9.5 / 8.5; batch 8, 384 rows 9.4 / 9.8, 512 rows 11.0 / 10.5;
+// batch 16, 384 rows 10.8 / 12.0.  64/8 heads, batch 8: 384 rows 9.9 / 11.6, 512 rows 11.5 / 12.3, 640 rows
+// 13.3 / 13.2.
+int kascade_gather_lone_rows(int group_size) { return group_size <= 4 ? 384 : 512; }
 
 // One workgroup pools a row's tokens for all query heads of its KV head, four heads at a time, where a
 // launch of its own spreads them over the chip: the saved launch (2 to 4 us) stops paying as tokens

@@ -11,7 +11,6 @@
 #include <ATen/ATen.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 
-#include <cmath>
 #include <map>
 
 #include "../../include/kascade_hip.h"
@@ -102,18 +101,11 @@ at::Tensor empty_like_type(at::IntArrayRef size, const at::Tensor& like, at::Sca
     return at::empty(size, like.options().dtype(type));
 }
 
-// kernels.default_num_split without known row counts (the same rule; see there for the reasons).
-int num_split(double total_rows, double max_rows, double cap_rows, double min_rows = 512) {
-    const int cus = kascade_device_cu_count() > 0 ? kascade_device_cu_count() : 256;
-    double per = std::max(min_rows, total_rows / (2.0 * cus));
-    if (cap_rows > 0) per = std::min(per, cap_rows);
-    if (total_rows / per < cus) per = std::max(std::min(128.0, min_rows), total_rows / cus);
-    return (int)std::max(1.0, std::min(256.0, std::nearbyint(max_rows / per)));
+// What kernels.default_num_split takes by default: two workgroups per compute unit, 512 rows each.
+int num_split(double total_rows, double max_rows, double cap_rows) {
+    const int cus = kascade_device_cu_count();
+    return kascade_decode_num_split(total_rows, max_rows, cus > 0 ? cus : 256, 2, 512, cap_rows);
 }
-constexpr double kGatherRowsPerSplit = 1664;
-// kernels.gather_lone_rows (see there)
-int64_t gather_lone_rows(const kascade_shape& s) { return s.group_size <= 4 ? 384 : 512; }
-constexpr int kFusedMergeMaxSplits = 32;
 
 // Arrival counters of the fused split merge: zero when made, and zero again after every launch, so
 // that launches on one stream share them; one array per stream.
@@ -196,11 +188,12 @@ const at::Tensor& head_map(PyObject* o, int64_t groups) {
 void hf_reuse(const HfTensors& h, const at::Tensor& idx, const at::Tensor& hm, PyObject* counters, const at::Tensor& out,
               int device, void* stream) {
     const int64_t topk = idx.size(-1);
-    const int ns = topk <= gather_lone_rows(h.shape) ? 1 : num_split((double)h.B * h.G * topk, (double)topk, kGatherRowsPerSplit);
+    const int ns = topk <= kascade_gather_lone_rows(h.shape.group_size)
+                       ? 1 : num_split((double)h.B * h.G * topk, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
     const int64_t parts = (h.B * h.H * ns + 63) / 64 * 64;
     const at::Tensor scratch = empty_like_type({parts + h.B * h.H * ns * h.D}, h.q, at::kFloat);
     at::Tensor sync;
-    if (ns <= kFusedMergeMaxSplits) sync = counters_for(counters, stream, h.B * h.G, h.q);
+    if (ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) sync = counters_for(counters, stream, h.B * h.G, h.q);
     const kascade_strides st = HfTensors::strides(h.k);
     check(kascade_decode_reuse_paged_shaped_call(
         &h.shape, half_ptr(h.q), half_ptr(h.k), half_ptr(h.v), nullptr, int_ptr(idx), int_ptr(hm), 0.f, float_ptr(scratch),
@@ -253,7 +246,7 @@ PyObject* hf_decode_anchor(PyObject* const* a) {
         agg = empty_like_type({h.B, h.G, stride}, h.q, at::kHalf);
         if (ws_bytes > 0) ws = empty_like_type({ws_bytes}, h.q, at::kByte);
     }
-    if (with_output && ns <= kFusedMergeMaxSplits) sync = counters_for(a[0], stream, h.B * h.G, h.q);
+    if (with_output && ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) sync = counters_for(a[0], stream, h.B * h.G, h.q);
     at::Tensor out = at::empty({h.B, 1, h.H, h.D}, h.q.options());
     at::Tensor idx = empty_like_type({h.B, h.G, width}, h.q, at::kInt);
     const kascade_strides st = HfTensors::strides(h.k);

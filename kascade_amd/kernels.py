@@ -90,18 +90,13 @@ def _blhd_strides(t: torch.Tensor, name: str) -> Strides:
     return Strides(t.stride(0), t.stride(1), t.stride(2))
 
 
-GATHER_ROWS_PER_SPLIT = 1664
+GATHER_ROWS_PER_SPLIT = 1664   # KASCADE_GATHER_ROWS_PER_SPLIT of the header
 
 
 def gather_lone_rows(group_size: int) -> int:
-    """Longest list a gather launch takes in one split per (sequence, KV head).  A lone split writes its
-    result itself; merging several costs about 3 us (partial results through device-coherent memory,
-    a counter, the way back), as much as 256 rows more in one workgroup, and more with more query
-    heads.  Us per launch, one split against the best of several: 32/8 heads, batch 1, 256 rows
-    6.9 / 8.0, 384 rows 8.2 / 8.4, 512 rows 9.5 / 8.5; batch 8, 384 rows 9.4 / 9.8, 512 rows 11.0 / 10.5;
-    batch 16, 384 rows 10.8 / 12.0.  64/8 heads, batch 8: 384 rows 9.9 / 11.6, 512 rows 11.5 / 12.3, 640 rows
-    13.3 / 13.2."""
-    return 384 if group_size <= 4 else 512
+    """Longest list a gather launch takes in one split per (sequence, KV head)
+    (kascade_gather_lone_rows, where the reasons are)."""
+    return _lib.load().kascade_gather_lone_rows(group_size)
 
 
 def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_rows: int = 512,
@@ -142,16 +137,7 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
             if not cap_rows or count(best)[1] <= 4096 or rounds >= 8:
                 return best
             rounds += 1
-    rows_per_split = max(min_rows, total_rows / target_wgs)
-    if cap_rows:
-        rows_per_split = min(rows_per_split, cap_rows)
-    if total_rows / rows_per_split < cus:
-        # small launch (short lists, small batch): latency, not set-up, is what counts, so
-        # spread down to 128 rows per workgroup to put one workgroup on every compute unit
-        rows_per_split = max(min(128, min_rows), total_rows / cus)
-    # round to nearest: one workgroup more than a whole number per compute unit costs a
-    # full extra wave of workgroups on a few units (tail), one fewer costs nothing
-    return int(max(1, min(256, round(max_rows / rows_per_split))))
+    return _lib.load().kascade_decode_num_split(total_rows, max_rows, cus, wgs_per_cu, min_rows, cap_rows or 0)
 
 
 # ---------------------------------------------------------------- decode

@@ -61,6 +61,27 @@ def test_one_launch_selection_ends_where_two_are_faster(lib):
     assert all(row(g, r) <= int(header.group(1)) for g in range(1, 17) for r in (1, 8, 1024))
 
 
+def test_split_rules_have_one_home(lib):
+    """The split counts of the Python wrappers and of the host extension come from the library; the two
+    numbers that Python holds itself are the header's."""
+    from kascade_amd import kernels, strategy
+    constants = dict(re.findall(r"#define (KASCADE_[A-Z_]+) (\d+)", open(HEADER).read()))
+    assert kernels.GATHER_ROWS_PER_SPLIT == int(constants["KASCADE_GATHER_ROWS_PER_SPLIT"])
+    assert strategy.FUSED_MERGE_MAX_SPLITS == int(constants["KASCADE_FUSED_MERGE_MAX_SPLITS"])
+    source = open(os.path.join(ROOT, "kascade_amd", "csrc", "native.cpp")).read()
+    assert not re.search(r"\b(1664|384|nearbyint)\b", source)
+    # the rule as the wrappers always had it
+    for total, longest, cus, per_cu, least, cap in ((128 * 6656, 6656, 256, 2, 512, 0), (8 * 1664, 1664, 256, 2, 512, 1664),
+                                                    (8 * 100, 100, 256, 2, 512, 0), (128 * 13184, 13184, 256, 2, 512, 1664),
+                                                    (3, 1, 256, 1, 1, 0), (8 * 524288, 524288, 256, 1, 64, 0), (0, 0, 256, 2, 0, 0)):
+        per = max(least, total / (per_cu * cus))
+        per = min(per, cap) if cap else per
+        if per and total / per < cus:
+            per = max(min(128, least), total / cus)
+        want = max(1, min(256, round(longest / per))) if per else 1
+        assert lib.kascade_decode_num_split(total, longest, cus, per_cu, least, cap) == want
+
+
 def _err(lib):
     return lib.kascade_get_last_error().decode()
 
