@@ -255,7 +255,8 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
  * kascade_decode_num_split: for lists or caches of up to max_rows rows per (sequence, KV head),
  *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
  *   least min_rows rows each, at most cap_rows (0: no cap); 1 to 256.
- * kascade_gather_lone_rows: the longest list a gather call takes in one split.
+ * kascade_gather_lone_rows: the longest list a gather call takes in one split, for so many query heads per
+ *   KV head and so many lists (batch times KV heads).
  * KASCADE_GATHER_ROWS_PER_SPLIT: cap_rows of gather calls.
  * KASCADE_FUSED_MERGE_MAX_SPLITS: up to this many splits the merge inside the launch (sync_counters)
  *   is the faster one. */
@@ -263,7 +264,7 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
 #define KASCADE_FUSED_MERGE_MAX_SPLITS 32
 int kascade_decode_num_split(double total_rows, double max_rows, int compute_units, double wgs_per_cu, double min_rows,
                              double cap_rows);
-int kascade_gather_lone_rows(int group_size);
+int kascade_gather_lone_rows(int group_size, int lists);
 
 /* An anchor pass and the selection over its pooled scores in one call: what
  * kascade_decode_recompute_paged_shaped_call followed by kascade_topk_rows_call gives, without the

@@ -565,13 +565,23 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     return per > 0 ? (int)fmax(1, fmin(256, nearbyint(max_rows / per))) : 1;
 }
 
-// A lone split writes its result itself; merging several costs about 3 us (partial results through
-// device-coherent memory, a counter, the way back), as much as 256 rows more in one workgroup, and more
-// with more query heads.  Us per launch, one split against the best of several: 32/8 heads, batch 1, 256
-// rows 6.9 / 8.0, 384 rows 8.2 / 8.4, 512 rows 9.5 / 8.5; batch 8, 384 rows 9.4 / 9.8, 512 rows 11.0 / 10.5;
-// batch 16, 384 rows 10.8 / 12.0.  64/8 heads, batch 8: 384 rows 9.9 / 11.6, 512 rows 11.5 / 12.3, 640 rows
-// 13.3 / 13.2.
-int kascade_gather_lone_rows(int group_size) { return group_size <= 4 ? 384 : 512; }
+// A lone split writes its result itself; merging several costs a trip through device-coherent memory, a
+// counter and the way back, the more the more query heads and workgroups there are.  Us per launch in a
+// captured graph, one split / as many as kascade_decode_num_split gives, 8 KV heads:
+//   rows   batch    1 head      2           4           5           7           8           16 heads per KV head
+//   256    1        6.0/7.2     6.1/7.2     6.2/7.7     6.5/8.8     6.6/9.2     6.8/9.3     7.8/13.1
+//   384    1        7.3/7.2     7.5/7.4     7.7/7.8     7.9/8.8     8.1/9.2     8.2/9.5     9.2/13.2
+//   384    4        7.8/7.6     7.9/7.7     8.1/8.2     8.3/9.4     8.6/10.0    8.6/10.1    9.6/13.9
+//   384    8        8.2/8.3     8.3/8.4     8.4/8.8     8.7/10.1    8.8/10.5    8.9/10.7    9.8/14.5
+//   512    1                                            9.2/9.0     9.5/9.5     9.5/9.6     10.5/13.4
+//   512    2                                            9.3/9.7     9.7/10.1    9.7/10.2    10.7/14.0
+//   512    8                                            10.1/10.5   10.3/11.0   10.4/11.0   11.4/15.0
+// (4 heads, 512 rows: 9.5/8.5 at batch 1, 11.0/10.5 at 8; with 2 or 4 KV heads one split of 384 rows is up to
+// 6 % behind for 1 and 2 heads, one of 512 up to 5 % for 5 to 7, from 64 and 16 lists on level.)
+int kascade_gather_lone_rows(int group_size, int lists) {
+    if (group_size <= 2) return lists >= 64 ? 384 : 256;
+    return group_size >= 8 || (group_size >= 5 && lists >= 16) ? 512 : 384;
+}
 
 // One workgroup pools a row's tokens for all query heads of its KV head, four heads at a time, where a
 // launch of its own spreads them over the chip: the saved launch (2 to 4 us) stops paying as tokens

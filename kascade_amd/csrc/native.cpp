@@ -188,7 +188,7 @@ const at::Tensor& head_map(PyObject* o, int64_t groups) {
 void hf_reuse(const HfTensors& h, const at::Tensor& idx, const at::Tensor& hm, PyObject* counters, const at::Tensor& out,
               int device, void* stream) {
     const int64_t topk = idx.size(-1);
-    const int ns = topk <= kascade_gather_lone_rows(h.shape.group_size)
+    const int ns = topk <= kascade_gather_lone_rows(h.shape.group_size, (int)(h.B * h.G))
                        ? 1 : num_split((double)h.B * h.G * topk, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
     const int64_t parts = (h.B * h.H * ns + 63) / 64 * 64;
     const at::Tensor scratch = empty_like_type({parts + h.B * h.H * ns * h.D}, h.q, at::kFloat);

@@ -93,10 +93,10 @@ def _blhd_strides(t: torch.Tensor, name: str) -> Strides:
 GATHER_ROWS_PER_SPLIT = 1664   # KASCADE_GATHER_ROWS_PER_SPLIT of the header
 
 
-def gather_lone_rows(group_size: int) -> int:
-    """Longest list a gather launch takes in one split per (sequence, KV head)
-    (kascade_gather_lone_rows, where the reasons are)."""
-    return _lib.load().kascade_gather_lone_rows(group_size)
+def gather_lone_rows(group_size: int, lists: int = 1 << 30) -> int:
+    """Longest list a gather launch takes in one split per (sequence, KV head), when it gathers so many
+    lists (default: many).  kascade_gather_lone_rows, where the reasons are."""
+    return _lib.load().kascade_gather_lone_rows(group_size, lists)
 
 
 def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_rows: int = 512,

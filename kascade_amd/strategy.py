@@ -317,7 +317,7 @@ class PagedKascadeDecoder:
         self.ns_reuse = num_split_reuse or kernels.default_num_split(
             G * budgets.decode_budget(total, k), self.max_topk, wgs_per_cu=1 if uniform else 2,
             cap_rows=kernels.GATHER_ROWS_PER_SPLIT, row_counts=reuse_rows, heads=G,
-            lone_rows=kernels.gather_lone_rows(group_size))
+            lone_rows=kernels.gather_lone_rows(group_size, max_batch * G))
         # The anchor passes (which also write their score codes) run 2 % faster with twice the
         # splits where two workgroups per compute unit leave a split more than 8192 rows
         # (16 x 65536: 795 / 508 us with 8 splits against 815 / 521 with 4); dense decode does not

@@ -197,3 +197,12 @@ def test_short_gather_lists_are_one_split(group, limit):
     # no device query below the limit; the general rule has the say above it
     assert kernels.default_num_split(8 * limit, limit, lone_rows=lone) == 1
     assert kernels.default_num_split(8 * 16 * 128, 128, row_counts=[128] * 16, lone_rows=lone) == 1
+
+
+@pytest.mark.parametrize("group,lists,limit", [(1, 8, 256), (2, 63, 256), (2, 64, 384), (3, 1, 384), (4, 8, 384), (5, 8, 384),
+                                               (7, 15, 384), (7, 16, 512), (8, 1, 512), (16, 8, 512)])
+def test_lone_gather_split_depends_on_the_number_of_lists(group, lists, limit):
+    """With few lists the workgroups of several splits find idle compute units: the groups whose merge is
+    the cheaper part go to several splits earlier there."""
+    from kascade_amd import kernels
+    assert kernels.gather_lone_rows(group, lists) == limit
