@@ -707,6 +707,30 @@ int kascade_topk_sorted_call(const kascade_half* scores, int32_t* out_idx, int r
 
 }  // extern "C"
 namespace {
+// 64 queries per wavefront in the K-only log-sum pass, or 32?  Units (workgroups) of 64 read every K tile for
+// twice the queries, 15 % less per query, but there are half as many and each is twice as long, so it is a
+// question of how the units fill the 512 places of the chip (two on each of 256 compute units), and of how
+// far their lengths spread: from q_start to q_start + q_len keys.  Us, 32 / 64 queries, 32/8 heads:
+//   units of 64   queries, position         32 / 64        why
+//   256           2048 at 8192              186 / 209      one workgroup per compute unit
+//   448, 512      3584 at 7168, 4096 at 0   347 / 291, 88 / 98: a residency nearly full of units about equally long
+//                                           wins; lengths that spread leave its places idle
+//   520, 576      4160 at 8320, 4608 at 1152  424 / 464, 169 / 158: equal lengths leave a second residency nearly
+//                                           empty, lengths that spread overlap
+//   520, 640      4160, 5120 at 0           93.7 / 102.8, 128.8 / 135.9 (whole prompts)
+//   768, 1024     6144, 8192 at 0           192 / 174, 315 / 281; at 4 times their length 1550 / 1465, 2725 / 2345
+//   704           11 x 512 at 0             28.8 / 34.3    short units: the set-up counts
+//   1024          16 x 512 at 0, at 512     37.3 / 40.8, 74.9 / 70.9
+// Sequences at different positions count as if all stood at the last one (the host knows no other).
+bool wide_log_sum_units(const Shape& sh, int batch, int q_start, int q_len) {
+    if (sh.D != 128) return false;
+    const long long units = (long long)((q_len + 63) / 64) * sh.G * ((sh.gs + 3) / 4) * batch;
+    const bool deep = (long long)q_start + q_len >= 2048;
+    if (units <= 512) return units >= 448 && q_start >= q_len;
+    if (units <= 640) return deep && q_start > 0 && q_start <= q_len;
+    return deep || (q_start >= q_len && units >= 800);
+}
+
 int prefill_dense_impl(const Shape& sh, const kascade_half* Q, const kascade_half* K, const kascade_half* V,
                                float* log_sum, kascade_half* Output, int batch, int seq_len,
                                kascade_strides q_strides, kascade_strides kv_strides,
@@ -724,13 +748,7 @@ int prefill_dense_impl(const Shape& sh, const kascade_half* Q, const kascade_hal
     p.q_sb = q_strides.b; p.q_sl = q_strides.l; p.q_sh = q_strides.h;
     p.k_sb = kv_strides.b; p.k_sl = kv_strides.l; p.k_sh = kv_strides.h;
     p.B = batch; p.L = seq_len; p.Lq = seq_len; p.T = (seq_len + kTile - 1) / kTile;
-    // The K-only pass takes 64 queries per wavefront where that leaves more units than are resident
-    // at once (two on each of 256 compute units): every K tile is read for twice the queries
-    // (32768 tokens, 32/8 heads: 4.20 ms against 4.67; two prompts of 3001: 90.5 against 94.8 us).  With
-    // fewer units nothing evens out their lengths, and units of half the size are faster (517 tokens
-    // 15.0 -> 10.6 us, 2048 44.9 -> 34.5, 4096 98.4 -> 89.8).
-    const long long units64 = (long long)((seq_len + 63) / 64) * sh.G * ((sh.gs + 3) / 4) * batch;
-    const int nqb = (with_output || sh.D != 128 || units64 <= 512) ? 1 : 2;
+    const int nqb = (!with_output && wide_log_sum_units(sh, batch, 0, seq_len)) ? 2 : 1;
     return check_hip(launch_prefill_attn(p, false, with_output != 0, nqb, static_cast<hipStream_t>(stream)), "prefill_dense");
 }
 }  // namespace
@@ -1062,12 +1080,7 @@ int prefill_chunk_dense_impl(const Shape& sh, const kascade_half* Q, const kasca
         return -1;
     p.K = E(K_pages); p.V = with_output ? E(V_pages) : E(K_pages);
     p.log_sum = log_sum; p.O = E(Output);
-    // 64 queries per wavefront in the K-only pass as for whole prompts, and from 512 units on (two per
-    // compute unit) where the chunk's units are about equally long: 4096 queries of 32/8 heads at
-    // position 12288 567 -> 489 us, 6144 334 -> 294; at position 0 87 -> 98, and 2048 queries (256 units)
-    // at 12288 261 -> 293, so those keep 32.
-    const long long units64 = (long long)((q_len + 63) / 64) * sh.G * ((sh.gs + 3) / 4) * batch;
-    const int nqb = (with_output || sh.D != 128 || units64 < 512 || (units64 == 512 && q_start < q_len)) ? 1 : 2;
+    const int nqb = (!with_output && wide_log_sum_units(sh, batch, q_start, q_len)) ? 2 : 1;
     return check_hip(launch_prefill_attn(p, false, with_output != 0, nqb,
                                          static_cast<hipStream_t>(stream)), "prefill_chunk_dense");
 }

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("B,L", [(1, 1), (16, 255), (16, 256), (16, 257), (17, 250), (13, 321)])
 def test_log_sums_on_both_sides_of_the_unit_size(cuda, B, L):
-    """32 queries per wavefront up to 512 units of 64 queries, 64 beyond (8 KV heads).  Tolerance as
+    """Batches of short prompts around 512 units of 64 queries (8 KV heads).  Tolerance as
     for the log-sums elsewhere: fp32 sums of exponentials of fp32-accumulated fp16 products."""
     from kascade_amd import kernels
     gen = torch.Generator().manual_seed(L)
@@ -51,8 +51,8 @@ def test_pooled_scores_do_not_depend_on_the_key_parts(cuda, L, heads, G, D):
 
 @pytest.mark.parametrize("B,n,start", [(16, 256, 256), (16, 250, 256), (16, 256, 0), (17, 225, 96)])
 def test_chunk_log_sums_do_not_depend_on_the_unit_size(cuda, B, n, start):
-    """A chunk's log-sums over the paged cache, in a batch large enough for 64 queries per wavefront
-    and alone (32 per wavefront): the same bits, and the oracle's values."""
+    """A chunk's log-sums over the paged cache, in a batch of about 512 units (64 queries per wavefront
+    where the units are equally long) and alone (32): the same bits, and the oracle's values."""
     from kascade_amd import kernels
     gen = torch.Generator().manual_seed(n)
     L, page = start + n, 16
@@ -74,3 +74,64 @@ def test_chunk_log_sums_do_not_depend_on_the_unit_size(cuda, B, n, start):
     assert all(torch.equal(one[0], m) for m in many)
     _, want = orc.dense_prefill(q, k, k)
     assert_close(one, want[:, start:], "chunk log_sum", atol=2e-3, rtol=1e-4)
+
+
+def _paged_copies(k, page, gen, B, cuda):
+    """k [1,L,G,D] in shuffled pages that B sequences share: (pages, block table)."""
+    L, G, D = k.shape[1:]
+    per = (L + page - 1) // page
+    rows = torch.zeros(per * page, G, D, dtype=k.dtype)
+    rows[:L] = k[0]
+    order = torch.randperm(per, generator=gen)
+    pages = torch.empty(per, page, G, D, dtype=k.dtype)
+    pages[order] = rows.view(per, page, G, D)
+    return pages.to(cuda), order.to(torch.int32).repeat(B, 1).to(cuda)
+
+
+# units of 64 queries: 440 and 448, 512 and 520 (about equal lengths), 640 twice (equal, spread), 648, 768 and 800
+# (short), 792 (whole prompts)
+@pytest.mark.parametrize("B,n,start", [(11, 320, 320), (14, 256, 256), (16, 256, 256), (13, 320, 320), (10, 512, 1536),
+                                       (5, 1024, 1024), (27, 192, 1888), (24, 256, 256), (25, 256, 256), (3, 2049, 0)])
+def test_log_sums_have_the_same_bits_on_every_line_of_the_unit_size(cuda, B, n, start):
+    """A batch of copies, whatever unit size the rule takes for it, against one of them alone (32 queries
+    per wavefront): the same bits, over the paged cache and, from position 0, for whole prompts."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(n + start)
+    q = torch.randn(1, start + n, 32, 128, generator=gen).half()
+    k = torch.randn(1, start + n, 8, 128, generator=gen).half()
+    kp, table = _paged_copies(k, 16, gen, B, cuda)
+    qd = q[:, start:].to(cuda)
+    one = kernels.prefill_chunk_dense(qd, kp, kp, table[:1], start, page_size=16, with_output=False)[0]
+    many = kernels.prefill_chunk_dense(qd.repeat(B, 1, 1, 1), kp, kp, table, start, page_size=16, with_output=False)[0]
+    assert all(torch.equal(one[0], m) for m in many)
+    if start == 0:
+        assert torch.equal(one, kernels.prefill_recompute1(qd, k.to(cuda)))
+        many = kernels.prefill_recompute1(qd.repeat(B, 1, 1, 1), k.to(cuda).repeat(B, 1, 1, 1))
+        assert all(torch.equal(one[0], m) for m in many)
+    _, want = orc.dense_prefill(q, k, k)
+    assert_close(one, want[:, start:], "log_sum", atol=2e-3, rtol=1e-4)
+
+
+def test_wide_log_sum_units_of_sequences_at_different_positions(cuda):
+    """512 units of 64 queries over a paged cache, each sequence with a start and a row count of its own
+    (none, a part of a unit, remainders): every sequence's rows have the bits of a call of its own, and
+    rows that belong to no sequence are not written."""
+    from kascade_amd import _lib, kernels
+    B, n, top = 16, 256, 256
+    gen = torch.Generator().manual_seed(7)
+    starts = [top, 0, 32, 224, 96, 256, 160, 64] * 2
+    lens = [256, 256, 1, 33, 64, 0, 127, 255, 65, 31, 250, 128, 0, 192, 200, 96]
+    k = torch.randn(1, top + n, 8, 128, generator=gen).half()
+    kp, table = _paged_copies(k, 16, gen, B, cuda)
+    q = torch.randn(B, n, 32, 128, generator=gen).half().to(cuda)
+    at = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda)
+    got, qs, ql = torch.full((B, n, 32), 7.0, device=cuda), at(starts), at(lens)
+    _lib.check(_lib.init().kascade_prefill_chunk_dense_call(
+        q.data_ptr(), kp.data_ptr(), None, got.data_ptr(), None, B, top, n, _lib.Strides(*q.stride()[:3]), table.data_ptr(),
+        table.shape[1], 16, kp.shape[0], 0, qs.data_ptr(), ql.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    for b in range(B):
+        assert bool((got[b, lens[b]:] == 7.0).all())
+        if lens[b]:
+            own = kernels.prefill_chunk_dense(q[b:b + 1, :lens[b]], kp, kp, table[b:b + 1], starts[b], page_size=16,
+                                              with_output=False)[0]
+            assert torch.equal(got[b, :lens[b]], own[0]), f"sequence {b}"
