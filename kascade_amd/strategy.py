@@ -94,10 +94,6 @@ class EfficientKascadeStrategy:
         self._hm_cache = {}
         self._budget_cache = {}
         self._merge_counters = None
-        cls = type(self)   # a subclass that replaces a seam gets its layers through it
-        self._own_seams = all(getattr(cls, name) is getattr(EfficientKascadeStrategy, name)
-                              for name in ("_prefill_recomp_forward", "_prefill_reuse_forward",
-                                           "_decode_recomp_forward", "_decode_reuse_forward"))
         if register:
             self.register_attention()
 
@@ -223,8 +219,10 @@ class EfficientKascadeStrategy:
         anchor = layer in self.recompute_layers
         if Lq != 1 and Lq != Lk:
             raise KascadeError("prefill needs Lq == Lk (no cached prefix), as in the reference kernels")
-        if not self._own_seams:
-            return self._through_seams(query, key, value, layer, anchor), None
+        name = _SEAM_NAMES[Lq == 1][anchor]
+        seam = getattr(self, name)
+        if getattr(seam, "__func__", None) is not _OWN_SEAMS[name]:   # replaced by a subclass, on the class or the instance
+            return self._through_seam(seam, query, key, value, layer, anchor), None
         # The reference copies the whole cache to [B,L,G,D] here on every decode step
         # (EfficientKascadeStrategy.py:149-150); the kernels take strided views of HF's head-major
         # tensors instead and read them in place.
@@ -239,21 +237,20 @@ class EfficientKascadeStrategy:
             o = self._hf_prefill_reuse(query, key, value, self.k, layer)
         return o, None
 
-    def _through_seams(self, query, key, value, layer, anchor):
-        """A layer of a subclass with seams of its own, which take [B,L,heads,D] views (decode: Q [B,H,D])."""
+    def _through_seam(self, seam, query, key, value, layer, anchor):
+        """A layer through a seam of the user's, which takes [B,L,heads,D] views (decode: Q [B,H,D])."""
         rounded_k = budgets.topk_width(key.shape[2], self.k)
         K, V = key.transpose(1, 2), value.transpose(1, 2)
         if query.shape[2] == 1:
             Q = query.squeeze(2).contiguous()
             if K.stride(-1) != 1 or V.stride() != K.stride():
                 K, V = K.contiguous(), V.contiguous()
-            o = self._decode_recomp_forward(Q, K, V, rounded_k, layer) if anchor else \
-                self._decode_reuse_forward(Q, K, V, layer)
+            o = seam(Q, K, V, rounded_k, layer) if anchor else seam(Q, K, V, layer)
             return o.unsqueeze(1)
         Q = query.transpose(1, 2)
         if anchor:
-            return self._prefill_recomp_forward(Q, K, V, rounded_k, self.tile_size, layer, self.k)
-        return self._prefill_reuse_forward(Q, K, V, self.k, layer)
+            return seam(Q, K, V, rounded_k, self.tile_size, layer, self.k)
+        return seam(Q, K, V, self.k, layer)
 
     def register_attention(self):
         """EfficientKascadeStrategy.py:163-168."""
@@ -265,6 +262,12 @@ class EfficientKascadeStrategy:
                                           dropout=dropout, **kwargs)
         ALL_MASK_ATTENTION_FUNCTIONS.register(self.name, ALL_MASK_ATTENTION_FUNCTIONS["sdpa"])
         ALL_ATTENTION_FUNCTIONS.register(self.name, _attention_forward)
+
+
+# The reference's seams, [decode][anchor], and this module's own: attention_forward goes past these to the
+# calls that take transformers tensors, and through whatever stands in their place.
+_SEAM_NAMES = (("_prefill_reuse_forward", "_prefill_recomp_forward"), ("_decode_reuse_forward", "_decode_recomp_forward"))
+_OWN_SEAMS = {name: getattr(EfficientKascadeStrategy, name) for pair in _SEAM_NAMES for name in pair}
 
 
 class PagedKascadeDecoder:

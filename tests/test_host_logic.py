@@ -206,3 +206,38 @@ def test_lone_gather_split_depends_on_the_number_of_lists(group, lists, limit):
     the cheaper part go to several splits earlier there."""
     from kascade_amd import kernels
     assert kernels.gather_lone_rows(group, lists) == limit
+
+
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+@pytest.mark.parametrize("Lq", [200, 1])
+@pytest.mark.parametrize("layer", [0, 1])
+def test_replaced_seams_are_called(monkeypatch, where, Lq, layer):
+    """EfficientKascadeStrategy.py:72-123: each layer kind runs through a method of its own, and one put in its
+    place -- in a subclass, on the class or on an instance that exists already -- gets the layer, with the
+    reference's arguments ([B,L,heads,D] tensors, decode Q [B,H,D])."""
+    from types import SimpleNamespace
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    L, p = 200, 10
+    name = {(200, 0): "_prefill_recomp_forward", (200, 1): "_prefill_reuse_forward",
+            (1, 0): "_decode_recomp_forward", (1, 1): "_decode_reuse_forward"}[Lq, layer]
+    seen = []
+
+    def mine(self, Q, *rest):
+        seen.append((self, Q, rest))
+        return Q + 1
+    kind = type("Mine", (EfficientKascadeStrategy,), {name: mine}) if where == "subclass" else EfficientKascadeStrategy
+    s = kind([0], None, k=p, tile_size=32, head_mapping=[list(range(8))] * 2, register=False)
+    if where == "class":
+        monkeypatch.setattr(EfficientKascadeStrategy, name, mine)
+    elif where == "instance":
+        s.__dict__[name] = lambda Q, *rest: mine(s, Q, *rest)
+    q = torch.randn(2, 32, Lq, 128).half()
+    k, v = torch.randn(2, 8, L, 128).half(), torch.randn(2, 8, L, 128).half()
+    o, none = s.attention_forward(SimpleNamespace(layer_idx=layer), q, k, v, None, 128 ** -0.5)
+    assert none is None and len(seen) == 1
+    who, Q, (K, V, *rest) = seen[0]
+    assert who is s and torch.equal(o, q.transpose(1, 2) + 1)
+    assert torch.equal(Q, q[:, :, 0] if Lq == 1 else q.transpose(1, 2))
+    assert torch.equal(K, k.transpose(1, 2)) and torch.equal(V, v.transpose(1, 2))
+    width = budgets.topk_width(L, p)
+    assert rest == {(200, 0): [width, 32, 0, p], (200, 1): [p, 1], (1, 0): [width, 0], (1, 1): [1]}[Lq, layer]
