@@ -219,10 +219,9 @@ class EfficientKascadeStrategy:
         anchor = layer in self.recompute_layers
         if Lq != 1 and Lq != Lk:
             raise KascadeError("prefill needs Lq == Lk (no cached prefix), as in the reference kernels")
-        name = _SEAM_NAMES[Lq == 1][anchor]
-        seam = getattr(self, name)
-        if getattr(seam, "__func__", None) is not _OWN_SEAMS[name]:   # replaced by a subclass, on the class or the instance
-            return self._through_seam(seam, query, key, value, layer, anchor), None
+        name, own = _SEAMS[Lq == 1][anchor]
+        if getattr(type(self), name) is not own or name in self.__dict__:   # replaced: in a subclass, on the class, here
+            return self._through_seam(getattr(self, name), query, key, value, layer, anchor), None
         # The reference copies the whole cache to [B,L,G,D] here on every decode step
         # (EfficientKascadeStrategy.py:149-150); the kernels take strided views of HF's head-major
         # tensors instead and read them in place.
@@ -264,10 +263,10 @@ class EfficientKascadeStrategy:
         ALL_ATTENTION_FUNCTIONS.register(self.name, _attention_forward)
 
 
-# The reference's seams, [decode][anchor], and this module's own: attention_forward goes past these to the
-# calls that take transformers tensors, and through whatever stands in their place.
-_SEAM_NAMES = (("_prefill_reuse_forward", "_prefill_recomp_forward"), ("_decode_reuse_forward", "_decode_recomp_forward"))
-_OWN_SEAMS = {name: getattr(EfficientKascadeStrategy, name) for pair in _SEAM_NAMES for name in pair}
+# The reference's seams, [decode][anchor], with this module's own methods: attention_forward goes past these to
+# the calls that take transformers tensors, and through whatever stands in their place.
+_SEAMS = tuple(tuple((name, getattr(EfficientKascadeStrategy, name)) for name in pair) for pair in
+               (("_prefill_reuse_forward", "_prefill_recomp_forward"), ("_decode_reuse_forward", "_decode_recomp_forward")))
 
 
 class PagedKascadeDecoder:
