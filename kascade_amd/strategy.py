@@ -171,6 +171,8 @@ class EfficientKascadeStrategy:
                                               self.rolling_prefill)
 
     def _prefill_recomp_forward(self, Q, K, V, topk, tile_size, layer, topk_percent):
+        if math.ceil(Q.shape[1] / tile_size) != math.ceil(Q.shape[1] / TILE):   # the score rows of other tiles
+            raise KascadeError(f"the kernels are specialised to tile_size={TILE}, got {tile_size}")
         return self._hf_prefill_recomp(Q.transpose(1, 2), K.transpose(1, 2), V.transpose(1, 2), topk, layer, topk_percent)
 
     def _prefill_reuse_forward(self, Q, K, V, topk_percent, layer):

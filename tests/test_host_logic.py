@@ -241,3 +241,14 @@ def test_replaced_seams_are_called(monkeypatch, where, Lq, layer):
     assert torch.equal(K, k.transpose(1, 2)) and torch.equal(V, v.transpose(1, 2))
     width = budgets.topk_width(L, p)
     assert rest == {(200, 0): [width, 32, 0, p], (200, 1): [p, 1], (1, 0): [width, 0], (1, 1): [1]}[Lq, layer]
+
+
+def test_prefill_seam_refuses_tiles_the_kernels_do_not_have():
+    """The reference's seam takes the tile size with each call; the kernels have one."""
+    from kascade_amd._lib import KascadeError
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    s = EfficientKascadeStrategy([0], None, k=10, tile_size=32, head_mapping=[list(range(8))], register=False)
+    q, k = torch.zeros(1, 200, 32, 128).half(), torch.zeros(1, 200, 8, 128).half()
+    for tile in (16, 64):
+        with pytest.raises(KascadeError, match="tile_size"):
+            s._prefill_recomp_forward(q, k, k, 128, tile, 0, 10)
