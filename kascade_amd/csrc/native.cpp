@@ -230,7 +230,7 @@ PyObject* hf_decode_anchor(PyObject* const* a) {
     const bool with_output = truth(a[4]);
     const int64_t width = integer(a[5]);
     const at::Tensor& hm = head_map(a[6], h.G);
-    need(width > 0 && width <= h.L, "the selection must lie within the cache");
+    need(width > 0, "the selection takes at least one token");
     const int device = device_of_caller();
     void* stream = stream_of(device);
     const int ns = num_split((double)h.B * h.G * h.L, (double)h.L, 0);
@@ -315,22 +315,23 @@ PyObject* hf_prefill_anchor(PyObject* const* a) {
 }
 
 // -------------------------------------------------------------------------- paged cache
-// q [B,H,D], pages [P,page,G,D]
+// q [B,H,D], pages [P,page,G,D]: any contiguous [...,G,D] view of that memory, where the call does not need
+// to know the number of pages
 struct PagedTensors {
     at::Tensor q, k, v;
     int64_t B, H, D, G, P, page;
     kascade_shape shape;
 };
 
-PagedTensors paged_tensors(PyObject* const* a, long long page) {
+PagedTensors paged_tensors(PyObject* const* a, long long page, bool counted) {
     PagedTensors t{tensor(a[0], "Q"), tensor(a[1], "K_pages"), tensor(a[2], "V_pages")};
-    need(t.q.dim() == 3 && t.k.dim() == 4, "Q must be [B,H,D] and pages [num_pages,page,G,D]");
+    need(t.q.dim() == 3 && t.k.dim() >= 2 && (t.k.dim() == 4 || !counted), "Q must be [B,H,D] and pages [num_pages,page,G,D]");
     need(t.q.is_cuda() && t.k.is_cuda() && t.v.is_cuda(), "Q, K_pages and V_pages must be device tensors");
     need(t.q.is_contiguous() && t.k.is_contiguous() && t.v.is_contiguous(), "Q, K_pages and V_pages must be contiguous");
     t.B = t.q.size(0); t.H = t.q.size(1); t.D = t.q.size(2);
-    t.P = t.k.size(0); t.page = page; t.G = t.k.size(2);
+    t.P = t.k.size(0); t.page = page; t.G = t.k.size(-2);
     t.shape = model_shape(t.q, t.k, t.H, t.G, t.D);
-    if (t.k.size(1) != page || t.k.size(3) != t.D || t.k.sizes() != t.v.sizes() || t.v.scalar_type() != t.k.scalar_type())
+    if ((counted && t.k.size(1) != page) || t.k.size(-1) != t.D || t.k.sizes() != t.v.sizes() || t.v.scalar_type() != t.k.scalar_type())
         fail("pages must be [num_pages,%lld,%lld,%lld]", page, (long long)t.G, (long long)t.D);
     return t;
 }
@@ -356,10 +357,12 @@ const at::Tensor& table_of(PyObject* o, int64_t B) {
     if (bt.dim() != 2 || bt.size(0) != B) fail("block_table must be [%lld,max_pages]", (long long)B);
     return bt;
 }
-const at::Tensor& lengths_of(PyObject* o, int64_t B) {
+// None: every sequence as long as the call says
+const int32_t* lengths_of(PyObject* o, int64_t B) {
+    if (o == Py_None) return nullptr;
     const at::Tensor& n = dense(o, at::kInt, "cache_seqlens");
     if (n.numel() != B) fail("cache_seqlens must have %lld entries", (long long)B);
-    return n;
+    return int_ptr(n);
 }
 int32_t* sync_of(PyObject* o, const PagedTensors& t) {
     if (o == Py_None) return nullptr;
@@ -378,8 +381,8 @@ void scratch_of(PyObject* lse, PyObject* part, const PagedTensors& t, int64_t ns
 // paged_reuse(Q, K_pages, V_pages, seqlens, cache_rows, head_mapping, percent, glse, Output_partial, num_split,
 //             block_table, page_size, out, sync, k_new, v_new) -> O
 PyObject* paged_reuse(PyObject* const* a) {
-    const PagedTensors t = paged_tensors(a, integer(a[11]));
-    const at::Tensor& lens = lengths_of(a[3], t.B);
+    const PagedTensors t = paged_tensors(a, integer(a[11]), true);
+    const int32_t* lens = lengths_of(a[3], t.B);
     const at::Tensor& rows = dense(a[4], at::kInt, "cache_rows");
     if (rows.dim() != 3 || rows.size(0) != t.B || rows.size(1) != t.G) fail("index lists must be [%lld,%lld,topk]", (long long)t.B, (long long)t.G);
     const at::Tensor& hm = head_map(a[5], t.G);
@@ -389,7 +392,7 @@ PyObject* paged_reuse(PyObject* const* a) {
     const at::Tensor& bt = table_of(a[10], t.B);
     at::Tensor out = out_buffer(a[12], t);
     check(kascade_decode_reuse_rows_shaped_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), int_ptr(lens), int_ptr(rows), int_ptr(hm), (float)number(a[6]),
+        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, int_ptr(rows), int_ptr(hm), (float)number(a[6]),
         lse, part, half_ptr(out), (int)t.B, (int)rows.size(2), (int)ns, int_ptr(bt), (int)bt.size(1), (int)t.page, (int)t.P,
         new_rows(a[14], t, "k_new"), new_rows(a[15], t, "v_new"), sync_of(a[13], t), nullptr, stream_of(device_of_caller())));
     return THPVariable_Wrap(out);
@@ -399,8 +402,8 @@ PyObject* paged_reuse(PyObject* const* a) {
 //              max_len, width, percent, valid_len, n_sel, block_table, page_size, out, sync, k_new, v_new, rows_out)
 // -> (O or None, topk_indices); cache rows are written to rows_out
 PyObject* paged_anchor(PyObject* const* a) {
-    const PagedTensors t = paged_tensors(a, integer(a[16]));
-    const at::Tensor& lens = lengths_of(a[3], t.B);
+    const PagedTensors t = paged_tensors(a, integer(a[16]), false);
+    const int32_t* lens = lengths_of(a[3], t.B);
     const bool with_output = truth(a[4]);
     const int64_t ns = integer(a[7]), max_len = integer(a[10]), width = integer(a[11]), stride = (max_len + 7) / 8 * 8;
     float *lse, *part;
@@ -428,7 +431,7 @@ PyObject* paged_anchor(PyObject* const* a) {
     }
     at::Tensor idx = empty_like_type({t.B, t.G, width}, t.q, at::kInt);
     check(kascade_decode_anchor_topk_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), int_ptr(lens), lse, part, float_ptr(sums), float_ptr(scores),
+        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, float_ptr(sums), float_ptr(scores),
         with_output ? half_ptr(out) : nullptr, agg.defined() ? half_ptr(agg) : nullptr, int_ptr(idx), int_ptr(rows),
         (int)t.B, (int)max_len, (int)stride, (int)ns, with_output, (int)max_len, (int)width, 0, (float)number(a[12]), valid,
         nsel, ws.defined() ? ws.data_ptr() : nullptr, int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr,
@@ -446,15 +449,15 @@ PyObject* paged_anchor(PyObject* const* a) {
 // paged_dense(Q, K_pages, V_pages, seqlens, glse, Output_partial, num_split, max_len, block_table, page_size, out, sync,
 //             k_new, v_new) -> O
 PyObject* paged_dense(PyObject* const* a) {
-    const PagedTensors t = paged_tensors(a, integer(a[9]));
-    const at::Tensor& lens = lengths_of(a[3], t.B);
+    const PagedTensors t = paged_tensors(a, integer(a[9]), false);
+    const int32_t* lens = lengths_of(a[3], t.B);
     const int64_t ns = integer(a[6]);
     float *lse, *part;
     scratch_of(a[4], a[5], t, ns, &lse, &part);
     const at::Tensor& bt = table_of(a[8], t.B);
     at::Tensor out = out_buffer(a[10], t);
     check(kascade_decode_dense_paged_shaped_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), int_ptr(lens), lse, part, half_ptr(out), (int)t.B,
+        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, half_ptr(out), (int)t.B,
         (int)integer(a[7]), (int)ns, int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr, new_rows(a[12], t, "k_new"),
         new_rows(a[13], t, "v_new"), sync_of(a[11], t), stream_of(device_of_caller())));
     return THPVariable_Wrap(out);

@@ -244,3 +244,44 @@ def test_captured_decode_keeps_its_own_merge_counters(cuda):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         assert all(bool((t == 5).all()) for t in held)
+
+
+@pytest.mark.parametrize("flat", [False, True])
+def test_paged_decoder_without_lengths(cuda, flat):
+    """A batch whose sequences all have max_len tokens needs no lengths on the device: dense, and anchor and
+    reuse layers of one row width, give what they give with them.  Dense and anchor layers address the
+    cache by the block table alone, so any contiguous [...,G,D] view of its memory does for them."""
+    from kascade_amd import workloads
+    from kascade_amd.strategy import PagedKascadeDecoder
+    n = 2100
+    c = workloads.paged_decode_inputs([n, n], seed=21, device=cuda)
+    maps = [list(range(G)), list(range(G)), c.head_mapping]
+    dec = PagedKascadeDecoder(10, maps, [0, 1], 2, n, page_size=c.page_size, device=cuda)
+    view = (lambda x: x.view(-1, G, D)) if flat else (lambda x: x)
+    full = [dec.dense(c.q, c.k_pages, c.v_pages, c.block_table, c.seqlens, n)]
+    bare = [dec.dense(c.q, view(c.k_pages), view(c.v_pages), c.block_table, None, n)]
+    for outs, lens, pages in ((full, c.seqlens, lambda x: x), (bare, None, view)):
+        outs.append(dec.forward(0, c.q, pages(c.k_pages), pages(c.v_pages), c.block_table, lens, n, ragged=False))
+        outs.append(dec._topk_to_reuse.clone())
+        outs.append(dec.forward(2, c.q, c.k_pages, c.v_pages, c.block_table, lens, n, ragged=False))
+        outs.append(dec.forward(1, c.q, c.k_pages, c.v_pages, c.block_table, lens, n, ragged=False))
+    assert all(torch.equal(a, b) for a, b in zip(full, bare))
+
+
+@pytest.mark.parametrize("L", [300, 19000])
+def test_decode_seam_takes_lists_longer_than_the_cache(cuda, L):
+    """The seam's topk is the caller's: a list wider than the cache names every token and the positions behind
+    them, as the selection call has it."""
+    from kascade_amd import kernels
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    g = torch.Generator().manual_seed(L)
+    q = torch.randn(1, H, D, generator=g).half().to(cuda)
+    k, v = (torch.randn(1, L, G, D, generator=g).half().to(cuda) for _ in range(2))
+    s = EfficientKascadeStrategy([0], None, k=10, tile_size=TILE, head_mapping=[list(range(G))] * 2, register=False)
+    o = s._decode_recomp_forward(q, k, v, L + 84, 1)
+    ns = 2
+    want, idx, _ = kernels.decode_full_kernel(q, k, v, L + 84, torch.empty(1, H, ns, device=cuda),
+                                              torch.empty(1, H, ns, D, device=cuda), torch.empty(1, H, device=cuda),
+                                              torch.empty(1, H, (L + 7) // 8 * 8, device=cuda), layer=1)
+    assert torch.equal(s._topk_to_reuse, idx)
+    assert_close(o, want, "output")
