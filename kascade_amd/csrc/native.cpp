@@ -3,7 +3,9 @@
 // ABI call on the current stream -- in one call.  The same steps as Python cost 20 to 35 us per layer,
 // several times what the layer's kernels take on short contexts.
 //
-// Positional arguments only (vectorcall); tensors are torch tensors.  Errors raise KascadeError.
+// Positional arguments only (vectorcall); tensors are torch tensors.  Errors raise KascadeError.  The
+// arguments are read with the interpreter lock held; it is released while memory is taken from the
+// allocator (which may wait for the device) and the kernels are launched.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
@@ -12,6 +14,7 @@
 #include <c10/core/impl/VirtualGuardImpl.h>
 
 #include <map>
+#include <string>
 
 #include "../../include/kascade_hip.h"
 
@@ -19,15 +22,27 @@ namespace {
 
 PyObject *g_error = nullptr, *g_raw_stream = nullptr, *g_capturing = nullptr;
 
-struct Fail {};   // a Python error is set
+struct Fail {};                             // a Python error is set
+struct Refused { std::string message; };    // becomes a KascadeError; thrown with or without the lock
 
 [[noreturn]] void fail(const char* fmt, ...) {
+    char text[1100];   // the library's own messages have up to 1023 characters
     va_list ap;
     va_start(ap, fmt);
-    PyErr_FormatV(g_error, fmt, ap);
+    vsnprintf(text, sizeof(text), fmt, ap);
     va_end(ap);
-    throw Fail{};
+    throw Refused{text};
 }
+
+// Without the interpreter lock until the end of the scope.
+class Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+public:
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    Unlocked& operator=(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 
 void need(bool ok, const char* msg) {
     if (!ok) fail("%s", msg);
@@ -125,6 +140,8 @@ void counters_dealloc(PyObject* o) {
 }
 PyTypeObject CountersType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// With the lock held, which also orders threads that share the object; two that miss at once make an array
+// each, and the later one stays.
 at::Tensor counters_for(PyObject* o, void* stream, int64_t n, const at::Tensor& like) {
     if (Py_TYPE(o) != &CountersType) fail("expected a _native.Counters object");
     PyObject* c = PyObject_CallNoArgs(g_capturing);
@@ -133,11 +150,15 @@ at::Tensor counters_for(PyObject* o, void* stream, int64_t n, const at::Tensor& 
     Py_DECREF(c);
     const auto options = like.options().dtype(at::kInt);
     // A graph replays on any stream and outlives this object: counters of its own, from its memory pool.
-    if (capturing) return at::zeros({n}, options);
+    auto zeros = [&](int64_t size) {
+        Unlocked unlocked;
+        return at::zeros({size}, options);
+    };
+    if (capturing) return zeros(n);
     auto& map = *reinterpret_cast<Counters*>(o)->by_stream;
     auto it = map.find(stream);
     if (it != map.end() && it->second.numel() >= n && it->second.device() == like.device()) return it->second;
-    const at::Tensor t = at::zeros({std::max<int64_t>(n, 1024)}, options);
+    const at::Tensor t = zeros(std::max<int64_t>(n, 1024));
     if (map.size() >= 16) map.clear();   // a program that keeps making streams
     map[stream] = t;
     return t;
@@ -185,31 +206,45 @@ const at::Tensor& head_map(PyObject* o, int64_t groups) {
     return hm;
 }
 
-void hf_reuse(const HfTensors& h, const at::Tensor& idx, const at::Tensor& hm, PyObject* counters, const at::Tensor& out,
-              int device, void* stream) {
-    const int64_t topk = idx.size(-1);
-    const int ns = topk <= kascade_gather_lone_rows(h.shape.group_size, (int)(h.B * h.G))
-                       ? 1 : num_split((double)h.B * h.G * topk, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
-    const int64_t parts = (h.B * h.H * ns + 63) / 64 * 64;
-    const at::Tensor scratch = empty_like_type({parts + h.B * h.H * ns * h.D}, h.q, at::kFloat);
+// Splits of a gather of lists of `topk` rows, and the merge counters it takes (lock held).
+struct Gather {
+    int64_t topk;
+    int ns;
     at::Tensor sync;
-    if (ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) sync = counters_for(counters, stream, h.B * h.G, h.q);
+};
+Gather plan_gather(const HfTensors& h, int64_t topk, PyObject* counters, void* stream) {
+    Gather g{topk, 1, {}};
+    if (topk > kascade_gather_lone_rows(h.shape.group_size, (int)(h.B * h.G)))
+        g.ns = num_split((double)h.B * h.G * topk, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
+    if (g.ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) g.sync = counters_for(counters, stream, h.B * h.G, h.q);
+    return g;
+}
+
+void hf_reuse(const HfTensors& h, const at::Tensor& idx, const at::Tensor& hm, const Gather& g, const at::Tensor& out,
+              void* stream) {
+    const int64_t parts = (h.B * h.H * g.ns + 63) / 64 * 64;
+    const at::Tensor scratch = empty_like_type({parts + h.B * h.H * g.ns * h.D}, h.q, at::kFloat);
     const kascade_strides st = HfTensors::strides(h.k);
     check(kascade_decode_reuse_paged_shaped_call(
         &h.shape, half_ptr(h.q), half_ptr(h.k), half_ptr(h.v), nullptr, int_ptr(idx), int_ptr(hm), 0.f, float_ptr(scratch),
-        float_ptr(scratch) + parts, half_ptr(out), (int)h.B, (int)h.L, (int)topk, ns, nullptr, 0, 1, &st, nullptr, nullptr,
-        sync.defined() ? int_ptr(sync) : nullptr, nullptr, stream));
+        float_ptr(scratch) + parts, half_ptr(out), (int)h.B, (int)h.L, (int)g.topk, g.ns, nullptr, 0, 1, &st, nullptr, nullptr,
+        g.sync.defined() ? int_ptr(g.sync) : nullptr, nullptr, stream));
 }
 
 // hf_decode_reuse(counters, query, key, value, topk_indices, head_mapping) -> O [B,1,H,D]
 PyObject* hf_decode_reuse(PyObject* const* a) {
     HfTensors h = hf_tensors(a + 1);
-    decode_layout(h);
     const at::Tensor& idx = index_lists(a[4], h);
     const at::Tensor& hm = head_map(a[5], h.G);
-    const int device = device_of_caller();
-    at::Tensor out = at::empty({h.B, 1, h.H, h.D}, h.q.options());
-    hf_reuse(h, idx, hm, a[0], out, device, stream_of(device));
+    void* stream = stream_of(device_of_caller());
+    const Gather g = plan_gather(h, idx.size(-1), a[0], stream);
+    at::Tensor out;
+    {
+        Unlocked unlocked;
+        decode_layout(h);
+        out = at::empty({h.B, 1, h.H, h.D}, h.q.options());
+        hf_reuse(h, idx, hm, g, out, stream);
+    }
     return THPVariable_Wrap(out);
 }
 
@@ -226,37 +261,43 @@ PyObject* pair(const at::Tensor& a, const at::Tensor& b) {
 // hf_decode_anchor(counters, query, key, value, with_output, width, identity_map) -> (O, topk_indices)
 PyObject* hf_decode_anchor(PyObject* const* a) {
     HfTensors h = hf_tensors(a + 1);
-    decode_layout(h);
     const bool with_output = truth(a[4]);
     const int64_t width = integer(a[5]);
     const at::Tensor& hm = head_map(a[6], h.G);
     need(width > 0, "the selection takes at least one token");
-    const int device = device_of_caller();
-    void* stream = stream_of(device);
+    void* stream = stream_of(device_of_caller());
     const int ns = num_split((double)h.B * h.G * h.L, (double)h.L, 0);
     const int64_t stride = (h.L + 7) / 8 * 8, heads = h.B * h.H;
     auto pad = [](int64_t x) { return (x + 63) / 64 * 64; };
     const int64_t n_lse = pad(heads * ns), n_part = with_output ? pad(heads * ns * h.D) : 0, n_sums = pad(heads);
-    const at::Tensor scratch = empty_like_type({n_lse + n_part + n_sums + heads * stride}, h.q, at::kFloat);
-    float* lse = float_ptr(scratch);
-    float *part = lse + n_lse, *sums = part + n_part, *scores = sums + n_sums;
-    const int64_t ws_bytes = kascade_topk_workspace_bytes((int)(h.B * h.G), h.L);
-    at::Tensor agg, ws, sync;
-    if (h.L > kascade_pool_select_row(h.shape.group_size, (int)(h.B * h.G))) {   // pooled and selected in two launches
-        agg = empty_like_type({h.B, h.G, stride}, h.q, at::kHalf);
-        if (ws_bytes > 0) ws = empty_like_type({ws_bytes}, h.q, at::kByte);
+    Gather g{};
+    at::Tensor sync;
+    if (!with_output) g = plan_gather(h, width, a[0], stream);
+    else if (ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) sync = counters_for(a[0], stream, h.B * h.G, h.q);
+    at::Tensor out, idx;
+    {
+        Unlocked unlocked;
+        decode_layout(h);
+        const at::Tensor scratch = empty_like_type({n_lse + n_part + n_sums + heads * stride}, h.q, at::kFloat);
+        float* lse = float_ptr(scratch);
+        float *part = lse + n_lse, *sums = part + n_part, *scores = sums + n_sums;
+        const int64_t ws_bytes = kascade_topk_workspace_bytes((int)(h.B * h.G), h.L);
+        at::Tensor agg, ws;
+        if (h.L > kascade_pool_select_row(h.shape.group_size, (int)(h.B * h.G))) {   // pooled and selected in two launches
+            agg = empty_like_type({h.B, h.G, stride}, h.q, at::kHalf);
+            if (ws_bytes > 0) ws = empty_like_type({ws_bytes}, h.q, at::kByte);
+        }
+        out = at::empty({h.B, 1, h.H, h.D}, h.q.options());
+        idx = empty_like_type({h.B, h.G, width}, h.q, at::kInt);
+        const kascade_strides st = HfTensors::strides(h.k);
+        check(kascade_decode_anchor_topk_call(
+            &h.shape, half_ptr(h.q), half_ptr(h.k), half_ptr(h.v), nullptr, lse, part, sums, scores,
+            with_output ? half_ptr(out) : nullptr, agg.defined() ? half_ptr(agg) : nullptr, int_ptr(idx), nullptr, (int)h.B,
+            (int)h.L, (int)stride, ns, with_output, (int)h.L, (int)width, 0, 0.f, nullptr, nullptr,
+            ws.defined() ? ws.data_ptr() : nullptr, nullptr, 0, 1, &st, nullptr, nullptr,
+            sync.defined() ? int_ptr(sync) : nullptr, stream));
+        if (!with_output) hf_reuse(h, idx, hm, g, out, stream);
     }
-    if (with_output && ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) sync = counters_for(a[0], stream, h.B * h.G, h.q);
-    at::Tensor out = at::empty({h.B, 1, h.H, h.D}, h.q.options());
-    at::Tensor idx = empty_like_type({h.B, h.G, width}, h.q, at::kInt);
-    const kascade_strides st = HfTensors::strides(h.k);
-    check(kascade_decode_anchor_topk_call(
-        &h.shape, half_ptr(h.q), half_ptr(h.k), half_ptr(h.v), nullptr, lse, part, sums, scores,
-        with_output ? half_ptr(out) : nullptr, agg.defined() ? half_ptr(agg) : nullptr, int_ptr(idx), nullptr, (int)h.B,
-        (int)h.L, (int)stride, ns, with_output, (int)h.L, (int)width, 0, 0.f, nullptr, nullptr,
-        ws.defined() ? ws.data_ptr() : nullptr, nullptr, 0, 1, &st, nullptr, nullptr,
-        sync.defined() ? int_ptr(sync) : nullptr, stream));
-    if (!with_output) hf_reuse(h, idx, hm, a[0], out, device, stream);
     return pair(out, idx);
 }
 
@@ -281,8 +322,15 @@ PyObject* hf_prefill_reuse(PyObject* const* a) {
     prompt_layout(h);
     const at::Tensor& idx = index_lists(a[3], h);
     const at::Tensor& hm = head_map(a[4], h.G);
-    at::Tensor out = at::empty({h.B, h.L, h.H, h.D}, h.q.options());
-    prompt_reuse(h, idx, hm, (float)number(a[5]), truth(a[6]), out, stream_of(device_of_caller()));
+    const float percent = (float)number(a[5]);
+    const bool rolling = truth(a[6]);
+    void* stream = stream_of(device_of_caller());
+    at::Tensor out;
+    {
+        Unlocked unlocked;
+        out = at::empty({h.B, h.L, h.H, h.D}, h.q.options());
+        prompt_reuse(h, idx, hm, percent, rolling, out, stream);
+    }
     return THPVariable_Wrap(out);
 }
 
@@ -297,20 +345,26 @@ PyObject* hf_prefill_anchor(PyObject* const* a) {
     const at::Tensor& nsel = dense(a[6], at::kInt, "n_sel");
     const at::Tensor& hm = head_map(a[7], h.G);
     need(valid.numel() == T && nsel.numel() == T, "valid_len and n_sel must have one entry per tile");
+    const float percent = (float)number(a[8]);
+    const bool rolling = truth(a[9]);
     void* stream = stream_of(device_of_caller());
     const kascade_strides qs = HfTensors::strides(h.q), ks = HfTensors::strides(h.k);
-    const at::Tensor log_sum = empty_like_type({h.B, h.L, h.H}, h.q, at::kFloat);
-    const at::Tensor scores = empty_like_type({h.B, h.G, T, h.L}, h.q, at::kHalf);
-    at::Tensor out = at::empty({h.B, h.L, h.H, h.D}, h.q.options());
-    at::Tensor idx = empty_like_type({h.B, h.G, T, width}, h.q, at::kInt);
-    check(kascade_prefill_dense_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), with_output ? half_ptr(h.v) : nullptr,
-                                            float_ptr(log_sum), with_output ? half_ptr(out) : nullptr, (int)h.B, (int)h.L,
-                                            qs, ks, with_output, stream));
-    check(kascade_prefill_aggregate_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), float_ptr(log_sum), half_ptr(scores),
-                                                (int)h.B, (int)h.L, qs, ks, 0, stream));
-    check(kascade_topk_call(half_ptr(scores), int_ptr(idx), (int)(h.B * h.G * T), h.L, (int)h.L, int_ptr(valid),
-                            int_ptr(nsel), (int)T, (int)width, (int)h.L - 1, nullptr, stream));
-    if (!with_output) prompt_reuse(h, idx, hm, (float)number(a[8]), truth(a[9]), out, stream);
+    at::Tensor out, idx;
+    {
+        Unlocked unlocked;
+        const at::Tensor log_sum = empty_like_type({h.B, h.L, h.H}, h.q, at::kFloat);
+        const at::Tensor scores = empty_like_type({h.B, h.G, T, h.L}, h.q, at::kHalf);
+        out = at::empty({h.B, h.L, h.H, h.D}, h.q.options());
+        idx = empty_like_type({h.B, h.G, T, width}, h.q, at::kInt);
+        check(kascade_prefill_dense_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), with_output ? half_ptr(h.v) : nullptr,
+                                                float_ptr(log_sum), with_output ? half_ptr(out) : nullptr, (int)h.B, (int)h.L,
+                                                qs, ks, with_output, stream));
+        check(kascade_prefill_aggregate_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), float_ptr(log_sum), half_ptr(scores),
+                                                    (int)h.B, (int)h.L, qs, ks, 0, stream));
+        check(kascade_topk_call(half_ptr(scores), int_ptr(idx), (int)(h.B * h.G * T), h.L, (int)h.L, int_ptr(valid),
+                                int_ptr(nsel), (int)T, (int)width, (int)h.L - 1, nullptr, stream));
+        if (!with_output) prompt_reuse(h, idx, hm, percent, rolling, out, stream);
+    }
     return pair(out, idx);
 }
 
@@ -336,13 +390,16 @@ PagedTensors paged_tensors(PyObject* const* a, long long page, bool counted) {
     return t;
 }
 
+// The caller's output, or none yet.
 at::Tensor out_buffer(PyObject* o, const PagedTensors& t) {
-    if (o == Py_None) return at::empty({t.B, t.H, t.D}, t.q.options());
+    if (o == Py_None) return {};
     const at::Tensor& out = dense(o, t.q.scalar_type(), "out");
     if (out.dim() != 3 || out.size(0) != t.B || out.size(1) != t.H || out.size(2) != t.D)
         fail("out must be [%lld,%lld,%lld]", (long long)t.B, (long long)t.H, (long long)t.D);
     return out;
 }
+
+at::Tensor fresh_out(const PagedTensors& t) { return at::empty({t.B, t.H, t.D}, t.q.options()); }
 
 const kascade_half* new_rows(PyObject* o, const PagedTensors& t, const char* name) {
     if (o == Py_None) return nullptr;
@@ -390,11 +447,19 @@ PyObject* paged_reuse(PyObject* const* a) {
     float *lse, *part;
     scratch_of(a[7], a[8], t, ns, &lse, &part);
     const at::Tensor& bt = table_of(a[10], t.B);
+    const float percent = (float)number(a[6]);
+    const kascade_half *k_new = new_rows(a[14], t, "k_new"), *v_new = new_rows(a[15], t, "v_new");
+    int32_t* sync = sync_of(a[13], t);
+    void* stream = stream_of(device_of_caller());
     at::Tensor out = out_buffer(a[12], t);
-    check(kascade_decode_reuse_rows_shaped_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, int_ptr(rows), int_ptr(hm), (float)number(a[6]),
-        lse, part, half_ptr(out), (int)t.B, (int)rows.size(2), (int)ns, int_ptr(bt), (int)bt.size(1), (int)t.page, (int)t.P,
-        new_rows(a[14], t, "k_new"), new_rows(a[15], t, "v_new"), sync_of(a[13], t), nullptr, stream_of(device_of_caller())));
+    {
+        Unlocked unlocked;
+        if (!out.defined()) out = fresh_out(t);
+        check(kascade_decode_reuse_rows_shaped_call(
+            &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, int_ptr(rows), int_ptr(hm), percent, lse, part,
+            half_ptr(out), (int)t.B, (int)rows.size(2), (int)ns, int_ptr(bt), (int)bt.size(1), (int)t.page, (int)t.P, k_new,
+            v_new, sync, nullptr, stream));
+    }
     return THPVariable_Wrap(out);
 }
 
@@ -421,21 +486,28 @@ PyObject* paged_anchor(PyObject* const* a) {
         valid = int_ptr(v);
         nsel = int_ptr(n);
     }
+    const float percent = (float)number(a[12]);
+    const kascade_half *k_new = new_rows(a[19], t, "k_new"), *v_new = new_rows(a[20], t, "v_new");
+    int32_t* sync = sync_of(a[18], t);
     void* stream = stream_of(device_of_caller());
-    at::Tensor out, agg, ws;
+    at::Tensor out, idx, agg, ws;
     if (with_output) out = out_buffer(a[17], t);
-    if (max_len > kascade_pool_select_row(t.shape.group_size, (int)(t.B * t.G))) {
-        agg = empty_like_type({t.B, t.G, stride}, t.q, at::kHalf);
-        const int64_t bytes = kascade_topk_workspace_bytes((int)(t.B * t.G), max_len);
-        if (bytes > 0) ws = empty_like_type({bytes}, t.q, at::kByte);
+    {
+        Unlocked unlocked;
+        if (with_output && !out.defined()) out = fresh_out(t);
+        if (max_len > kascade_pool_select_row(t.shape.group_size, (int)(t.B * t.G))) {
+            agg = empty_like_type({t.B, t.G, stride}, t.q, at::kHalf);
+            const int64_t bytes = kascade_topk_workspace_bytes((int)(t.B * t.G), max_len);
+            if (bytes > 0) ws = empty_like_type({bytes}, t.q, at::kByte);
+        }
+        idx = empty_like_type({t.B, t.G, width}, t.q, at::kInt);
+        check(kascade_decode_anchor_topk_call(
+            &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, float_ptr(sums), float_ptr(scores),
+            with_output ? half_ptr(out) : nullptr, agg.defined() ? half_ptr(agg) : nullptr, int_ptr(idx), int_ptr(rows),
+            (int)t.B, (int)max_len, (int)stride, (int)ns, with_output, (int)max_len, (int)width, 0, percent, valid,
+            nsel, ws.defined() ? ws.data_ptr() : nullptr, int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr, k_new, v_new, sync,
+            stream));
     }
-    at::Tensor idx = empty_like_type({t.B, t.G, width}, t.q, at::kInt);
-    check(kascade_decode_anchor_topk_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, float_ptr(sums), float_ptr(scores),
-        with_output ? half_ptr(out) : nullptr, agg.defined() ? half_ptr(agg) : nullptr, int_ptr(idx), int_ptr(rows),
-        (int)t.B, (int)max_len, (int)stride, (int)ns, with_output, (int)max_len, (int)width, 0, (float)number(a[12]), valid,
-        nsel, ws.defined() ? ws.data_ptr() : nullptr, int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr,
-        new_rows(a[19], t, "k_new"), new_rows(a[20], t, "v_new"), sync_of(a[18], t), stream));
     if (!with_output) {
         PyObject* i = THPVariable_Wrap(idx);
         if (!i) throw Fail{};
@@ -455,11 +527,18 @@ PyObject* paged_dense(PyObject* const* a) {
     float *lse, *part;
     scratch_of(a[4], a[5], t, ns, &lse, &part);
     const at::Tensor& bt = table_of(a[8], t.B);
+    const int max_len = (int)integer(a[7]);
+    const kascade_half *k_new = new_rows(a[12], t, "k_new"), *v_new = new_rows(a[13], t, "v_new");
+    int32_t* sync = sync_of(a[11], t);
+    void* stream = stream_of(device_of_caller());
     at::Tensor out = out_buffer(a[10], t);
-    check(kascade_decode_dense_paged_shaped_call(
-        &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, half_ptr(out), (int)t.B,
-        (int)integer(a[7]), (int)ns, int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr, new_rows(a[12], t, "k_new"),
-        new_rows(a[13], t, "v_new"), sync_of(a[11], t), stream_of(device_of_caller())));
+    {
+        Unlocked unlocked;
+        if (!out.defined()) out = fresh_out(t);
+        check(kascade_decode_dense_paged_shaped_call(
+            &t.shape, half_ptr(t.q), half_ptr(t.k), half_ptr(t.v), lens, lse, part, half_ptr(out), (int)t.B, max_len, (int)ns,
+            int_ptr(bt), (int)bt.size(1), (int)t.page, nullptr, k_new, v_new, sync, stream));
+    }
     return THPVariable_Wrap(out);
 }
 
@@ -479,6 +558,9 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
     try {
         return F(args);
     } catch (const Fail&) {
+        return nullptr;
+    } catch (const Refused& e) {
+        PyErr_SetString(g_error, e.message.c_str());
         return nullptr;
     }
     END_HANDLE_TH_ERRORS

@@ -285,3 +285,40 @@ def test_decode_seam_takes_lists_longer_than_the_cache(cuda, L):
                                               torch.empty(1, H, (L + 7) // 8 * 8, device=cuda), layer=1)
     assert torch.equal(s._topk_to_reuse, idx)
     assert_close(o, want, "output")
+
+
+def test_other_threads_run_during_a_layer_call(cuda):
+    """A layer call lets go of the interpreter lock while it takes memory and launches.  With a switch interval
+    beyond the test's length a waiting thread runs only where this one lets go by itself."""
+    import sys
+    import threading
+    import time
+    from kascade_amd import _lib
+    native = _lib.native()
+    q = torch.randn(1, H, 1, D, device=cuda).half()
+    k = torch.randn(1, G, 2000, D, device=cuda).half()
+    idx = torch.arange(256, device=cuda, dtype=torch.int32).expand(1, G, 256).contiguous()
+    same = torch.arange(G, device=cuda, dtype=torch.int32)
+    counters = native.Counters()
+    turns, stop, ready = [0], [False], threading.Event()
+
+    def other():
+        ready.set()
+        while not stop[0]:
+            turns[0] += 1
+            time.sleep(0)
+    before = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    try:
+        sys.setswitchinterval(1000.0)   # before the thread first waits for the lock
+        thread.start()
+        ready.wait()
+        start = turns[0]
+        held = []   # dropping a tensor may let go of the lock too
+        while turns[0] == start and len(held) < 5000:
+            held.append(native.hf_decode_reuse(counters, q, k, k, idx, same))
+        assert turns[0] > start
+    finally:
+        stop[0] = True
+        sys.setswitchinterval(before)
+        thread.join()
