@@ -2,11 +2,14 @@
 _native (host code against torch's C++ interface, linked to that library) with g++.
 
 Both are built in-tree (kascade_amd/libkascade_hip.so, kascade_amd/_native.so).  ``build()``
-always recompiles; ``ensure_built()`` compiles only when no library exists.
+always recompiles; ``ensure_built()`` compiles only when no library exists.  The library needs hipcc
+alone; without torch the extension, which only the Python strategies use, is left out, and without g++
+ROCm's own clang builds it.
 Run ``python -m kascade_amd.build`` to build from a shell.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -67,16 +70,27 @@ def build(verbose: bool = False, extra_flags=()) -> Path:
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wno-unused-command-line-argument",
           *map(str, objs), "-o", str(tmp)])
     os.replace(tmp, LIB_PATH)
-    build_native()
+    if _torch_root() is None:
+        print(f"torch is not installed: {LIB_PATH.name} is built, {NATIVE_PATH.name} (the Python strategies) is not")
+    else:
+        build_native()
     return LIB_PATH
+
+
+def _torch_root():
+    spec = importlib.util.find_spec("torch")
+    return Path(spec.origin).resolve().parent if spec and spec.origin else None
+
+
+def _host_compiler() -> str:
+    return shutil.which("g++") or str(Path(_hipcc()).resolve().parent / "amdclang++")
 
 
 def build_native() -> Path:
     """The host extension: plain C++ (no device code), so g++ builds it."""
-    import torch
-    root = Path(torch.__file__).resolve().parent
+    root = _torch_root()
     tmp = NATIVE_PATH.with_suffix(".so.tmp")
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{root / 'include'}",
+    _run([_host_compiler(), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{root / 'include'}",
           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "native.cpp"), f"-L{PKG_DIR}", "-l:libkascade_hip.so",
           f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN", "-o", str(tmp)])
     os.replace(tmp, NATIVE_PATH)
@@ -84,7 +98,7 @@ def build_native() -> Path:
 
 
 def ensure_built() -> Path:
-    if not (LIB_PATH.exists() and NATIVE_PATH.exists()):
+    if not LIB_PATH.exists() or not (NATIVE_PATH.exists() or _torch_root() is None):
         build()
     return LIB_PATH
 

@@ -252,3 +252,37 @@ def test_prefill_seam_refuses_tiles_the_kernels_do_not_have():
     for tile in (16, 64):
         with pytest.raises(KascadeError, match="tile_size"):
             s._prefill_recomp_forward(q, k, k, 128, tile, 0, 10)
+
+
+@pytest.mark.parametrize("torch_here", [True, False])
+@pytest.mark.parametrize("gxx_here", [True, False])
+def test_library_builds_with_hipcc_alone(monkeypatch, tmp_path, torch_here, gxx_here):
+    """The C library needs hipcc only; the extension module of the Python strategies needs torch, and any host
+    compiler, ROCm's among them."""
+    import shutil
+    from pathlib import Path
+    from kascade_amd import build
+    ran = []
+
+    def run(cmd):
+        ran.append([str(x) for x in cmd])
+        Path(ran[-1][ran[-1].index("-o") + 1]).touch()
+        return ""
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "PKG_DIR", tmp_path)
+    monkeypatch.setattr(build, "LIB_PATH", tmp_path / "libkascade_hip.so")
+    monkeypatch.setattr(build, "NATIVE_PATH", tmp_path / "_native.so")
+    monkeypatch.setattr(build, "_hipcc", lambda: "/opt/rocm/bin/hipcc")
+    if not torch_here:
+        monkeypatch.setattr(build, "_torch_root", lambda: None)
+    which = shutil.which
+    monkeypatch.setattr(shutil, "which", lambda name: (which(name) if gxx_here or name != "g++" else None))
+    assert build.build() == tmp_path / "libkascade_hip.so" and build.LIB_PATH.exists()
+    native = [c for c in ran if any("native.cpp" in x for x in c)]
+    assert len(native) == (1 if torch_here else 0) and build.NATIVE_PATH.exists() == torch_here
+    assert all(c[0] == "/opt/rocm/bin/hipcc" for c in ran if c not in native)
+    if native and not gxx_here:
+        assert native[0][0].endswith("amdclang++")
+    count = len(ran)
+    build.ensure_built()
+    assert len(ran) == count
