@@ -1,11 +1,15 @@
 // Exact per-row top-n selection over fp16 scores (radix select on the 16-bit
-// order-preserving key), one 1024-thread workgroup per row:
+// order-preserving key):
 //   pass 1  LDS histogram of the high 11 key bits, suffix scan -> threshold bin
 //   pass 2  LDS histogram of the low 5 bits inside that bin -> exact threshold
 //           key T and the number r of entries equal to T that still fit
 //   pass 3  ordered compaction: entries > T and the first r entries == T, written
 //           in ascending index order (deterministic, ties to the lower index)
-// The row is streamed from L2/HBM three times as 16-byte loads.
+// Rows of up to 131072 entries are held in the registers of one workgroup of 256 to 1024 threads
+// (topk_select_reg_kernel; decode anchors pool into those registers, decode_pool_select_kernel).  Longer
+// rows run the passes over chunks on several workgroups per row (topk_split_*), given a workspace.  What
+// is left -- longer rows without one, tensors that start off a 16-byte boundary -- streams the row three
+// times through one workgroup (topk_select_kernel).
 #include "topk.h"
 
 #include <type_traits>
@@ -272,8 +276,9 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(
 //    above / equal to T are sums of min(sat(key - (T-1)), 2) over packed halves.
 //  * The selected positions are staged in LDS in their final order, so that the list leaves as
 //    full-width stores.
-// Causal prompt tiles (8 heads x L/32 rows, ragged): L = 4096 18.2 -> 10.2 us, 8192 34 -> 20, 16384
-// 73 -> 48, 32768 178 -> 151, 65536 905 -> 584 us; 2048 full rows of 65536: 141 us = 1.9 TB/s.
+// Causal prompt tiles (8 heads x L/32 rows, ragged), against one size of workgroup with a scan over all
+// (chunk, wavefront) pairs: L = 4096 18.6 -> 9.4 us, 8192 34.6 -> 20.5, 16384 73.6 -> 48.8, 32768 179 -> 150,
+// 65536 907 -> 587 us; 2048 full rows of 65536: 175 -> 143 us = 1.9 TB/s.
 // Sum of the entries of s_wave before `wave`, and of all of them (one per wavefront, in LDS).
 template <int THREADS>
 __device__ __forceinline__ void scan_waves(const uint32_t* s_wave, int wave, uint32_t& before, uint32_t& all) {

@@ -25,8 +25,19 @@ def _check_rows(scores, idx, n_of, valid_of, what):
 @pytest.mark.parametrize("L", [1, 8, 511, 513, 2048, 2049, 4096, 4097, 8193, 16384, 16385, 32768, 32769, 65536])
 @pytest.mark.parametrize("rows", [3, 257])
 def test_register_selection_edges(cuda, L, rows):
-    """Longest row of every workgroup size and chunk count, one more entry, and both sides of the
-    row count at which long rows change the workgroup size.  The selection is exact: no tolerance."""
+    """Longest row of every workgroup size and chunk count, one more entry, and both sides of the 256 rows
+    at which rows beyond 32768 entries change the workgroup size.  The selection is exact: no tolerance."""
+    _check_selection(cuda, L, rows)
+
+
+@pytest.mark.parametrize("L", [16384, 16385, 32768])
+@pytest.mark.parametrize("rows", [512, 513])
+def test_register_selection_on_both_sides_of_512_rows(cuda, L, rows):
+    """Rows of 16385 to 32768 entries take workgroups of 1024 threads up to 512 rows and of 512 beyond."""
+    _check_selection(cuda, L, rows)
+
+
+def _check_selection(cuda, L, rows):
     from kascade_amd import kernels
     gen = torch.Generator().manual_seed(L)
     base = (torch.rand(3, L, generator=gen) ** 4 * 512).round().half() / 512      # many ties

@@ -322,3 +322,32 @@ def test_other_threads_run_during_a_layer_call(cuda):
         stop[0] = True
         sys.setswitchinterval(before)
         thread.join()
+
+
+@pytest.mark.parametrize("streams", [2, 17])
+def test_eager_decode_on_several_streams(cuda, streams):
+    """Merge counters belong to a stream: layers of one strategy that run on several at the same time give the
+    bits of one stream, and so do the calls after the seventeenth stream, where the arrays kept for the others
+    are let go."""
+    from kascade_amd.strategy import EfficientKascadeStrategy
+    L = 9000
+    g = torch.Generator(device=cuda).manual_seed(6)
+    q = torch.randn(2, H, 1, D, device=cuda, generator=g).half()
+    k, v = (torch.randn(2, G, L, D, device=cuda, generator=g).half() for _ in range(2))
+    s = EfficientKascadeStrategy([0], None, k=10, tile_size=TILE, head_mapping=[list(range(G))] * 2, register=False)
+
+    def step():
+        o0, _ = s.attention_forward(_Module(0), q, k, v, None, D ** -0.5)
+        idx = s._topk_to_reuse
+        return o0, idx, s.attention_forward(_Module(1), q, k, v, None, D ** -0.5)[0]
+    want = step()
+    torch.cuda.synchronize()
+    all_streams = [torch.cuda.Stream() for _ in range(streams)]
+    got = []
+    for _ in range(6):
+        for st in all_streams:
+            with torch.cuda.stream(st):
+                got.append(step())
+    torch.cuda.synchronize()
+    assert len({st.cuda_stream for st in all_streams}) == streams
+    assert all(torch.equal(a, b) for one in got for a, b in zip(one, want))
