@@ -605,7 +605,9 @@ void topk_select_reg_kernel(
 // sum_h exp2(score - lse_h), rounded to fp16 as decode_aggregate_kernel rounds it, and goes straight
 // into the selection's registers: no pooled row in memory, one launch instead of two (merge of the
 // log-sums included).  Masked tokens need no test of their own (one per code costs a quarter of the
-// pooling, 1.1 us at 16384 tokens of 4 heads, 3.3 of 8): see kScoreNone in decode.h.  Bound by the latency of one workgroup: its exponentials (8 per head and lane and
+// pooling, 1.1 us at 16384 tokens of 4 heads, 3.3 of 8) unless a log-sum leaves the range the codes are
+// made for: a row with nothing but masked tokens, or scores so large that their sum came out as nothing.
+// See kScoreNone in decode.h.  Bound by the latency of one workgroup: its exponentials (8 per head and lane and
 // chunk) and the selection's scans; kascade_pool_select_row has the line up to which the saved launch
 // pays for the few compute units it uses, with both sides measured.
 template <int THREADS, int MAXC>
@@ -649,12 +651,11 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
             for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
             const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
             if (lane == 0) {
-                s_lse[h] = (v == -INFINITY) ? 0.f : v;   // nothing but masked tokens: every reference is -inf
+                s_lse[h] = v;
                 p.row_sums[head] = v;
             }
         } else if (lane == 0) {
-            const float v = p.row_sums[head];
-            s_lse[h] = (v == -INFINITY) ? 0.f : v;
+            s_lse[h] = p.row_sums[head];
         }
     }
     if (row_len <= n || n == 0) {
@@ -679,6 +680,24 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
             bt.q[u] = *reinterpret_cast<const uint4_t*>(reinterpret_cast<const uint16_t*>(hr) + jc);
             bt.ref[u] = hr[p.scores_stride / 2 + (jc >> 6)];
         }
+    };
+    // packed order keys of a piece: no entry is negative, so the key is the value with the top bit set
+    auto keys_of = [&](const float (&sum)[8], int j0) {
+        uint4_t d;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const half2_t x = {(half_t)sum[e], (half_t)sum[e + 1]};
+            d[e >> 1] = __builtin_bit_cast(uint32_t, x) | 0x80008000u;
+        }
+        if (j0 + 8 > len) {   // the piece at the tokens' end and those behind it: probability 0, or no entry
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int sh = 16 * (e & 1);
+                const uint32_t key = j0 + e < len ? (d[e >> 1] >> sh) & 0xFFFFu : j0 + e < row_len ? 0x8000u : 0u;
+                d[e >> 1] = (d[e >> 1] & (0xFFFF0000u >> sh)) | (key << sh);
+            }
+        }
+        return d;
     };
     uint4_t data[MAXC];
     Batch cur, n1, n2;
@@ -711,22 +730,35 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
                     }
                 }
             }
-            // packed order keys: no entry is negative, so the key is the value with the top bit set
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const half2_t x = {(half_t)sum[e], (half_t)sum[e + 1]};
-                data[c][e >> 1] = __builtin_bit_cast(uint32_t, x) | 0x80008000u;
-            }
-            if (j0 + 8 > len) {   // the piece at the tokens' end and those behind it: probability 0, or no entry
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int sh = 16 * (e & 1);
-                    const uint32_t key = j0 + e < len ? (data[c][e >> 1] >> sh) & 0xFFFFu : j0 + e < row_len ? 0x8000u : 0u;
-                    data[c][e >> 1] = (data[c][e >> 1] & (0xFFFF0000u >> sh)) | (key << sh);
-                }
-            }
+            data[c] = keys_of(sum, j0);
         }
     });
+    // A log-sum outside the range the codes are made for: the same sums again, every code tested for the mark.
+    // (Up to kSane a reference lies less than one step above its log-sum, whatever their rounding.)
+    constexpr float kSane = 1048576.f;
+    const bool odd = lane < p.group_size && !(fabsf(s_lse[min(lane, kMaxGroup - 1)]) < kSane);
+    if (__ballot(odd) != 0) {   // the same in every wavefront
+        static_for<0, MAXC>([&](auto c_c) {
+            constexpr int c = decltype(c_c)::value;
+            const int j0 = first + c * 512, jc = min(j0, last_piece);
+            if (c < nch) {
+                float sum[8] = {};
+#pragma clang loop unroll(disable)
+                for (int h = 0; h < p.group_size; ++h) {
+                    const float* hr = base + (long long)h * p.scores_stride;
+                    const uint4_t codes = *reinterpret_cast<const uint4_t*>(reinterpret_cast<const uint16_t*>(hr) + jc);
+                    const float ref = hr[p.scores_stride / 2 + (jc >> 6)] - s_lse[h];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const uint32_t q = (e & 1) ? codes[e >> 1] >> 16 : codes[e >> 1] & 0xFFFFu;
+                        const float pr = fast_exp2(__builtin_fmaf((float)q, -1.f / kScoreSteps, ref));
+                        sum[e] += (q == kScoreNone) ? 0.f : pr;
+                    }
+                }
+                data[c] = keys_of(sum, j0);
+            }
+        });
+    }
     select_row<THREADS, MAXC, true>(data, nch, 0, row_len, n, k, fill, out, row, ro);
 }
 

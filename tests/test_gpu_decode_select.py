@@ -216,3 +216,23 @@ def test_anchor_selection_with_and_without_buffers_for_two_launches(cuda, H, G, 
         torch.cuda.synchronize()
         got.append((idx, rows, sums))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("H,G,L", [(8, 8, 700), (32, 8, 2100), (16, 1, 9001)])
+def test_scores_beyond_the_codes_range_in_one_call(cuda, H, G, L):
+    """bf16 scores around 1e19, where a sum of exponentials in 32 bits can come out as nothing, with tokens whose
+    score overflows to -inf for some heads only: the lists are those of the two-launch route all the same."""
+    from kascade_amd import _lib, kernels
+    D, k_sel = 128, 128
+    gen = torch.Generator().manual_seed(L)
+    q, k = torch.randn(1, H, 1, D, generator=gen), torch.randn(1, G, L, D, generator=gen)
+    q[:, ::2, :, 3], q[:, 1::2, :, 3] = 1e20, 1.0
+    k[:, :, 100:300, 3] = -1e30
+    q, k = q.bfloat16().to(cuda), k.bfloat16().to(cuda)
+    glse, sums = torch.empty(1, H, 3, device=cuda), torch.empty(1, H, device=cuda)
+    scores = torch.empty(1, H, (L + 7) // 8 * 8, device=cuda)
+    _, agg = kernels.decode_recompute(q[:, :, 0], k.transpose(1, 2), k.transpose(1, 2), glse, None, sums, scores, 1)
+    want = kernels.topk_indices(agg[:, :, :L], k_sel, fill_value=0)
+    native = _lib.native()
+    _, idx = native.hf_decode_anchor(native.Counters(), q, k, k, False, k_sel, torch.arange(G, device=cuda, dtype=torch.int32))
+    assert torch.equal(idx, want)
