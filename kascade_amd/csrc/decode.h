@@ -13,9 +13,8 @@ namespace kascade {
 // below what survives the pooled sum's fp16 rounding.  65535 marks a masked position (score -inf);
 // the reference of a granule with nothing else is -inf, so that even a reader that takes the mark for
 // a code gets probability 0 there and, next to a real maximum, 2^-32 of that -- under a finite log-sum.
-// Splits start at
-// multiples of 64 tokens, so a granule belongs to one workgroup.  Half the bytes of fp32 scores: their
-// write-back to HBM, interleaved with the K stream, costs several times its size.
+// Splits start at multiples of 64 tokens, so a granule belongs to one workgroup.  Half the bytes of
+// fp32 scores: their write-back to HBM, interleaved with the K stream, costs several times its size.
 constexpr float kScoreSteps = 2048.f;
 constexpr uint32_t kScoreNone = 65535u;
 

@@ -607,9 +607,9 @@ void topk_select_reg_kernel(
 // log-sums included).  Masked tokens need no test of their own (one per code costs a quarter of the
 // pooling, 1.1 us at 16384 tokens of 4 heads, 3.3 of 8) unless a log-sum leaves the range the codes are
 // made for: a row with nothing but masked tokens, or scores so large that their sum came out as nothing.
-// See kScoreNone in decode.h.  Bound by the latency of one workgroup: its exponentials (8 per head and lane and
-// chunk) and the selection's scans; kascade_pool_select_row has the line up to which the saved launch
-// pays for the few compute units it uses, with both sides measured.
+// See kScoreNone in decode.h.  Bound by the latency of one workgroup: its exponentials (8 per head and
+// lane and chunk) and the selection's scans; kascade_pool_select_row has the line up to which the saved
+// launch pays for the few compute units it uses, with both sides measured.
 template <int THREADS, int MAXC>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS > 512 ? 4 : THREADS > 256 ? 2 : 1, 4)))
 void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restrict__ out, RowsOut ro) {
