@@ -526,32 +526,50 @@ void prefill_attn_kernel_q64(PrefillParams p) {
 
 // Pooled tile scores: out[b,g,t,key] = sum over the 32 queries of tile t and the 4 q-heads of g
 // of exp2(s*scale - log_sum), for keys before the tile's first (global) position.
-// Two workgroups per compute unit (register budget 256): one wavefront's exponentials run
-// under the other's matrix instructions.
 //
-// A wavefront takes 32 keys of every 128-key tile and nobody else reads them.  Their rows go
+// A wavefront takes 32 keys (a slice) of every 128-key tile and nobody else reads them.  Their rows go
 // from global memory straight into the wavefront's own LDS area (whole rows per load: read as
 // B operands directly, a 16-byte piece of 32 different rows per instruction, the same bytes kept
 // the data-return path of the memory pipeline busy 96 % of the kernel) and come back as B
 // operands (lane = key, 8 elements at d = 16 ks + 8 lg) from the chunk-permuted rows.  Two buffers
-// per wavefront, no barrier in the tile loop: the loads of the next tile are issued one per
-// contraction step and waited for at the top of that tile.
+// per wavefront, no barrier in the tile loop.
+//
+// What bounds it: the chip's power (long calls run at 1.6 GHz) and the issue of vector instructions, three per
+// score (multiply-add, exponential, sum).  So
+//  * the products are 16x16x32: at the power limit, random operands in registers, that instruction
+//    sustains 1.84 PFLOP/s, 32x32x16 1.59 (both 2.4 on zeros).
+//  * the loop spends next to nothing on anything but scores: a row address is one 64-bit addition, a pointer
+//    per lane that never changes plus an offset in scalar registers.
+//  * the exponentials of one head's scores run between the next head's matrix instructions, across the tile
+//    boundary too.  A slice's rows are in registers from the tile before on, so a buffer is free for the
+//    slice after the next one a quarter into the tile and its loads have more than a tile's time.
+// 32/8 heads, against 32x32x16 products with the row addresses formed per lane and the last head's exponentials at the
+// tile's end: 1024 tokens 11.1 -> 9.9 us, 4096 83.2 -> 75.0, 8192 314 -> 275, 32768 4.63 -> 4.06 ms (1.08 PFLOP/s),
+// chunks at position 14336 of 2048 queries 318 -> 292, of 512 at 15872 96.3 -> 87.9.
 template <bool PAGED, int D, typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_aggregate_kernel(PrefillParams p) {
     typedef typename Elem<T>::x8 x8_t;
-    constexpr int kKS = D / 16;
+    constexpr int kSteps = D / 32;              // contraction steps
     constexpr int kChunks = D / 8;
     constexpr int kRPL = 64 / kChunks;          // rows per load instruction
     constexpr int kLoads = 32 / kRPL;           // load instructions per wavefront and tile
     constexpr int kWaveElems = 32 * D;          // a wavefront's 32 rows
+    constexpr int kBufBytes = 4 * kWaveElems * 2;
+    constexpr int kPatterns = kLoads / 2;       // chunk permutations: loads j and j + kPatterns have the same
+    static_assert(kLoads == 2 * kSteps, "a load behind every second matrix instruction of a head");
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
     const int kvh = p.G, nheads = p.G * hs.gs;
     const T* Qp = (const T*)p.Q;
     const T* Kp = (const T*)p.K;
-    __shared__ __attribute__((aligned(1024))) T sK[2 * 4 * kWaveElems];
-    __shared__ __attribute__((aligned(16))) float s_lse[128];
+    // the log-sums in front, where the LDS instructions' offsets reach them
+    __shared__ struct alignas(1024) {
+        float lse[128];
+        alignas(1024) T k[2 * 4 * kWaveElems];
+    } s_mem;
+    float* s_lse = s_mem.lse;
+    T* sK = s_mem.k;
 
     const int Ls = p.L;                  // width of a row of pooled scores
     const int Lq = p.Lq;
@@ -561,15 +579,12 @@ void prefill_aggregate_kernel(PrefillParams p) {
     blk -= part * p.T;
     int q_start, Lqv;                    // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
-    const int L = q_start + Lqv;         // keys of this sequence
     const int t = p.T - 1 - blk;
     const int tid = threadIdx.x;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int li = lane & 31;
-    const int lg = lane >> 5;
     const int tl = t * kTile;            // first query row of the tile
-    const int ts = q_start + tl;         // its global position
+    const int ts = q_start + tl;         // its global position: a multiple of 32
     half_t* out = p.agg + (((long long)b * kvh + g) * p.T + t) * Ls;
     const half_t neg_inf = (half_t)(-INFINITY);
 
@@ -584,34 +599,71 @@ void prefill_aggregate_kernel(PrefillParams p) {
             s_lse[tid] = counts ? p.log_sum_in[((long long)b * Lq + q) * nheads + head0 + (tid >> 5)] : INFINITY;
         }
 
-        // ---- staging: load j of a tile covers rows j kRPL + lrow of the wavefront's 32 ----
-        const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+        // ---- staging: load j of a slice covers rows j kRPL + lrow of its 32.  The wavefront's slices are
+        // those of tiles ti0 .. ti0 + n - 1: all of their keys lie before the query tile, none past the
+        // sequence's end ----
+        const int n = min(ti1 - ti0, (ts / 32 - (4 * ti0 + wave) + 3) / 4);
+        const int key0 = ti0 * kAggKT + 32 * wave;         // first key of slice 0
         const int lrow = lane / kChunks;
         const int lchunk = lane % kChunks;
-        const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
         const unsigned row_stride = PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl;
+        const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
+        const char* lane_ptr[kPatterns];
+#pragma unroll
+        for (int j = 0; j < kPatterns; ++j)
+            lane_ptr[j] = (const char*)(kbase + (long long)((unsigned long long)(unsigned)lrow * row_stride) +
+                                        (lchunk ^ swz16<D>(j * kRPL + lrow)) * 8);
         const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
         const int page_mask = (1 << p.page_shift) - 1;
-        const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * 4 * kWaveElems * 2
-        const T* my_k = sK + wave * kWaveElems;
-        // block-table entry of the key this lane stands for (row lane & 31 of the wavefront's 32),
-        // fetched a tile ahead; the lanes of a load pick theirs up with a lane permutation
-        int pg_next = 0;
-        auto fetch_page = [&](int ti) {
-            if (PAGED) pg_next = bt_row[min(ti * kAggKT + 32 * wave + li, L - 1) >> p.page_shift];
-        };
-        int pg_cur = 0;   // entries of the tile whose loads are being issued
-        auto issue_load = [&](int ti, int j, int buf) {
-            const int row = j * kRPL + lrow;
-            const int key = min(ti * kAggKT + 32 * wave + row, L - 1);
-            int src = key;
+        const uint32_t lds_w = lds_address(sK) + wave * (kWaveElems * 2);   // + buf * kBufBytes
+        // Block-table entries of 64 pages, one per lane (pages are at least four tokens, 64 of them two tiles),
+        // and of the 64 behind them
+        int pages = 0, pages_next = 0, page_group = 0;
+        auto fetch_pages = [&](int group) { return bt_row[min(64 * group + lane, p.max_pages - 1)]; };
+        if (PAGED && n > 0) {
+            page_group = (key0 >> p.page_shift) >> 6;
+            pages = fetch_pages(page_group);
+            pages_next = fetch_pages(page_group + 1);
+        }
+        unsigned long long row_off = 0;   // strided: offset of the next load's first row
+        const unsigned long long row_step = (unsigned long long)row_stride * (2 * kRPL);
+        auto offset_of_key = [&](int key) {   // uniform
+            int row = key;
             if (PAGED) {
-                const int pgv = __builtin_amdgcn_ds_bpermute(row << 2, pg_cur);
-                src = (pgv << p.page_shift) + (key & page_mask);
+                const int page = __builtin_amdgcn_readlane(pages, (key >> p.page_shift) & 63);
+                row = (page << p.page_shift) + (key & page_mask);
             }
-            const T* gp = kbase + (long long)((unsigned long long)(unsigned)src * row_stride) +
-                          (lchunk ^ swz<D>(row)) * 8;
-            load_to_lds_16(gp, lds_w + buf * (4 * kWaveElems * 2) + j * 1024);
+            unsigned long long off = (unsigned long long)(unsigned)row * row_stride * 2;
+            asm("" : "+s"(off));   // stays in scalar registers: the compiler would multiply once per lane
+            return off;
+        };
+        auto enter_slice = [&](int i) {   // before the loads of slice i, slices in order
+            if (PAGED) {
+                const int group = ((key0 + i * kAggKT) >> p.page_shift) >> 6;
+                if (group != page_group) {   // uniform
+                    page_group = group;
+                    pages = pages_next;
+                    pages_next = fetch_pages(group + 1);
+                }
+            } else {
+                row_off = offset_of_key(key0 + i * kAggKT);
+            }
+        };
+        auto issue_load = [&](int i, auto j_c, uint32_t lds_buf) {   // loads of a slice in order
+            constexpr int j = decltype(j_c)::value;
+            unsigned long long off = row_off;
+            if (PAGED) {
+                const int key = key0 + i * kAggKT + j * kRPL;
+                off = offset_of_key(key);
+                if (D == 64 && p.page_shift == 2) {   // eight rows per load, four per page
+                    const unsigned long long off4 = offset_of_key(key + 4) - 8ull * row_stride;
+                    load_to_lds_16(lane_ptr[j % kPatterns] + (lrow < 4 ? off : off4), lds_buf + j * 1024);
+                    return;
+                }
+            } else {
+                row_off += row_step;
+            }
+            load_to_lds_16<j * 1024>(lane_ptr[j % kPatterns], off, lds_buf);
         };
         // The tile's Q rows, head slot `wave` of the sub-group by this wavefront: whole rows into the
         // other buffer, chunks permuted like the keys' (fragments read from memory directly, every
@@ -621,94 +673,135 @@ void prefill_aggregate_kernel(PrefillParams p) {
         for (int j = 0; j < kLoads; ++j) {
             const int row = j * kRPL + lrow;
             const T* qp = Qp + (long long)b * p.q_sb + (long long)min(tl + row, Lqv - 1) * p.q_sl +
-                          (long long)min(head0 + wave_u, g * hs.gs + hs.gs - 1) * p.q_sh;
-            load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_w + ((ti0 + 1) & 1) * (4 * kWaveElems * 2) + j * 1024);
+                          (long long)min(head0 + wave, g * hs.gs + hs.gs - 1) * p.q_sh;
+            load_to_lds_16(qp + (lchunk ^ swz16<D>(row)) * 8, lds_w + kBufBytes + j * 1024);
         }
-        fetch_page(ti0);
-        pg_cur = pg_next;
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) issue_load(ti0, j, ti0 & 1);
-        if (ti0 + 1 < ti1) fetch_page(ti0 + 1);
-        const int kx = lg ^ swz<D>(li);
+        if (n > 0) {
+            enter_slice(0);
+            static_for<0, kLoads>([&](auto j) { issue_load(0, j, lds_w); });
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // own rows have landed
         __syncthreads();                                   // everybody's, and s_lse
-        // A operands: row block rb = head slot rb, row li = query tl + li
-        x8_t qa[kGroupSize][kKS];
-        const T* sQ = sK + ((ti0 + 1) & 1) * (4 * kWaveElems);
+        // Operands of 16 rows: lane (dq, col) holds row col, elements [32 ks + 8 dq, +8).  Offset of step 0's
+        // 16 bytes within 32 staged rows; step ks: bits 6 and up flipped, rows 16 .. 31: 16 rows further on
+        const int col = lane & 15, dq = lane >> 4;
+        const uint32_t at_lane = (uint32_t)(col * D + (dq ^ swz16<D>(col)) * 8) * 2;
+        auto read_op = [&](uint32_t addr, int half, int ks) {
+            return *(__attribute__((address_space(3))) const x8_t*)(size_t)((addr ^ (64 * ks)) + half * (16 * D * 2));
+        };
+        // A operands: head slot rb, query rows tl + 16 half + col
+        x8_t qa[kGroupSize][2][kSteps];
+        const uint32_t q_addr = lds_address(sK) + kBufBytes + at_lane;
 #pragma unroll
         for (int rb = 0; rb < kGroupSize; ++rb)
 #pragma unroll
-            for (int ks = 0; ks < kKS; ++ks) {
-                PackT<T> x;
-                x.v8 = *reinterpret_cast<const x8_t*>(&sQ[rb * kWaveElems + li * D + ((2 * ks) ^ kx) * 8]);
-                if (tl + li >= Lqv) x.u = uint4_t{0, 0, 0, 0};
-                qa[rb][ks] = x.v8;
-            }
-        __syncthreads();   // the other buffer takes the next tile's keys from here on
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int ks = 0; ks < kSteps; ++ks) {
+                    PackT<T> x;
+                    x.v8 = read_op(q_addr + rb * (kWaveElems * 2), half, ks);
+                    if (tl + 16 * half + col >= Lqv) x.u = uint4_t{0, 0, 0, 0};
+                    qa[rb][half][ks] = x.v8;
+                }
+        __syncthreads();   // the other buffer takes slice 1 from here on
 
-        for (int ti = ti0; ti < ti1; ++ti) {
-            // this tile's rows have landed (and the next tile's block-table entries arrived)
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            const T* bK = my_k + (ti & 1) * (4 * kWaveElems);
-            const int tn = min(ti + 1, ti1 - 1);   // after the last tile: its rows once more, unused
-            const int nbuf = (ti + 1) & 1;
-            pg_cur = pg_next;
-            if (ti + 2 < ti1) fetch_page(ti + 2);
-
-            // Head by head, the exponentials of one head's scores between the matrix instructions of the
-            // next head's: a wavefront's vector and matrix work overlap within itself, which counts where
-            // few wavefronts share a SIMD (512 tokens 10.1 -> 9.1 us, 1024 12.0 -> 10.7; 32768 4.56 -> 4.44
-            // ms, where the clock follows the power limit).  Two heads' scores are live instead of four,
-            // which makes room for the tile's eight key operands.
-            float16_t acc[2];
-            float16_t zero16;   // the first product of a head starts from a constant zero
-#pragma unroll
-            for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
-            x8_t kb[kKS];
-#pragma unroll
-            for (int ks = 0; ks < kKS; ++ks) kb[ks] = *reinterpret_cast<const x8_t*>(&bK[li * D + ((2 * ks) ^ kx) * 8]);
-            float4_t ls[4];   // log-sums of the rows of the head whose exponentials are next
-            float sum = 0.f;
-            // accumulator v of head rb is query row 8(v/4) + 4lg + v%4, column = key li
-            auto exponentials = [&](const float16_t& s, int v0, int v1) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    if (v >= v0 && v < v1) sum += fast_exp2(s[v] * kScaleLog2 - ls[v >> 2][v & 3]);
+        if (n > 0) {
+            auto read_lse = [&](int rb, int half) {
+                return *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 16 * half + 4 * dq]);
             };
+            // log-sums of the rows of the head whose exponentials are next
+            float4_t ls[2] = {read_lse(kGroupSize - 1, 0), read_lse(kGroupSize - 1, 1)};
+            x8_t kb[2][kSteps];     // B operands: the slice's keys 16 kh + col
+            const uint32_t k_lane = lds_w + at_lane;
 #pragma unroll
-            for (int rb = 0; rb < kGroupSize; ++rb) {
+            for (int ks = 0; ks < kSteps; ++ks)
 #pragma unroll
-                for (int ks = 0; ks < kKS; ++ks) {
-                    acc[rb & 1] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks], ks == 0 ? zero16 : acc[rb & 1]);
-                    if (rb == 0 && ks < kLoads) issue_load(tn, ks, nbuf);
-                    if (rb > 0 && ks > 0) exponentials(acc[(rb - 1) & 1], 16 * (ks - 1) / (kKS - 1), 16 * ks / (kKS - 1));
-                    if (ks == kKS - 1) {
+                for (int kh = 0; kh < 2; ++kh) kb[kh][ks] = read_op(k_lane, kh, ks);
+            enter_slice(min(1, n - 1));
+            static_for<0, kLoads>([&](auto j) { issue_load(min(1, n - 1), j, lds_w + kBufBytes); });
+            // A head's scores: acc[..][half][kh][v] is query row 16 half + 4 dq + v, key 16 kh + col.  It takes
+            // kProducts matrix instructions, and behind each of those of the next head kPer of them move on: scores
+            // into the exponent's arguments, the arguments of the step before through the exponential, the
+            // exponentials before those into the sums.  No instruction waits for the one in front of it, and
+            // none of the vector instructions for the matrix unit.
+            constexpr int kProducts = 4 * kSteps, kPer = 16 / kProducts;
+            float4_t acc[2][2][2];
+            const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+            acc[1][0][0] = acc[1][0][1] = acc[1][1][0] = acc[1][1][1] = zero4;
+            float sum[2] = {}, arg[kPer] = {}, ex[kPer] = {};   // sum: of the keys col and 16 + col
+            auto add_step = [&](int step) {   // score e: row block e / 8, row e / 2 % 4, key block e % 2
 #pragma unroll
-                        for (int v4 = 0; v4 < 4; ++v4)
-                            ls[v4] = *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 8 * v4 + 4 * lg]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int u = 0; u < kPer; ++u) sum[(step * kPer + u) & 1] += ex[u];
+                asm volatile("" : "+v"(sum[0]), "+v"(sum[1]));   // here, not where the sums are used
+#pragma unroll
+                for (int u = 0; u < kPer; ++u) ex[u] = fast_exp2(arg[u]);
+            };
+            auto exponentials = [&](const float4_t (&s)[2][2], int step, int head) {
+                add_step(step);
+#pragma unroll
+                for (int u = 0; u < kPer; ++u) {
+                    const int e = step * kPer + u, half = e >> 3, v = (e >> 1) & 3;
+                    arg[u] = s[half][e & 1][v] * kScaleLog2 - ls[half][v];
+                }
+                if (((step + 1) * kPer) % 8 == 0) {   // a row block's log-sums are free for the next head's
+                    const int half = ((step + 1) * kPer - 1) >> 3;
+                    ls[half] = read_lse((head + 1) % kGroupSize, half);
+                }
+            };
+            auto store_sum = [&](int i) {   // lane (dq, col): key 16 (dq & 1) + col, which quarters 0 and 1 write
+                float total[2];
+#pragma unroll
+                for (int kh = 0; kh < 2; ++kh) {
+                    const uint32_t u = __builtin_bit_cast(uint32_t, sum[kh]);
+                    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+                    total[kh] = sum_with_other_half(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
+                }
+                half_t* o = out + key0 + i * kAggKT + (lane & 31);
+                if (lane < 32) {   // a later sub-group of the KV head adds to what the earlier ones left
+                    float x = dq & 1 ? total[1] : total[0];
+                    if (p.accumulate) x += (float)*o;
+                    *o = (half_t)x;
+                }
+            };
+            for (int i = 0; i < n; ++i) {   // slice i, in registers; its buffer takes slice i + 2
+                const uint32_t buf = lds_w + (i & 1) * kBufBytes;
+                const uint32_t k_addr = k_lane + (~i & 1) * kBufBytes;   // of slice i + 1
+                const int in = min(i + 2, n - 1);       // after the last slice: its rows once more, unused
+                enter_slice(in);
+                tile_phase<KASCADE_PRIO_AGG>(2);
+#pragma unroll
+                for (int rb = 0; rb < kGroupSize; ++rb) {
+                    // the next slice's rows have landed: only the loads issued in this one may be on their way
+                    if (rb == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "i"(kLoads) : "memory");
+                    static_for<0, kProducts>([&](auto st_c) {
+                        constexpr int st = decltype(st_c)::value;
+                        const int ks = st >> 2, half = (st >> 1) & 1, kh = st & 1;
+                        acc[rb & 1][half][kh] = Elem<T>::mma_16x16x32(qa[rb][half][ks], kb[kh][ks], ks == 0 ? zero4 : acc[rb & 1][half][kh]);
+                        asm volatile("" :: "v"(acc[rb & 1][half][kh]));   // here, not where the scores are used
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (rb == 1 && kh == 0) issue_load(in, std::integral_constant<int, st / 2>{}, buf);
+                        if (rb == 3 && half == 1) kb[kh][ks] = read_op(k_addr, kh, ks);
+                        exponentials(acc[(rb + 1) & 1], st, (rb + kGroupSize - 1) % kGroupSize);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (rb == 1 && st == 1) {   // the slice before this one is summed up
+                            if (i > 0) store_sum(i - 1);
+                            sum[0] = sum[1] = 0.f;
+                        }
+                    });
                 }
             }
-#pragma unroll
-            for (int j = kKS; j < kLoads; ++j) issue_load(tn, j, nbuf);
             tile_phase<KASCADE_PRIO_AGG>(1);
-            exponentials(acc[(kGroupSize - 1) & 1], 0, 16);
-            sum = sum_with_other_half(sum);
-            tile_phase<KASCADE_PRIO_AGG>(2);
-            const int key = ti * kAggKT + 32 * wave + li;
-            if (lg == 0 && key < Ls) {
-                if (key < ts)   // a later sub-group of the KV head adds to what the earlier ones left
-                    out[key] = (half_t)(p.accumulate ? sum + (float)out[key] : sum);
-                else if (p.fill_invalid)
-                    out[key] = neg_inf;
-            }
+#pragma unroll
+            for (int st = 0; st < kProducts; ++st) exponentials(acc[1], st, kGroupSize - 1);
+            add_step(0);
+            add_step(1);
+            store_sum(n - 1);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
     }
     if (p.fill_invalid) {
         const int end = part == p.key_parts - 1 ? Ls : min(Ls, (ti0 + p.part_tiles) * kAggKT);
-        for (int key = max(ntiles, ti0) * kAggKT + tid; key < end; key += kThreads) out[key] = neg_inf;
+        for (int key = max(tl < Lqv ? ts : 0, ti0 * kAggKT) + tid; key < end; key += kThreads) out[key] = neg_inf;
     }
 }
 

@@ -135,3 +135,26 @@ def test_wide_log_sum_units_of_sequences_at_different_positions(cuda):
             own = kernels.prefill_chunk_dense(q[b:b + 1, :lens[b]], kp, kp, table[b:b + 1], starts[b], page_size=16,
                                               with_output=False)[0]
             assert torch.equal(got[b, :lens[b]], own[0]), f"sequence {b}"
+
+
+@pytest.mark.parametrize("page", [4, 8, 64])
+@pytest.mark.parametrize("heads,G,D,dtype", [(32, 8, 128, torch.float16), (14, 2, 64, torch.bfloat16)])
+def test_pooled_scores_over_pages_of_every_size(cuda, page, heads, G, D, dtype):
+    """Tiles of a chunk read their keys through 64 block-table entries at a time (256 tokens with the smallest
+    pages; at head_dim 64 a load then covers two pages): the bits of the whole prompt over a strided cache,
+    for chunks whose keys start and end in different groups of entries."""
+    from kascade_amd import kernels
+    L = 1300
+    gen = torch.Generator().manual_seed(page + D)
+    q = torch.randn(1, L, heads, D, generator=gen).to(dtype).to(cuda)
+    k = torch.randn(1, L, G, D, generator=gen).to(dtype)
+    kp, table = _paged_copies(k, page, gen, 1, cuda)
+    k = k.to(cuda)
+    log_sum = kernels.prefill_recompute1(q, k)
+    whole = torch.empty(1, G, (L + 31) // 32, L, device=cuda, dtype=torch.float16)
+    kernels.prefill_aggregate(q, k, log_sum, whole, fill_invalid=True)
+    for start, end in ((0, 96), (96, 512), (512, 1300), (1280, 1300)):
+        got = torch.empty(1, G, (end - start + 31) // 32, end, device=cuda, dtype=torch.float16)
+        kernels.prefill_chunk_aggregate(q[:, start:end], kp, log_sum[:, start:end].contiguous(), got, table, start, page,
+                                        fill_invalid=True)
+        assert torch.equal(got, whole[:, :, start // 32:(end + 31) // 32, :end]), f"rows {start}..{end}"
