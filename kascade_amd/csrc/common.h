@@ -112,6 +112,17 @@ __device__ __forceinline__ float sum_with_other_half(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
+// The same over the four lanes of equal lane % 16
+__device__ __forceinline__ float max_over_quarters(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return max_with_other_half(fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])));
+}
+__device__ __forceinline__ float sum_over_quarters(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return sum_with_other_half(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
+}
 
 __device__ __forceinline__ uint4_t ld_global_16(const void* p) {
     return *reinterpret_cast<const uint4_t*>(p);

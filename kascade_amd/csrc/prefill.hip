@@ -1,4 +1,4 @@
-// Prefill attention kernels for gfx950 (fp16/bf16 MFMA 32x32x16, fp32 softmax).
+// Prefill attention kernels for gfx950 (fp16/bf16 MFMA 16x16x32, fp32 softmax).
 //
 // prefill_attn_kernel -- flash attention over one (query block, KV head, batch)
 //   per workgroup; 4 wavefronts, wavefront w owns q-head 4g+w and 32*NQB queries,
@@ -20,6 +20,15 @@
 //   product O^T = V^T P^T -- P never leaves registers.  The A operand of that product,
 //   V^T, comes out of the row-major V tile through the transposing LDS read
 //   ds_read_b64_tr_b16 (two per operand: four keys each).
+//
+//   What bounds long calls is the chip's power, and per product 16x16x32 takes less of it than 32x32x16 (1.84
+//   against 1.59 PFLOP/s on random operands in registers).  Against 32x32x16 products, row addresses formed by a
+//   64-bit product per tensor and row, and list entries requested behind the tile's loads, 32/8 heads: dense
+//   2048 tokens 47.5 -> 44.4 us, 8192 524 -> 490, 32768 8.1 -> 7.6 ms, chunks at position 14336 of 512 queries
+//   324 -> 260 us, of 2048 501 -> 462; reuse 4096 36.4 -> 35.3 us, 32768 982 -> 948, but 517 9.48 -> 9.68 and 2048
+//   12.9 -> 13.2 (units of a few tiles: chains of latencies); log-sums alone 2048 30.8 -> 28.6, 32768 4.21 -> 3.85
+//   ms, chunk of 512 205 -> 168 us, of 2048 299 -> 266, but 1024 tokens of 64 heads 19.5 -> 21.0 (three units on
+//   a compute unit instead of four; held to the registers of four, 1024 tokens of 32 heads take 16.9 instead of 16.0).
 //
 // prefill_aggregate_kernel -- pooled tile scores: S = Q_tile K^T with the 128
 //   (query, head) rows of a tile held as A operands in registers by every
@@ -76,6 +85,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     typedef typename Elem<T>::x2 x2_t;
     typedef AttnTile<D> G_;
     constexpr int kKT = G_::kKT, kKS = G_::kKS, kDB = G_::kDB, kKB = G_::kKB, kChunks = G_::kChunks;
+    constexpr int NQ = 2 * NQB;     // blocks of 16 queries
     constexpr int kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
@@ -89,7 +99,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
     // resident per compute unit: two with V (64 KB of LDS, 256 registers), K only by the registers
-    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : PAGED ? 3 : 4;
+    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : 3;
     unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
@@ -103,8 +113,8 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
-    const int li = lane & 31;
-    const int lg = lane >> 5;
+    const int col = lane & 15;          // of an operand or result of 16 rows or columns
+    const int dq = lane >> 4;
     const int q0l = tq * QT;            // first query row of this block
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
@@ -142,13 +152,10 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // the masks need to know (both products contract over the same order).
     const int slot0 = wave * 4 * kRPL + lrow;
     const int pos0 = 4 * (wave * kRPL + lrow);
-    int coff[4];                                 // element offset of the chunk this lane fetches for row j
-#pragma unroll
-    for (int j = 0; j < 4; ++j) coff[j] = (lchunk ^ swz<D>(slot0 + j * kRPL)) * 8;
     // tile position of LDS row `slot`
     auto pos_of_slot = [](int slot) { return 4 * ((slot / (4 * kRPL)) * kRPL + slot % kRPL) + (slot / kRPL) % 4; };
     const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
-    const T* vbase = PAGED ? Vp + (long long)g * D : Vp + (long long)b * p.k_sb + (long long)g * p.k_sh;
+    const unsigned long long v_from_k = (unsigned long long)Vp - (unsigned long long)Kp;   // V shares K's layout
     const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
     const int page_mask = (1 << p.page_shift) - 1;
     const int max_row = PAGED ? (p.num_pages << p.page_shift) - 1 : 0;
@@ -165,7 +172,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // strided: nothing (addresses follow from the tile index).
     int ids[4];
     int pend_ti = 0;        // tile the ids belong to
-    const unsigned row_stride = PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl;   // host checks < 2^31
+    const unsigned row_bytes = 2 * (PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl);   // host checks stride < 2^31
     auto fetch_ids = [&](int ti) {
         pend_ti = ti;
         if (sparse && ti < ng) {   // values are bounded at use
@@ -181,42 +188,61 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
             ids[0] = bt_row[tile_key(ti, pos0) >> p.page_shift];
         }
     };
-    // Row addresses of the tile whose ids are held (element offsets from kbase / vbase).  The
+    // K row addresses of the tile whose ids are held; V's are a scalar offset away.  The
     // loads themselves are issued one at a time between the matrix instructions of the first
     // product: a wavefront that issued all eight at once would sit in front of the memory
     // pipeline, which takes 16 cycles per 1 KB load, with nothing running behind it.
-    long long off[4];
-    auto next_offsets = [&]() {
-        if (sparse && pend_ti < ng) {
+    // lane_ptr: the chunk this lane fetches for row j of key 0 (REUSE) or of the position's row within a tile,
+    // within a page if PAGED (passes over consecutive keys alone: one addition a row and tile, a product a page).
+    const char* lane_ptr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz16<D>(slot0 + j * kRPL)) * 8);
+        if (!REUSE) lane_ptr[j] += (unsigned long long)row_bytes * (unsigned)(PAGED ? (pos0 + j) & page_mask : pos0 + j);
+    }
+    const char* row_ptr[4];
+    auto next_rows = [&]() {
+        if (REUSE && sparse && pend_ti < ng) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {   // a corrupt index must not leave the tensor
                 const int row = max(0, min(ids[j], PAGED ? max_row : L - 1));
-                off[j] = (long long)((unsigned long long)(unsigned)row * row_stride) + coff[j];
+                row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
             }
+        } else if (!REUSE && (pend_ti + 1) * kKT <= L) {   // uniform
+            const int k0 = pend_ti * kKT;
+            const unsigned long long off = PAGED ? (unsigned long long)row_bytes * (unsigned)((ids[0] << p.page_shift) + (k0 & page_mask))
+                                                 : (unsigned long long)row_bytes * (unsigned)k0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) row_ptr[j] = lane_ptr[j] + off;
         } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int key = tile_key(pend_ti, pos0 + j);
-                const int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
-                off[j] = (long long)((unsigned long long)(unsigned)row * row_stride) + coff[j];
+                int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
+                if (REUSE) {
+                    row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
+                } else {   // lane_ptr is ahead by the position's row: may be a step back
+                    row -= PAGED ? (pos0 + j) & page_mask : pos0 + j;
+                    row_ptr[j] = lane_ptr[j] + (long long)row_bytes * row;
+                }
             }
         }
     };
     constexpr int kNumLoads = WITH_V ? 8 : 4;
-    auto issue_load = [&](int i, int buf) {   // i < 4: K row group i; else V row group i - 4
-        if (i < 4) load_to_lds_16(kbase + off[i], lds_k + buf * (kTileElems * 2) + i * 1024);
-        else load_to_lds_16(vbase + off[i - 4], lds_v + buf * (kTileElems * 2) + (i - 4) * 1024);
+    auto issue_load = [&](auto i_c, int buf) {   // i < 4: K row group i; else V row group i - 4
+        constexpr int i = decltype(i_c)::value;
+        if constexpr (i < 4) load_to_lds_16(row_ptr[i], lds_k + buf * (kTileElems * 2) + i * 1024);
+        else load_to_lds_16<(i - 4) * 1024>(row_ptr[i - 4], v_from_k, lds_v + buf * (kTileElems * 2));
     };
-    // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 32 kb + li,
-    // chunk 2 ks + lg.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):
-    // the 16 lanes of a group address rows 16 s + 8 h + 4 lg + (0..3) of a key block, 16 columns
-    // of V from column 32 db + 16 (group & 1) on, and receive one column of the four rows each.
-    const int kx = lg ^ swz<D>(li);
-    const int krd = li * D;
-    const int vcol = lane & 15;
-    const int vrow = 4 * lg + (vcol >> 2);                          // + 32 kb + 16 s + 8 h
-    const int vchunk = 2 * ((lane >> 4) & 1) + ((vcol >> 1) & 1);    // + 4 db
-    const int vrd = vrow * D + 4 * (vcol & 1);
+    // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 16 kb + col,
+    // chunk 4 ks + dq.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):
+    // the 16 lanes of a quarter address rows 32 s + 16 h + 4 dq + (0..3), 16 columns
+    // of V from column 16 db on, and receive one column of the four rows each.
+    const int kx = dq ^ swz16<D>(col);
+    const int krd = col * D;
+    const int vrow = 4 * dq + (col >> 2);                // + 32 s + 16 h, which do not enter swz16
+    const int vchunk = ((col >> 1) & 1) ^ swz16<D>(vrow);   // ^ 2 db
+    const int vrd = vrow * D + 4 * (col & 1);
 
     // Softmax state.  m[] is the reference the exponentials are taken against, in log2 units of
     // the scaled scores.  It follows the running maximum lazily: a tile moves it only when one of
@@ -229,16 +255,16 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // Reuse units sum the exponentials as they enter the second product (rounded to the element
     // type, two per instruction); the passes whose log-sum feeds the selection sum them in fp32.
     constexpr bool kPairSum = REUSE && WITH_V && !EXACT_SUM;
-    float m[NQB], l[NQB];
-    float16_t oT[NQB][kDB];
+    float m[NQ];
+    float l[NQ];
+    float4_t oT[NQ][kDB];      // query block, 16 output columns
+    const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        m[qb] = -INFINITY;
-        l[qb] = 0.f;
+    for (int q = 0; q < NQ; ++q) {
+        m[q] = -INFINITY;
+        l[q] = 0.f;
 #pragma unroll
-        for (int db = 0; db < kDB; ++db)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) oT[qb][db][v] = 0.f;
+        for (int db = 0; db < kDB; ++db) oT[q][db] = zero4;
     }
 
     // Order of the tiles.  A sparse unit takes its diagonal tile first: the keys q0 .. q0+31 need
@@ -248,26 +274,25 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // average under rolling budgets).  Softmax is accumulated online, so the order is free.
     auto tile_at = [&](int s) { return (REUSE && sparse) ? (s == 0 ? ng : s - 1) : s; };
     fetch_ids(tile_at(0));
-    next_offsets();
-#pragma unroll
-    for (int i = 0; i < kNumLoads; ++i) issue_load(i, 0);
+    next_rows();
+    static_for<0, kNumLoads>([&](auto i) { issue_load(i, 0); });
     if (ntiles > 1) fetch_ids(tile_at(1));
 
-    // ---- Q fragments (B operand of S^T): query li (+32 qb), d chunk 16*ks + 8*lg; requested after
+    // ---- Q fragments (B operand of S^T): query col (+ 16 q), d chunk 32*ks + 8*dq; requested after
     // the first tile's rows, which the first barrier waits for ----
-    x8_t qf[NQB][kKS];
+    x8_t qf[NQ][kKS];
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        const int ql = q0l + 32 * qb + li;
+    for (int q = 0; q < NQ; ++q) {
+        const int ql = q0l + 16 * q + col;
         const bool ok = ql < Lqv;
         const T* qp = Qp + (long long)b * p.q_sb + (long long)min(ql, Lqv - 1) * p.q_sl +
-                      (long long)head * p.q_sh + lg * 8;
+                      (long long)head * p.q_sh + dq * 8;
 #pragma unroll
         for (int ks = 0; ks < kKS; ++ks) {
             PackT<T> t;
-            t.u = ld_global_16(qp + ks * 16);
+            t.u = ld_global_16(qp + ks * 32);
             if (!ok) t.u = uint4_t{0, 0, 0, 0};
-            qf[qb][ks] = t.v8;
+            qf[q][ks] = t.v8;
         }
     }
 
@@ -278,7 +303,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     constexpr int kFull = 0, kMasked = 1, kDiag = 2;
     auto run_tile = [&](int sq, auto mode_c) {
         constexpr int MODE = decltype(mode_c)::value;
-        constexpr int nkb = (MODE == kDiag && QT == 32) ? 1 : kKB;
+        constexpr int nkb = (MODE == kDiag && QT == 32) ? 2 : kKB;
         const int ti = tile_at(sq);
         const T* bK = sK + (sq & 1) * kTileElems;
         const T* bV = sV + (sq & 1) * kTileElems;
@@ -289,27 +314,30 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         // The next tile's loads go out between the products below, unconditionally: after the last
         // tile they fetch its rows once more into the idle buffer (1/28 of the traffic on average,
         // from the cache) rather than put a branch between the matrix instructions.
-        if (sq + 1 < ntiles) next_offsets();
+        // The ids of the tile behind that one are requested before those loads: the compiler waits for every
+        // load on its way when it writes registers that one of its own loads may still fill, and behind the
+        // tile's loads that wait was a whole trip to memory.
+        if (sq + 1 < ntiles) next_rows();
+        if (sq + 2 < ntiles) fetch_ids(tile_at(sq + 2));
         const int nbuf = (sq + 1) & 1;
 
         tile_phase<kPrio>(0);
-        // ---- S^T = K_tile Q^T.  Step c = (key block c / kKS, contraction step c % kKS); operands are
-        // read from LDS two windows (four steps) ahead of the products that use them, in program
-        // order, because LDS reads do not move across the load statements ----
+        // ---- S^T = K_tile Q^T.  Step c = 16 keys and 32 elements of the contraction, two key blocks in turn;
+        // operands are read from LDS two windows (four steps) ahead of the products that use them, in
+        // program order, because LDS reads do not move across the load statements ----
         constexpr int kSteps = nkb * kKS;
-        float16_t sT[NQB][nkb];
-        float16_t zero16;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
+        float4_t sT[NQ][nkb];
+        auto key_block = [](int c) { return 2 * (c / (2 * kKS)) + (c & 1); };
+        auto k_step = [](int c) { return (c % (2 * kKS)) >> 1; };
         auto read_a = [&](int c) {
-            return *reinterpret_cast<const x8_t*>(&bK[32 * (c / kKS) * D + krd + ((2 * (c % kKS)) ^ kx) * 8]);
+            return *reinterpret_cast<const x8_t*>(&bK[16 * key_block(c) * D + krd + ((4 * k_step(c)) ^ kx) * 8]);
         };
-        constexpr int kAhead = (kKB <= 2) ? 2 : 1;   // windows read ahead (registers are scarcer at D = 64)
+        constexpr int kAhead = (D == 128) ? 2 : 1;   // windows read ahead (registers are scarcer at D = 64)
         x8_t aw[kAhead + 1][2];
 #pragma unroll
         for (int c = 0; c < 2 * kAhead && c < kSteps; ++c) aw[c >> 1][c & 1] = read_a(c);
-#pragma unroll
-        for (int w = 0; w < kSteps / 2; ++w) {
+        static_for<0, kSteps / 2>([&](auto w_c) {
+            constexpr int w = decltype(w_c)::value;
             if (2 * (w + kAhead) < kSteps) {
                 aw[(w + kAhead) % (kAhead + 1)][0] = read_a(2 * (w + kAhead));
                 aw[(w + kAhead) % (kAhead + 1)][1] = read_a(2 * (w + kAhead) + 1);
@@ -317,118 +345,164 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
             __builtin_amdgcn_sched_barrier(0);   // the scheduler would sink the reads to their use
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int kb = (2 * w + i) / kKS, ks = (2 * w + i) % kKS;
+                const int kb = key_block(2 * w + i), ks = k_step(2 * w + i);
 #pragma unroll
-                for (int qb = 0; qb < NQB; ++qb)   // the first product starts from a constant zero
-                    sT[qb][kb] = Elem<T>::mma_32x32x16(aw[w % (kAhead + 1)][i], qf[qb][ks], ks == 0 ? zero16 : sT[qb][kb]);
+                for (int q = 0; q < NQ; ++q)   // the first product starts from a constant zero
+                    sT[q][kb] = Elem<T>::mma_16x16x32(aw[w % (kAhead + 1)][i], qf[q][ks], ks == 0 ? zero4 : sT[q][kb]);
             }
-            if (w < kNumLoads) issue_load(w, nbuf);
-        }
-#pragma unroll
-        for (int i = kSteps / 2; i < kNumLoads; ++i) issue_load(i, nbuf);
-        if (sq + 2 < ntiles) fetch_ids(tile_at(sq + 2));
-        // ---- masks: accumulator v of key block kb is LDS row 32kb + 8(v/4) + 4lg + v%4 of the tile ----
+            if constexpr (w < kNumLoads) issue_load(w_c, nbuf);
+        });
+        static_for<kSteps / 2, kNumLoads>([&](auto i) { issue_load(i, nbuf); });
+        // ---- masks: accumulator v of key block kb is LDS row 16 kb + 4 dq + v of the tile ----
         if (MODE != kFull) {
             const bool diag_here = MODE == kDiag || (sparse && ti == ng);
             if (sparse && !diag_here) {   // a selection that ends inside this tile
 #pragma unroll
-                for (int qb = 0; qb < NQB; ++qb)
+                for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                    for (int kb = 0; kb < nkb; ++kb)
+                    for (int v = 0; v < 4; ++v) {
+                        const int pos = ti * kKT + pos_of_slot(16 * kb + 4 * dq + v);
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            const int pos = ti * kKT + pos_of_slot(32 * kb + 8 * (v >> 2) + 4 * lg + (v & 3));
-                            if (pos >= n) sT[qb][kb][v] = -INFINITY;
-                        }
+                        for (int q = 0; q < NQ; ++q)
+                            if (pos >= n) sT[q][kb][v] = -INFINITY;
+                    }
             } else {                           // the causal edge and the end of the sequence
                 const int kstart = diag_here ? q0 : ti * kKT;
 #pragma unroll
-                for (int qb = 0; qb < NQB; ++qb) {
-                    const int q = q0 + 32 * qb + li;   // global position
+                for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                    for (int kb = 0; kb < nkb; ++kb)
+                    for (int v = 0; v < 4; ++v) {
+                        const int key = kstart + pos_of_slot(16 * kb + 4 * dq + v);
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            const int key = kstart + pos_of_slot(32 * kb + 8 * (v >> 2) + 4 * lg + (v & 3));
-                            if (key > q || key >= L) sT[qb][kb][v] = -INFINITY;
-                        }
-                }
+                        for (int q = 0; q < NQ; ++q)   // q0 + 16 q + col: the query's global position
+                            if (key > q0 + 16 * q + col || key >= L) sT[q][kb][v] = -INFINITY;
+                    }
             }
         }
-        // ---- online softmax (one query column per lane pair: lanes li and li + 32) ----
+        // ---- online softmax (one query column per four lanes: those of equal col) ----
         tile_phase<kPrio>(1);
-        x8_t pf[NQB][2 * nkb];
-#pragma unroll
-        for (int qb = 0; qb < NQB; ++qb) {
+        x8_t pf[NQ][nkb / 2];
+        auto maximum = [&](int q) {
             float mx = -INFINITY;
 #pragma unroll
             for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sT[qb][kb][v]);
-            const float ms = mx * kScaleLog2;
-            if (__any(ms > m[qb] + kRefSlack)) {   // wavefront-uniform
-                const float mnew = fmaxf(m[qb], max_with_other_half(ms));   // the same in both lanes of a column
-                const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[qb] - mnew);
-                m[qb] = mnew;
-                l[qb] *= corr;
+                for (int v = 0; v < 4; ++v) mx = fmaxf(mx, sT[q][kb][v]);
+            return mx * kScaleLog2;
+        };
+        // 32 queries' references, from their scores' maxima
+        auto move_references = [&](int q0, const float (&ms)[2]) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int q = q0 + i;
+                const float mnew = fmaxf(m[q], max_over_quarters(ms[i]));   // the same in the four lanes of a column
+                const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
+                m[q] = mnew;
+                l[q] *= corr;
                 if (WITH_V) {
 #pragma unroll
-                    for (int db = 0; db < kDB; ++db)
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) oT[qb][db][v] *= corr;
+                    for (int db = 0; db < kDB; ++db) oT[q][db] *= corr;
                 }
             }
-            const float mu = (m[qb] == -INFINITY) ? 0.f : m[qb];
+        };
+        if constexpr (!WITH_V) {
+            // Log-sums alone: the same rule, but the maximum is only formed on the first tiles and where a lane's
+            // sum says that a score may lie kRefSlack above its reference (its exponential alone is 2^kRefSlack
+            // then), or is no number (the reference still is -inf); then the exponentials are formed anew.
+            constexpr float kSumLimit = 250.f;
+            // A unit's first tiles move it often, and forming the exponentials twice costs more than the maximum:
+            // 16 tiles of 64 keys (517 tokens 10.6 -> 9.9 us, 1024 17.5 -> 16.1, the long calls unchanged), all
+            // tiles of 128 (4096 tokens at head_dim 64: 36.1 -> 34.5).
+            constexpr int kEarly = D == 64 ? 0x7fffffff : 16;
+#pragma unroll
+            for (int q = 0; q < NQ; q += 2) {
+                float sum[2];
+                auto sums = [&](float mu0, float mu1) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        sum[i] = 0.f;
+#pragma unroll
+                        for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                sum[i] += fast_exp2(__builtin_fmaf(sT[q + i][kb][v], kScaleLog2, -(i ? mu1 : mu0)));
+                    }
+                };
+                bool look = sq < kEarly;   // wavefront-uniform
+                if (!look) {
+                    sums(m[q], m[q + 1]);
+                    look = __any(!(sum[0] <= kSumLimit) || !(sum[1] <= kSumLimit));
+                }
+                if (look) {
+                    const float ms[2] = {maximum(q), maximum(q + 1)};
+                    if (__any(ms[0] > m[q] + kRefSlack || ms[1] > m[q + 1] + kRefSlack)) move_references(q, ms);
+                    sums(m[q] == -INFINITY ? 0.f : m[q], m[q + 1] == -INFINITY ? 0.f : m[q + 1]);
+                }
+                l[q] += sum[0];
+                l[q + 1] += sum[1];
+            }
+            tile_phase<kPrio>(2);
+            return;
+        }
+        {
+            const float ms[2] = {maximum(0), maximum(1)};
+            if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) move_references(0, ms);   // wavefront-uniform
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const float mu = (m[q] == -INFINITY) ? 0.f : m[q];
+            float sum = 0.f;
+            float4_t e[nkb];
 #pragma unroll
             for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    sT[qb][kb][v] = fast_exp2(__builtin_fmaf(sT[qb][kb][v], kScaleLog2, -mu));
-            float sum = 0.f;
+                for (int v = 0; v < 4; ++v) e[kb][v] = fast_exp2(__builtin_fmaf(sT[q][kb][v], kScaleLog2, -mu));
             if (WITH_V) {
 #pragma unroll
-                for (int s = 0; s < 2 * nkb; ++s) {
+                for (int s = 0; s < nkb / 2; ++s) {
                     x8_t t;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) t[e] = (T)sT[qb][s >> 1][8 * (s & 1) + e];
-                    pf[qb][s] = t;
+                    for (int i = 0; i < 8; ++i) t[i] = (T)e[2 * s + (i >> 2)][i & 3];
+                    pf[q][s] = t;
                 }
             }
             if (kPairSum) {
 #pragma unroll
-                for (int s = 0; s < 2 * nkb; ++s)
+                for (int s = 0; s < nkb / 2; ++s)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const x2_t pr = {pf[qb][s][2 * e], pf[qb][s][2 * e + 1]};
+                    for (int i = 0; i < 4; ++i) {
+                        const x2_t pr = {pf[q][s][2 * i], pf[q][s][2 * i + 1]};
                         sum = Elem<T>::add_pair(pr, sum);
                     }
             } else {
 #pragma unroll
                 for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) sum += sT[qb][kb][v];
+                    for (int v = 0; v < 4; ++v) sum += e[kb][v];
             }
-            l[qb] += sum;   // per-lane partial sum (own key positions)
+            l[q] += sum;   // per-lane partial sum (own key positions)
         }
         tile_phase<kPrio>(2);
-        // ---- O^T += V^T P^T: step s covers the keys of accumulators 8(s&1) .. 8(s&1)+7 of key block
-        // s/2, i.e. rows 16 s + 8 h + 4 lg + (0..3), h = 0, 1, of the tile.  The operands of a block
-        // of 32 output rows are read while the block before it is multiplied ----
+        // ---- O^T += V^T P^T: step s covers the keys of blocks 2 s and 2 s + 1, whose scores lane dq holds: rows
+        // 32 s + 16 h + 4 dq + (0..3), h = 0, 1, of the tile.  The operands of a group of steps are read
+        // while the group before it is multiplied ----
         if (WITH_V) {
-            constexpr int kPS = 2 * nkb;
+            constexpr int kPS = nkb / 2;
             auto read_v = [&](int db, int s, int h) {
-                const int row = 16 * s + 8 * h;   // + vrow; only its low four bits enter swz
-                const T* vp = bV + row * D + vrd + ((4 * db + vchunk) ^ swz<D>(row + vrow)) * 8;
+                const T* vp = bV + (32 * s + 16 * h) * D + vrd + ((2 * db) ^ vchunk) * 8;
                 return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
             };
-            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block)
-            constexpr int kGrp = (kKB <= 2) ? 4 : 2;
+            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block),
+            // two column blocks in turn
+            constexpr int kGrp = (D == 128) ? 4 : 2;
             constexpr int kGroupsPV = kDB * kPS / kGrp;
+            auto out_block = [](int t) { return 2 * (t / (2 * kPS)) + (t & 1); };
+            auto p_step = [](int t) { return (t % (2 * kPS)) >> 1; };
             short4_t av[2][kGrp][2];
 #pragma unroll
             for (int i = 0; i < kGrp; ++i)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(i / kPS, i % kPS, h);
+                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(out_block(i), p_step(i), h);
 #pragma unroll
             for (int gq = 0; gq < kGroupsPV; ++gq) {
                 if (gq + 1 < kGroupsPV) {
@@ -436,17 +510,17 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
                     for (int i = 0; i < kGrp; ++i)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
-                            av[(gq + 1) & 1][i][h] = read_v((kGrp * (gq + 1) + i) / kPS, (kGrp * (gq + 1) + i) % kPS, h);
+                            av[(gq + 1) & 1][i][h] = read_v(out_block(kGrp * (gq + 1) + i), p_step(kGrp * (gq + 1) + i), h);
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int i = 0; i < kGrp; ++i) {
-                    const int db = (kGrp * gq + i) / kPS, s = (kGrp * gq + i) % kPS;
+                    const int db = out_block(kGrp * gq + i), s = p_step(kGrp * gq + i);
                     const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
                     const x8_t a = __builtin_bit_cast(x8_t, both);
 #pragma unroll
-                    for (int qb = 0; qb < NQB; ++qb)
-                        oT[qb][db] = Elem<T>::mma_32x32x16(a, pf[qb][s], oT[qb][db]);
+                    for (int q = 0; q < NQ; ++q)
+                        oT[q][db] = Elem<T>::mma_16x16x32(a, pf[q][s], oT[q][db]);
                 }
             }
         }
@@ -455,7 +529,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     {
         int sq = 0;
         if (REUSE && sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
-            if (kKB <= 2) run_tile(0, std::integral_constant<int, kDiag>{});
+            if (kKT == 64) run_tile(0, std::integral_constant<int, kDiag>{});
             else run_tile(0, std::integral_constant<int, kMasked>{});
             sq = 1;
         }
@@ -471,33 +545,33 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // leave as whole rows: 16-byte stores, four rows per instruction ----
     static_assert(!WITH_V || NQB == 1, "the output pass is written for 32 queries per wavefront");
     if (WITH_V) __syncthreads();   // everybody is done with the tile buffers
+    T* so = sK + wave * (32 * D);
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        const int ql = q0l + 32 * qb + li;
-        const float lt = sum_with_other_half(l[qb]);
-        if (p.log_sum && lg == 0 && ql < Lqv && real_head)
-            p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[qb];
+    for (int q = 0; q < NQ; ++q) {
+        const int ql = q0l + 16 * q + col;
+        const float lt = sum_over_quarters(l[q]);
+        if (p.log_sum && dq == 0 && ql < Lqv && real_head)
+            p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[q];
         if (WITH_V) {
-            T* so = sK + wave * (32 * D);
             const float inv = 1.f / lt;
+            const int row = 16 * q + col;
 #pragma unroll
-            for (int db = 0; db < kDB; ++db)
-#pragma unroll
-                for (int v4 = 0; v4 < 4; ++v4) {   // d = 32 db + 8 v4 + 4 lg .. +3: chunk 4 db + v4 of row li
-                    x4_t o = {(T)(oT[qb][db][4 * v4 + 0] * inv), (T)(oT[qb][db][4 * v4 + 1] * inv),
-                              (T)(oT[qb][db][4 * v4 + 2] * inv), (T)(oT[qb][db][4 * v4 + 3] * inv)};
-                    *reinterpret_cast<x4_t*>(&so[li * D + (((4 * db + v4) ^ (li & (kChunks - 1))) * 8) + 4 * lg]) = o;
-                }
-            __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
-#pragma unroll
-            for (int j = 0; j < 32 / kRPL; ++j) {
-                const int r = j * kRPL + lrow;
-                const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
-                const int qr = q0l + r;
-                if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
-                    __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
-                        (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
+            for (int db = 0; db < kDB; ++db) {   // d = 16 db + 4 dq .. +3: half of chunk 2 db + dq / 2
+                const x4_t o = {(T)(oT[q][db][0] * inv), (T)(oT[q][db][1] * inv), (T)(oT[q][db][2] * inv), (T)(oT[q][db][3] * inv)};
+                *reinterpret_cast<x4_t*>(&so[row * D + (((2 * db + (dq >> 1)) ^ (row & (kChunks - 1))) * 8) + 4 * (dq & 1)]) = o;
             }
+        }
+    }
+    if (WITH_V) {
+        __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
+#pragma unroll
+        for (int j = 0; j < 32 / kRPL; ++j) {
+            const int r = j * kRPL + lrow;
+            const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
+            const int qr = q0l + r;
+            if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
+                __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
+                    (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
         }
     }
 }
@@ -749,13 +823,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
                 }
             };
             auto store_sum = [&](int i) {   // lane (dq, col): key 16 (dq & 1) + col, which quarters 0 and 1 write
-                float total[2];
-#pragma unroll
-                for (int kh = 0; kh < 2; ++kh) {
-                    const uint32_t u = __builtin_bit_cast(uint32_t, sum[kh]);
-                    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-                    total[kh] = sum_with_other_half(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
-                }
+                const float total[2] = {sum_over_quarters(sum[0]), sum_over_quarters(sum[1])};
                 half_t* o = out + key0 + i * kAggKT + (lane & 31);
                 if (lane < 32) {   // a later sub-group of the KV head adds to what the earlier ones left
                     float x = dq & 1 ? total[1] : total[0];

@@ -12,9 +12,9 @@ namespace {
 // and the score registers a narrower head frees hold the extra keys.
 template <int D> struct AttnTile {
     static constexpr int kKT = 64 * 128 / D;     // keys per tile
-    static constexpr int kKS = D / 16;           // contraction steps of S^T = K Q^T
-    static constexpr int kDB = D / 32;           // 32-row blocks of O^T
-    static constexpr int kKB = kKT / 32;         // 32-key blocks of a tile
+    static constexpr int kKS = D / 32;           // contraction steps of S^T = K Q^T
+    static constexpr int kDB = D / 16;           // 16-row blocks of O^T
+    static constexpr int kKB = kKT / 16;         // 16-key blocks of a tile
     static constexpr int kChunks = D / 8;        // 16-byte chunks of a row
     static constexpr int kRowsPerLoad = 64 / kChunks;   // rows one wavefront-wide 16-byte load covers
     static constexpr int kTileElems = kKT * D;   // 16 KB of K (and of V) whatever D
@@ -84,9 +84,14 @@ __device__ __forceinline__ void unit_of_workgroup(int B, int G, int nblocks, int
 }
 
 __device__ __forceinline__ int rolling_budget(float pct, int tile_start) {
-    long long fl = (long long)floor((double)pct * (double)tile_start / 100.0);
-    if (fl < 128) fl = 128;
-    return (int)(((fl + 127) / 128) * 128);
+    // floor(pct tile_start / 100) without a division, which every unit's first list entry would wait for (517 tokens
+    // 9.80 -> 9.68 us).  x is exact, and where it is no multiple of 100 it lies a relative 2^-44 or more off
+    // the next one: the quotient's rounding does not reach it, so this is the floor of the rounded quotient too.
+    const double x = (double)pct * (double)tile_start;
+    int fl = (int)(x * 0.01);
+    fl += (double)(fl + 1) * 100.0 <= x;
+    fl -= (double)fl * 100.0 > x;
+    return max(128, (fl + 127) & ~127);
 }
 
 // Index-row width the host gives a prompt of L keys: min(128 ceil(min(max(128, floor(pct L / 100)), L) / 128), L).

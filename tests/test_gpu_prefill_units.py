@@ -158,3 +158,32 @@ def test_pooled_scores_over_pages_of_every_size(cuda, page, heads, G, D, dtype):
         kernels.prefill_chunk_aggregate(q[:, start:end], kp, log_sum[:, start:end].contiguous(), got, table, start, page,
                                         fill_invalid=True)
         assert torch.equal(got, whole[:, :, start // 32:(end + 31) // 32, :end]), f"rows {start}..{end}"
+
+
+@pytest.mark.parametrize("heads,G,D,dtype", [(32, 8, 128, torch.float16), (32, 8, 128, torch.bfloat16), (14, 2, 64, torch.float16)])
+@pytest.mark.parametrize("batch", [1, 9])
+def test_log_sums_alone_follow_late_maxima(cuda, batch, heads, G, D, dtype):
+    """The pass for log-sums alone forms a tile's maximum only where the tile's sums ask for it: scores that
+    rise step by step far behind the first tiles, by less and by more than the reference may lag and once beyond the
+    range of the exponentials, give the bits of the pass with an output and the log-sum of float64.  Nine sequences
+    of 32 heads take units of 64 queries."""
+    from kascade_amd import kernels
+    L = 4200 if batch == 1 else 1500
+    gen = torch.Generator().manual_seed(D + batch)
+    q = torch.randn(batch, L, heads, D, generator=gen).to(dtype).to(cuda)
+    k = torch.randn(batch, L, G, D, generator=gen)
+    for at, size in ((1, 3.0), (700, 6.0), (1100, 12.0), (1101, 24.0), (1290, 200.0)):
+        k[:, at] *= size
+    k = k.to(dtype).to(cuda)
+    alone = kernels.prefill_recompute1(q, k)
+    log_sum, _ = kernels.prefill_recompute0(q, k, k)
+    assert torch.equal(alone, log_sum)
+    b = batch - 1
+    rows = torch.tensor([0, 1, 63, 64, 699, 700, 1023, 1099, 1101, 1289, 1290, 1299, L - 1], device=cuda)
+    for h in (0, heads - 1):
+        s = (q[b, rows, h].double() @ k[b, :, h // (heads // G)].double().t().contiguous()) * D ** -0.5
+        s.masked_fill_(torch.arange(L, device=cuda)[None, :] > rows[:, None], float("-inf"))
+        want = torch.logsumexp(s, 1) / 0.6931471805599453
+        # scores are fp32 sums of D products of up to 200 x 4 x 4, the log-sum has 24 bits: 1e-6 of the largest
+        bound = 1e-6 * s.masked_fill(s.isinf(), 0).abs().amax(1) / 0.69 + 4e-6 * want.abs() + 1e-5
+        assert ((alone[b, rows, h].double() - want).abs() <= bound).all()
