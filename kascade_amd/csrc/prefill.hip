@@ -10,12 +10,12 @@
 //   registers, no LDS store instructions) into one of two buffers, so a tile costs one
 //   barrier: wait for the own loads, barrier, start the next tile's loads into the other
 //   buffer, compute.  Rows lie in LDS as they lie in memory; the 16-byte chunk c of row R
-//   sits at chunk c ^ swz(R), chosen by the lane that fetches it (each lane picks the global
+//   sits at chunk c ^ swz16(R), chosen by the lane that fetches it (each lane picks the global
 //   chunk that belongs at its LDS position), which makes both read patterns below free of
 //   bank conflicts without padding.
 //
-//   The kernel works on S^T = K Q^T so that each lane owns one query column:
-//   row max / row sum are in-lane reductions plus one cross-half exchange, and
+//   The kernel works on S^T = K Q^T so that four lanes (equal lane % 16) own one query column:
+//   row max / row sum are in-lane reductions plus two exchanges, and
 //   the exponentiated scores are already in the B-operand layout of the second
 //   product O^T = V^T P^T -- P never leaves registers.  The A operand of that product,
 //   V^T, comes out of the row-major V tile through the transposing LDS read

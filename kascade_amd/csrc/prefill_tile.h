@@ -21,18 +21,15 @@ template <int D> struct AttnTile {
 };
 
 // Chunk permutation of a tile row in LDS (see the head of the file).  What it must give:
-// 16 lanes reading the same chunk of 16 consecutive rows (A operand of S^T), and 32 lanes
-// reading 4 consecutive rows x 4 consecutive chunks in 8-byte halves (transposing read of V),
+// lane (dq, col) reading chunk 4 ks + dq of row col (A operand of S^T), and the 16 lanes of each quarter dq reading
+// rows 4 dq .. 4 dq + 3 x 2 consecutive chunks in 8-byte halves (transposing read of V),
 // each touch all 64 banks once.  Rows are 256 bytes (D = 128: the row does not move the bank)
-// or 128 bytes (D = 64: the row parity picks the bank half, three more row bits permute).
-template <int D> __device__ __forceinline__ int swz(int row);
-template <> __device__ __forceinline__ int swz<128>(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-template <> __device__ __forceinline__ int swz<64>(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
-
-// The same for operands of 16 rows (lane (dq, col) reads chunk 4 ks + dq of row col).  The hardware serves
-// a 16-byte read in groups that mix lanes 0-3 and 12-15 of one quarter with lanes 4-11 of the next, whose chunks
-// differ in bit 0: with swz() they share banks.
-template <int D> __device__ __forceinline__ int swz16(int row) { return (swz<D>(row) & ~3) | (-(row >> 2) & 3); }
+// or 128 bytes (D = 64: the row parity picks the bank half, three more row bits permute).  The hardware serves a
+// 16-byte read in groups that mix lanes 0-3 and 12-15 of one quarter with lanes 4-11 of the next, whose chunks
+// differ in bit 0: hence -(row / 4), not row / 4, in the low bits.
+template <int D> __device__ __forceinline__ int swz16(int row);
+template <> __device__ __forceinline__ int swz16<128>(int row) { return ((row & 3) << 2) | (-(row >> 2) & 3); }
+template <> __device__ __forceinline__ int swz16<64>(int row) { return (((row >> 1) & 1) << 2) | (-(row >> 2) & 3); }
 
 // One wavefront-wide load of 16 bytes per lane from global memory into LDS: lane i's bytes
 // land at lds_base + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
