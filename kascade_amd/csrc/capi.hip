@@ -708,28 +708,25 @@ int kascade_topk_sorted_call(const kascade_half* scores, int32_t* out_idx, int r
 }  // extern "C"
 namespace {
 // 64 queries per wavefront in the K-only log-sum pass, or 32?  Units (workgroups) of 64 read every K tile for
-// twice the queries, but there are half as many and each is twice as long, so it is a
-// question of how the units fill the places of the chip (two of 64 or three of 32 on each of 256 compute units), and
-// of how far their lengths spread: from q_start to q_start + q_len keys.  Us, 32 / 64 queries, 32/8 heads:
-//   units of 64   queries, position              32 / 64        why
-//   256, 384      2048, 3072 at 14336            266 / 327, 409 / 434
-//   448           3584 at 14336, at 2048         546 / 462, 147 / 135   a residency nearly full of units about equally
-//   512           4096 at 14336, at 2048         574 / 510, 172 / 150   long wins; lengths that spread
-//                 4096 at 512, at 0              101 / 109, 78 / 94     leave its places idle
-//   520, 576      4160 at 8320, 4608 at 1152     424 / 464, 169 / 158 (another build): equal lengths leave a second
-//                                                residency nearly empty, lengths that spread overlap
-//   640           5120 at 0                      128 / 131 (whole prompts)
-//   768, 2048     6144, 16384 at 0               174 / 166, 1067 / 1037
-//   752, 1024     3001, 4096 at 0, 64 heads       88 / 93, 159 / 158: units of up to 64 tiles
-//   1024          8192 at 0                      285 / 294
-//   704, 1024     11 x 512 at 0, 16 x 512 at 0, at 512: 28.8 / 34.3, 37.3 / 40.8, 74.9 / 70.9 (another build): short
-//                                                units, the set-up counts
+// twice the queries, 15 % less per query, but there are half as many and each is twice as long, so it is a
+// question of how the units fill the 512 places of the chip (two on each of 256 compute units), and of how
+// far their lengths spread: from q_start to q_start + q_len keys.  Us, 32 / 64 queries, 32/8 heads:
+//   units of 64   queries, position         32 / 64        why
+//   256           2048 at 8192              186 / 209      one workgroup per compute unit
+//   448, 512      3584 at 7168, 4096 at 0   347 / 291, 88 / 98: a residency nearly full of units about equally long
+//                                           wins; lengths that spread leave its places idle
+//   520, 576      4160 at 8320, 4608 at 1152  424 / 464, 169 / 158: equal lengths leave a second residency nearly
+//                                           empty, lengths that spread overlap
+//   520, 640      4160, 5120 at 0           93.7 / 102.8, 128.8 / 135.9 (whole prompts)
+//   768, 1024     6144, 8192 at 0           192 / 174, 315 / 281; at 4 times their length 1550 / 1465, 2725 / 2345
+//   704           11 x 512 at 0             28.8 / 34.3    short units: the set-up counts
+//   1024          16 x 512 at 0, at 512     37.3 / 40.8, 74.9 / 70.9
 // Sequences at different positions count as if all stood at the last one (the host knows no other).
 bool wide_log_sum_units(const Shape& sh, int batch, int q_start, int q_len) {
     if (sh.D != 128) return false;
     const long long units = (long long)((q_len + 63) / 64) * sh.G * ((sh.gs + 3) / 4) * batch;
-    const bool deep = (long long)q_start + q_len > 4096;
-    if (units <= 512) return units >= 448 && 2LL * q_start >= q_len;
+    const bool deep = (long long)q_start + q_len >= 2048;
+    if (units <= 512) return units >= 448 && q_start >= q_len;
     if (units <= 640) return deep && q_start > 0 && q_start <= q_len;
     return deep || (q_start >= q_len && units >= 800);
 }

@@ -19,6 +19,7 @@ typedef _Float16 half_t;
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 typedef int int4_t __attribute__((ext_vector_type(4)));
@@ -49,6 +50,9 @@ template <> struct Elem<half_t> {
     static __device__ __forceinline__ float4_t mma_16x16x16(short4_t a, x4 b, float4_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(x4, a), b, c, 0, 0, 0);
     }
+    static __device__ __forceinline__ float16_t mma_32x32x16(x8 a, x8 b, float16_t c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    }
     // acc + p.x + p.y in fp32 (one instruction for two elements)
     static __device__ __forceinline__ float add_pair(x2 p, float acc) {
         const x2 ones = {(half_t)1.f, (half_t)1.f};
@@ -62,6 +66,9 @@ template <> struct Elem<bf16_t> {
     }
     static __device__ __forceinline__ float4_t mma_16x16x16(short4_t a, x4 b, float4_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, __builtin_bit_cast(short4_t, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float16_t mma_32x32x16(x8 a, x8 b, float16_t c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ float add_pair(x2 p, float acc) {
         const x2 ones = {(bf16_t)1.f, (bf16_t)1.f};

@@ -76,16 +76,17 @@ template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
 // Queries are rows [0, Lq) of Q at global positions q_start + row (q_start a multiple of 32);
 // keys are positions [0, L) with L = q_start + Lq.  PAGED: K/V are pages [P, page, G, D]
 // addressed through the block table, and gathered index rows hold physical row numbers.
+//
+// Sparse passes (and the dense tiles of their first units): products 16x16x32.
 // EXACT_SUM: the softmax denominators are summed in fp32 from the unrounded exponentials (the
-// passes whose log-sum is an output); otherwise reuse units sum them as they enter the second product.
-template <int NQB, bool REUSE, bool WITH_V, bool PAGED, int D, typename T, bool EXACT_SUM = false>
-__device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK, T* sV) {
+// passes whose log-sum is an output); otherwise units sum them as they enter the second product.
+template <bool PAGED, int D, typename T, bool EXACT_SUM>
+__device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
     typedef typename Elem<T>::x2 x2_t;
     typedef AttnTile<D> G_;
     constexpr int kKT = G_::kKT, kKS = G_::kKS, kDB = G_::kDB, kKB = G_::kKB, kChunks = G_::kChunks;
-    constexpr int NQ = 2 * NQB;     // blocks of 16 queries
     constexpr int kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
@@ -94,13 +95,12 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     const T* Kp = (const T*)p.K;
     const T* Vp = (const T*)p.V;
 
-    constexpr int QT = 32 * NQB;
+    constexpr int QT = 32, NQ = 2;   // blocks of 16 queries
     const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
-    // resident per compute unit: two with V (64 KB of LDS, 256 registers), K only by the registers
-    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : 3;
-    unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
+    // two workgroups are resident on a compute unit (64 KB of LDS, 256 registers)
+    unit_of_workgroup(p.B, p.G * hs.subs, nqt, 2, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
     const int L = q_start + Lqv;    // keys of this sequence
@@ -109,6 +109,11 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         sub = g % hs.subs;
         g /= hs.subs;               // the KV head
     }
+    // Whose lists a sparse unit reads: a scalar load, on its way while the first rows' addresses are formed (as a vector
+    // load every sparse unit waited for it before it requested anything: 3001 tokens 24.3 -> 23.9 us, head_dim 64
+    // at 4096 12.4 -> 12.2)
+    typedef const __attribute__((address_space(4))) int* ConstantPtr;
+    const int mapped = *(ConstantPtr)(p.head_map + __builtin_amdgcn_readfirstlane(g));
     const int tq = nqt - 1 - blk;   // long (late) query blocks first
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
@@ -125,7 +130,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     bool sparse = false;
     int n = 0, ng = 0;
     const int* idx_row = nullptr;
-    if (REUSE) {
+    {
         // a sequence of a mixed batch keeps the budget it has on its own (the rows are as wide as
         // the longest sequence needs)
         const int width = p.q_start_rows ? min(p.max_topk, topk_width_of(p.topk_percent, L)) : p.max_topk;
@@ -134,12 +139,10 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         if (q0 > n) {
             sparse = true;
             ng = (n + kKT - 1) / kKT;
-            const int src = max(0, min(p.head_map[g], kvh - 1));   // a map built for another head count must not leave the tensor
-            idx_row = p.idx + (((long long)b * kvh + src) * p.T + tq) * p.max_topk;
         }
     }
     const int ntiles = sparse ? ng + 1 : (min(q0 + QT, L) + kKT - 1) / kKT;
-    const bool idx_vec = REUSE && (p.max_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(p.idx) & 15) == 0;
+    const bool idx_vec = (p.max_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(p.idx) & 15) == 0;
 
     // ---- tile staging: wavefront w fills rows [4w R, 4(w+1) R) of a tile with four loads of R rows
     // each (R = 4 at D = 128, 8 at D = 64); lane = (row within the load, chunk position) ----
@@ -160,7 +163,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     const int page_mask = (1 << p.page_shift) - 1;
     const int max_row = PAGED ? (p.num_pages << p.page_shift) - 1 : 0;
     const uint32_t lds_k = lds_address(sK) + wave_u * 4096;   // this wavefront's 4 KB of a K buffer
-    const uint32_t lds_v = WITH_V ? lds_address(sV) + wave_u * 4096 : 0;
+    const uint32_t lds_v = lds_address(sV) + wave_u * 4096;
 
     // key position `pos` of tile `ti` -> key id (contiguous and diagonal tiles)
     auto tile_key = [&](int ti, int pos) {
@@ -192,43 +195,30 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // loads themselves are issued one at a time between the matrix instructions of the first
     // product: a wavefront that issued all eight at once would sit in front of the memory
     // pipeline, which takes 16 cycles per 1 KB load, with nothing running behind it.
-    // lane_ptr: the chunk this lane fetches for row j of key 0 (REUSE) or of the position's row within a tile,
-    // within a page if PAGED (passes over consecutive keys alone: one addition a row and tile, a product a page).
+    // lane_ptr: the chunk this lane fetches for row j, of cache row 0.
     const char* lane_ptr[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz16<D>(slot0 + j * kRPL)) * 8);
-        if (!REUSE) lane_ptr[j] += (unsigned long long)row_bytes * (unsigned)(PAGED ? (pos0 + j) & page_mask : pos0 + j);
     }
     const char* row_ptr[4];
     auto next_rows = [&]() {
-        if (REUSE && sparse && pend_ti < ng) {
+        if (sparse && pend_ti < ng) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {   // a corrupt index must not leave the tensor
                 const int row = max(0, min(ids[j], PAGED ? max_row : L - 1));
                 row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
             }
-        } else if (!REUSE && (pend_ti + 1) * kKT <= L) {   // uniform
-            const int k0 = pend_ti * kKT;
-            const unsigned long long off = PAGED ? (unsigned long long)row_bytes * (unsigned)((ids[0] << p.page_shift) + (k0 & page_mask))
-                                                 : (unsigned long long)row_bytes * (unsigned)k0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) row_ptr[j] = lane_ptr[j] + off;
         } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int key = tile_key(pend_ti, pos0 + j);
-                int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
-                if (REUSE) {
-                    row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
-                } else {   // lane_ptr is ahead by the position's row: may be a step back
-                    row -= PAGED ? (pos0 + j) & page_mask : pos0 + j;
-                    row_ptr[j] = lane_ptr[j] + (long long)row_bytes * row;
-                }
+                const int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
+                row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
             }
         }
     };
-    constexpr int kNumLoads = WITH_V ? 8 : 4;
+    constexpr int kNumLoads = 8;
     auto issue_load = [&](auto i_c, int buf) {   // i < 4: K row group i; else V row group i - 4
         constexpr int i = decltype(i_c)::value;
         if constexpr (i < 4) load_to_lds_16(row_ptr[i], lds_k + buf * (kTileElems * 2) + i * 1024);
@@ -250,11 +240,11 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // (representable in fp16 and bf16, sums and products are kept in fp32) and the rescaling of the
     // accumulators -- 64 products per lane -- runs on the first tiles of a unit and then almost
     // never.  The quotient is the same: numerator and denominator carry the same factor.
-    constexpr int kPrio = WITH_V ? KASCADE_PRIO_V : KASCADE_PRIO_K;
+    constexpr int kPrio = KASCADE_PRIO_V;
     constexpr float kRefSlack = 8.f;
     // Reuse units sum the exponentials as they enter the second product (rounded to the element
     // type, two per instruction); the passes whose log-sum feeds the selection sum them in fp32.
-    constexpr bool kPairSum = REUSE && WITH_V && !EXACT_SUM;
+    constexpr bool kPairSum = !EXACT_SUM;
     float m[NQ];
     float l[NQ];
     float4_t oT[NQ][kDB];      // query block, 16 output columns
@@ -272,11 +262,10 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // the first gathered tile and then its rows are still on their way -- one dependent trip to
     // memory less before the first product of every unit, and units are short (28 tiles on
     // average under rolling budgets).  Softmax is accumulated online, so the order is free.
-    auto tile_at = [&](int s) { return (REUSE && sparse) ? (s == 0 ? ng : s - 1) : s; };
+    auto tile_at = [&](int s) { return sparse ? (s == 0 ? ng : s - 1) : s; };
     fetch_ids(tile_at(0));
     next_rows();
     static_for<0, kNumLoads>([&](auto i) { issue_load(i, 0); });
-    if (ntiles > 1) fetch_ids(tile_at(1));
 
     // ---- Q fragments (B operand of S^T): query col (+ 16 q), d chunk 32*ks + 8*dq; requested after
     // the first tile's rows, which the first barrier waits for ----
@@ -296,6 +285,12 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         }
     }
 
+    if (sparse) {
+        const int src = max(0, min(mapped, kvh - 1));   // a map built for another head count must not leave the tensor
+        idx_row = p.idx + (((long long)b * kvh + src) * p.T + tq) * p.max_topk;
+    }
+    if (ntiles > 1) fetch_ids(tile_at(1));
+
     // One tile: registers -> LDS, next tile's loads, both products, softmax.  Three copies of
     // the code, each straight-line: tiles that need no mask (all but one or two of a unit), tiles
     // that do (the causal edge, the end of the sequence, a selection that ends inside a tile), and
@@ -303,7 +298,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     constexpr int kFull = 0, kMasked = 1, kDiag = 2;
     auto run_tile = [&](int sq, auto mode_c) {
         constexpr int MODE = decltype(mode_c)::value;
-        constexpr int nkb = (MODE == kDiag && QT == 32) ? 2 : kKB;
+        constexpr int nkb = (MODE == kDiag) ? 2 : kKB;
         const int ti = tile_at(sq);
         const T* bK = sK + (sq & 1) * kTileElems;
         const T* bV = sV + (sq & 1) * kTileElems;
@@ -399,51 +394,12 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
                 const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
                 m[q] = mnew;
                 l[q] *= corr;
-                if (WITH_V) {
+                {
 #pragma unroll
                     for (int db = 0; db < kDB; ++db) oT[q][db] *= corr;
                 }
             }
         };
-        if constexpr (!WITH_V) {
-            // Log-sums alone: the same rule, but the maximum is only formed on the first tiles and where a lane's
-            // sum says that a score may lie kRefSlack above its reference (its exponential alone is 2^kRefSlack
-            // then), or is no number (the reference still is -inf); then the exponentials are formed anew.
-            constexpr float kSumLimit = 250.f;
-            // A unit's first tiles move it often, and forming the exponentials twice costs more than the maximum:
-            // 16 tiles of 64 keys (517 tokens 10.6 -> 9.9 us, 1024 17.5 -> 16.1, the long calls unchanged), all
-            // tiles of 128 (4096 tokens at head_dim 64: 36.1 -> 34.5).
-            constexpr int kEarly = D == 64 ? 0x7fffffff : 16;
-#pragma unroll
-            for (int q = 0; q < NQ; q += 2) {
-                float sum[2];
-                auto sums = [&](float mu0, float mu1) {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        sum[i] = 0.f;
-#pragma unroll
-                        for (int kb = 0; kb < nkb; ++kb)
-#pragma unroll
-                            for (int v = 0; v < 4; ++v)
-                                sum[i] += fast_exp2(__builtin_fmaf(sT[q + i][kb][v], kScaleLog2, -(i ? mu1 : mu0)));
-                    }
-                };
-                bool look = sq < kEarly;   // wavefront-uniform
-                if (!look) {
-                    sums(m[q], m[q + 1]);
-                    look = __any(!(sum[0] <= kSumLimit) || !(sum[1] <= kSumLimit));
-                }
-                if (look) {
-                    const float ms[2] = {maximum(q), maximum(q + 1)};
-                    if (__any(ms[0] > m[q] + kRefSlack || ms[1] > m[q + 1] + kRefSlack)) move_references(q, ms);
-                    sums(m[q] == -INFINITY ? 0.f : m[q], m[q + 1] == -INFINITY ? 0.f : m[q + 1]);
-                }
-                l[q] += sum[0];
-                l[q + 1] += sum[1];
-            }
-            tile_phase<kPrio>(2);
-            return;
-        }
         {
             const float ms[2] = {maximum(0), maximum(1)};
             if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) move_references(0, ms);   // wavefront-uniform
@@ -457,7 +413,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
             for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) e[kb][v] = fast_exp2(__builtin_fmaf(sT[q][kb][v], kScaleLog2, -mu));
-            if (WITH_V) {
+            {
 #pragma unroll
                 for (int s = 0; s < nkb / 2; ++s) {
                     x8_t t;
@@ -486,7 +442,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         // ---- O^T += V^T P^T: step s covers the keys of blocks 2 s and 2 s + 1, whose scores lane dq holds: rows
         // 32 s + 16 h + 4 dq + (0..3), h = 0, 1, of the tile.  The operands of a group of steps are read
         // while the group before it is multiplied ----
-        if (WITH_V) {
+        {
             constexpr int kPS = nkb / 2;
             auto read_v = [&](int db, int s, int h) {
                 const T* vp = bV + (32 * s + 16 * h) * D + vrd + ((2 * db) ^ vchunk) * 8;
@@ -528,13 +484,13 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
 
     {
         int sq = 0;
-        if (REUSE && sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
+        if (sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
             if (kKT == 64) run_tile(0, std::integral_constant<int, kDiag>{});
             else run_tile(0, std::integral_constant<int, kMasked>{});
             sq = 1;
         }
         // tiles wholly below the unit's first query and inside the sequence / wholly inside the selection
-        const int full_end = (REUSE && sparse) ? 1 + n / kKT : min((q0 + 1) / kKT, L / kKT);
+        const int full_end = sparse ? 1 + n / kKT : min((q0 + 1) / kKT, L / kKT);
         for (; sq < full_end; ++sq) run_tile(sq, std::integral_constant<int, kFull>{});
         for (; sq < ntiles; ++sq) run_tile(sq, std::integral_constant<int, kMasked>{});
     }
@@ -543,8 +499,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
     // ---- epilogue (rows are local to this call).  A lane holds one query's output spread over its
     // registers; the rows go through the wavefront's share of the (now idle) K buffers so that they
     // leave as whole rows: 16-byte stores, four rows per instruction ----
-    static_assert(!WITH_V || NQB == 1, "the output pass is written for 32 queries per wavefront");
-    if (WITH_V) __syncthreads();   // everybody is done with the tile buffers
+        __syncthreads();   // everybody is done with the tile buffers
     T* so = sK + wave * (32 * D);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -552,7 +507,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
         const float lt = sum_over_quarters(l[q]);
         if (p.log_sum && dq == 0 && ql < Lqv && real_head)
             p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[q];
-        if (WITH_V) {
+        {
             const float inv = 1.f / lt;
             const int row = 16 * q + col;
 #pragma unroll
@@ -562,7 +517,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
             }
         }
     }
-    if (WITH_V) {
+    {
         __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
 #pragma unroll
         for (int j = 0; j < 32 / kRPL; ++j) {
@@ -577,6 +532,386 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillParams& p, T* sK,
 }
 
 
+// Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
+// tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and the
+// last bits of the log-sums decide between tokens whose pooled scores lie within one step at a selection's threshold.
+template <int NQB, bool WITH_V, bool PAGED, int D, typename T>
+__device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK, T* sV) {
+    typedef typename Elem<T>::x8 x8_t;
+    typedef typename Elem<T>::x4 x4_t;
+    typedef AttnTile<D> G_;
+    constexpr int kKT = G_::kKT, kKS = D / 16, kDB = D / 32, kKB = kKT / 32, kChunks = G_::kChunks;
+    constexpr int kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
+    constexpr float kScaleLog2 = ScaleLog2<D>::value;
+    const HeadSlots hs = head_slots(p.gs);
+    const int kvh = p.G, nheads = p.G * hs.gs;
+    const T* Qp = (const T*)p.Q;
+    const T* Kp = (const T*)p.K;
+    const T* Vp = (const T*)p.V;
+
+    // All arguments in one trip to memory: left alone, the compiler loads them in three, each where it is first used
+    // (log-sums alone, 1024 tokens: 15.9 -> 15.7 us; dense 2048 45.1 -> 44.5).  Sparse units have more arguments than
+    // registers to keep them in: 4096 tokens 31.2 -> 31.8.
+    asm volatile("" :: "s"(p.q_start_rows), "s"(p.q_len_rows), "s"(p.q_sb), "s"(p.q_sl), "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_sl),
+                 "s"(p.k_sh), "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.L), "s"(p.gs));
+    constexpr int QT = 32 * NQB;
+    const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
+    const int nqt = (Lq + QT - 1) / QT;
+    int blk, g, b;
+    // resident per compute unit: two with V (64 KB of LDS, 256 registers), K only by the registers
+    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : PAGED && D == 64 ? 3 : 4;
+    unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
+    int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
+    chunk_of_sequence(p, b, q_start, Lqv);
+    const int L = q_start + Lqv;    // keys of this sequence
+    int sub = 0;
+    if (hs.subs > 1) {
+        sub = g % hs.subs;
+        g /= hs.subs;               // the KV head
+    }
+    const int tq = nqt - 1 - blk;   // long (late) query blocks first
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6;
+    const int lane = tid & 63;
+    const int li = lane & 31;
+    const int lg = lane >> 5;
+    const int q0l = tq * QT;            // first query row of this block
+    if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
+    const int q0 = q_start + q0l;       // its global position
+    const int head = g * hs.gs + min(4 * sub + wave, hs.gs - 1);
+    const bool real_head = 4 * sub + wave < hs.gs;   // a slot beyond the last head computes along and stores nothing
+
+    const int ntiles = (min(q0 + QT, L) + kKT - 1) / kKT;
+
+    // ---- tile staging: wavefront w fills rows [4w R, 4(w+1) R) of a tile with four loads of R rows
+    // each (R = 4 at D = 128, 8 at D = 64); lane = (row within the load, chunk position) ----
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int lrow = lane / kChunks;
+    const int lchunk = lane % kChunks;
+    // This lane's four rows sit at LDS rows slot0 + j R (j = load) and hold the four consecutive
+    // tile positions pos0 + j: one 16-byte load brings their four indices, one block-table entry
+    // covers their page, and the rows of a tile in LDS are a permutation of its keys -- which only
+    // the masks need to know (both products contract over the same order).
+    const int slot0 = wave * 4 * kRPL + lrow;
+    const int pos0 = 4 * (wave * kRPL + lrow);
+    // tile position of LDS row `slot`
+    auto pos_of_slot = [](int slot) { return 4 * ((slot / (4 * kRPL)) * kRPL + slot % kRPL) + (slot / kRPL) % 4; };
+    const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
+    const unsigned long long v_from_k = (unsigned long long)Vp - (unsigned long long)Kp;   // V shares K's layout
+    const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
+    const int page_mask = (1 << p.page_shift) - 1;
+    const uint32_t lds_k = lds_address(sK) + wave_u * 4096;   // this wavefront's 4 KB of a K buffer
+    const uint32_t lds_v = WITH_V ? lds_address(sV) + wave_u * 4096 : 0;
+    const unsigned row_bytes = 2 * (PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl);   // host checks stride < 2^31
+
+    // PAGED: block-table entry of this lane's rows of a tile (four consecutive keys from a multiple of four on: one
+    // page), fetched a tile ahead so that the loads never wait on it
+    int page = 0;
+    auto fetch_page = [&](int ti) {
+        if (PAGED) page = bt_row[min(ti * kKT + pos0, L - 1) >> p.page_shift];
+    };
+    // K row addresses of a tile; V's are a scalar offset away.  The
+    // loads themselves are issued one at a time between the matrix instructions of the first
+    // product: a wavefront that issued all eight at once would sit in front of the memory
+    // pipeline, which takes 16 cycles per 1 KB load, with nothing running behind it.
+    // lane_ptr: the chunk this lane fetches for row j of a tile, within a page if PAGED: one addition a row and
+    // tile, one product a tile.
+    const char* lane_ptr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz<D>(slot0 + j * kRPL)) * 8) +
+                      (unsigned long long)row_bytes * (unsigned)(PAGED ? (pos0 + j) & page_mask : pos0 + j);
+    const char* row_ptr[4];
+    auto next_rows = [&](int ti) {
+        const int k0 = ti * kKT;
+        if (k0 + kKT <= L) {   // uniform
+            const unsigned long long off = (unsigned long long)row_bytes *
+                                           (unsigned)(PAGED ? (page << p.page_shift) + (k0 & page_mask) : k0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) row_ptr[j] = lane_ptr[j] + off;
+        } else {               // rows past the sequence's end: the last one again
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int key = min(k0 + pos0 + j, L - 1);
+                const int row = PAGED ? (page << p.page_shift) + (key & page_mask) - ((pos0 + j) & page_mask) : key - (pos0 + j);
+                row_ptr[j] = lane_ptr[j] + (long long)row_bytes * row;
+            }
+        }
+    };
+    constexpr int kNumLoads = WITH_V ? 8 : 4;
+    auto issue_load = [&](auto i_c, int buf) {   // i < 4: K row group i; else V row group i - 4
+        constexpr int i = decltype(i_c)::value;
+        if constexpr (i < 4) load_to_lds_16(row_ptr[i], lds_k + buf * (kTileElems * 2) + i * 1024);
+        else load_to_lds_16<(i - 4) * 1024>(row_ptr[i - 4], v_from_k, lds_v + buf * (kTileElems * 2));
+    };
+    // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 32 kb + li,
+    // chunk 2 ks + lg.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):
+    // the 16 lanes of a group address rows 16 s + 8 h + 4 lg + (0..3) of a key block, 16 columns
+    // of V from column 32 db + 16 (group & 1) on, and receive one column of the four rows each.
+    const int kx = lg ^ swz<D>(li);
+    const int krd = li * D;
+    const int vcol = lane & 15;
+    const int vrow = 4 * lg + (vcol >> 2);                          // + 32 kb + 16 s + 8 h
+    const int vchunk = 2 * ((lane >> 4) & 1) + ((vcol >> 1) & 1);    // + 4 db
+    const int vrd = vrow * D + 4 * (vcol & 1);
+
+    // Softmax state.  m[] is the reference the exponentials are taken against, in log2 units of
+    // the scaled scores.  It follows the running maximum lazily: a tile moves it only when one of
+    // its scores lies more than kRefSlack above it, so an exponential never exceeds 2^kRefSlack
+    // (representable in fp16 and bf16, sums and products are kept in fp32) and the rescaling of the
+    // accumulators -- 64 products per lane -- runs on the first tiles of a unit and then almost
+    // never.  The quotient is the same: numerator and denominator carry the same factor.
+    constexpr int kPrio = WITH_V ? KASCADE_PRIO_V : KASCADE_PRIO_K;
+    constexpr float kRefSlack = 8.f;
+    float m[NQB], l[NQB];
+    float16_t oT[NQB][kDB];
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+        m[qb] = -INFINITY;
+        l[qb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < kDB; ++db)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) oT[qb][db][v] = 0.f;
+    }
+
+    fetch_page(0);
+    next_rows(0);
+    static_for<0, kNumLoads>([&](auto i) { issue_load(i, 0); });
+    if (ntiles > 1) fetch_page(1);
+
+    // ---- Q fragments (B operand of S^T): query li (+32 qb), d chunk 16*ks + 8*lg; requested after
+    // the first tile's rows, which the first barrier waits for ----
+    x8_t qf[NQB][kKS];
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+        const int ql = q0l + 32 * qb + li;
+        const bool ok = ql < Lqv;
+        const T* qp = Qp + (long long)b * p.q_sb + (long long)min(ql, Lqv - 1) * p.q_sl +
+                      (long long)head * p.q_sh + lg * 8;
+#pragma unroll
+        for (int ks = 0; ks < kKS; ++ks) {
+            PackT<T> t;
+            t.u = ld_global_16(qp + ks * 16);
+            if (!ok) t.u = uint4_t{0, 0, 0, 0};
+            qf[qb][ks] = t.v8;
+        }
+    }
+
+    // One tile: next tile's loads, both products, softmax.  Two copies of
+    // the code, each straight-line: tiles that need no mask (all but one or two of a unit) and tiles
+    // that do (the causal edge, the end of the sequence).
+    auto run_tile = [&](int sq, auto masked_c) {
+        constexpr bool MASKED = decltype(masked_c)::value;
+        constexpr int nkb = kKB;
+        const T* bK = sK + (sq & 1) * kTileElems;
+        const T* bV = sV + (sq & 1) * kTileElems;
+        // own loads of this tile landed; after the barrier everybody's have, and everybody is done
+        // reading the other buffer (the tile before), which the next tile's loads may now fill
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        // The next tile's loads go out between the products below, unconditionally: after the last
+        // tile they fetch its rows once more into the idle buffer (1/28 of the traffic on average,
+        // from the cache) rather than put a branch between the matrix instructions.
+        // The block-table entry of the tile behind that one is requested before those loads: the compiler waits for
+        // every load on its way before it lets one of its own overwrite a register, and behind the
+        // tile's loads that wait was a whole trip to memory (chunk of 512 queries at 14336: 324 -> 260 us).
+        if (sq + 1 < ntiles) next_rows(sq + 1);
+        if (sq + 2 < ntiles) fetch_page(sq + 2);
+        const int nbuf = (sq + 1) & 1;
+
+        tile_phase<kPrio>(0);
+        // ---- S^T = K_tile Q^T.  Step c = (key block c / kKS, contraction step c % kKS); operands are
+        // read from LDS two windows (four steps) ahead of the products that use them, in program
+        // order, because LDS reads do not move across the load statements ----
+        constexpr int kSteps = nkb * kKS;
+        float16_t sT[NQB][nkb];
+        float16_t zero16;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
+        auto read_a = [&](int c) {
+            return *reinterpret_cast<const x8_t*>(&bK[32 * (c / kKS) * D + krd + ((2 * (c % kKS)) ^ kx) * 8]);
+        };
+        constexpr int kAhead = (kKB <= 2) ? 2 : 1;   // windows read ahead (registers are scarcer at D = 64)
+        x8_t aw[kAhead + 1][2];
+#pragma unroll
+        for (int c = 0; c < 2 * kAhead && c < kSteps; ++c) aw[c >> 1][c & 1] = read_a(c);
+        static_for<0, kSteps / 2>([&](auto w_c) {
+            constexpr int w = decltype(w_c)::value;
+            if (2 * (w + kAhead) < kSteps) {
+                aw[(w + kAhead) % (kAhead + 1)][0] = read_a(2 * (w + kAhead));
+                aw[(w + kAhead) % (kAhead + 1)][1] = read_a(2 * (w + kAhead) + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // the scheduler would sink the reads to their use
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int kb = (2 * w + i) / kKS, ks = (2 * w + i) % kKS;
+#pragma unroll
+                for (int qb = 0; qb < NQB; ++qb)   // the first product starts from a constant zero
+                    sT[qb][kb] = Elem<T>::mma_32x32x16(aw[w % (kAhead + 1)][i], qf[qb][ks], ks == 0 ? zero16 : sT[qb][kb]);
+            }
+            if constexpr (w < kNumLoads) issue_load(w_c, nbuf);
+        });
+        static_for<kSteps / 2, kNumLoads>([&](auto i) { issue_load(i, nbuf); });
+        // ---- masks: accumulator v of key block kb is LDS row 32kb + 8(v/4) + 4lg + v%4 of the tile ----
+        if (MASKED) {   // the causal edge and the end of the sequence
+#pragma unroll
+            for (int qb = 0; qb < NQB; ++qb) {
+                const int q = q0 + 32 * qb + li;   // global position
+#pragma unroll
+                for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int key = sq * kKT + pos_of_slot(32 * kb + 8 * (v >> 2) + 4 * lg + (v & 3));
+                        if (key > q || key >= L) sT[qb][kb][v] = -INFINITY;
+                    }
+            }
+        }
+        // ---- online softmax (one query column per lane pair: lanes li and li + 32) ----
+        tile_phase<kPrio>(1);
+        x8_t pf[NQB][2 * nkb];
+#pragma unroll
+        for (int qb = 0; qb < NQB; ++qb) {
+            float sum;
+            auto exponentials = [&](float mu) {
+                sum = 0.f;
+                float e[nkb][16];
+#pragma unroll
+                for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        e[kb][v] = fast_exp2(__builtin_fmaf(sT[qb][kb][v], kScaleLog2, -mu));
+                        sum += e[kb][v];
+                    }
+                if (WITH_V) {
+#pragma unroll
+                    for (int s = 0; s < 2 * nkb; ++s) {
+                        x8_t t;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) t[i] = (T)e[s >> 1][8 * (s & 1) + i];
+                        pf[qb][s] = t;
+                    }
+                }
+            };
+            // Log-sums alone: the maximum is only formed on a unit's first tiles, which move the reference often (16 of 64
+            // keys, all of 128), and where a lane's sum says that a score may lie kRefSlack above the reference (its
+            // exponential alone is 2^kRefSlack then), or is no number (the reference still is -inf); then the
+            // exponentials are formed anew.  The rule is the same: the log-sums have the bits of the pass with an output.
+            constexpr float kSumLimit = 250.f;
+            bool look = WITH_V || D == 64 || sq < 16;   // wavefront-uniform
+            if (!look) {
+                exponentials(m[qb]);
+                look = __any(!(sum <= kSumLimit));
+            }
+            if (look) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sT[qb][kb][v]);
+                const float ms = mx * kScaleLog2;
+                if (__any(ms > m[qb] + kRefSlack)) {   // wavefront-uniform
+                    const float mnew = fmaxf(m[qb], max_with_other_half(ms));   // the same in both lanes of a column
+                    const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[qb] - mnew);
+                    m[qb] = mnew;
+                    l[qb] *= corr;
+                    if (WITH_V) {
+#pragma unroll
+                        for (int db = 0; db < kDB; ++db)
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) oT[qb][db][v] *= corr;
+                    }
+                }
+                exponentials((m[qb] == -INFINITY) ? 0.f : m[qb]);
+            }
+            l[qb] += sum;   // per-lane partial sum (own key positions)
+        }
+        tile_phase<kPrio>(2);
+        // ---- O^T += V^T P^T: step s covers the keys of accumulators 8(s&1) .. 8(s&1)+7 of key block
+        // s/2, i.e. rows 16 s + 8 h + 4 lg + (0..3), h = 0, 1, of the tile.  The operands of a block
+        // of 32 output rows are read while the block before it is multiplied ----
+        if (WITH_V) {
+            constexpr int kPS = 2 * nkb;
+            auto read_v = [&](int db, int s, int h) {
+                const int row = 16 * s + 8 * h;   // + vrow; only its low four bits enter swz
+                const T* vp = bV + row * D + vrd + ((4 * db + vchunk) ^ swz<D>(row + vrow)) * 8;
+                return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
+            };
+            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block)
+            constexpr int kGrp = (kKB <= 2) ? 4 : 2;
+            constexpr int kGroupsPV = kDB * kPS / kGrp;
+            short4_t av[2][kGrp][2];
+#pragma unroll
+            for (int i = 0; i < kGrp; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(i / kPS, i % kPS, h);
+#pragma unroll
+            for (int gq = 0; gq < kGroupsPV; ++gq) {
+                if (gq + 1 < kGroupsPV) {
+#pragma unroll
+                    for (int i = 0; i < kGrp; ++i)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+                            av[(gq + 1) & 1][i][h] = read_v((kGrp * (gq + 1) + i) / kPS, (kGrp * (gq + 1) + i) % kPS, h);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kGrp; ++i) {
+                    const int db = (kGrp * gq + i) / kPS, s = (kGrp * gq + i) % kPS;
+                    const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    const x8_t a = __builtin_bit_cast(x8_t, both);
+#pragma unroll
+                    for (int qb = 0; qb < NQB; ++qb)
+                        oT[qb][db] = Elem<T>::mma_32x32x16(a, pf[qb][s], oT[qb][db]);
+                }
+            }
+        }
+    };
+
+    // tiles wholly below the unit's first query and inside the sequence need no mask
+    const int full_end = min((q0 + 1) / kKT, L / kKT);
+    int sq = 0;
+    for (; sq < full_end; ++sq) run_tile(sq, std::false_type{});
+    for (; sq < ntiles; ++sq) run_tile(sq, std::true_type{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
+
+    // ---- epilogue (rows are local to this call).  A lane holds one query's output spread over its
+    // registers; the rows go through the wavefront's share of the (now idle) K buffers so that they
+    // leave as whole rows: 16-byte stores, four rows per instruction ----
+    static_assert(!WITH_V || NQB == 1, "the output pass is written for 32 queries per wavefront");
+    if (WITH_V) __syncthreads();   // everybody is done with the tile buffers
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+        const int ql = q0l + 32 * qb + li;
+        const float lt = sum_with_other_half(l[qb]);
+        if (p.log_sum && lg == 0 && ql < Lqv && real_head)
+            p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[qb];
+        if (WITH_V) {
+            T* so = sK + wave * (32 * D);
+            const float inv = 1.f / lt;
+#pragma unroll
+            for (int db = 0; db < kDB; ++db)
+#pragma unroll
+                for (int v4 = 0; v4 < 4; ++v4) {   // d = 32 db + 8 v4 + 4 lg .. +3: chunk 4 db + v4 of row li
+                    x4_t o = {(T)(oT[qb][db][4 * v4 + 0] * inv), (T)(oT[qb][db][4 * v4 + 1] * inv),
+                              (T)(oT[qb][db][4 * v4 + 2] * inv), (T)(oT[qb][db][4 * v4 + 3] * inv)};
+                    *reinterpret_cast<x4_t*>(&so[li * D + (((4 * db + v4) ^ (li & (kChunks - 1))) * 8) + 4 * lg]) = o;
+                }
+            __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
+#pragma unroll
+            for (int j = 0; j < 32 / kRPL; ++j) {
+                const int r = j * kRPL + lrow;
+                const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
+                const int qr = q0l + r;
+                if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
+                    __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
+                        (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
+            }
+        }
+    }
+}
+
+
 // 32 queries per wavefront: register budget capped so that two workgroups share a
 // compute unit (64 KB of LDS each: two K and two V tile buffers).
 template <bool REUSE, bool WITH_V, bool PAGED, int D, typename T, bool EXACT_SUM = false>
@@ -584,7 +919,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_attn_kernel_q32(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
     __shared__ __attribute__((aligned(1024))) T sV[WITH_V ? 2 * AttnTile<D>::kTileElems : 8];
-    prefill_attn_body<1, REUSE, WITH_V, PAGED, D, T, EXACT_SUM>(p, sK, sV);
+    if constexpr (REUSE) prefill_reuse_body<PAGED, D, T, EXACT_SUM>(p, sK, sV);
+    else prefill_dense_body<1, WITH_V, PAGED, D, T>(p, sK, sV);
 }
 
 // 64 queries per wavefront for the K-only log-sum pass, whose state fits 256 registers: two
@@ -595,55 +931,40 @@ template <bool PAGED, int D, typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_attn_kernel_q64(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
-    prefill_attn_body<2, false, false, PAGED, D, T>(p, sK, static_cast<T*>(nullptr));
+    prefill_dense_body<2, false, PAGED, D, T>(p, sK, static_cast<T*>(nullptr));
 }
 
 // Pooled tile scores: out[b,g,t,key] = sum over the 32 queries of tile t and the 4 q-heads of g
 // of exp2(s*scale - log_sum), for keys before the tile's first (global) position.
+// Two workgroups per compute unit (register budget 256): one wavefront's exponentials run
+// under the other's matrix instructions.  With 16x16x32 products, row addresses from scalar registers and the last
+// head's exponentials across the tile boundary 32768 tokens took 4.1 ms instead of 4.6, but a key's sum was then spread
+// over four lanes instead of two, and its last bits decide between tokens whose pooled scores lie within one
+// step at a selection's threshold.
 //
-// A wavefront takes 32 keys (a slice) of every 128-key tile and nobody else reads them.  Their rows go
+// A wavefront takes 32 keys of every 128-key tile and nobody else reads them.  Their rows go
 // from global memory straight into the wavefront's own LDS area (whole rows per load: read as
 // B operands directly, a 16-byte piece of 32 different rows per instruction, the same bytes kept
 // the data-return path of the memory pipeline busy 96 % of the kernel) and come back as B
 // operands (lane = key, 8 elements at d = 16 ks + 8 lg) from the chunk-permuted rows.  Two buffers
-// per wavefront, no barrier in the tile loop.
-//
-// What bounds it: the chip's power (long calls run at 1.6 GHz) and the issue of vector instructions, three per
-// score (multiply-add, exponential, sum).  So
-//  * the products are 16x16x32: at the power limit, random operands in registers, that instruction
-//    sustains 1.84 PFLOP/s, 32x32x16 1.59 (both 2.4 on zeros).
-//  * the loop spends next to nothing on anything but scores: a row address is one 64-bit addition, a pointer
-//    per lane that never changes plus an offset in scalar registers.
-//  * the exponentials of one head's scores run between the next head's matrix instructions, across the tile
-//    boundary too.  A slice's rows are in registers from the tile before on, so a buffer is free for the
-//    slice after the next one a quarter into the tile and its loads have more than a tile's time.
-// 32/8 heads, against 32x32x16 products with the row addresses formed per lane and the last head's exponentials at the
-// tile's end: 1024 tokens 11.1 -> 9.9 us, 4096 83.2 -> 75.0, 8192 314 -> 275, 32768 4.63 -> 4.06 ms (1.08 PFLOP/s),
-// chunks at position 14336 of 2048 queries 318 -> 292, of 512 at 15872 96.3 -> 87.9.
+// per wavefront, no barrier in the tile loop: the loads of the next tile are issued one per
+// contraction step and waited for at the top of that tile.
 template <bool PAGED, int D, typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_aggregate_kernel(PrefillParams p) {
     typedef typename Elem<T>::x8 x8_t;
-    constexpr int kSteps = D / 32;              // contraction steps
+    constexpr int kKS = D / 16;
     constexpr int kChunks = D / 8;
     constexpr int kRPL = 64 / kChunks;          // rows per load instruction
     constexpr int kLoads = 32 / kRPL;           // load instructions per wavefront and tile
     constexpr int kWaveElems = 32 * D;          // a wavefront's 32 rows
-    constexpr int kBufBytes = 4 * kWaveElems * 2;
-    constexpr int kPatterns = kLoads / 2;       // chunk permutations: loads j and j + kPatterns have the same
-    static_assert(kLoads == 2 * kSteps, "a load behind every second matrix instruction of a head");
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
     const int kvh = p.G, nheads = p.G * hs.gs;
     const T* Qp = (const T*)p.Q;
     const T* Kp = (const T*)p.K;
-    // the log-sums in front, where the LDS instructions' offsets reach them
-    __shared__ struct alignas(1024) {
-        float lse[128];
-        alignas(1024) T k[2 * 4 * kWaveElems];
-    } s_mem;
-    float* s_lse = s_mem.lse;
-    T* sK = s_mem.k;
+    __shared__ __attribute__((aligned(1024))) T sK[2 * 4 * kWaveElems];
+    __shared__ __attribute__((aligned(16))) float s_lse[128];
 
     const int Ls = p.L;                  // width of a row of pooled scores
     const int Lq = p.Lq;
@@ -653,12 +974,15 @@ void prefill_aggregate_kernel(PrefillParams p) {
     blk -= part * p.T;
     int q_start, Lqv;                    // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
+    const int L = q_start + Lqv;         // keys of this sequence
     const int t = p.T - 1 - blk;
     const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = tid >> 6;
     const int lane = tid & 63;
+    const int li = lane & 31;
+    const int lg = lane >> 5;
     const int tl = t * kTile;            // first query row of the tile
-    const int ts = q_start + tl;         // its global position: a multiple of 32
+    const int ts = q_start + tl;         // its global position
     half_t* out = p.agg + (((long long)b * kvh + g) * p.T + t) * Ls;
     const half_t neg_inf = (half_t)(-INFINITY);
 
@@ -673,71 +997,34 @@ void prefill_aggregate_kernel(PrefillParams p) {
             s_lse[tid] = counts ? p.log_sum_in[((long long)b * Lq + q) * nheads + head0 + (tid >> 5)] : INFINITY;
         }
 
-        // ---- staging: load j of a slice covers rows j kRPL + lrow of its 32.  The wavefront's slices are
-        // those of tiles ti0 .. ti0 + n - 1: all of their keys lie before the query tile, none past the
-        // sequence's end ----
-        const int n = min(ti1 - ti0, (ts / 32 - (4 * ti0 + wave) + 3) / 4);
-        const int key0 = ti0 * kAggKT + 32 * wave;         // first key of slice 0
+        // ---- staging: load j of a tile covers rows j kRPL + lrow of the wavefront's 32 ----
+        const int wave_u = __builtin_amdgcn_readfirstlane(wave);
         const int lrow = lane / kChunks;
         const int lchunk = lane % kChunks;
-        const unsigned row_stride = PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl;
         const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
-        const char* lane_ptr[kPatterns];
-#pragma unroll
-        for (int j = 0; j < kPatterns; ++j)
-            lane_ptr[j] = (const char*)(kbase + (long long)((unsigned long long)(unsigned)lrow * row_stride) +
-                                        (lchunk ^ swz16<D>(j * kRPL + lrow)) * 8);
+        const unsigned row_stride = PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl;
         const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
         const int page_mask = (1 << p.page_shift) - 1;
-        const uint32_t lds_w = lds_address(sK) + wave * (kWaveElems * 2);   // + buf * kBufBytes
-        // Block-table entries of 64 pages, one per lane (pages are at least four tokens, 64 of them two tiles),
-        // and of the 64 behind them
-        int pages = 0, pages_next = 0, page_group = 0;
-        auto fetch_pages = [&](int group) { return bt_row[min(64 * group + lane, p.max_pages - 1)]; };
-        if (PAGED && n > 0) {
-            page_group = (key0 >> p.page_shift) >> 6;
-            pages = fetch_pages(page_group);
-            pages_next = fetch_pages(page_group + 1);
-        }
-        unsigned long long row_off = 0;   // strided: offset of the next load's first row
-        const unsigned long long row_step = (unsigned long long)row_stride * (2 * kRPL);
-        auto offset_of_key = [&](int key) {   // uniform
-            int row = key;
-            if (PAGED) {
-                const int page = __builtin_amdgcn_readlane(pages, (key >> p.page_shift) & 63);
-                row = (page << p.page_shift) + (key & page_mask);
-            }
-            unsigned long long off = (unsigned long long)(unsigned)row * row_stride * 2;
-            asm("" : "+s"(off));   // stays in scalar registers: the compiler would multiply once per lane
-            return off;
+        const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * 4 * kWaveElems * 2
+        const T* my_k = sK + wave * kWaveElems;
+        // block-table entry of the key this lane stands for (row lane & 31 of the wavefront's 32),
+        // fetched a tile ahead; the lanes of a load pick theirs up with a lane permutation
+        int pg_next = 0;
+        auto fetch_page = [&](int ti) {
+            if (PAGED) pg_next = bt_row[min(ti * kAggKT + 32 * wave + li, L - 1) >> p.page_shift];
         };
-        auto enter_slice = [&](int i) {   // before the loads of slice i, slices in order
+        int pg_cur = 0;   // entries of the tile whose loads are being issued
+        auto issue_load = [&](int ti, int j, int buf) {
+            const int row = j * kRPL + lrow;
+            const int key = min(ti * kAggKT + 32 * wave + row, L - 1);
+            int src = key;
             if (PAGED) {
-                const int group = ((key0 + i * kAggKT) >> p.page_shift) >> 6;
-                if (group != page_group) {   // uniform
-                    page_group = group;
-                    pages = pages_next;
-                    pages_next = fetch_pages(group + 1);
-                }
-            } else {
-                row_off = offset_of_key(key0 + i * kAggKT);
+                const int pgv = __builtin_amdgcn_ds_bpermute(row << 2, pg_cur);
+                src = (pgv << p.page_shift) + (key & page_mask);
             }
-        };
-        auto issue_load = [&](int i, auto j_c, uint32_t lds_buf) {   // loads of a slice in order
-            constexpr int j = decltype(j_c)::value;
-            unsigned long long off = row_off;
-            if (PAGED) {
-                const int key = key0 + i * kAggKT + j * kRPL;
-                off = offset_of_key(key);
-                if (D == 64 && p.page_shift == 2) {   // eight rows per load, four per page
-                    const unsigned long long off4 = offset_of_key(key + 4) - 8ull * row_stride;
-                    load_to_lds_16(lane_ptr[j % kPatterns] + (lrow < 4 ? off : off4), lds_buf + j * 1024);
-                    return;
-                }
-            } else {
-                row_off += row_step;
-            }
-            load_to_lds_16<j * 1024>(lane_ptr[j % kPatterns], off, lds_buf);
+            const T* gp = kbase + (long long)((unsigned long long)(unsigned)src * row_stride) +
+                          (lchunk ^ swz<D>(row)) * 8;
+            load_to_lds_16(gp, lds_w + buf * (4 * kWaveElems * 2) + j * 1024);
         };
         // The tile's Q rows, head slot `wave` of the sub-group by this wavefront: whole rows into the
         // other buffer, chunks permuted like the keys' (fragments read from memory directly, every
@@ -747,129 +1034,94 @@ void prefill_aggregate_kernel(PrefillParams p) {
         for (int j = 0; j < kLoads; ++j) {
             const int row = j * kRPL + lrow;
             const T* qp = Qp + (long long)b * p.q_sb + (long long)min(tl + row, Lqv - 1) * p.q_sl +
-                          (long long)min(head0 + wave, g * hs.gs + hs.gs - 1) * p.q_sh;
-            load_to_lds_16(qp + (lchunk ^ swz16<D>(row)) * 8, lds_w + kBufBytes + j * 1024);
+                          (long long)min(head0 + wave_u, g * hs.gs + hs.gs - 1) * p.q_sh;
+            load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_w + ((ti0 + 1) & 1) * (4 * kWaveElems * 2) + j * 1024);
         }
-        if (n > 0) {
-            enter_slice(0);
-            static_for<0, kLoads>([&](auto j) { issue_load(0, j, lds_w); });
-        }
+        fetch_page(ti0);
+        pg_cur = pg_next;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) issue_load(ti0, j, ti0 & 1);
+        if (ti0 + 1 < ti1) fetch_page(ti0 + 1);
+        const int kx = lg ^ swz<D>(li);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // own rows have landed
         __syncthreads();                                   // everybody's, and s_lse
-        // Operands of 16 rows: lane (dq, col) holds row col, elements [32 ks + 8 dq, +8).  Offset of step 0's
-        // 16 bytes within 32 staged rows; step ks: bits 6 and up flipped, rows 16 .. 31: 16 rows further on
-        const int col = lane & 15, dq = lane >> 4;
-        const uint32_t at_lane = (uint32_t)(col * D + (dq ^ swz16<D>(col)) * 8) * 2;
-        auto read_op = [&](uint32_t addr, int half, int ks) {
-            return *(__attribute__((address_space(3))) const x8_t*)(size_t)((addr ^ (64 * ks)) + half * (16 * D * 2));
-        };
-        // A operands: head slot rb, query rows tl + 16 half + col
-        x8_t qa[kGroupSize][2][kSteps];
-        const uint32_t q_addr = lds_address(sK) + kBufBytes + at_lane;
+        // A operands: row block rb = head slot rb, row li = query tl + li
+        x8_t qa[kGroupSize][kKS];
+        const T* sQ = sK + ((ti0 + 1) & 1) * (4 * kWaveElems);
 #pragma unroll
         for (int rb = 0; rb < kGroupSize; ++rb)
 #pragma unroll
-            for (int half = 0; half < 2; ++half)
-#pragma unroll
-                for (int ks = 0; ks < kSteps; ++ks) {
-                    PackT<T> x;
-                    x.v8 = read_op(q_addr + rb * (kWaveElems * 2), half, ks);
-                    if (tl + 16 * half + col >= Lqv) x.u = uint4_t{0, 0, 0, 0};
-                    qa[rb][half][ks] = x.v8;
-                }
-        __syncthreads();   // the other buffer takes slice 1 from here on
+            for (int ks = 0; ks < kKS; ++ks) {
+                PackT<T> x;
+                x.v8 = *reinterpret_cast<const x8_t*>(&sQ[rb * kWaveElems + li * D + ((2 * ks) ^ kx) * 8]);
+                if (tl + li >= Lqv) x.u = uint4_t{0, 0, 0, 0};
+                qa[rb][ks] = x.v8;
+            }
+        __syncthreads();   // the other buffer takes the next tile's keys from here on
 
-        if (n > 0) {
-            auto read_lse = [&](int rb, int half) {
-                return *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 16 * half + 4 * dq]);
+        for (int ti = ti0; ti < ti1; ++ti) {
+            // this tile's rows have landed (and the next tile's block-table entries arrived)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const T* bK = my_k + (ti & 1) * (4 * kWaveElems);
+            const int tn = min(ti + 1, ti1 - 1);   // after the last tile: its rows once more, unused
+            const int nbuf = (ti + 1) & 1;
+            pg_cur = pg_next;
+            if (ti + 2 < ti1) fetch_page(ti + 2);
+
+            // Head by head, the exponentials of one head's scores between the matrix instructions of the
+            // next head's: a wavefront's vector and matrix work overlap within itself, which counts where
+            // few wavefronts share a SIMD (512 tokens 10.1 -> 9.1 us, 1024 12.0 -> 10.7; 32768 4.56 -> 4.44
+            // ms, where the clock follows the power limit).  Two heads' scores are live instead of four,
+            // which makes room for the tile's eight key operands.
+            float16_t acc[2];
+            float16_t zero16;   // the first product of a head starts from a constant zero
+#pragma unroll
+            for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
+            x8_t kb[kKS];
+#pragma unroll
+            for (int ks = 0; ks < kKS; ++ks) kb[ks] = *reinterpret_cast<const x8_t*>(&bK[li * D + ((2 * ks) ^ kx) * 8]);
+            float4_t ls[4];   // log-sums of the rows of the head whose exponentials are next
+            float sum = 0.f;
+            // accumulator v of head rb is query row 8(v/4) + 4lg + v%4, column = key li
+            auto exponentials = [&](const float16_t& s, int v0, int v1) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (v >= v0 && v < v1) sum += fast_exp2(s[v] * kScaleLog2 - ls[v >> 2][v & 3]);
             };
-            // log-sums of the rows of the head whose exponentials are next
-            float4_t ls[2] = {read_lse(kGroupSize - 1, 0), read_lse(kGroupSize - 1, 1)};
-            x8_t kb[2][kSteps];     // B operands: the slice's keys 16 kh + col
-            const uint32_t k_lane = lds_w + at_lane;
 #pragma unroll
-            for (int ks = 0; ks < kSteps; ++ks)
+            for (int rb = 0; rb < kGroupSize; ++rb) {
 #pragma unroll
-                for (int kh = 0; kh < 2; ++kh) kb[kh][ks] = read_op(k_lane, kh, ks);
-            enter_slice(min(1, n - 1));
-            static_for<0, kLoads>([&](auto j) { issue_load(min(1, n - 1), j, lds_w + kBufBytes); });
-            // A head's scores: acc[..][half][kh][v] is query row 16 half + 4 dq + v, key 16 kh + col.  It takes
-            // kProducts matrix instructions, and behind each of those of the next head kPer of them move on: scores
-            // into the exponent's arguments, the arguments of the step before through the exponential, the
-            // exponentials before those into the sums.  No instruction waits for the one in front of it, and
-            // none of the vector instructions for the matrix unit.
-            constexpr int kProducts = 4 * kSteps, kPer = 16 / kProducts;
-            float4_t acc[2][2][2];
-            const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
-            acc[1][0][0] = acc[1][0][1] = acc[1][1][0] = acc[1][1][1] = zero4;
-            float sum[2] = {}, arg[kPer] = {}, ex[kPer] = {};   // sum: of the keys col and 16 + col
-            auto add_step = [&](int step) {   // score e: row block e / 8, row e / 2 % 4, key block e % 2
+                for (int ks = 0; ks < kKS; ++ks) {
+                    acc[rb & 1] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks], ks == 0 ? zero16 : acc[rb & 1]);
+                    if (rb == 0 && ks < kLoads) issue_load(tn, ks, nbuf);
+                    if (rb > 0 && ks > 0) exponentials(acc[(rb - 1) & 1], 16 * (ks - 1) / (kKS - 1), 16 * ks / (kKS - 1));
+                    if (ks == kKS - 1) {
 #pragma unroll
-                for (int u = 0; u < kPer; ++u) sum[(step * kPer + u) & 1] += ex[u];
-                asm volatile("" : "+v"(sum[0]), "+v"(sum[1]));   // here, not where the sums are used
-#pragma unroll
-                for (int u = 0; u < kPer; ++u) ex[u] = fast_exp2(arg[u]);
-            };
-            auto exponentials = [&](const float4_t (&s)[2][2], int step, int head) {
-                add_step(step);
-#pragma unroll
-                for (int u = 0; u < kPer; ++u) {
-                    const int e = step * kPer + u, half = e >> 3, v = (e >> 1) & 3;
-                    arg[u] = s[half][e & 1][v] * kScaleLog2 - ls[half][v];
-                }
-                if (((step + 1) * kPer) % 8 == 0) {   // a row block's log-sums are free for the next head's
-                    const int half = ((step + 1) * kPer - 1) >> 3;
-                    ls[half] = read_lse((head + 1) % kGroupSize, half);
-                }
-            };
-            auto store_sum = [&](int i) {   // lane (dq, col): key 16 (dq & 1) + col, which quarters 0 and 1 write
-                const float total[2] = {sum_over_quarters(sum[0]), sum_over_quarters(sum[1])};
-                half_t* o = out + key0 + i * kAggKT + (lane & 31);
-                if (lane < 32) {   // a later sub-group of the KV head adds to what the earlier ones left
-                    float x = dq & 1 ? total[1] : total[0];
-                    if (p.accumulate) x += (float)*o;
-                    *o = (half_t)x;
-                }
-            };
-            for (int i = 0; i < n; ++i) {   // slice i, in registers; its buffer takes slice i + 2
-                const uint32_t buf = lds_w + (i & 1) * kBufBytes;
-                const uint32_t k_addr = k_lane + (~i & 1) * kBufBytes;   // of slice i + 1
-                const int in = min(i + 2, n - 1);       // after the last slice: its rows once more, unused
-                enter_slice(in);
-                tile_phase<KASCADE_PRIO_AGG>(2);
-#pragma unroll
-                for (int rb = 0; rb < kGroupSize; ++rb) {
-                    // the next slice's rows have landed: only the loads issued in this one may be on their way
-                    if (rb == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "i"(kLoads) : "memory");
-                    static_for<0, kProducts>([&](auto st_c) {
-                        constexpr int st = decltype(st_c)::value;
-                        const int ks = st >> 2, half = (st >> 1) & 1, kh = st & 1;
-                        acc[rb & 1][half][kh] = Elem<T>::mma_16x16x32(qa[rb][half][ks], kb[kh][ks], ks == 0 ? zero4 : acc[rb & 1][half][kh]);
-                        asm volatile("" :: "v"(acc[rb & 1][half][kh]));   // here, not where the scores are used
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (rb == 1 && kh == 0) issue_load(in, std::integral_constant<int, st / 2>{}, buf);
-                        if (rb == 3 && half == 1) kb[kh][ks] = read_op(k_addr, kh, ks);
-                        exponentials(acc[(rb + 1) & 1], st, (rb + kGroupSize - 1) % kGroupSize);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (rb == 1 && st == 1) {   // the slice before this one is summed up
-                            if (i > 0) store_sum(i - 1);
-                            sum[0] = sum[1] = 0.f;
-                        }
-                    });
+                        for (int v4 = 0; v4 < 4; ++v4)
+                            ls[v4] = *reinterpret_cast<const float4_t*>(&s_lse[rb * 32 + 8 * v4 + 4 * lg]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            tile_phase<KASCADE_PRIO_AGG>(1);
 #pragma unroll
-            for (int st = 0; st < kProducts; ++st) exponentials(acc[1], st, kGroupSize - 1);
-            add_step(0);
-            add_step(1);
-            store_sum(n - 1);
+            for (int j = kKS; j < kLoads; ++j) issue_load(tn, j, nbuf);
+            tile_phase<KASCADE_PRIO_AGG>(1);
+            exponentials(acc[(kGroupSize - 1) & 1], 0, 16);
+            sum = sum_with_other_half(sum);
+            tile_phase<KASCADE_PRIO_AGG>(2);
+            const int key = ti * kAggKT + 32 * wave + li;
+            if (lg == 0 && key < Ls) {
+                if (key < ts)   // a later sub-group of the KV head adds to what the earlier ones left
+                    out[key] = (half_t)(p.accumulate ? sum + (float)out[key] : sum);
+                else if (p.fill_invalid)
+                    out[key] = neg_inf;
+            }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
     }
     if (p.fill_invalid) {
         const int end = part == p.key_parts - 1 ? Ls : min(Ls, (ti0 + p.part_tiles) * kAggKT);
-        for (int key = max(tl < Lqv ? ts : 0, ti0 * kAggKT) + tid; key < end; key += kThreads) out[key] = neg_inf;
+        for (int key = max(ntiles, ti0) * kAggKT + tid; key < end; key += kThreads) out[key] = neg_inf;
     }
 }
 

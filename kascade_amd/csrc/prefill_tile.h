@@ -12,7 +12,7 @@ namespace {
 // and the score registers a narrower head frees hold the extra keys.
 template <int D> struct AttnTile {
     static constexpr int kKT = 64 * 128 / D;     // keys per tile
-    static constexpr int kKS = D / 32;           // contraction steps of S^T = K Q^T
+    static constexpr int kKS = D / 32;           // contraction steps of S^T = K Q^T, 16x16x32 products
     static constexpr int kDB = D / 16;           // 16-row blocks of O^T
     static constexpr int kKB = kKT / 16;         // 16-key blocks of a tile
     static constexpr int kChunks = D / 8;        // 16-byte chunks of a row
@@ -30,6 +30,11 @@ template <int D> struct AttnTile {
 template <int D> __device__ __forceinline__ int swz16(int row);
 template <> __device__ __forceinline__ int swz16<128>(int row) { return ((row & 3) << 2) | (-(row >> 2) & 3); }
 template <> __device__ __forceinline__ int swz16<64>(int row) { return (((row >> 1) & 1) << 2) | (-(row >> 2) & 3); }
+
+// The same for operands of 32 rows (lane (lg, li) reads chunk 2 ks + lg of row li; V in quarters of 4 rows x 4 chunks)
+template <int D> __device__ __forceinline__ int swz(int row);
+template <> __device__ __forceinline__ int swz<128>(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+template <> __device__ __forceinline__ int swz<64>(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 
 // One wavefront-wide load of 16 bytes per lane from global memory into LDS: lane i's bytes
 // land at lds_base + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
