@@ -997,34 +997,77 @@ void prefill_aggregate_kernel(PrefillParams p) {
             s_lse[tid] = counts ? p.log_sum_in[((long long)b * Lq + q) * nheads + head0 + (tid >> 5)] : INFINITY;
         }
 
-        // ---- staging: load j of a tile covers rows j kRPL + lrow of the wavefront's 32 ----
+        // ---- staging: load j of a tile covers rows j kRPL + lrow of the wavefront's 32.  Its slices of tiles
+        // ti0 .. ti0 + n - 1 hold keys before the query tile (all inside the sequence), in whole slices; for a tile behind
+        // those it stages the last one again.  A row address is one addition, a pointer per lane that never
+        // changes plus an offset in scalar registers (formed per lane, addresses were one vector instruction in four) ----
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+        const int n = min(ti1 - ti0, (ts / 32 - (4 * ti0 + wave_u) + 3) / 4);
+        auto key_of_tile = [&](int ti) { return n > 0 ? min(ti, ti0 + n - 1) * kAggKT + 32 * wave_u : 0; };
         const int lrow = lane / kChunks;
         const int lchunk = lane % kChunks;
-        const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
+        constexpr int kPatterns = kLoads / 2;       // chunk permutations: loads j and j + kPatterns have the same
         const unsigned row_stride = PAGED ? (unsigned)(kvh * D) : (unsigned)p.k_sl;
+        const T* kbase = PAGED ? Kp + (long long)g * D : Kp + (long long)b * p.k_sb + (long long)g * p.k_sh;
+        const char* lane_ptr[kPatterns];
+#pragma unroll
+        for (int j = 0; j < kPatterns; ++j)
+            lane_ptr[j] = (const char*)(kbase + (long long)((unsigned long long)(unsigned)lrow * row_stride) +
+                                        (lchunk ^ swz<D>(j * kRPL + lrow)) * 8);
         const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
         const int page_mask = (1 << p.page_shift) - 1;
         const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * 4 * kWaveElems * 2
         const T* my_k = sK + wave * kWaveElems;
-        // block-table entry of the key this lane stands for (row lane & 31 of the wavefront's 32),
-        // fetched a tile ahead; the lanes of a load pick theirs up with a lane permutation
-        int pg_next = 0;
-        auto fetch_page = [&](int ti) {
-            if (PAGED) pg_next = bt_row[min(ti * kAggKT + 32 * wave + li, L - 1) >> p.page_shift];
-        };
-        int pg_cur = 0;   // entries of the tile whose loads are being issued
-        auto issue_load = [&](int ti, int j, int buf) {
-            const int row = j * kRPL + lrow;
-            const int key = min(ti * kAggKT + 32 * wave + row, L - 1);
-            int src = key;
+        // Block-table entries of 64 pages, one per lane (pages are at least four tokens, 64 of them two tiles),
+        // and of the 64 behind them
+        int pages = 0, pages_next = 0, page_group = 0;
+        auto fetch_pages = [&](int group) { return bt_row[min(64 * group + lane, p.max_pages - 1)]; };
+        if (PAGED) {
+            page_group = (key_of_tile(ti0) >> p.page_shift) >> 6;
+            pages = fetch_pages(page_group);
+            pages_next = fetch_pages(page_group + 1);
+        }
+        unsigned long long row_off = 0;   // strided: offset of the next load's first row
+        const unsigned long long row_step = (unsigned long long)row_stride * (2 * kRPL);
+        int key0 = 0;                     // first key of the tile whose loads are being issued
+        auto offset_of_key = [&](int key) {   // uniform
+            int row = key;
             if (PAGED) {
-                const int pgv = __builtin_amdgcn_ds_bpermute(row << 2, pg_cur);
-                src = (pgv << p.page_shift) + (key & page_mask);
+                const int page = __builtin_amdgcn_readlane(pages, (key >> p.page_shift) & 63);
+                row = (page << p.page_shift) + (key & page_mask);
             }
-            const T* gp = kbase + (long long)((unsigned long long)(unsigned)src * row_stride) +
-                          (lchunk ^ swz<D>(row)) * 8;
-            load_to_lds_16(gp, lds_w + buf * (4 * kWaveElems * 2) + j * 1024);
+            unsigned long long off = (unsigned long long)(unsigned)row * row_stride * 2;
+            asm("" : "+s"(off));   // stays in scalar registers: the compiler would multiply once per lane
+            return off;
+        };
+        auto enter_tile = [&](int ti) {   // before the loads of a tile, tiles in order
+            key0 = key_of_tile(ti);
+            if (PAGED) {
+                const int group = (key0 >> p.page_shift) >> 6;
+                if (group != page_group) {   // uniform
+                    page_group = group;
+                    pages = pages_next;
+                    pages_next = fetch_pages(group + 1);
+                }
+            } else {
+                row_off = offset_of_key(key0);
+            }
+        };
+        auto issue_load = [&](int j, int buf) {   // loads of a tile in order
+            const uint32_t lds = lds_w + buf * (4 * kWaveElems * 2) + j * 1024;
+            unsigned long long off = row_off;
+            if (PAGED) {
+                const int key = key0 + j * kRPL;
+                off = offset_of_key(key);
+                if (D == 64 && p.page_shift == 2) {   // eight rows per load, four per page
+                    const unsigned long long off4 = offset_of_key(key + 4) - 8ull * row_stride;
+                    load_to_lds_16(lane_ptr[j % kPatterns] + (lrow < 4 ? off : off4), lds);
+                    return;
+                }
+            } else {
+                row_off += row_step;
+            }
+            load_to_lds_16<0>(lane_ptr[j % kPatterns], off, lds);
         };
         // The tile's Q rows, head slot `wave` of the sub-group by this wavefront: whole rows into the
         // other buffer, chunks permuted like the keys' (fragments read from memory directly, every
@@ -1037,11 +1080,9 @@ void prefill_aggregate_kernel(PrefillParams p) {
                           (long long)min(head0 + wave_u, g * hs.gs + hs.gs - 1) * p.q_sh;
             load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_w + ((ti0 + 1) & 1) * (4 * kWaveElems * 2) + j * 1024);
         }
-        fetch_page(ti0);
-        pg_cur = pg_next;
+        enter_tile(ti0);
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) issue_load(ti0, j, ti0 & 1);
-        if (ti0 + 1 < ti1) fetch_page(ti0 + 1);
+        for (int j = 0; j < kLoads; ++j) issue_load(j, ti0 & 1);
         const int kx = lg ^ swz<D>(li);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // own rows have landed
         __syncthreads();                                   // everybody's, and s_lse
@@ -1065,8 +1106,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
             const T* bK = my_k + (ti & 1) * (4 * kWaveElems);
             const int tn = min(ti + 1, ti1 - 1);   // after the last tile: its rows once more, unused
             const int nbuf = (ti + 1) & 1;
-            pg_cur = pg_next;
-            if (ti + 2 < ti1) fetch_page(ti + 2);
+            enter_tile(tn);
 
             // Head by head, the exponentials of one head's scores between the matrix instructions of the
             // next head's: a wavefront's vector and matrix work overlap within itself, which counts where
@@ -1093,7 +1133,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
 #pragma unroll
                 for (int ks = 0; ks < kKS; ++ks) {
                     acc[rb & 1] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks], ks == 0 ? zero16 : acc[rb & 1]);
-                    if (rb == 0 && ks < kLoads) issue_load(tn, ks, nbuf);
+                    if (rb == 0 && ks < kLoads) issue_load(ks, nbuf);
                     if (rb > 0 && ks > 0) exponentials(acc[(rb - 1) & 1], 16 * (ks - 1) / (kKS - 1), 16 * ks / (kKS - 1));
                     if (ks == kKS - 1) {
 #pragma unroll
@@ -1104,7 +1144,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
                 }
             }
 #pragma unroll
-            for (int j = kKS; j < kLoads; ++j) issue_load(tn, j, nbuf);
+            for (int j = kKS; j < kLoads; ++j) issue_load(j, nbuf);
             tile_phase<KASCADE_PRIO_AGG>(1);
             exponentials(acc[(kGroupSize - 1) & 1], 0, 16);
             sum = sum_with_other_half(sum);
