@@ -1,4 +1,4 @@
-// Prefill attention kernels for gfx950 (fp16/bf16 MFMA 16x16x32, fp32 softmax).
+// Prefill attention kernels for gfx950 (fp16/bf16 MFMA 32x32x16 and 16x16x32, fp32 softmax).
 //
 // prefill_attn_kernel -- flash attention over one (query block, KV head, batch)
 //   per workgroup; 4 wavefronts, wavefront w owns q-head 4g+w and 32*NQB queries,
@@ -10,25 +10,23 @@
 //   registers, no LDS store instructions) into one of two buffers, so a tile costs one
 //   barrier: wait for the own loads, barrier, start the next tile's loads into the other
 //   buffer, compute.  Rows lie in LDS as they lie in memory; the 16-byte chunk c of row R
-//   sits at chunk c ^ swz16(R), chosen by the lane that fetches it (each lane picks the global
+//   sits at chunk c ^ swz(R) (swz16 in sparse units), chosen by the lane that fetches it (each lane picks the global
 //   chunk that belongs at its LDS position), which makes both read patterns below free of
 //   bank conflicts without padding.
 //
-//   The kernel works on S^T = K Q^T so that four lanes (equal lane % 16) own one query column:
-//   row max / row sum are in-lane reductions plus two exchanges, and
+//   The kernel works on S^T = K Q^T so that two lanes (four in sparse units) own one query column:
+//   row max / row sum are in-lane reductions plus one or two exchanges, and
 //   the exponentiated scores are already in the B-operand layout of the second
 //   product O^T = V^T P^T -- P never leaves registers.  The A operand of that product,
 //   V^T, comes out of the row-major V tile through the transposing LDS read
 //   ds_read_b64_tr_b16 (two per operand: four keys each).
 //
 //   What bounds long calls is the chip's power, and per product 16x16x32 takes less of it than 32x32x16 (1.84
-//   against 1.59 PFLOP/s on random operands in registers).  Against 32x32x16 products, row addresses formed by a
-//   64-bit product per tensor and row, and list entries requested behind the tile's loads, 32/8 heads: dense
-//   2048 tokens 47.5 -> 44.4 us, 8192 524 -> 490, 32768 8.1 -> 7.6 ms, chunks at position 14336 of 512 queries
-//   324 -> 260 us, of 2048 501 -> 462; reuse 4096 36.4 -> 35.3 us, 32768 982 -> 948, but 517 9.48 -> 9.68 and 2048
-//   12.9 -> 13.2 (units of a few tiles: chains of latencies); log-sums alone 2048 30.8 -> 28.6, 32768 4.21 -> 3.85
-//   ms, chunk of 512 205 -> 168 us, of 2048 299 -> 266, but 1024 tokens of 64 heads 19.5 -> 21.0 (three units on
-//   a compute unit instead of four; held to the registers of four, 1024 tokens of 32 heads take 16.9 instead of 16.0).
+//   against 1.59 PFLOP/s on random operands in registers): sparse units use it (32/8 heads, 4096 tokens 36.4 -> 35.3
+//   us, 32768 982 -> 935).  Dense passes and pooling keep 32x32x16 (see there).  Against row addresses formed by a
+//   64-bit product per tensor and row and block-table entries requested behind the tile's loads: dense 517 tokens
+//   14.6 -> 13.5 us, 2048 49.4 -> 46.9, chunks at position 14336 of 512 queries 326 -> 247 us, of 2048 532 -> 520;
+//   log-sums alone 517 10.2 -> 9.6 us, 32768 4.39 -> 4.24 ms, chunks of 512 205 -> 173 us, of 2048 310 -> 301.
 //
 // prefill_aggregate_kernel -- pooled tile scores: S = Q_tile K^T with the 128
 //   (query, head) rows of a tile held as A operands in registers by every
@@ -533,8 +531,9 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
 
 
 // Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
-// tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and the
-// last bits of the log-sums decide between tokens whose pooled scores lie within one step at a selection's threshold.
+// tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and
+// the last bits of the log-sums decide between tokens whose pooled scores lie within one step at a selection's
+// threshold: single output rows of a 32768-token prompt moved by up to 0.27 of the outputs' root mean square.
 template <int NQB, bool WITH_V, bool PAGED, int D, typename T>
 __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
@@ -550,8 +549,8 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     const T* Vp = (const T*)p.V;
 
     // All arguments in one trip to memory: left alone, the compiler loads them in three, each where it is first used
-    // (log-sums alone, 1024 tokens: 15.9 -> 15.7 us; dense 2048 45.1 -> 44.5).  Sparse units have more arguments than
-    // registers to keep them in: 4096 tokens 31.2 -> 31.8.
+    // (with 16x16x32 products: log-sums alone, 1024 tokens 15.9 -> 15.7 us; dense 2048 45.1 -> 44.5).  Sparse units have
+    // more arguments than registers to keep them in: 4096 tokens 31.2 -> 31.8.
     asm volatile("" :: "s"(p.q_start_rows), "s"(p.q_len_rows), "s"(p.q_sb), "s"(p.q_sl), "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_sl),
                  "s"(p.k_sh), "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.L), "s"(p.gs));
     constexpr int QT = 32 * NQB;
