@@ -40,16 +40,12 @@ template <> __device__ __forceinline__ int swz<64>(int row) { return (((row >> 1
 // land at lds_base + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
 // compiler does not know that it writes LDS, so whoever reads the bytes waits for vmcnt and
 // passes a barrier first (the tile loop does both once per tile).
+// No vector ALU instruction belongs in here: the compiler puts no wait states between the matrix instructions and a
+// register that inline assembly writes, nor between the restore of a spilled scalar register and its use in there.
+// Addresses are formed by the callers, in C++.
 __device__ __forceinline__ void load_to_lds_16(const void* gptr, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :: "v"(gptr), "s"(lds_base) : "m0");
-}
-// The same from lane_ptr + off (off wavefront-uniform) to lds_base + OFF: the addition takes the place of the
-// wait between writing m0 and reading it.
-template <int OFF> __device__ __forceinline__ void load_to_lds_16(const void* lane_ptr, unsigned long long off, uint32_t lds_base) {
-    const void* ptr;
-    asm volatile("s_add_u32 m0, %2, %4\n\tv_lshl_add_u64 %0, %3, 0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                 : "=&v"(ptr) : "v"(lane_ptr), "s"(lds_base), "s"(off), "i"(OFF) : "m0", "scc");
 }
 template <typename P> __device__ __forceinline__ uint32_t lds_address(P* ptr) {
     return (uint32_t)(size_t)(__attribute__((address_space(3))) void*)ptr;
