@@ -775,12 +775,18 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
             auto exponentials = [&](float mu) {
                 sum = 0.f;
                 float e[nkb][16];
+                // At head_dim 64 a tile's 64 additions stand behind all of its exponentials: mixed with them, as at 128,
+                // their chain holds these up (14/2 heads, 4096 tokens: log-sums alone 48.6 -> 45.6 us, dense 66.7 ->
+                // 60.6; 32/8 heads: 53.2 -> 51.7 and 88.7 -> 84.0; a chunk of 2048 queries at 14336 196 -> 181 and 293
+                // -> 277; slower at 3001 tokens of 32/8 heads, log-sums alone 32.7 -> 33.7, and 8192 of 14/2, dense 188
+                // -> 193).  The order of addition is the same.
+                constexpr bool kSumsBehind = D == 64;
 #pragma unroll
                 for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         e[kb][v] = fast_exp2(__builtin_fmaf(sT[qb][kb][v], kScaleLog2, -mu));
-                        sum += e[kb][v];
+                        if (!kSumsBehind) sum += e[kb][v];
                     }
                 if (WITH_V) {
 #pragma unroll
@@ -790,6 +796,13 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
                         for (int i = 0; i < 8; ++i) t[i] = (T)e[s >> 1][8 * (s & 1) + i];
                         pf[qb][s] = t;
                     }
+                }
+                if (kSumsBehind) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) sum += e[kb][v];
                 }
             };
             // Log-sums alone: the maximum is only formed on a unit's first tiles, which move the reference often (16 of 64
