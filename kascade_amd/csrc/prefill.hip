@@ -557,8 +557,8 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
-    // resident per compute unit: two with V (64 KB of LDS, 256 registers), K only by the registers
-    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : PAGED && D == 64 ? 3 : 4;
+    // resident per compute unit: two with V (64 KB of LDS, 256 registers), four with K only (32 KB, 128 registers)
+    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : 4;
     unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
@@ -615,9 +615,11 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     // pipeline, which takes 16 cycles per 1 KB load, with nothing running behind it.
     // lane_ptr: the chunk this lane fetches for row j of a tile, within a page if PAGED: one addition a row and
     // tile, one product a tile.
-    const char* lane_ptr[4];
+    // At D = 64 rows j and j + 2 are permuted alike: over the paged cache, where registers are scarcer, two pointers do.
+    constexpr int kPtrs = PAGED && D == 64 ? 2 : 4;
+    const char* lane_ptr[kPtrs];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < kPtrs; ++j)
         lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz<D>(slot0 + j * kRPL)) * 8) +
                       (unsigned long long)row_bytes * (unsigned)(PAGED ? (pos0 + j) & page_mask : pos0 + j);
     const char* row_ptr[4];
@@ -627,13 +629,14 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
             const unsigned long long off = (unsigned long long)row_bytes *
                                            (unsigned)(PAGED ? (page << p.page_shift) + (k0 & page_mask) : k0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) row_ptr[j] = lane_ptr[j] + off;
+            for (int j = 0; j < 4; ++j) row_ptr[j] = lane_ptr[j % kPtrs] + (off + (unsigned long long)row_bytes * (j - j % kPtrs));
         } else {               // rows past the sequence's end: the last one again
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int key = min(k0 + pos0 + j, L - 1);
-                const int row = PAGED ? (page << p.page_shift) + (key & page_mask) - ((pos0 + j) & page_mask) : key - (pos0 + j);
-                row_ptr[j] = lane_ptr[j] + (long long)row_bytes * row;
+                const int pos = pos0 + j % kPtrs;   // the row that lane_ptr holds
+                const int row = PAGED ? (page << p.page_shift) + (key & page_mask) - (pos & page_mask) : key - pos;
+                row_ptr[j] = lane_ptr[j % kPtrs] + (long long)row_bytes * row;
             }
         }
     };
@@ -925,9 +928,10 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
 
 
 // 32 queries per wavefront: register budget capped so that two workgroups share a
-// compute unit (64 KB of LDS each: two K and two V tile buffers).
+// compute unit (64 KB of LDS each: two K and two V tile buffers), four without V (log-sums alone over the paged
+// cache at head_dim 64, in 134 registers and three: four chunks of 1024 queries at 4096, 32/8 heads, 122.5 -> 116.5 us).
 template <bool REUSE, bool WITH_V, bool PAGED, int D, typename T, bool EXACT_SUM = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(REUSE || WITH_V ? 2 : 4)))
 void prefill_attn_kernel_q32(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
     __shared__ __attribute__((aligned(1024))) T sV[WITH_V ? 2 * AttnTile<D>::kTileElems : 8];

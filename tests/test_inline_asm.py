@@ -9,6 +9,8 @@ registers (five wait states after a vector instruction that wrote them)."""
 import re
 import subprocess
 
+import pytest
+
 from kascade_amd import build
 
 SGPR = re.compile(r"\bs(\d+\b|\[\d+:\d+\])")
@@ -32,11 +34,24 @@ def _hazards(assembly):
     return kernels, found
 
 
-def test_inline_assembly_of_the_matrix_kernels_needs_no_wait_states(tmp_path):
-    out = tmp_path / "prefill.s"
+@pytest.fixture(scope="module")
+def assembly(tmp_path_factory):
+    out = tmp_path_factory.mktemp("asm") / "prefill.s"
     subprocess.run([build._hipcc(), *build.COMMON_FLAGS, "--cuda-device-only", "-S", str(build.CSRC / "prefill.hip"),
                     "-o", str(out)], check=True, capture_output=True)
-    assembly = out.read_text()
+    return out.read_text()
+
+
+def test_inline_assembly_of_the_matrix_kernels_needs_no_wait_states(assembly):
     kernels, found = _hazards(assembly)
     assert len(kernels) > 20 and "global_load_lds_dwordx4" in assembly   # the scan met what it looks for
     assert not found, f"{len(found)} lines, first {found[:3]}"
+
+
+def test_log_sum_units_of_32_queries_fit_four_to_a_compute_unit(assembly):
+    """The order of the units counts on four workgroups of the pass for log-sums alone per compute unit: 128
+    vector registers, none of them spilled, strided and paged, at both head dims."""
+    kernels = re.findall(r"\.name: +(\S+prefill_attn_kernel_q32ILb0ELb0E\S+)\n.*?\.private_segment_fixed_size: (\d+)"
+                         r".*?\.vgpr_count: +(\d+)", assembly, re.S)
+    assert len(kernels) == 8
+    assert all(int(vgprs) <= 128 and scratch == "0" for _, scratch, vgprs in kernels), kernels
