@@ -1016,7 +1016,11 @@ void prefill_aggregate_kernel(PrefillParams p) {
         // ---- staging: load j of a tile covers rows j kRPL + lrow of the wavefront's 32.  Its slices of tiles
         // ti0 .. ti0 + n - 1 hold keys before the query tile (all inside the sequence), in whole slices; for a tile behind
         // those it stages the last one again.  A row address is one addition, a pointer per lane that never
-        // changes plus an offset in scalar registers (formed per lane, addresses were one vector instruction in four) ----
+        // changes plus an offset in scalar registers (formed per lane, addresses were one vector instruction in four).
+        // kLanePages: rows over the paged cache at D = 64, whose loads take eight rows and so up to two pages, are formed
+        // per lane all the same (14/2 heads, 512 tokens 15.1 -> 14.2 us, 2048 queries at 14336 128.5 -> 127.6; 32/8
+        // heads: 512 queries at 2048 12.5 -> 12.1) ----
+        constexpr bool kLanePages = PAGED && D == 64;
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
         const int n = min(ti1 - ti0, (ts / 32 - (4 * ti0 + wave_u) + 3) / 4);
         auto key_of_tile = [&](int ti) { return n > 0 ? min(ti, ti0 + n - 1) * kAggKT + 32 * wave_u : 0; };
@@ -1028,17 +1032,20 @@ void prefill_aggregate_kernel(PrefillParams p) {
         const char* lane_ptr[kPatterns];
 #pragma unroll
         for (int j = 0; j < kPatterns; ++j)
-            lane_ptr[j] = (const char*)(kbase + (long long)((unsigned long long)(unsigned)lrow * row_stride) +
+            lane_ptr[j] = (const char*)(kbase + (kLanePages ? 0ll : (long long)((unsigned long long)(unsigned)lrow * row_stride)) +
                                         (lchunk ^ swz<D>(j * kRPL + lrow)) * 8);
         const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
         const int page_mask = (1 << p.page_shift) - 1;
         const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * 4 * kWaveElems * 2
         const T* my_k = sK + wave * kWaveElems;
         // Block-table entries of 64 pages, one per lane (pages are at least four tokens, 64 of them two tiles),
-        // and of the 64 behind them
+        // and of the 64 behind them; with kLanePages the entries of the slice's 32 keys and of the next slice's
         int pages = 0, pages_next = 0, page_group = 0;
         auto fetch_pages = [&](int group) { return bt_row[min(64 * group + lane, p.max_pages - 1)]; };
-        if (PAGED) {
+        auto fetch_slice = [&](int ti) { return bt_row[(key_of_tile(ti) + li) >> p.page_shift]; };
+        if (kLanePages) {
+            pages_next = fetch_slice(ti0);
+        } else if (PAGED) {
             page_group = (key_of_tile(ti0) >> p.page_shift) >> 6;
             pages = fetch_pages(page_group);
             pages_next = fetch_pages(page_group + 1);
@@ -1058,7 +1065,10 @@ void prefill_aggregate_kernel(PrefillParams p) {
         };
         auto enter_tile = [&](int ti) {   // before the loads of a tile, tiles in order
             key0 = key_of_tile(ti);
-            if (PAGED) {
+            if (kLanePages) {
+                pages = pages_next;
+                pages_next = fetch_slice(ti + 1);
+            } else if (PAGED) {
                 const int group = (key0 >> p.page_shift) >> 6;
                 if (group != page_group) {   // uniform
                     page_group = group;
@@ -1074,12 +1084,13 @@ void prefill_aggregate_kernel(PrefillParams p) {
             unsigned long long off = row_off;
             if (PAGED) {
                 const int key = key0 + j * kRPL;
-                off = offset_of_key(key);
-                if (D == 64 && p.page_shift == 2) {   // eight rows per load, four per page
-                    const unsigned long long off4 = offset_of_key(key + 4) - 8ull * row_stride;
-                    load_to_lds_16(lane_ptr[j % kPatterns] + (lrow < 4 ? off : off4), lds);
+                if (kLanePages) {
+                    const int page = __builtin_amdgcn_ds_bpermute((j * kRPL + lrow) << 2, pages);
+                    const unsigned row = (unsigned)((page << p.page_shift) + ((key + lrow) & page_mask));
+                    load_to_lds_16(lane_ptr[j % kPatterns] + (unsigned long long)row * row_stride * 2, lds);
                     return;
                 }
+                off = offset_of_key(key);
             } else {
                 row_off += row_step;
             }
