@@ -160,6 +160,49 @@ def test_pooled_scores_over_pages_of_every_size(cuda, page, heads, G, D, dtype):
         assert torch.equal(got, whole[:, :, start // 32:(end + 31) // 32, :end]), f"rows {start}..{end}"
 
 
+@pytest.mark.parametrize("page", [4, 8, 128, 256])
+@pytest.mark.parametrize("heads,G,D,dtype", [(32, 8, 128, torch.float16), (14, 2, 64, torch.bfloat16), (32, 8, 64, torch.float16)])
+def test_attention_over_pages_of_every_size(cuda, page, heads, G, D, dtype):
+    """Pages smaller than a tile (64 keys, 128 at head_dim 64), as large and larger: chunks that start in the middle of
+    a page and end inside a tile have the bits of the whole prompt over a strided cache, dense, log-sums alone and
+    sparse (with and without log-sums)."""
+    from kascade_amd import budgets, kernels
+    L, p = 1300, 10
+    gen = torch.Generator().manual_seed(page + D)
+    q = torch.randn(1, L, heads, D, generator=gen).to(dtype).to(cuda)
+    k, v = (torch.randn(1, L, G, D, generator=gen).to(dtype) for _ in range(2))
+    kp, table = _paged_copies(k, page, gen, 1, cuda)
+    vp = torch.empty_like(kp)
+    rows = torch.zeros(kp.shape[0] * page, G, D, dtype=dtype)
+    rows[:L] = v[0]
+    vp[table[0].long()] = rows.view(-1, page, G, D).to(cuda)
+    k, v = k.to(cuda), v.to(cuda)
+    log_sum, out = kernels.prefill_recompute0(q, k, v)
+    T, W = (L + 31) // 32, budgets.topk_width(L, p)
+    idx = torch.zeros(1, G, T, W, dtype=torch.int32)
+    for t in range(1, T):
+        n = min(32 * t, W)
+        for g in range(G):
+            idx[0, g, t, :n] = torch.randperm(32 * t, generator=gen)[:n].sort().values
+    idx = idx.to(cuda)
+    maps = torch.arange(G - 1, -1, -1, dtype=torch.int32, device=cuda)
+    sparse, sparse_sums = kernels.prefill_reuse(q, k, v, idx, maps, float(p), True, return_log_sum=True)
+    sparse_alone = kernels.prefill_reuse(q, k, v, idx, maps, float(p), True)
+    for start, end in ((0, 96), (96, 500), (480, 1300), (1280, 1300)):
+        qc = q[:, start:end]
+        sums, o = kernels.prefill_chunk_dense(qc, kp, vp, table, start, page)
+        assert torch.equal(sums, log_sum[:, start:end]) and torch.equal(o, out[:, start:end]), f"rows {start}..{end}"
+        alone, _ = kernels.prefill_chunk_dense(qc, kp, vp, table, start, page, with_output=False)
+        assert torch.equal(alone, sums), f"log-sums alone, rows {start}..{end}"
+        width = budgets.topk_width(end, p)
+        lists = kernels.translate_indices(idx[:, :, start // 32:(end + 31) // 32, :width].contiguous(), table, end, page)
+        o, sums = kernels.prefill_chunk_reuse(qc, kp, vp, lists, maps, float(p), end > 128, table, start, page,
+                                              return_log_sum=True)
+        assert torch.equal(o, sparse[:, start:end]) and torch.equal(sums, sparse_sums[:, start:end]), f"sparse rows {start}..{end}"
+        o = kernels.prefill_chunk_reuse(qc, kp, vp, lists, maps, float(p), end > 128, table, start, page)
+        assert torch.equal(o, sparse_alone[:, start:end]), f"sparse rows {start}..{end}, no log-sums"
+
+
 @pytest.mark.parametrize("heads,G,D,dtype", [(32, 8, 128, torch.float16), (32, 8, 128, torch.bfloat16), (14, 2, 64, torch.float16)])
 @pytest.mark.parametrize("batch", [1, 9])
 def test_log_sums_alone_follow_late_maxima(cuda, batch, heads, G, D, dtype):
