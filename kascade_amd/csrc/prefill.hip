@@ -219,8 +219,8 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     constexpr int kNumLoads = 8;
     auto issue_load = [&](auto i_c, int buf) {   // i < 4: K row group i; else V row group i - 4
         constexpr int i = decltype(i_c)::value;
-        if constexpr (i < 4) load_to_lds_16(row_ptr[i], lds_k + buf * (kTileElems * 2) + i * 1024);
-        else load_to_lds_16(row_ptr[i - 4] + v_from_k, lds_v + buf * (kTileElems * 2) + (i - 4) * 1024);
+        if constexpr (i < 4) load_to_lds_16<i * 1024>(row_ptr[i], lds_k + buf * (kTileElems * 2));
+        else load_to_lds_16<(i - 4) * 1024>(row_ptr[i - 4] + v_from_k, lds_v + buf * (kTileElems * 2));
     };
     // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 16 kb + col,
     // chunk 4 ks + dq.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):
@@ -643,8 +643,8 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     constexpr int kNumLoads = WITH_V ? 8 : 4;
     auto issue_load = [&](auto i_c, int buf) {   // i < 4: K row group i; else V row group i - 4
         constexpr int i = decltype(i_c)::value;
-        if constexpr (i < 4) load_to_lds_16(row_ptr[i], lds_k + buf * (kTileElems * 2) + i * 1024);
-        else load_to_lds_16(row_ptr[i - 4] + v_from_k, lds_v + buf * (kTileElems * 2) + (i - 4) * 1024);
+        if constexpr (i < 4) load_to_lds_16<i * 1024>(row_ptr[i], lds_k + buf * (kTileElems * 2));
+        else load_to_lds_16<(i - 4) * 1024>(row_ptr[i - 4] + v_from_k, lds_v + buf * (kTileElems * 2));
     };
     // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 32 kb + li,
     // chunk 2 ks + lg.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):

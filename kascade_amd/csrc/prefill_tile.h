@@ -37,15 +37,16 @@ template <> __device__ __forceinline__ int swz<128>(int row) { return ((row & 3)
 template <> __device__ __forceinline__ int swz<64>(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 
 // One wavefront-wide load of 16 bytes per lane from global memory into LDS: lane i's bytes
-// land at lds_base + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
+// land at lds_base + OFF + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
 // compiler does not know that it writes LDS, so whoever reads the bytes waits for vmcnt and
 // passes a barrier first (the tile loop does both once per tile).
 // No vector ALU instruction belongs in here: the compiler puts no wait states between the matrix instructions and a
 // register that inline assembly writes, nor between the restore of a spilled scalar register and its use in there.
-// Addresses are formed by the callers, in C++.
-__device__ __forceinline__ void load_to_lds_16(const void* gptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :: "v"(gptr), "s"(lds_base) : "m0");
+// Addresses are formed by the callers, in C++.  OFF is added to lds_base on the way into m0, which takes no scalar register
+// per call (sparse units spill theirs: 16384 tokens 266 -> 262 us, 4096 30.8 -> 30.4).
+template <int OFF = 0> __device__ __forceinline__ void load_to_lds_16(const void* gptr, uint32_t lds_base) {
+    asm volatile("s_add_u32 m0, %1, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :: "v"(gptr), "s"(lds_base), "i"(OFF) : "m0", "scc");
 }
 template <typename P> __device__ __forceinline__ uint32_t lds_address(P* ptr) {
     return (uint32_t)(size_t)(__attribute__((address_space(3))) void*)ptr;
