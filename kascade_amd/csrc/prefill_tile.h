@@ -1,6 +1,7 @@
 // Pieces of the prefill attention kernels (prefill.hip): tile geometry, the
-// LDS chunk permutation, direct-to-LDS loads, the workgroup -> unit mapping and the budgets.
+// LDS chunk permutation, direct-to-LDS loads and the workgroup -> unit mapping.
 #pragma once
+#include "budgets.h"
 #include "prefill.h"
 
 namespace kascade {
@@ -80,26 +81,6 @@ __device__ __forceinline__ void unit_of_workgroup(int B, int G, int nblocks, int
         g = blockIdx.y;
         b = blockIdx.z;
     }
-}
-
-__device__ __forceinline__ int rolling_budget(float pct, int tile_start) {
-    // floor(pct tile_start / 100) without a division, which every unit's first list entry would wait for (517 tokens
-    // 9.80 -> 9.68 us).  x is exact, and where it is no multiple of 100 it lies a relative 2^-44 or more off
-    // the next one: the quotient's rounding does not reach it, so this is the floor of the rounded quotient too.
-    const double x = (double)pct * (double)tile_start;
-    int fl = (int)(x * 0.01);
-    fl += (double)(fl + 1) * 100.0 <= x;
-    fl -= (double)fl * 100.0 > x;
-    return max(128, (fl + 127) & ~127);
-}
-
-// Index-row width the host gives a prompt of L keys: min(128 ceil(min(max(128, floor(pct L / 100)), L) / 128), L).
-__device__ __forceinline__ int topk_width_of(float pct, int L) {
-    long long k = (long long)floor((double)pct * (double)L / 100.0);
-    if (k < 128) k = 128;
-    if (k > L) k = L;
-    k = ((k + 127) / 128) * 128;
-    return (int)(k > L ? L : k);
 }
 
 // Where sequence b's rows of a chunked call stand: first global position and number of rows.
