@@ -84,8 +84,9 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     typedef typename Elem<T>::x4 x4_t;
     typedef typename Elem<T>::x2 x2_t;
     typedef AttnTile<D> G_;
-    constexpr int kKT = G_::kKT, kKS = G_::kKS, kDB = G_::kDB, kKB = G_::kKB, kChunks = G_::kChunks;
-    constexpr int kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
+    constexpr int kKT = G_::kKT, kChunks = G_::kChunks, kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
+    // products 16x16x32: contraction steps of S^T, 16-row blocks of O^T, 16-key blocks of a tile
+    constexpr int kKS = D / 32, kDB = D / 16, kKB = kKT / 16;
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
     const int kvh = p.G, nheads = p.G * hs.gs;
@@ -126,18 +127,15 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
 
     // ---- key regime of this block ----
     bool sparse = false;
-    int n = 0, ng = 0;
+    int ng = 0;
     const int* idx_row = nullptr;
-    {
-        // a sequence of a mixed batch keeps the budget it has on its own (the rows are as wide as
-        // the longest sequence needs)
-        const int width = p.q_start_rows ? min(p.max_topk, topk_width_of(p.topk_percent, L)) : p.max_topk;
-        n = (p.rolling && L > 128) ? rolling_budget(p.topk_percent, q0) : width;
-        n = min(n, width);
-        if (q0 > n) {
-            sparse = true;
-            ng = (n + kKT - 1) / kKT;
-        }
+    // a sequence of a mixed batch keeps the budget it has on its own (the rows are as wide as
+    // the longest sequence needs)
+    const int width = p.q_start_rows ? min(p.max_topk, topk_width_of(p.topk_percent, L)) : p.max_topk;
+    const int n = min((p.rolling && L > 128) ? rolling_budget(p.topk_percent, q0) : width, width);
+    if (q0 > n) {
+        sparse = true;
+        ng = (n + kKT - 1) / kKT;
     }
     const int ntiles = sparse ? ng + 1 : (min(q0 + QT, L) + kKT - 1) / kKT;
     const bool idx_vec = (p.max_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(p.idx) & 15) == 0;
@@ -383,24 +381,17 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 for (int v = 0; v < 4; ++v) mx = fmaxf(mx, sT[q][kb][v]);
             return mx * kScaleLog2;
         };
-        // 32 queries' references, from their scores' maxima
-        auto move_references = [&](int q0, const float (&ms)[2]) {
+        const float ms[NQ] = {maximum(0), maximum(1)};
+        if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) {   // wavefront-uniform
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int q = q0 + i;
-                const float mnew = fmaxf(m[q], max_over_quarters(ms[i]));   // the same in the four lanes of a column
+            for (int q = 0; q < NQ; ++q) {
+                const float mnew = fmaxf(m[q], max_over_quarters(ms[q]));   // the same in the four lanes of a column
                 const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
                 m[q] = mnew;
                 l[q] *= corr;
-                {
 #pragma unroll
-                    for (int db = 0; db < kDB; ++db) oT[q][db] *= corr;
-                }
+                for (int db = 0; db < kDB; ++db) oT[q][db] *= corr;
             }
-        };
-        {
-            const float ms[2] = {maximum(0), maximum(1)};
-            if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) move_references(0, ms);   // wavefront-uniform
         }
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -411,14 +402,12 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
             for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) e[kb][v] = fast_exp2(__builtin_fmaf(sT[q][kb][v], kScaleLog2, -mu));
-            {
 #pragma unroll
-                for (int s = 0; s < nkb / 2; ++s) {
-                    x8_t t;
+            for (int s = 0; s < nkb / 2; ++s) {
+                x8_t t;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) t[i] = (T)e[2 * s + (i >> 2)][i & 3];
-                    pf[q][s] = t;
-                }
+                for (int i = 0; i < 8; ++i) t[i] = (T)e[2 * s + (i >> 2)][i & 3];
+                pf[q][s] = t;
             }
             if (kPairSum) {
 #pragma unroll
@@ -440,64 +429,60 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         // ---- O^T += V^T P^T: step s covers the keys of blocks 2 s and 2 s + 1, whose scores lane dq holds: rows
         // 32 s + 16 h + 4 dq + (0..3), h = 0, 1, of the tile.  The operands of a group of steps are read
         // while the group before it is multiplied ----
-        {
-            constexpr int kPS = nkb / 2;
-            auto read_v = [&](int db, int s, int h) {
-                const T* vp = bV + (32 * s + 16 * h) * D + vrd + ((2 * db) ^ vchunk) * 8;
-                return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
-            };
-            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block),
-            // two column blocks in turn
-            constexpr int kGrp = (D == 128) ? 4 : 2;
-            constexpr int kGroupsPV = kDB * kPS / kGrp;
-            auto out_block = [](int t) { return 2 * (t / (2 * kPS)) + (t & 1); };
-            auto p_step = [](int t) { return (t % (2 * kPS)) >> 1; };
-            short4_t av[2][kGrp][2];
+        constexpr int kPS = nkb / 2;
+        auto read_v = [&](int db, int s, int h) {
+            const T* vp = bV + (32 * s + 16 * h) * D + vrd + ((2 * db) ^ vchunk) * 8;
+            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
+        };
+        // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block),
+        // two column blocks in turn
+        constexpr int kGrp = (D == 128) ? 4 : 2;
+        constexpr int kGroupsPV = kDB * kPS / kGrp;
+        auto out_block = [](int t) { return 2 * (t / (2 * kPS)) + (t & 1); };
+        auto p_step = [](int t) { return (t % (2 * kPS)) >> 1; };
+        short4_t av[2][kGrp][2];
 #pragma unroll
-            for (int i = 0; i < kGrp; ++i)
+        for (int i = 0; i < kGrp; ++i)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(out_block(i), p_step(i), h);
+            for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(out_block(i), p_step(i), h);
 #pragma unroll
-            for (int gq = 0; gq < kGroupsPV; ++gq) {
-                if (gq + 1 < kGroupsPV) {
+        for (int gq = 0; gq < kGroupsPV; ++gq) {
+            if (gq + 1 < kGroupsPV) {
 #pragma unroll
-                    for (int i = 0; i < kGrp; ++i)
+                for (int i = 0; i < kGrp; ++i)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            av[(gq + 1) & 1][i][h] = read_v(out_block(kGrp * (gq + 1) + i), p_step(kGrp * (gq + 1) + i), h);
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int h = 0; h < 2; ++h)
+                        av[(gq + 1) & 1][i][h] = read_v(out_block(kGrp * (gq + 1) + i), p_step(kGrp * (gq + 1) + i), h);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < kGrp; ++i) {
-                    const int db = out_block(kGrp * gq + i), s = p_step(kGrp * gq + i);
-                    const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    const x8_t a = __builtin_bit_cast(x8_t, both);
+            for (int i = 0; i < kGrp; ++i) {
+                const int db = out_block(kGrp * gq + i), s = p_step(kGrp * gq + i);
+                const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                const x8_t a = __builtin_bit_cast(x8_t, both);
 #pragma unroll
-                    for (int q = 0; q < NQ; ++q)
-                        oT[q][db] = Elem<T>::mma_16x16x32(a, pf[q][s], oT[q][db]);
-                }
+                for (int q = 0; q < NQ; ++q)
+                    oT[q][db] = Elem<T>::mma_16x16x32(a, pf[q][s], oT[q][db]);
             }
         }
     };
 
-    {
-        int sq = 0;
-        if (sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
-            if (kKT == 64) run_tile(0, std::integral_constant<int, kDiag>{});
-            else run_tile(0, std::integral_constant<int, kMasked>{});
-            sq = 1;
-        }
-        // tiles wholly below the unit's first query and inside the sequence / wholly inside the selection
-        const int full_end = sparse ? 1 + n / kKT : min((q0 + 1) / kKT, L / kKT);
-        for (; sq < full_end; ++sq) run_tile(sq, std::integral_constant<int, kFull>{});
-        for (; sq < ntiles; ++sq) run_tile(sq, std::integral_constant<int, kMasked>{});
+    int sq = 0;
+    if (sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
+        if (kKT == 64) run_tile(0, std::integral_constant<int, kDiag>{});
+        else run_tile(0, std::integral_constant<int, kMasked>{});
+        sq = 1;
     }
+    // tiles wholly below the unit's first query and inside the sequence / wholly inside the selection
+    const int full_end = sparse ? 1 + n / kKT : min((q0 + 1) / kKT, L / kKT);
+    for (; sq < full_end; ++sq) run_tile(sq, std::integral_constant<int, kFull>{});
+    for (; sq < ntiles; ++sq) run_tile(sq, std::integral_constant<int, kMasked>{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
 
     // ---- epilogue (rows are local to this call).  A lane holds one query's output spread over its
     // registers; the rows go through the wavefront's share of the (now idle) K buffers so that they
     // leave as whole rows: 16-byte stores, four rows per instruction ----
-        __syncthreads();   // everybody is done with the tile buffers
+    __syncthreads();   // everybody is done with the tile buffers
     T* so = sK + wave * (32 * D);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -505,30 +490,25 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         const float lt = sum_over_quarters(l[q]);
         if (p.log_sum && dq == 0 && ql < Lqv && real_head)
             p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[q];
-        {
-            const float inv = 1.f / lt;
-            const int row = 16 * q + col;
+        const float inv = 1.f / lt;
+        const int row = 16 * q + col;
 #pragma unroll
-            for (int db = 0; db < kDB; ++db) {   // d = 16 db + 4 dq .. +3: half of chunk 2 db + dq / 2
-                const x4_t o = {(T)(oT[q][db][0] * inv), (T)(oT[q][db][1] * inv), (T)(oT[q][db][2] * inv), (T)(oT[q][db][3] * inv)};
-                *reinterpret_cast<x4_t*>(&so[row * D + (((2 * db + (dq >> 1)) ^ (row & (kChunks - 1))) * 8) + 4 * (dq & 1)]) = o;
-            }
+        for (int db = 0; db < kDB; ++db) {   // d = 16 db + 4 dq .. +3: half of chunk 2 db + dq / 2
+            const x4_t o = {(T)(oT[q][db][0] * inv), (T)(oT[q][db][1] * inv), (T)(oT[q][db][2] * inv), (T)(oT[q][db][3] * inv)};
+            *reinterpret_cast<x4_t*>(&so[row * D + (((2 * db + (dq >> 1)) ^ (row & (kChunks - 1))) * 8) + 4 * (dq & 1)]) = o;
         }
     }
-    {
-        __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
+    __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
 #pragma unroll
-        for (int j = 0; j < 32 / kRPL; ++j) {
-            const int r = j * kRPL + lrow;
-            const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
-            const int qr = q0l + r;
-            if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
-                __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
-                    (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
-        }
+    for (int j = 0; j < 32 / kRPL; ++j) {
+        const int r = j * kRPL + lrow;
+        const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
+        const int qr = q0l + r;
+        if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
+            __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
+                (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
     }
 }
-
 
 // Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
 // tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and
@@ -539,8 +519,9 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
     typedef AttnTile<D> G_;
-    constexpr int kKT = G_::kKT, kKS = D / 16, kDB = D / 32, kKB = kKT / 32, kChunks = G_::kChunks;
-    constexpr int kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
+    constexpr int kKT = G_::kKT, kChunks = G_::kChunks, kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
+    // products 32x32x16: contraction steps of S^T, 32-row blocks of O^T, 32-key blocks of a tile
+    constexpr int kKS = D / 16, kDB = D / 32, kKB = kKT / 32;
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
     const int kvh = p.G, nheads = p.G * hs.gs;
@@ -925,7 +906,6 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
         }
     }
 }
-
 
 // 32 queries per wavefront: register budget capped so that two workgroups share a
 // compute unit (64 KB of LDS each: two K and two V tile buffers), four without V (log-sums alone over the paged

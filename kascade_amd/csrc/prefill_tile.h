@@ -7,15 +7,12 @@
 namespace kascade {
 namespace {
 
-// Tile geometry of the attention kernel per head dimension.  A tile is 16 KB of K (and of V)
-// whatever D: 64 keys at D = 128, 128 keys at D = 64, so a wavefront always stages a tile with
-// four 1 KB loads per tensor, both products issue 16 matrix instructions per tile and wavefront,
+// Tile geometry of the attention kernels per head dimension, whatever products they use.  A tile is 16 KB of K (and of
+// V) whatever D: 64 keys at D = 128, 128 keys at D = 64, so a wavefront always stages a tile with four 1 KB loads per
+// tensor, each product takes as many matrix instructions per tile and 32 queries (16 of 32x32x16, 32 of 16x16x32),
 // and the score registers a narrower head frees hold the extra keys.
 template <int D> struct AttnTile {
     static constexpr int kKT = 64 * 128 / D;     // keys per tile
-    static constexpr int kKS = D / 32;           // contraction steps of S^T = K Q^T, 16x16x32 products
-    static constexpr int kDB = D / 16;           // 16-row blocks of O^T
-    static constexpr int kKB = kKT / 16;         // 16-key blocks of a tile
     static constexpr int kChunks = D / 8;        // 16-byte chunks of a row
     static constexpr int kRowsPerLoad = 64 / kChunks;   // rows one wavefront-wide 16-byte load covers
     static constexpr int kTileElems = kKT * D;   // 16 KB of K (and of V) whatever D
