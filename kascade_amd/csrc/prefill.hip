@@ -22,8 +22,9 @@
 //   ds_read_b64_tr_b16 (two per operand: four keys each).
 //
 //   What bounds long calls is the chip's power, and per product 16x16x32 takes less of it than 32x32x16 (1.84
-//   against 1.59 PFLOP/s on random operands in registers): sparse units use it (32/8 heads, 4096 tokens 36.4 -> 35.3
-//   us, 32768 982 -> 935).  Dense passes and pooling keep 32x32x16 (see there).  Against row addresses formed by a
+//   against 1.59 PFLOP/s on random operands in registers): sparse units use it (32/8 heads: 3001 tokens 23.8 -> 23.1 us,
+//   4096 31.6 -> 30.4, 16384 277 -> 262, 32768 982 -> 933; no gain at 2048 tokens, 12.8 both and in bf16 12.6 -> 12.8, nor
+//   below).  Dense passes and pooling keep 32x32x16 (see there).  Against row addresses formed by a
 //   64-bit product per tensor and row and block-table entries requested behind the tile's loads: dense 517 tokens
 //   14.6 -> 13.5 us, 2048 49.4 -> 46.9, chunks at position 14336 of 512 queries 326 -> 247 us, of 2048 532 -> 520;
 //   log-sums alone 517 10.2 -> 9.6 us, 32768 4.39 -> 4.24 ms, chunks of 512 205 -> 173 us, of 2048 310 -> 301.
@@ -513,7 +514,9 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
 // Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
 // tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and
 // the last bits of the log-sums decide between tokens whose pooled scores lie within one step at a selection's
-// threshold: single output rows of a 32768-token prompt moved by up to 0.27 of the outputs' root mean square.
+// threshold: single output rows of a 32768-token prompt moved by up to 0.27 of the outputs' root mean square.  The order
+// of the additions is all that differs: four chained 16x16x32 products and eight 32x32x16 ones gave the same bits in
+// all of 524288 dot products of 128 elements.
 template <int NQB, bool WITH_V, bool PAGED, int D, typename T>
 __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
@@ -936,7 +939,7 @@ void prefill_attn_kernel_q64(PrefillParams p) {
 // under the other's matrix instructions.  With 16x16x32 products, row addresses from scalar registers and the last
 // head's exponentials across the tile boundary 32768 tokens took 4.1 ms instead of 4.6, but a key's sum was then spread
 // over four lanes instead of two, and its last bits decide between tokens whose pooled scores lie within one
-// step at a selection's threshold.
+// step at a selection's threshold (the products' own bits are the same, see the dense passes).
 //
 // A wavefront takes 32 keys of every 128-key tile and nobody else reads them.  Their rows go
 // from global memory straight into the wavefront's own LDS area (whole rows per load: read as
