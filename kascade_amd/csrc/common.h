@@ -124,6 +124,33 @@ __device__ __forceinline__ float sum_over_quarters(float x) {
     return sum_with_other_half(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
+// x over the 64 lanes, in every lane: pairs 32, 16, 8, 4, 2 and 1 lanes apart in turn, by swaps of lane halves and rows
+// and DPP moves (through LDS, as __shfl_xor goes, a step is a trip of about 130 cycles).  The rotations by 8 and 4 within
+// a row of 16 are exchanges across that distance: by then a row has period 16 and 8.
+__device__ __forceinline__ float wave_max(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, max_with_other_half(x));
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false)));  // row_ror:8
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, false)));  // row_ror:4
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false)));   // quad_perm [2,3,0,1]
+    return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false)));  // quad_perm [1,0,3,2]
+}
+__device__ __forceinline__ float wave_sum(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, sum_with_other_half(x));
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false));   // row_ror:8
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, false));   // row_ror:4
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false));    // quad_perm [2,3,0,1]
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));    // quad_perm [1,0,3,2]
+    return x;
+}
+// x of lane `l`, the same in the whole wavefront (l uniform)
+__device__ __forceinline__ float lane_value(float x, int l) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
+}
+
 __device__ __forceinline__ uint4_t ld_global_16(const void* p) {
     return *reinterpret_cast<const uint4_t*>(p);
 }

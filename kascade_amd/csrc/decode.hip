@@ -331,10 +331,7 @@ void decode_split_kernel(DecodeParams p) {
         for (int e = 0; e < 4; ++e)
             if (key0 + e >= cn) sc[e] = -INFINITY;
         float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-        if (WITH_V) {
-            mx = fmaxf(mx, __shfl_xor(mx, 16));
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-        }
+        if (WITH_V) mx = max_over_quarters(mx);
         mx = fmaxf(mx, mcol);
         const float mref = (mx == -INFINITY) ? 0.f : mx * kScaleLog2;
         const float corr = fast_exp2(mcol * kScaleLog2 - mref);   // mcol = -inf -> 0
@@ -373,8 +370,7 @@ void decode_split_kernel(DecodeParams p) {
         float mx = -INFINITY;
 #pragma unroll
         for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fmaxf(fmaxf(sc[j][0], sc[j][1]), fmaxf(sc[j][2], sc[j][3])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = max_over_quarters(mx);
         const float base = (mx == -INFINITY) ? 0.f : mx;
         if (col < gs) {
 #pragma unroll
@@ -603,15 +599,18 @@ void decode_split_kernel(DecodeParams p) {
 
     // ---- the wavefront's state: columns 0-3, the four parts of a column in lanes col + 16*dq ----
     if (WITH_V) {   // one reference per column: the partial sums just add
-        lcol += __shfl_xor(lcol, 16);
-        lcol += __shfl_xor(lcol, 32);
-    } else {
+        lcol = sum_over_quarters(lcol);
+    } else {   // lane dq = 0 is the one that counts: rows 0 and 1, then the halves
 #pragma unroll
         for (int sh = 16; sh <= 32; sh <<= 1) {
-            const float mo = __shfl_xor(mcol, sh), lo = __shfl_xor(lcol, sh);
-            const float mx = fmaxf(mcol, mo);
+            const uint32_t mu = __builtin_bit_cast(uint32_t, mcol), lu = __builtin_bit_cast(uint32_t, lcol);
+            const auto m2 = sh == 16 ? __builtin_amdgcn_permlane16_swap(mu, mu, false, false) : __builtin_amdgcn_permlane32_swap(mu, mu, false, false);
+            const auto l2 = sh == 16 ? __builtin_amdgcn_permlane16_swap(lu, lu, false, false) : __builtin_amdgcn_permlane32_swap(lu, lu, false, false);
+            const float m0 = __builtin_bit_cast(float, (uint32_t)m2[0]), mo = __builtin_bit_cast(float, (uint32_t)m2[1]);
+            const float l0 = __builtin_bit_cast(float, (uint32_t)l2[0]), lo = __builtin_bit_cast(float, (uint32_t)l2[1]);
+            const float mx = fmaxf(m0, mo);
             const float mref = (mx == -INFINITY) ? 0.f : mx * kScaleLog2;
-            lcol = lcol * fast_exp2(mcol * kScaleLog2 - mref) + lo * fast_exp2(mo * kScaleLog2 - mref);
+            lcol = l0 * fast_exp2(m0 * kScaleLog2 - mref) + lo * fast_exp2(mo * kScaleLog2 - mref);
             mcol = mx;
         }
     }
@@ -714,13 +713,11 @@ void decode_split_kernel(DecodeParams p) {
         const float g0 = (lane < ns) ? load_device(gl + lane) : -INFINITY;   // splits [0, 64)
         float mx = g0;
         for (int s = lane + 64; s < ns; s += 64) mx = fmaxf(mx, load_device(gl + s));
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        mx = wave_max(mx);
         const float mref = (mx == -INFINITY) ? 0.f : mx;
         float sum = fast_exp2(g0 - mref);
         for (int s = lane + 64; s < ns; s += 64) sum += fast_exp2(load_device(gl + s) - mref);
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+        sum = wave_sum(sum);
         const float lse = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
         if (p.row_sums && lane == 0) p.row_sums[(size_t)b * nheads + head] = lse;
         if (WITH_V) {
@@ -737,7 +734,7 @@ void decode_split_kernel(DecodeParams p) {
                 }
 #pragma unroll
                 for (int j = 0; j < kEarly; ++j) {
-                    const float w = __shfl(wl, (s0 & 63) + j);   // 0 for splits that do not exist
+                    const float w = lane_value(wl, (s0 & 63) + j);   // 0 for splits that do not exist
                     o0 += w * xe[j].x;
                     o1 += w * xe[j].y;
                 }
@@ -754,11 +751,7 @@ void decode_split_kernel(DecodeParams p) {
 constexpr int kCombineLds = 512;   // splits whose weights fit the LDS buffer
 
 __device__ __forceinline__ float combine_reduce(float x, bool is_max, float* s_red) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float y = __shfl_xor(x, o);
-        x = is_max ? fmaxf(x, y) : x + y;
-    }
+    x = is_max ? wave_max(x) : wave_sum(x);
     __syncthreads();   // s_red may still be read from the previous reduction
     if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = x;
     __syncthreads();
@@ -844,13 +837,11 @@ __global__ __launch_bounds__(256) void decode_aggregate_kernel(const float* __re
             const float* gl = glse + ((size_t)b * nheads + g * gs + h) * num_split;
             float mx = -INFINITY;
             for (int sidx = lane; sidx < num_split; sidx += 64) mx = fmaxf(mx, gl[sidx]);
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            mx = wave_max(mx);
             const float mref = (mx == -INFINITY) ? 0.f : mx;
             float sum = 0.f;
             for (int sidx = lane; sidx < num_split; sidx += 64) sum += fast_exp2(gl[sidx] - mref);
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+            sum = wave_sum(sum);
             const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
             if (lane == 0) {
                 s_lse[h] = v;

@@ -642,13 +642,11 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
             const float g0 = lane < p.num_split ? gl[lane] : -INFINITY;
             float mx = g0;
             for (int s = lane + 64; s < p.num_split; s += 64) mx = fmaxf(mx, gl[s]);
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            mx = wave_max(mx);
             const float mref = (mx == -INFINITY) ? 0.f : mx;
             float sum = fast_exp2(g0 - mref);
             for (int s = lane + 64; s < p.num_split; s += 64) sum += fast_exp2(gl[s] - mref);
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+            sum = wave_sum(sum);
             const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
             if (lane == 0) {
                 s_lse[h] = v;
