@@ -12,8 +12,7 @@ struct PrefillParams {
     // KV head: the KV head's gs query heads are taken four at a time, ceil(gs/4) "sub-groups" --
     // the attention kernels launch one workgroup per (KV head, sub-group), the pooling kernel is
     // launched once per sub-group (vsub) and adds to the pooled scores of the earlier ones.  A
-    // slot beyond the KV head's last query head computes along on that head's data and leaves
-    // nothing behind: no output, no log-sum, nothing in the pooled sums.
+    // slot beyond the KV head's last query head fills its share of the tiles and computes nothing.
     const void* Q;            // [B,Lq,H,D] through (q_sb, q_sl, q_sh)
     const void* K;            // [B,L,G,D] through (k_sb, k_sl, k_sh); V shares the strides.
     const void* V;            //   Paged: [num_pages, page, G, D] contiguous, strides unused

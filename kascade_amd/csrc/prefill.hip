@@ -77,9 +77,14 @@ template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
 // addressed through the block table, and gathered index rows hold physical row numbers.
 //
 // Sparse passes (and the dense tiles of their first units): products 16x16x32.
+// SPARE: the KV head's last sub-group may have fewer than four query heads (gs no multiple of four).  Its wavefronts
+// without a head only stage their rows of every tile, which leaves the matrix unit and the power to the others: 28/4
+// heads bf16, two prompts of 3001 tokens, eight layers with pooling over the heads there are 780 -> 737 us.  A variant of its own, because
+// the second loop costs the allocation of the first (32/8 heads, 517 tokens 119.2 -> 120.4 us).  Rotating the slots over
+// the wavefronts, so that the idle one is not always the same SIMD's, gave nothing.
 // EXACT_SUM: the softmax denominators are summed in fp32 from the unrounded exponentials (the
 // passes whose log-sum is an output); otherwise units sum them as they enter the second product.
-template <bool PAGED, int D, typename T, bool EXACT_SUM>
+template <bool PAGED, int D, typename T, bool SPARE, bool EXACT_SUM>
 __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
@@ -124,7 +129,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
     const int head = g * hs.gs + min(4 * sub + wave, hs.gs - 1);
-    const bool real_head = 4 * sub + wave < hs.gs;   // a slot beyond the last head computes along and stores nothing
+    const bool has_head = !SPARE || 4 * sub + __builtin_amdgcn_readfirstlane(wave) < hs.gs;
 
     // ---- key regime of this block ----
     bool sparse = false;
@@ -468,6 +473,20 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         }
     };
 
+    if (SPARE && !has_head) {   // wavefront-uniform: this slot only fills its quarter of every tile
+#pragma clang loop unroll(disable)
+        for (int s = 0; s < ntiles; ++s) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (s + 1 < ntiles) {
+                next_rows();
+                if (s + 2 < ntiles) fetch_ids(tile_at(s + 2));
+                static_for<0, kNumLoads>([&](auto i) { issue_load(i, (s + 1) & 1); });
+            }
+        }
+        __syncthreads();   // the one behind the last tile
+        return;
+    }
     int sq = 0;
     if (sparse) {   // a copy of its own where it halves the tile's products (64-key tiles)
         if (kKT == 64) run_tile(0, std::integral_constant<int, kDiag>{});
@@ -489,7 +508,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     for (int q = 0; q < NQ; ++q) {
         const int ql = q0l + 16 * q + col;
         const float lt = sum_over_quarters(l[q]);
-        if (p.log_sum && dq == 0 && ql < Lqv && real_head)
+        if (p.log_sum && dq == 0 && ql < Lqv)
             p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[q];
         const float inv = 1.f / lt;
         const int row = 16 * q + col;
@@ -505,7 +524,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         const int r = j * kRPL + lrow;
         const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
         const int qr = q0l + r;
-        if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
+        if (qr < Lqv)   // the output is not read again by these kernels: keep it out of the caches
             __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
                 (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
     }
@@ -517,7 +536,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
 // threshold: single output rows of a 32768-token prompt moved by up to 0.27 of the outputs' root mean square.  The order
 // of the additions is all that differs: four chained 16x16x32 products and eight 32x32x16 ones gave the same bits in
 // all of 524288 dot products of 128 elements.
-template <int NQB, bool WITH_V, bool PAGED, int D, typename T>
+template <int NQB, bool WITH_V, bool PAGED, int D, typename T, bool SPARE>
 __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
@@ -562,7 +581,7 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
     const int head = g * hs.gs + min(4 * sub + wave, hs.gs - 1);
-    const bool real_head = 4 * sub + wave < hs.gs;   // a slot beyond the last head computes along and stores nothing
+    const bool has_head = !SPARE || 4 * sub + __builtin_amdgcn_readfirstlane(wave) < hs.gs;
 
     const int ntiles = (min(q0 + QT, L) + kKT - 1) / kKT;
 
@@ -867,6 +886,20 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
         }
     };
 
+    if (SPARE && !has_head) {   // wavefront-uniform: this slot only fills its quarter of every tile
+#pragma clang loop unroll(disable)
+        for (int s = 0; s < ntiles; ++s) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (s + 1 < ntiles) {
+                next_rows(s + 1);
+                if (s + 2 < ntiles) fetch_page(s + 2);
+                static_for<0, kNumLoads>([&](auto i) { issue_load(i, (s + 1) & 1); });
+            }
+        }
+        if (WITH_V) __syncthreads();   // the one behind the last tile
+        return;
+    }
     // tiles wholly below the unit's first query and inside the sequence need no mask
     const int full_end = min((q0 + 1) / kKT, L / kKT);
     int sq = 0;
@@ -883,7 +916,7 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     for (int qb = 0; qb < NQB; ++qb) {
         const int ql = q0l + 32 * qb + li;
         const float lt = sum_with_other_half(l[qb]);
-        if (p.log_sum && lg == 0 && ql < Lqv && real_head)
+        if (p.log_sum && lg == 0 && ql < Lqv)
             p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[qb];
         if (WITH_V) {
             T* so = sK + wave * (32 * D);
@@ -902,7 +935,7 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
                 const int r = j * kRPL + lrow;
                 const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
                 const int qr = q0l + r;
-                if (qr < Lqv && real_head)   // the output is not read again by these kernels: keep it out of the caches
+                if (qr < Lqv)   // the output is not read again by these kernels: keep it out of the caches
                     __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
                         (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
             }
@@ -913,28 +946,30 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
 // 32 queries per wavefront: register budget capped so that two workgroups share a
 // compute unit (64 KB of LDS each: two K and two V tile buffers), four without V (log-sums alone over the paged
 // cache at head_dim 64, in 134 registers and three: four chunks of 1024 queries at 4096, 32/8 heads, 122.5 -> 116.5 us).
-template <bool REUSE, bool WITH_V, bool PAGED, int D, typename T, bool EXACT_SUM = false>
+template <bool REUSE, bool WITH_V, bool PAGED, int D, typename T, bool SPARE, bool EXACT_SUM = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(REUSE || WITH_V ? 2 : 4)))
 void prefill_attn_kernel_q32(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
     __shared__ __attribute__((aligned(1024))) T sV[WITH_V ? 2 * AttnTile<D>::kTileElems : 8];
-    if constexpr (REUSE) prefill_reuse_body<PAGED, D, T, EXACT_SUM>(p, sK, sV);
-    else prefill_dense_body<1, WITH_V, PAGED, D, T>(p, sK, sV);
+    if constexpr (REUSE) prefill_reuse_body<PAGED, D, T, SPARE, EXACT_SUM>(p, sK, sV);
+    else prefill_dense_body<1, WITH_V, PAGED, D, T, SPARE>(p, sK, sV);
 }
 
 // 64 queries per wavefront for the K-only log-sum pass, whose state fits 256 registers: two
 // workgroups per compute unit, and the MFMA results stay in ordinary registers (with the full
 // 512-register budget the compiler parks them in accumulation registers and copies each one out
 // before the softmax).
-template <bool PAGED, int D, typename T>
+template <bool PAGED, int D, typename T, bool SPARE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_attn_kernel_q64(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
-    prefill_dense_body<2, false, PAGED, D, T>(p, sK, static_cast<T*>(nullptr));
+    prefill_dense_body<2, false, PAGED, D, T, SPARE>(p, sK, static_cast<T*>(nullptr));
 }
 
 // Pooled tile scores: out[b,g,t,key] = sum over the 32 queries of tile t and the 4 q-heads of g
 // of exp2(s*scale - log_sum), for keys before the tile's first (global) position.
+// NH: query heads of the launch's sub-group (three of the second one at seven per KV head: its launches 54.3 -> 48.1 us
+// at two prompts of 3001 tokens).
 // Two workgroups per compute unit (register budget 256): one wavefront's exponentials run
 // under the other's matrix instructions.  With 16x16x32 products, row addresses from scalar registers and the last
 // head's exponentials across the tile boundary 32768 tokens took 4.1 ms instead of 4.6, but a key's sum was then spread
@@ -948,7 +983,7 @@ void prefill_attn_kernel_q64(PrefillParams p) {
 // operands (lane = key, 8 elements at d = 16 ks + 8 lg) from the chunk-permuted rows.  Two buffers
 // per wavefront, no barrier in the tile loop: the loads of the next tile are issued one per
 // contraction step and waited for at the top of that tile.
-template <bool PAGED, int D, typename T>
+template <bool PAGED, int D, typename T, int NH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_aggregate_kernel(PrefillParams p) {
     typedef typename Elem<T>::x8 x8_t;
@@ -1097,10 +1132,10 @@ void prefill_aggregate_kernel(PrefillParams p) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // own rows have landed
         __syncthreads();                                   // everybody's, and s_lse
         // A operands: row block rb = head slot rb, row li = query tl + li
-        x8_t qa[kGroupSize][kKS];
+        x8_t qa[NH][kKS];
         const T* sQ = sK + ((ti0 + 1) & 1) * (4 * kWaveElems);
 #pragma unroll
-        for (int rb = 0; rb < kGroupSize; ++rb)
+        for (int rb = 0; rb < NH; ++rb)
 #pragma unroll
             for (int ks = 0; ks < kKS; ++ks) {
                 PackT<T> x;
@@ -1139,7 +1174,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
                     if (v >= v0 && v < v1) sum += fast_exp2(s[v] * kScaleLog2 - ls[v >> 2][v & 3]);
             };
 #pragma unroll
-            for (int rb = 0; rb < kGroupSize; ++rb) {
+            for (int rb = 0; rb < NH; ++rb) {
 #pragma unroll
                 for (int ks = 0; ks < kKS; ++ks) {
                     acc[rb & 1] = Elem<T>::mma_32x32x16(qa[rb][ks], kb[ks], ks == 0 ? zero16 : acc[rb & 1]);
@@ -1156,7 +1191,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
 #pragma unroll
             for (int j = kKS; j < kLoads; ++j) issue_load(j, nbuf);
             tile_phase<KASCADE_PRIO_AGG>(1);
-            exponentials(acc[(kGroupSize - 1) & 1], 0, 16);
+            exponentials(acc[(NH - 1) & 1], 0, 16);
             sum = sum_with_other_half(sum);
             tile_phase<KASCADE_PRIO_AGG>(2);
             const int key = ti * kAggKT + 32 * wave + li;
@@ -1191,33 +1226,26 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
         if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
         grid = dim3((unsigned)total);
     }
-    if (reuse && p.log_sum) {   // a reuse pass that also reports its log-sums: fp32 sums
-        if (paged)
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, true, D, T, true>), grid, block, 0, stream, p);
-        else
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, false, D, T, true>), grid, block, 0, stream, p);
-    } else if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
-        if constexpr (D == 128) {
-            if (paged) hipLaunchKernelGGL((prefill_attn_kernel_q64<true, D, T>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((prefill_attn_kernel_q64<false, D, T>), grid, block, 0, stream, p);
+    auto launch = [&](auto paged_c, auto spare_c) -> hipError_t {
+        constexpr bool kPaged = decltype(paged_c)::value, kSpare = decltype(spare_c)::value;
+        if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
+            if constexpr (D == 128) hipLaunchKernelGGL((prefill_attn_kernel_q64<kPaged, D, T, kSpare>), grid, block, 0, stream, p);
+            else return hipErrorInvalidValue;
+        } else if (reuse && p.log_sum) {   // a reuse pass that also reports its log-sums: fp32 sums, any group
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, true, true>), grid, block, 0, stream, p);
+        } else if (reuse) {
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
+        } else if (with_v) {
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         } else {
-            return hipErrorInvalidValue;
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         }
-    } else if (paged) {
-        if (reuse)
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, true, D, T>), grid, block, 0, stream, p);
-        else if (with_v)
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, true, D, T>), grid, block, 0, stream, p);
-        else
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, true, D, T>), grid, block, 0, stream, p);
-    } else if (reuse) {
-        hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, false, D, T>), grid, block, 0, stream, p);
-    } else {
-        if (with_v)
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, false, D, T>), grid, block, 0, stream, p);
-        else
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, false, D, T>), grid, block, 0, stream, p);
-    }
+        return hipSuccess;
+    };
+    const bool spare = head_slots(p.gs).gs % 4 != 0;
+    const hipError_t e = paged ? (spare ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{}))
+                               : (spare ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{}));
+    if (e != hipSuccess) return e;
     return hipGetLastError();
 }
 
@@ -1229,10 +1257,19 @@ hipError_t launch_aggregate_t(const PrefillParams& p, hipStream_t stream) {
         if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
         grid = dim3((unsigned)total);
     }
-    if (p.block_table)
-        hipLaunchKernelGGL((prefill_aggregate_kernel<true, D, T>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((prefill_aggregate_kernel<false, D, T>), grid, block, 0, stream, p);
+    auto launch = [&](auto heads) {
+        constexpr int kHeads = decltype(heads)::value;
+        if (p.block_table)
+            hipLaunchKernelGGL((prefill_aggregate_kernel<true, D, T, kHeads>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((prefill_aggregate_kernel<false, D, T, kHeads>), grid, block, 0, stream, p);
+    };
+    switch (head_slots(p.gs).gs - 4 * p.vsub) {   // the sub-group's query heads, at most four of them
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    default: launch(std::integral_constant<int, 4>{});
+    }
     return hipGetLastError();
 }
 

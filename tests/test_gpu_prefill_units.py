@@ -230,3 +230,40 @@ def test_log_sums_alone_follow_late_maxima(cuda, batch, heads, G, D, dtype):
         # scores are fp32 sums of D products of up to 200 x 4 x 4, the log-sum has 24 bits: 1e-6 of the largest
         bound = 1e-6 * s.masked_fill(s.isinf(), 0).abs().amax(1) / 0.69 + 4e-6 * want.abs() + 1e-5
         assert ((alone[b, rows, h].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("gs", [1, 2, 3, 5, 6, 7])
+@pytest.mark.parametrize("G,D,L", [(8, 128, 700), (4, 64, 1063), (3, 128, 31)])
+def test_spare_head_slots_change_no_head(cuda, gs, G, D, L):
+    """Groups that fill no whole four head slots leave wavefronts without a head.  Against the same call whose groups
+    are filled up with copies of their last head (log-sum +inf in pooling: exp2(-inf) = 0 each): the same bits."""
+    from kascade_amd import budgets, kernels
+    gen = torch.Generator().manual_seed(10 * gs + L)
+    q = torch.randn(2, L, G, gs, D, generator=gen).half()
+    full = (gs + 3) // 4 * 4
+    qf = torch.cat([q] + [q[:, :, :, -1:]] * (full - gs), dim=3).flatten(2, 3).to(cuda)
+    q = q.flatten(2, 3).to(cuda)
+    k, v = (torch.randn(2, L, G, D, generator=gen).half().to(cuda) for _ in range(2))
+
+    def real(x):   # [B,L,G*full,...] without the copies
+        return x.unflatten(2, (G, full))[:, :, :, :gs].flatten(2, 3)
+    ls, out = kernels.prefill_recompute0(q, k, v)
+    lsf, outf = kernels.prefill_recompute0(qf, k, v)
+    assert torch.equal(ls, real(lsf)) and torch.equal(out, real(outf))
+    assert torch.equal(kernels.prefill_recompute1(q, k), real(kernels.prefill_recompute1(qf, k)))
+
+    T = (L + 31) // 32
+    sc, scf = (torch.zeros(2, G, T, L, device=cuda, dtype=torch.float16) for _ in range(2))
+    lsf = lsf.unflatten(2, (G, full)).clone()
+    lsf[:, :, :, gs:] = float("inf")
+    kernels.prefill_aggregate(q, k, ls, sc)
+    kernels.prefill_aggregate(qf, k, lsf.flatten(2, 3).contiguous(), scf)
+    assert torch.equal(sc, scf)
+
+    width = budgets.topk_width(L, 10)
+    valid, nsel = budgets.prefill_tile_budgets(L, 32, 10, True, width)
+    idx = kernels.topk_indices(sc, width, valid_len=torch.tensor(valid, dtype=torch.int32, device=cuda),
+                               n_sel=torch.tensor(nsel, dtype=torch.int32, device=cuda))
+    hm = torch.arange(G, dtype=torch.int32, device=cuda).flip(0)
+    assert torch.equal(kernels.prefill_reuse(q, k, v, idx, hm, 10.0, True),
+                       real(kernels.prefill_reuse(qf, k, v, idx, hm, 10.0, True)))
