@@ -50,6 +50,12 @@ __device__ __forceinline__ float2 load_device2(const float* p) {
     return make_float2(x.f[0], x.f[1]);
 }
 
+// An entry of a table that no launch reading it writes, at an address that is the same in the whole wavefront: a scalar load
+__device__ __forceinline__ int scalar_entry(const int* table, long long i) {
+    typedef const __attribute__((address_space(4))) int* ConstantPtr;
+    return ((ConstantPtr)table)[i];
+}
+
 template <int D, int HS>
 struct alignas(16) MergeState {  // one per wavefront after the in-wave merge
     float m[HS];
@@ -100,6 +106,15 @@ void decode_split_kernel(DecodeParams p) {
     __shared__ __attribute__((aligned(16))) T s_kt[4][16 * kKtStride];
     __shared__ __attribute__((aligned(16))) T s_vt[WITH_V ? 4 : 1][WITH_V ? 16 * kVtStride : 8];
 
+    // A launch of a few rows per workgroup is a chain of dependent trips to memory, and its start was six of them: arguments
+    // in four trips, each where the compiler first uses one, then Q, then the list.  Now all arguments come at once, Q
+    // is not waited for before the first product, the newest token's rows are requested with it, and the list's first
+    // entries go out in front of it (captured step of 24 layers at 16384 tokens 352 -> 344 us, eager step of 8 x
+    // 3000 tokens 64/8 heads 143.0 -> 139.6).
+    asm volatile("" :: "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.seqlens), "s"(p.idx), "s"(p.block_table), "s"(p.k_new), "s"(p.v_new),
+                 "s"(p.kv_stride_b), "s"(p.kv_stride_h), "s"(p.kv_stride_l), "s"(p.max_pages), "s"(p.topk), "s"(p.num_split),
+                 "s"(p.max_row), "s"(p.gs), "s"(p.glse), "s"(p.opart), "s"(p.k_cache), "s"(p.v_cache), "s"(p.counters),
+                 "s"(p.out), "s"(p.row_sums));
     const int g = blockIdx.x;       // the 8 KV heads of one token range are adjacent in dispatch order
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
@@ -107,7 +122,7 @@ void decode_split_kernel(DecodeParams p) {
 
     // Gather mode: requested at once, together with the lengths (it decides where the list is, the next
     // trip to memory).  A map built for another KV-head count must not leave the index tensor.
-    const int map_g = GATHER ? max(0, min(p.head_map[g], kvh - 1)) : 0;
+    const int map_g = GATHER ? max(0, min(scalar_entry(p.head_map, g), kvh - 1)) : 0;
 
     // The longest context memory allows a sequence that claims `len` tokens: lengths live in device
     // memory, the host sized every buffer from its own arguments, so each length is cut down to
@@ -149,7 +164,7 @@ void decode_split_kernel(DecodeParams p) {
     // at once or whose lists all have the same length (launch_decode_split decides); beyond
     // kMaxNumbered sequences the workgroups keep their grid position.
     constexpr int kMapRounds = kMaxNumbered / 64;
-    int b, split, nsplit_b, seqlen;
+    int b, split, nsplit_b, seqlen, n;   // n: rows this (b, g) pair attends to
     bool len_cut;
     if (p.number_splits) {
         // every wavefront works it out for itself: lane l holds sequences l, l + 64, ...; no LDS,
@@ -165,12 +180,13 @@ void decode_split_kernel(DecodeParams p) {
             cut[r] = __ballot(lens[r] != raw);
         }
         int carry = 0;   // splits of the sequences of earlier rounds (wavefront-uniform)
-        b = -1; split = 0; nsplit_b = 1; seqlen = 0; len_cut = false;
+        b = -1; split = 0; nsplit_b = 1; seqlen = 0; n = 0; len_cut = false;
 #pragma unroll
         for (int r = 0; r < kMapRounds; ++r) {
             if (64 * r < p.B && b < 0) {   // uniform
                 const int bi = 64 * r + lane;
-                const int cnt = bi < p.B ? split_count(rows_for(lens[r])) : 0;
+                const int rows = rows_for(lens[r]);
+                const int cnt = bi < p.B ? split_count(rows) : 0;
                 int incl = cnt;
 #pragma unroll
                 for (int o = 1; o < 64; o <<= 1) {
@@ -185,6 +201,7 @@ void decode_split_kernel(DecodeParams p) {
                     split = __builtin_amdgcn_readfirstlane(w - __shfl(excl, src));
                     nsplit_b = __builtin_amdgcn_readfirstlane(__shfl(cnt, src));
                     seqlen = __builtin_amdgcn_readfirstlane(__shfl(lens[r], src));
+                    n = __builtin_amdgcn_readfirstlane(__shfl(rows, src));
                     len_cut = (cut[r] >> src) & 1;
                 }
                 carry += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
@@ -195,15 +212,15 @@ void decode_split_kernel(DecodeParams p) {
         b = blockIdx.z;
         split = blockIdx.y;
         nsplit_b = p.num_split;
-        const int raw = p.seqlens ? p.seqlens[b] : p.kv_stride_tokens;
+        const int raw = p.seqlens ? scalar_entry(p.seqlens, b) : p.kv_stride_tokens;
         seqlen = safe_len(raw);
         len_cut = seqlen != raw;
+        n = rows_for(seqlen);
         if (p.seqlens != nullptr) {
-            nsplit_b = split_count(rows_for(seqlen));
+            nsplit_b = split_count(n);
             if (split >= nsplit_b) return;   // the first split marks the missing ones as empty
         }
     }
-    const int n = rows_for(seqlen);  // rows this (b, g) pair attends to
     // contiguous range of this split; every split covers rows_per_split rows, sequences
     // shorter than num_split*rows_per_split leave their last splits empty, and the last split of
     // a sequence runs to the sequence's end
@@ -218,35 +235,33 @@ void decode_split_kernel(DecodeParams p) {
     // A length that had to be cut down names a slot that does not exist: nothing is appended.
     const int newest = seqlen - 1;
     const bool can_append = p.k_new != nullptr && newest >= 0 && !len_cut;
-    int newest_row = -1;   // PHYS: the cache row of the newest token, what a list names it by
-    if (PHYS && can_append)
-        newest_row = (p.block_table[(size_t)b * p.max_pages + (newest >> p.page_shift)] << p.page_shift) +
-                     (newest & ((1 << p.page_shift) - 1));
+    // the page of the newest token and this thread's 16-byte chunk of its K or V row: requested here, used much later
+    // (without a page to ask for, the first word of Q: a load under a branch would be waited for at the branch's end)
+    const int newest_page = scalar_entry(can_append && p.block_table
+                                             ? p.block_table + ((long long)b * p.max_pages + (newest >> p.page_shift))
+                                             : (const int*)p.Q, 0);
+    uint4_t new_chunk = {0, 0, 0, 0};
+    if (can_append) {   // uniform
+        const int t = min(tid, 2 * (D / 8) - 1), part = t / (D / 8), c = t % (D / 8);
+        new_chunk = ld_global_16((part ? (const T*)p.v_new : (const T*)p.k_new) + ((size_t)b * kvh + g) * D + c * 8);
+    }
     auto write_newest = [&]() {
         if (tid < 2 * (D / 8)) {   // one 16-byte chunk of the K row or of the V row per thread
             const int part = tid / (D / 8), c = tid % (D / 8);
             size_t off;
             if (p.block_table) {
-                const int pg = p.block_table[(size_t)b * p.max_pages + (newest >> p.page_shift)];
-                const int row = (pg << p.page_shift) + (newest & ((1 << p.page_shift) - 1));
+                const int row = (newest_page << p.page_shift) + (newest & ((1 << p.page_shift) - 1));
                 off = (size_t)row * (kvh * D) + (size_t)g * D + c * 8;
             } else {
                 off = (size_t)b * p.kv_stride_b + (size_t)g * p.kv_stride_h + (size_t)newest * p.kv_stride_l + c * 8;
             }
-            const T* src = (part ? (const T*)p.v_new : (const T*)p.k_new) + ((size_t)b * kvh + g) * D + c * 8;
             T* dst = (part ? (T*)p.v_cache : (T*)p.k_cache) + off;
-            *reinterpret_cast<uint4_t*>(dst) = ld_global_16(src);
+            *reinterpret_cast<uint4_t*>(dst) = new_chunk;
         }
     };
-    if (can_append) {
-        if (!GATHER) {
-            if (newest >= r0 && newest < r1) {   // the split that streams the newest row
-                write_newest();
-                __syncthreads();
-            }
-        } else if (split == 0) {
-            write_newest();   // lists that do not name the newest token still leave it cached
-        }
+    if (!GATHER && can_append && newest >= r0 && newest < r1) {   // the split that streams the newest row
+        write_newest();
+        __syncthreads();
     }
     if (GATHER && tid == 0) s_found = -1;
 
@@ -255,7 +270,7 @@ void decode_split_kernel(DecodeParams p) {
     // of rows 4i + dq of a tile, i = 0..3, so 16 lanes fetch one 256-byte row and an instruction
     // four rows.  Computing: the same lane is key `col` / part dq of the A operand of
     // S^T = K Q^T (v_mfma_f32_16x16x32_f16: 16 keys x 16 columns, d contracted 32 at a time; the
-    // four query heads are columns 0-3, the rest zero) and ends up with S^T[4dq .. 4dq+3][col]:
+    // four query heads are columns 0-3, the rest the last of them again, unused) and ends up with S^T[4dq .. 4dq+3][col]:
     // exactly the B-operand layout of O^T += V^T P^T (v_mfma_f32_16x16x16_f16, the tile's 16 keys
     // contracted), whose A operand V^T is read out of the row-major V tile by the transposing LDS
     // read.  The tiles pass through wavefront-private LDS (no workgroup barrier).  Nothing here is
@@ -267,13 +282,25 @@ void decode_split_kernel(DecodeParams p) {
     // (lr, lc) takes chunk lc of rows kRowsPerLoad * i + lr.
     constexpr int kChunks = D / 8, kRowsPerLoad = 64 / kChunks, kLoads = 16 / kRowsPerLoad;
     const int lc = lane % kChunks, lr = lane / kChunks;
+    // This thread's first entries of the list, in front of Q and outside the sub-chunks' loop: in there the compiler waits
+    // for every load on its way before it lets one overwrite registers, which put a trip for Q before the list's.
+    constexpr int kPre = 2;
+    const int* idx_row = nullptr;
+    int pre[kPre];
+    if (GATHER) {
+        idx_row = p.idx + ((size_t)b * kvh + map_g) * p.topk;
+        if (r0 < r1 && r1 - r0 <= kPre * kThreads) {   // uniform: a split whose list is staged in one or two steps
+#pragma unroll
+            for (int j = 0; j < kPre; ++j) pre[j] = idx_row[min(r0 + tid + j * kThreads, r1 - 1)];
+        }
+        KASCADE_SCHED_FENCE();
+    }
     x8_t qb[D / 32];   // B operand of the first product: Q[col][32*st + 8*dq, +8)
 #pragma unroll
     for (int st = 0; st < D / 32; ++st) {
         PackT<T> t;
         t.u = ld_global_16((const T*)p.Q + ((size_t)b * nheads + g * gs + min(col, gs - 1)) * D + 32 * st + 8 * dq);
-        if (col >= gs) t.u = uint4_t{0, 0, 0, 0};
-        qb[st] = t.v8;
+        qb[st] = t.v8;   // columns past the last head: that head again, not used
     }
     // Online softmax state of this lane's column.  With V one running maximum per column (the
     // second product needs a common reference: two cross-lane exchanges per tile); without V
@@ -284,8 +311,6 @@ void decode_split_kernel(DecodeParams p) {
 #pragma unroll
     for (int blk = 0; blk < (WITH_V ? kOBlocks : 1); ++blk) oacc[blk] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    const int* idx_row = nullptr;
-    if (GATHER) idx_row = p.idx + ((size_t)b * kvh + map_g) * p.topk;
     const int page_mask = (1 << p.page_shift) - 1;
     const unsigned stride_l = p.kv_stride_l;
     T* kt = &s_kt[wave][0];
@@ -460,11 +485,16 @@ void decode_split_kernel(DecodeParams p) {
             // all of a thread's index loads first, then all of its block-table loads: two trips to
             // memory per sub-chunk instead of two per entry (the count per thread is a compile-time
             // constant per case, so that short lists do not pay for eight loads)
+            // what a list names the newest token by
+            const int newest_name = !PHYS ? newest : can_append ? (newest_page << p.page_shift) + (newest & page_mask) : -1;
             auto stage = [&](auto per_tag) {
                 constexpr int kPer = decltype(per_tag)::value;
                 int toks[kPer], rows[kPer];
 #pragma unroll
-                for (int j = 0; j < kPer; ++j) toks[j] = idx_row[c0 + min(tid + j * kThreads, cn - 1)];
+                for (int j = 0; j < kPer; ++j) {
+                    if (kPer <= kPre && c0 == r0) toks[j] = pre[j % kPre];   // uniform
+                    else toks[j] = idx_row[c0 + min(tid + j * kThreads, cn - 1)];
+                }
                 early_tiles();
 #pragma unroll
                 for (int j = 0; j < kPer; ++j) {
@@ -476,7 +506,7 @@ void decode_split_kernel(DecodeParams p) {
                 for (int j = 0; j < kPer; ++j) {
                     const int i = tid + j * kThreads;
                     if (i < cn) {
-                        if (toks[j] == (PHYS ? newest_row : newest)) s_found = c0;
+                        if (toks[j] == newest_name) s_found = c0;
                         s_row[i] = (PAGED && !PHYS) ? (rows[j] << p.page_shift) + (toks[j] & page_mask) : rows[j];
                     }
                 }
@@ -489,6 +519,8 @@ void decode_split_kernel(DecodeParams p) {
             if (can_append && s_found == c0) {   // c0 differs per sub-chunk: no reset needed
                 write_newest();
                 __syncthreads();
+            } else if (can_append && split == 0 && c0 == r0) {
+                write_newest();   // lists that do not name the newest token still leave it cached
             }
             auto issue = [&](int t, Tile& tb) {   // tile t: rows [16t, 16t+16) of the sub-chunk
 #pragma unroll
@@ -520,6 +552,7 @@ void decode_split_kernel(DecodeParams p) {
             }
         }
         };
+        if (can_append && split == 0 && r0 >= r1) write_newest();   // no list at all
         if (p.block_table) run(std::true_type{}); else run(std::false_type{});
     } else {
         // Token range [r0, r1) (dense baseline, anchor passes): no staging.  A wavefront owns one strip

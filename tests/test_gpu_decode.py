@@ -731,3 +731,56 @@ def test_reuse_from_translated_rows_equals_reuse_from_token_lists(cuda, seqlens,
     out = kernels.decode_reuse_rows(q, kp, vp, lens, bad, hm, pct, glse, part, bt, page_size=ps)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("named", [True, False])
+@pytest.mark.parametrize("n,ns", [(1, 1), (128, 1), (256, 1), (257, 1), (512, 1), (513, 1), (513, 2), (2049, 1), (2560, 2)])
+@pytest.mark.parametrize("form", ["tokens", "rows", "strided"])
+def test_gather_lists_of_every_staging_with_and_without_the_newest_token(cuda, form, n, ns, named):
+    """A list is staged from registers (up to two entries per thread), or in sub-chunks of 2048; the newest token's
+    rows arrive beside the cache.  Against the same call on a cache that holds them: the same bits, and both caches
+    are equal afterwards, whether or not the list names that token."""
+    from kascade_amd import kernels
+    G, H, D, page = 4, 12, 128, 16
+    L = 2 * n + 40
+    gen = torch.Generator().manual_seed(n)
+    q = torch.randn(1, H, D, generator=gen).half().to(cuda)
+    k, v = (torch.randn(1, L, G, D, generator=gen).half().to(cuda) for _ in range(2))
+    idx = torch.stack([torch.randperm(L - 1, generator=gen)[:n].sort().values for _ in range(G)])
+    if named:
+        idx[:, -1] = L - 1
+    idx = idx[None].to(torch.int32).contiguous().to(cuda)
+    hm = torch.tensor([2, 0, 3, 1], dtype=torch.int32, device=cuda)
+    lens = torch.tensor([L], dtype=torch.int32, device=cuda)
+    table = None
+    kn, vn = k[:, L - 1].contiguous(), v[:, L - 1].contiguous()
+    row = L - 1
+    if form != "strided":
+        per = -(-L // page)
+        order = torch.randperm(per, generator=gen)
+
+        def paged(x):
+            out = torch.zeros(per, page, G, D, dtype=x.dtype, device=cuda)
+            flat = torch.zeros(per * page, G, D, dtype=x.dtype, device=cuda)
+            flat[:L] = x[0]
+            out[order.to(cuda)] = flat.view(per, page, G, D)
+            return out
+        k, v, table = paged(k), paged(v), order.to(torch.int32)[None].contiguous().to(cuda)
+        row = int(order[(L - 1) // page]) * page + (L - 1) % page
+    if form == "rows":
+        t = idx.long()
+        idx = (table[0].long()[t // page] * page + t % page).to(torch.int32).contiguous()
+
+    def call(kc, vc, **new):
+        glse = torch.empty(1, H, ns, device=cuda)
+        part = torch.empty(1, H, ns, D, device=cuda)
+        if form == "rows":
+            return kernels.decode_reuse_rows(q, kc, vc, lens, idx, hm, 0.0, glse, part, table, page, **new)
+        return kernels.decode_reuse_paged(q, kc, vc, lens, idx, hm, 0.0, glse, part, table, page, **new)
+    want = call(k, v)
+    kc, vc = k.clone(), v.clone()
+    for c in (kc, vc):
+        c.view(-1, G, D)[row] = 7.0
+    got = call(kc, vc, k_new=kn, v_new=vn)
+    assert torch.equal(got, want)
+    assert torch.equal(kc, k) and torch.equal(vc, v)
