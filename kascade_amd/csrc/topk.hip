@@ -272,13 +272,16 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(
 //    exponent bins).  The bin of +0 and the 31 smallest subnormals, where pooled probabilities
 //    underflow to by the thousand, is not counted at all: its count is the row length minus the
 //    sum of the others.  NONNEG: no entry is below +0 (pooled probabilities), half the bins.
-//  * The fine histogram tests both halves of a word against the threshold bin at once; the counts
-//    above / equal to T are sums of min(sat(key - (T-1)), 2) over packed halves.
+//  * The fine histogram knows of +0 only where its bin is the threshold's.  min(sat(key - (T-1)), 2) over packed
+//    halves, two bits an entry, gives the counts above / equal to T and, kept, the masks of the compaction.
 //  * The selected positions are staged in LDS in their final order, so that the list leaves as
 //    full-width stores.
 // Causal prompt tiles (8 heads x L/32 rows, ragged), against one size of workgroup with a scan over all
 // (chunk, wavefront) pairs: L = 4096 18.6 -> 9.4 us, 8192 34.6 -> 20.5, 16384 73.6 -> 48.8, 32768 179 -> 150,
 // 65536 907 -> 587 us; 2048 full rows of 65536: 175 -> 143 us = 1.9 TB/s.
+// One row on one compute unit (decode anchors, pooling included, 16384 tokens of 4 heads): 13.4 -> 12.3 us with the log-sums'
+// parts requested before the length is known, the histograms cleared under the row's loads, counters addressed by the key's
+// bits in place, and the codes kept.
 // Sum of the entries of s_wave before `wave`, and of all of them (one per wavefront, in LDS).
 template <int THREADS>
 __device__ __forceinline__ void scan_waves(const uint32_t* s_wave, int wave, uint32_t& before, uint32_t& all) {
@@ -289,12 +292,26 @@ __device__ __forceinline__ void scan_waves(const uint32_t* s_wave, int wave, uin
     before = wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)inc, wave - 1) : 0u;
 }
 
+// A workgroup's histograms.  Cleared by the caller a barrier before select_row, under the loads of the row.
+template <int THREADS, bool NONNEG>
+struct SelectLds {
+    static constexpr int kCopies = 4;
+    static constexpr int kNB = NONNEG ? 1024 : 2048;                 // coarse bins
+    uint32_t hist[kNB * kCopies];
+    uint32_t hist2[32];
+    __device__ __forceinline__ void clear() {
+        for (int i = threadIdx.x * 4; i < kNB * kCopies; i += THREADS * 4) *reinterpret_cast<uint4_t*>(&hist[i]) = uint4_t{0, 0, 0, 0};
+        if (threadIdx.x < 32) hist2[threadIdx.x] = 0;
+    }
+};
+
 template <int THREADS, int MAXC, bool NONNEG>
-__device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch, int lead, int row_len, int n, int k,
-                                           int fill, int* __restrict__ out, long long row, const RowsOut& ro) {
+__device__ __forceinline__ void select_row(SelectLds<THREADS, NONNEG>& lds, const uint4_t (&data)[MAXC], int nch, int lead,
+                                           int row_len, int n, int k, int fill, int* __restrict__ out, long long row,
+                                           const RowsOut& ro) {
     constexpr int kW = THREADS / 64;
-    constexpr int kCopies = 4;
-    constexpr int kNB = NONNEG ? 1024 : 2048;                        // coarse bins ...
+    constexpr int kCopies = SelectLds<THREADS, NONNEG>::kCopies;
+    constexpr int kNB = SelectLds<THREADS, NONNEG>::kNB;             // coarse bins ...
     constexpr uint32_t kBin0 = NONNEG ? 1024 : 0;                    // ... from this one on
     constexpr int kStage = kNB * kCopies;                            // positions staged in the histogram's LDS
     constexpr uint32_t kOne = 0x00010001u, kTwo = 0x00020002u;
@@ -302,8 +319,8 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
     constexpr uint32_t kSkipBin = kZeroKey >> 5;                     // coarse bin of +0: counted by subtraction
     constexpr int kBPT = kNB / THREADS > 0 ? kNB / THREADS : 1;      // bins per thread in the scan
     static_assert(kNB % THREADS == 0 || kNB < THREADS, "whole bins per thread");
-    __shared__ __attribute__((aligned(16))) uint32_t s_hist[kNB * kCopies];
-    __shared__ uint32_t s_hist2[32];
+    uint32_t* s_hist = lds.hist;
+    uint32_t* s_hist2 = lds.hist2;
     __shared__ uint32_t s_wave[kW], s_gt[kW], s_eq[kW];
     __shared__ uint32_t s_sel[2];  // b1, cum_above
 
@@ -314,21 +331,23 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
     int* rdst = ro.rows ? ro.rows + row * (long long)k : nullptr;
 
     // ---- pass 1: coarse histogram ----
-    for (int i = tid * 4; i < kNB * kCopies; i += THREADS * 4) *reinterpret_cast<uint4_t*>(&s_hist[i]) = uint4_t{0, 0, 0, 0};
-    if (tid < 32) s_hist2[tid] = 0;
-    __syncthreads();
-    const uint32_t copy = tid & (kCopies - 1);
-    auto count1 = [&](uint32_t key) {   // absent entries and the bin of +0 are not counted
-        const uint32_t bin = key >> 5;
-        if (NONNEG ? bin > kSkipBin : (key != 0 && bin != kSkipBin)) atomicAdd(&s_hist[(bin - kBin0) * kCopies + copy], 1u);
+    // A bin's copies are 16 bytes: the byte offset of a key's counter is its bin in place, shifted by one, and the copy.
+    // (NONNEG: the top bit of every bin is set and left out.)
+    static_assert(kCopies == 4, "a bin is 16 bytes");
+    constexpr uint32_t kBinBytes = NONNEG ? 0x3FF0u : 0x7FF0u;
+    const uint32_t copy = (tid & (kCopies - 1)) * 4;
+    auto count1 = [&](uint16_t key, uint32_t bytes) {   // absent entries and the bin of +0 are not counted
+        if (NONNEG ? key >= kZeroKey + 32 : (key != 0 && key >> 5 != kSkipBin))
+            atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_hist) + bytes), 1u);
     };
     static_for<0, MAXC>([&](auto c_c) {
         constexpr int c = decltype(c_c)::value;
         if (c < nch) {   // uniform
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                count1(data[c][j] & 0xFFFFu);
-                count1(data[c][j] >> 16);
+                const uint32_t w = data[c][j];
+                count1((uint16_t)w, ((w >> 1) & kBinBytes) | copy);
+                count1((uint16_t)(w >> 16), ((w >> 17) & kBinBytes) | copy);
             }
         }
     });
@@ -369,33 +388,34 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
     const uint32_t b1 = s_sel[0];
     const uint32_t cum_above = s_sel[1];
 
-    // ---- pass 2: fine histogram inside the threshold bin.  Few entries match: both halves of a word
-    // are tested at once.  +0 is left out of the atomics (that many on one address would serialise)
-    // and counted per wavefront where its bin is the threshold's ----
+    // ---- pass 2: fine histogram inside the threshold bin.  +0 is left out of the atomics (that many on one
+    // address would serialise) and counted per wavefront where its bin is the threshold's ----
     {
         const uint32_t bb = (b1 << 5) | (b1 << 21);
-        uint32_t nonzero = 0;   // per half: slots of this thread that do not hold +0 (<= 4 MAXC)
-        static_for<0, MAXC>([&](auto c_c) {
-            constexpr int c = decltype(c_c)::value;
-            if (c < nch) {
+        auto fine = [&](auto with_zero) {
+            constexpr bool ZERO = decltype(with_zero)::value;
+            uint32_t nonzero = 0;   // per half: slots of this thread that do not hold +0 (<= 4 MAXC)
+            static_for<0, MAXC>([&](auto c_c) {
+                constexpr int c = decltype(c_c)::value;
+                if (c < nch) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t w = data[c][j];
-                    const uint32_t x = (w ^ bb) & 0xFFE0FFE0u;   // a half is 0 iff its key lies in the bin
-                    nonzero = pk_add_u16(nonzero, pk_min_u16(w ^ 0x80008000u, kOne));
-                    if (pk_min_u16(x, kOne) != kOne) {
-                        if ((x & 0xFFFFu) == 0 && (w & 0xFFFFu) != kZeroKey) atomicAdd(&s_hist2[w & 31u], 1u);
-                        if ((x >> 16) == 0 && (w >> 16) != kZeroKey) atomicAdd(&s_hist2[(w >> 16) & 31u], 1u);
+                    for (int j = 0; j < 4; ++j) {
+                        const uint32_t w = data[c][j];
+                        const uint32_t x = (w ^ bb) & 0xFFE0FFE0u;   // a half is 0 iff its key lies in the bin
+                        if (ZERO) nonzero = pk_add_u16(nonzero, pk_min_u16(w ^ 0x80008000u, kOne));
+                        if ((uint16_t)x == 0 && (!ZERO || (uint16_t)w != kZeroKey)) atomicAdd(&s_hist2[w & 31u], 1u);
+                        if (x < 0x10000u && (!ZERO || w >> 16 != kZeroKey)) atomicAdd(&s_hist2[(w >> 16) & 31u], 1u);
                     }
                 }
-            }
-        });
-        if (b1 == kSkipBin) {
-            uint32_t z = 8u * (uint32_t)nch - (nonzero & 0xFFFFu) - (nonzero >> 16);
+            });
+            if (ZERO) {
+                uint32_t z = 8u * (uint32_t)nch - (nonzero & 0xFFFFu) - (nonzero >> 16);
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) z += __shfl_xor(z, o);
-            if (lane == 0 && z) atomicAdd(&s_hist2[kZeroKey & 31u], z);
-        }
+                for (int o = 32; o >= 1; o >>= 1) z += __shfl_xor(z, o);
+                if (lane == 0 && z) atomicAdd(&s_hist2[kZeroKey & 31u], z);
+            }
+        };
+        if (b1 == kSkipBin) fine(std::true_type{}); else fine(std::false_type{});   // uniform
     }
     __syncthreads();
     uint32_t T, r;   // threshold key and the number of entries equal to it to take: every wavefront for itself
@@ -415,23 +435,29 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
     const uint32_t tm1 = (T - 1u) | ((T - 1u) << 16);   // T >= 1
 
     // ---- pass 3: ordered compaction ----
-    // code of a half: min(sat(key - (T-1)), 2) = 0 below T, 1 equal to T, 2 above T
+    // code of a half: min(sat(key - (T-1)), 2) = 0 below T, 1 equal to T, 2 above T.  Kept for both uses, two bits an
+    // entry: word j of a chunk at bits 2 j and 16 + 2 j, an odd chunk 8 bits above the even one before it.
+    constexpr uint32_t kAbove = 0xAAAAAAAAu, kEqual = 0x55555555u;
+    uint32_t codes[(MAXC + 1) / 2];
     {
-        uint32_t sum = 0, ties = 0;   // per half: sum of the codes (<= 8 MAXC), number of ones (<= 4 MAXC)
+        uint32_t gt = 0, eq = 0;
+#pragma unroll
+        for (int i = 0; i < (MAXC + 1) / 2; ++i) codes[i] = 0;
         static_for<0, MAXC>([&](auto c_c) {
             constexpr int c = decltype(c_c)::value;
             if (c < nch) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1), kTwo);
-                    sum = pk_add_u16(sum, code);
-                    ties = pk_add_u16(ties, code & kOne);
-                }
+                for (int j = 0; j < 4; ++j)
+                    codes[c / 2] |= pk_min_u16(pk_sub_sat_u16(data[c][j], tm1), kTwo) << (8 * (c & 1) + 2 * j);
             }
         });
-        const uint32_t eq = (ties & 0xFFFFu) + (ties >> 16);
+#pragma unroll
+        for (int i = 0; i < (MAXC + 1) / 2; ++i) {
+            gt += (uint32_t)__popc(codes[i] & kAbove);
+            eq += (uint32_t)__popc(codes[i] & kEqual);
+        }
         // above T in the low half, equal to T in the high half (a wavefront holds at most 8192 entries)
-        const uint32_t all = wave_incl_scan((((sum & 0xFFFFu) + (sum >> 16) - eq) >> 1) | (eq << 16));
+        const uint32_t all = wave_incl_scan(gt | (eq << 16));
         if (lane == 63) {
             s_gt[wave] = all & 0xFFFFu;
             s_eq[wave] = all >> 16;
@@ -446,20 +472,15 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
     const int base0 = wave * nch * 512 + lane * 8 - lead;      // position of this thread's first entry
 #pragma clang loop unroll(disable)
     for (uint32_t lo = 0; lo < (uint32_t)n; lo += kStage) {
-        // opaque copy: the codes are recomputed per round instead of being kept in registers across rounds
-        uint32_t tm1_r = tm1;
-        asm volatile("" : "+v"(tm1_r));
         uint32_t carry = 0;   // entries of the wavefront's part before the chunk: above T / equal to T, packed
         static_for<0, MAXC>([&](auto c_c) {
             constexpr int c = decltype(c_c)::value;
             if (c < nch) {
-                uint32_t above = 0, equal = 0;   // bit e: entry e of the chunk is above / equal to T
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t code = pk_min_u16(pk_sub_sat_u16(data[c][j], tm1_r), kTwo);
-                    above |= (((code >> 1) & 1u) | ((code >> 16) & 2u)) << (2 * j);
-                    equal |= ((code & 1u) | ((code >> 15) & 2u)) << (2 * j);
-                }
+                // bit e: entry e of the chunk is above / equal to T (entries 2 j in the low half, 2 j + 1 in the high one)
+                const uint32_t cc = codes[c / 2] >> (8 * (c & 1));
+                const uint32_t gt2 = (cc & kAbove) >> 1, eq2 = cc & kEqual;
+                const uint32_t above = (gt2 | (gt2 >> 15)) & 0xFFu;
+                uint32_t equal = (eq2 | (eq2 >> 15)) & 0xFFu;
                 const uint32_t cnt = (uint32_t)__popc(above) | ((uint32_t)__popc(equal) << 16);
                 const uint32_t v = wave_incl_scan(cnt);
                 if (cnt) {
@@ -469,6 +490,7 @@ __device__ __forceinline__ void select_row(const uint4_t (&data)[MAXC], int nch,
                     // earlier ties taken
                     uint32_t pos = gt_before + (ex & 0xFFFFu) + min(my_eq, r) - lo;
                     const uint32_t room = r - min(my_eq, r);             // ties that still fit, the lower positions first
+                    equal = room == 0 ? 0u : equal;
 #pragma clang loop unroll(disable)
                     while ((uint32_t)__popc(equal) > room) equal &= ~(0x80000000u >> __clz(equal));
 #pragma clang loop unroll(disable)
@@ -562,6 +584,8 @@ void topk_select_reg_kernel(
         if (c < nch && slots >= 8)   // uniform
             data[c] = *reinterpret_cast<const uint4_t*>(src + min(first + c * 512, last_full));
     });
+    __shared__ __attribute__((aligned(16))) SelectLds<THREADS, false> s_sel_lds;
+    s_sel_lds.clear();
     // the pieces at the row's two ends, one thread each, entry by entry (0: no entry)
     const int tail = slots & ~7;    // first slot of the partial piece at the end
     auto piece = [&](int s0) {
@@ -596,7 +620,8 @@ void topk_select_reg_kernel(
             }
         }
     });
-    select_row<THREADS, MAXC, false>(data, nch, lead, len, n, k, fill, out, row, ro);
+    __syncthreads();   // cleared histograms
+    select_row<THREADS, MAXC, false>(s_sel_lds, data, nch, lead, len, n, k, fill, out, row, ro);
 }
 
 // Decode anchors: pooling and selection of a (sequence, KV head) row in one workgroup.  What the
@@ -615,8 +640,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
 void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restrict__ out, RowsOut ro) {
     constexpr int kMaxGroup = 16;
     __shared__ float s_lse[kMaxGroup];
+    __shared__ __attribute__((aligned(16))) SelectLds<THREADS, true> s_sel_lds;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row = blockIdx.x, b = row / p.groups;
+    // The first parts of the log-sums are requested together with the length, the first scores before those parts have
+    // arrived: one trip to memory less each, and the histograms are cleared meanwhile.
+    float first_part = -INFINITY;
+    if (p.glse && wave < p.group_size && lane < p.num_split)
+        first_part = p.glse[((long long)row * p.group_size + wave) * p.num_split + lane];
     const int raw = p.seqlens ? p.seqlens[b] : p.uniform_len;
     const float* base = p.scores + (long long)row * p.group_size * p.scores_stride;   // heads of a KV head are adjacent
     const int len = max(0, min(raw, p.len_cap));           // tokens whose scores were written
@@ -628,35 +659,32 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
         row_len = p.uniform_len;                           // every row the same: positions past a sequence pool to 0
     }
     n = max(0, n);
-    if (row_len <= n || n == 0) {
-        if (p.glse == nullptr) {
-            list_head<THREADS>(n, k, fill, out, row, ro);
-            return;
-        }
-    }
     // the heads' log-sums: merged from the splits' parts by a wavefront per head, or ready
-    for (int h = wave; h < p.group_size; h += THREADS / 64) {
-        const long long head = (long long)row * p.group_size + h;
-        if (p.glse) {
-            const float* gl = p.glse + head * p.num_split;
-            const float g0 = lane < p.num_split ? gl[lane] : -INFINITY;
-            float mx = g0;
-            for (int s = lane + 64; s < p.num_split; s += 64) mx = fmaxf(mx, gl[s]);
-            mx = wave_max(mx);
-            const float mref = (mx == -INFINITY) ? 0.f : mx;
-            float sum = fast_exp2(g0 - mref);
-            for (int s = lane + 64; s < p.num_split; s += 64) sum += fast_exp2(gl[s] - mref);
-            sum = wave_sum(sum);
-            const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
-            if (lane == 0) {
-                s_lse[h] = v;
-                p.row_sums[head] = v;
+    auto merge_log_sums = [&]() {
+        for (int h = wave; h < p.group_size; h += THREADS / 64) {
+            const long long head = (long long)row * p.group_size + h;
+            if (p.glse) {
+                const float* gl = p.glse + head * p.num_split;
+                const float g0 = h == wave ? first_part : lane < p.num_split ? gl[lane] : -INFINITY;
+                float mx = g0;
+                for (int s = lane + 64; s < p.num_split; s += 64) mx = fmaxf(mx, gl[s]);
+                mx = wave_max(mx);
+                const float mref = (mx == -INFINITY) ? 0.f : mx;
+                float sum = fast_exp2(g0 - mref);
+                for (int s = lane + 64; s < p.num_split; s += 64) sum += fast_exp2(gl[s] - mref);
+                sum = wave_sum(sum);
+                const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
+                if (lane == 0) {
+                    s_lse[h] = v;
+                    p.row_sums[head] = v;
+                }
+            } else if (lane == 0) {
+                s_lse[h] = p.row_sums[head];
             }
-        } else if (lane == 0) {
-            s_lse[h] = p.row_sums[head];
         }
-    }
+    };
     if (row_len <= n || n == 0) {
+        if (p.glse) merge_log_sums();
         list_head<THREADS>(n, k, fill, out, row, ro);
         return;
     }
@@ -701,7 +729,9 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
     Batch cur, n1, n2;
     load_batch(0, n1);
     load_batch(1, n2);
-    __syncthreads();   // s_lse
+    s_sel_lds.clear();
+    merge_log_sums();
+    __syncthreads();   // s_lse, cleared histograms
     static_for<0, MAXC>([&](auto c_c) {
         constexpr int c = decltype(c_c)::value;
         data[c] = uint4_t{0, 0, 0, 0};
@@ -757,7 +787,7 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
             }
         });
     }
-    select_row<THREADS, MAXC, true>(data, nch, 0, row_len, n, k, fill, out, row, ro);
+    select_row<THREADS, MAXC, true>(s_sel_lds, data, nch, 0, row_len, n, k, fill, out, row, ro);
 }
 
 // --------------------------------------------------------------------------
