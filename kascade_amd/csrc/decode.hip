@@ -848,6 +848,10 @@ __global__ __launch_bounds__(128) void decode_combine_kernel(const float* __rest
 // (glse [B,H,num_split]): then every workgroup merges them itself -- a wavefront per head, four
 // heads at a time -- and the first workgroup of a (sequence, KV head) also writes them to
 // row_sums_out, which saves the combine launch of an anchor pass that produces no output.
+// scores_stride is a multiple of 8 (host).
+// Bound by trips to memory, not by its bytes: the log-sums' parts and the codes of four heads at a time are requested together
+// (one after the other, 16 sequences of 65536 tokens took 23.3 us and four of 131072 to 524288 28.6; 17.4 and 21.4 now).
+// Workgroups past the sequence write their zeros and leave.
 __global__ __launch_bounds__(256) void decode_aggregate_kernel(const float* __restrict__ scores,
                                                               const float* __restrict__ row_sums_in,
                                                               const float* __restrict__ glse, int num_split,
@@ -861,67 +865,73 @@ __global__ __launch_bounds__(256) void decode_aggregate_kernel(const float* __re
     const int g = blockIdx.y;
     const int b = blockIdx.z;
     const int kvh = gridDim.y, nheads = gridDim.y * gs;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const long long head0 = (long long)b * nheads + g * gs;
+    // this wavefront's first head: its first 64 parts, or its log-sum (the last head again where there is none)
+    const long long mine = head0 + min(wave, gs - 1);
+    const float first_part = glse ? glse[mine * num_split + min(lane, num_split - 1)] : row_sums_in[mine];
     // the same bound the streaming launch applied to the length: codes beyond it were never written
     const int len = max(0, min(seqlens ? seqlens[b] : uniform_len, len_cap));
     const int j0 = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (glse != nullptr) {   // uniform over the launch
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        for (int h = wave; h < gs; h += 4) {
-            const float* gl = glse + ((size_t)b * nheads + g * gs + h) * num_split;
-            float mx = -INFINITY;
-            for (int sidx = lane; sidx < num_split; sidx += 64) mx = fmaxf(mx, gl[sidx]);
+    half_t* ap = agg + ((size_t)b * kvh + g) * scores_stride + j0;
+    if (blockIdx.x > 0 && (int)blockIdx.x * 2048 >= len) {   // uniform
+        if (j0 < scores_stride) *reinterpret_cast<uint4_t*>(ap) = uint4_t{0, 0, 0, 0};
+        return;
+    }
+    const int jc = min(j0, max(0, len - 1) & ~7);   // past the tokens: codes that exist, dropped below
+    uint4_t q[4];
+    float ref[4];
+    auto request = [&](int h0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float* row = scores + (head0 + min(h0 + u, gs - 1)) * scores_stride;
+            q[u] = ld_global_16(reinterpret_cast<const uint16_t*>(row) + jc);
+            ref[u] = row[scores_stride / 2 + (jc >> 6)];
+        }
+    };
+    request(0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int h = wave; h < gs; h += 4) {
+        float v;
+        if (glse != nullptr) {   // uniform over the launch
+            const float* gl = glse + (head0 + h) * num_split;
+            const float g0 = lane >= num_split ? -INFINITY : h == wave ? first_part : gl[lane];
+            float mx = g0;
+            for (int s = lane + 64; s < num_split; s += 64) mx = fmaxf(mx, gl[s]);
             mx = wave_max(mx);
             const float mref = (mx == -INFINITY) ? 0.f : mx;
-            float sum = 0.f;
-            for (int sidx = lane; sidx < num_split; sidx += 64) sum += fast_exp2(gl[sidx] - mref);
+            float sum = fast_exp2(g0 - mref);
+            for (int s = lane + 64; s < num_split; s += 64) sum += fast_exp2(gl[s] - mref);
             sum = wave_sum(sum);
-            const float v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
-            if (lane == 0) {
-                s_lse[h] = v;
-                if (blockIdx.x == 0 && row_sums_out) row_sums_out[(size_t)b * nheads + g * gs + h] = v;
-            }
+            v = (sum > 0.f) ? fast_log2(sum) + mref : -INFINITY;
+            if (lane == 0 && blockIdx.x == 0 && row_sums_out) row_sums_out[head0 + h] = v;
+        } else {
+            v = h == wave ? first_part : row_sums_in[head0 + h];
         }
-    } else if (threadIdx.x < gs) {
-        s_lse[threadIdx.x] = row_sums_in[(size_t)b * nheads + g * gs + threadIdx.x];
+        if (lane == 0) s_lse[h] = v;
     }
     __syncthreads();
-    if (j0 >= scores_stride) return;
-    float sum[8];
+    float sum[8] = {};
+    for (int h0 = 0; h0 < gs; h0 += 4) {
+        if (h0 > 0) request(h0);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sum[e] = 0.f;
-    const bool full = (j0 + 8 <= scores_stride) && ((scores_stride & 7) == 0);
-    if (j0 < len) {   // codes and references beyond the sequence were never written
-        for (int h = 0; h < gs; ++h) {
-            const float* row = scores + ((size_t)b * nheads + g * gs + h) * scores_stride;
-            const uint16_t* sp = reinterpret_cast<const uint16_t*>(row) + j0;
-            const float ref = row[scores_stride / 2 + (j0 >> 6)] - s_lse[h];
-            uint32_t q[8];
-            if (full) {
-                const uint4_t raw = ld_global_16(sp);
+        for (int u = 0; u < 4; ++u) {
+            if (h0 + u < gs) {   // uniform
+                const float r = ref[u] - s_lse[h0 + u];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) q[e] = (raw[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) q[e] = (j0 + e < len) ? sp[e] : kScoreNone;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pr = fast_exp2(ref - (float)q[e] * (1.f / kScoreSteps));
-                sum[e] += (q[e] == kScoreNone) ? 0.f : pr;
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t c = (q[u][e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
+                    const float pr = fast_exp2(r - (float)c * (1.f / kScoreSteps));
+                    sum[e] += (c == kScoreNone) ? 0.f : pr;
+                }
             }
         }
     }
-    half_t* ap = agg + ((size_t)b * kvh + g) * scores_stride + j0;
-    if (full && ((scores_stride & 7) == 0)) {
-        Pack16 o;
+    if (j0 >= scores_stride) return;
+    Pack16 o;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o.h[e] = (j0 + e < len) ? (half_t)sum[e] : (half_t)0.f;
-        *reinterpret_cast<uint4_t*>(ap) = o.u;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (j0 + e < scores_stride) ap[e] = (j0 + e < len) ? (half_t)sum[e] : (half_t)0.f;
-    }
+    for (int e = 0; e < 8; ++e) o.h[e] = (j0 + e < len) ? (half_t)sum[e] : (half_t)0.f;
+    *reinterpret_cast<uint4_t*>(ap) = o.u;
 }
 
 }  // namespace

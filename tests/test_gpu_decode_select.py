@@ -236,3 +236,39 @@ def test_scores_beyond_the_codes_range_in_one_call(cuda, H, G, L):
     native = _lib.native()
     _, idx = native.hf_decode_anchor(native.Counters(), q, k, k, False, k_sel, torch.arange(G, device=cuda, dtype=torch.int32))
     assert torch.equal(idx, want)
+
+
+@pytest.mark.parametrize("H,G,lens,ns", [(5, 1, [1], 1), (28, 4, [2047, 9], 3), (8, 8, [2048, 2049], 2), (16, 1, [2056, 1], 65),
+                                         (40, 4, [6145, 2048, 4097], 70), (32, 8, [4096, 700], 64), (9, 1, [333], 5)])
+@pytest.mark.parametrize("layer", [0, 1])
+def test_pooling_launch_follows_the_scores_it_is_given(cuda, H, G, lens, ns, layer):
+    """The pooled scores of an anchor pass from the 16-bit codes in its scratch and its log-sums: groups of 1 to 16 heads
+    (not only multiples of the four that are requested together), lengths at the edges of a workgroup's 2048 tokens, more
+    and fewer splits than a wavefront has lanes.  In float64; an fp32 sum of up to 16 exponentials whose arguments are
+    below 32 in size is off by less than 2^-18, so one step of fp16 covers rounding and ties."""
+    from kascade_amd import kernels
+    D, page = 128, 16
+    gen = torch.Generator().manual_seed(H + lens[0])
+    B, L = len(lens), max(lens)
+    pages, stride = math.ceil(L / page), (L + 7) // 8 * 8 + 2048
+    q = torch.randn(B, H, D, generator=gen).half().to(cuda)
+    kp = torch.randn(B * pages, page, G, D, generator=gen).half().to(cuda)
+    bt = torch.randperm(B * pages, generator=gen).to(torch.int32).view(B, pages).to(cuda)
+    seq = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    glse, part = torch.empty(B, H, ns, device=cuda), torch.empty(B, H, ns, D, device=cuda)
+    sums, scores = torch.empty(B, H, device=cuda), torch.empty(B, H, stride, device=cuda)
+    _, agg = kernels.decode_recompute(q, kp, kp, glse, part, sums, scores, layer, cache_seqlens=seq, block_table=bt,
+                                      page_size=page, kv_len=L)
+    torch.cuda.synchronize()
+    agg = agg.cpu()
+    codes = scores.cpu().view(torch.int16).view(B, H, 2 * stride)[..., :stride].to(torch.int32) & 0xFFFF
+    refs = scores.cpu()[..., stride // 2:].double()
+    total = torch.logsumexp(glse.cpu().double() * math.log(2.0), -1) / math.log(2.0)
+    assert float((sums.cpu().double() - total).abs().max()) < 1e-5
+    for b, n in enumerate(lens):
+        ref = refs[b, :, :(n + 63) // 64].repeat_interleave(64, -1)[:, :n]
+        p = torch.exp2(ref - codes[b, :, :n].double() / 2048.0 - total[b, :, None])
+        want = p.view(G, H // G, n).sum(1)
+        step = torch.clamp(want, min=2.0 ** -14) * 2.0 ** -10
+        assert bool(((agg[b, :, :n].double() - want).abs() <= step).all())
+        assert not bool(agg[b, :, n:].any())
