@@ -808,6 +808,9 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
 // device-coherent atomics, stores and loads.  With thousands of rows (prefill) the counter's
 // round trip at the end of every workgroup costs more than the launches, so the scans stay
 // kernels of their own.
+// Bound by dependent trips to memory and the counters' turns in LDS, not by bytes.  32 rows of 131072 to 524288 entries:
+// coarse pass 26.2 -> 19.9 us with the row's loads in front of its length and behind no branch and a bin's copies side by
+// side, fine pass 21.8 -> 18.2 with the same loads, four copies and the scan's sums by DPP instead of LDS exchanges.
 // --------------------------------------------------------------------------
 constexpr int kSplitU = 4;
 constexpr int kSplitChunk = kSplitU * kChunk;   // 32768 entries per workgroup
@@ -840,12 +843,28 @@ __device__ __forceinline__ void row_params(const int* valid_len, const int* n_se
 }
 
 // The chunk [c0, c1) of a row as order keys: thread t holds entries c0 + u*8192 + 8t .. +8 for
-// u = 0..kSplitU-1 (every load instruction covers consecutive 16-byte pieces).
+// u = 0..kSplitU-1 (every load instruction covers consecutive 16-byte pieces).  Where no piece crosses the chunk's end the
+// loads stand behind no branch (pieces past the end take the last one again): under a branch each waited for the one before.
 __device__ __forceinline__ void load_chunk(const uint16_t* __restrict__ src, bool aligned, int c0, int c1,
                                            uint32_t (&keys)[kSplitU][8], int (&nv)[kSplitU]) {
+    const int first = c0 + (int)threadIdx.x * 8;
+    if (aligned && c1 >= 8 && (c1 & 7) == 0) {   // uniform (a chunk behind the row's end has c1 < c0: nothing is taken)
+        uint4_t v[kSplitU];
+#pragma unroll
+        for (int u = 0; u < kSplitU; ++u) {
+            v[u] = ld_global_16(src + min(first + u * kChunk, c1 - 8));
+            nv[u] = first + u * kChunk < c1 ? 8 : 0;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < kSplitU; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) keys[u][e] = order_key((uint16_t)(v[u][e >> 1] >> (16 * (e & 1))));
+        return;
+    }
 #pragma unroll
     for (int u = 0; u < kSplitU; ++u) {
-        const int base = c0 + u * kChunk + (int)threadIdx.x * 8;
+        const int base = first + u * kChunk;
         nv[u] = 0;
         if (base < c1) nv[u] = load_keys(src, aligned, base, c1, keys[u]);
     }
@@ -892,11 +911,21 @@ template <bool FUSED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void topk_split_hist1_kernel(
     const uint16_t* __restrict__ scores, long long row_stride, int uniform_len,
     const int* __restrict__ valid_len, const int* __restrict__ n_sel, int period, int k, SplitWs ws) {
-    __shared__ uint32_t s_hist[kHistCopies][kBins1];
+    // a bin's copies lie side by side: in one bank each, lanes that count in the same bin took turns whatever their copy
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist[kBins1][kHistCopies];
     __shared__ uint32_t s_wave[kWaves];
     __shared__ int s_flag;
+    static_assert(kHistCopies == 4, "a bin is 16 bytes");
     const int tid = threadIdx.x;
     const long long row = blockIdx.y;
+    const int c0 = blockIdx.x * kSplitChunk;
+    if (c0 >= uniform_len) return;
+    // requested for the row's full width before its length has arrived, cut down below
+    const uint16_t* src = scores + row * row_stride;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(src) & 15) == 0);
+    uint32_t keys[kSplitU][8];
+    int nv[kSplitU];
+    load_chunk(src, aligned, c0, min(uniform_len, c0 + kSplitChunk), keys, nv);
     int len, n;
     row_params(valid_len, n_sel, period, uniform_len, k, row, len, n);
     uint32_t* sel = ws.sel + row * kSelWords;
@@ -904,27 +933,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
         if (FUSED && blockIdx.x == 0 && tid == 0) { sel[0] = 0; sel[5] = (uint32_t)n; sel[6] = (uint32_t)len; }
         return;
     }
-    const int c0 = blockIdx.x * kSplitChunk;
     if (c0 >= len) return;
     const int c1 = min(len, c0 + kSplitChunk);
-    const uint16_t* src = scores + row * row_stride;
-    const bool aligned = ((reinterpret_cast<uintptr_t>(src) & 15) == 0);
-    uint32_t keys[kSplitU][8];
-    int nv[kSplitU];
-    load_chunk(src, aligned, c0, c1, keys, nv);
-    for (int i = tid; i < kHistCopies * kBins1; i += kThreads) (&s_hist[0][0])[i] = 0;
+#pragma unroll
+    for (int u = 0; u < kSplitU; ++u) nv[u] = max(0, min(nv[u], len - (c0 + u * kChunk + tid * 8)));
+    for (int i = tid; i < kBins1; i += kThreads) *reinterpret_cast<uint4_t*>(s_hist[i]) = uint4_t{0, 0, 0, 0};
     __syncthreads();
     // +0 (pooled probabilities underflow to it by the thousand) is not counted: its number is
     // the chunk's length minus the sum of the others.  The other entries go to one of four
     // copies of the histogram, chosen by the lane, which spreads the crowded bins.
-    uint32_t* mine = s_hist[tid & (kHistCopies - 1)];
+    uint32_t* mine = &s_hist[0][tid & (kHistCopies - 1)];
     uint32_t counted = 0;
 #pragma unroll
     for (int u = 0; u < kSplitU; ++u)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             if (e < nv[u] && keys[u][e] != 0x8000u) {
-                atomicAdd(&mine[keys[u][e] >> 5], 1u);
+                atomicAdd(&mine[(keys[u][e] >> 5) * kHistCopies], 1u);
                 ++counted;
             }
 #pragma unroll
@@ -933,9 +958,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
     __syncthreads();
     uint32_t* gh = ws.hist1 + row * kBins1;
     for (int i = tid; i < kBins1; i += kThreads) {
-        uint32_t c = 0;
-#pragma unroll
-        for (int j = 0; j < kHistCopies; ++j) c += s_hist[j][i];
+        const uint4_t h = *reinterpret_cast<const uint4_t*>(s_hist[i]);
+        uint32_t c = h[0] + h[1] + h[2] + h[3];
         if (i == (int)(0x8000u >> 5)) {
             uint32_t all = 0;
 #pragma unroll
@@ -982,18 +1006,17 @@ __device__ __forceinline__ void split_scan2(uint32_t* sel, const uint32_t* rinfo
         }
     }
 #pragma unroll
-    for (int j = 0; j < 32; ++j)
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) h[j] += __shfl_xor(h[j], o);
+    for (int j = 0; j < 32; ++j) h[j] = wave_incl_scan(h[j]);   // the sum in the last lane
     // the fine bin of the n-th largest entry, from the top (bin 0 takes whatever is left)
     uint32_t above = sel[2];
     int b2 = 0;
     bool found = false;
 #pragma unroll
     for (int j = 31; j >= 1; --j) {
+        const uint32_t hj = (uint32_t)__builtin_amdgcn_readlane((int)h[j], 63);
         if (!found) {
-            if (above + h[j] >= n) { found = true; b2 = j; }
-            else above += h[j];
+            if (above + hj >= n) { found = true; b2 = j; }
+            else above += hj;
         }
     }
     const uint32_t r = n - above;
@@ -1025,7 +1048,7 @@ __device__ __forceinline__ void split_scan2(uint32_t* sel, const uint32_t* rinfo
 template <bool FUSED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void topk_split_hist2_kernel(
     const uint16_t* __restrict__ scores, long long row_stride, int uniform_len, int max_chunks, SplitWs ws) {
-    __shared__ uint32_t s_hist2[32];
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist2[32][kHistCopies];
     __shared__ uint32_t s_gt1;
     __shared__ int s_flag;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1043,9 +1066,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
     const uint32_t b1 = sel[1];
 #pragma unroll
     for (int u = 0; u < kSplitU; ++u) nv[u] = max(0, min(nv[u], len - (c0 + u * kChunk + tid * 8)));
-    if (tid < 32) s_hist2[tid] = 0;
+    if (tid < 32) *reinterpret_cast<uint4_t*>(s_hist2[tid]) = uint4_t{0, 0, 0, 0};
     if (tid == 32) s_gt1 = 0;
     __syncthreads();
+    uint32_t* mine = &s_hist2[0][tid & (kHistCopies - 1)];
     uint32_t gt1 = 0, zeros = 0;
     const bool zero_bin = b1 == (0x8000u >> 5);   // uniform: the threshold lies among +0 and the smallest subnormals
 #pragma unroll
@@ -1057,19 +1081,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
             if (zero_bin) {   // that many atomics on one address would serialise: a ballot per wavefront
                 const bool zero = in && keys[u][e] == 0x8000u;
                 zeros += (uint32_t)__popcll(__ballot(zero));
-                if (in && !zero && hb == b1) atomicAdd(&s_hist2[keys[u][e] & 31u], 1u);
+                if (in && !zero && hb == b1) atomicAdd(&mine[(keys[u][e] & 31u) * kHistCopies], 1u);
             } else if (in && hb == b1) {
-                atomicAdd(&s_hist2[keys[u][e] & 31u], 1u);
+                atomicAdd(&mine[(keys[u][e] & 31u) * kHistCopies], 1u);
             }
             gt1 += (in && hb > b1);
         }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) gt1 += __shfl_xor(gt1, o);
     if (lane == 0 && gt1) atomicAdd(&s_gt1, gt1);
-    if (lane == 0 && zeros) atomicAdd(&s_hist2[0], zeros);   // +0 is entry 0 of its bin
+    if (lane == 0 && zeros) atomicAdd(&s_hist2[0][0], zeros);   // +0 is entry 0 of its bin
     __syncthreads();
     uint32_t* info = ws.cinfo + (row * max_chunks + blockIdx.x) * kInfoWords;
-    if (tid < 32) store_device_u32(info + tid, s_hist2[tid]);
+    if (tid < 32) {
+        const uint4_t h = *reinterpret_cast<const uint4_t*>(s_hist2[tid]);
+        store_device_u32(info + tid, h[0] + h[1] + h[2] + h[3]);
+    }
     if (tid == 32) store_device_u32(info + 32, s_gt1);
     if (!FUSED) return;
     const int nchunks = (len + kSplitChunk - 1) / kSplitChunk;

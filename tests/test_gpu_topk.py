@@ -202,3 +202,33 @@ def test_topk_second_output_as_cache_rows(cuda, L, k, rows_per_seq):
                                          block_table=bt, page_size=page)
         assert torch.equal(got, want)
         assert torch.equal(rows, kernels.translate_indices(want, bt, Lv, page))
+
+
+@pytest.mark.parametrize("L", [131073, 131080, 163840, 163841, 163848])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rows_over_several_workgroups_at_the_edges_of_chunks(cuda, L, offset):
+    """Rows that end inside, at and just behind a chunk of 32768 entries or a piece of 8, lengths from one entry to all of
+    them, most scores in a few subnormal bins (as pooled probabilities of long rows are), aligned rows and not: the same
+    lists as the streaming kernel's, whose code is separate."""
+    from kascade_amd import kernels, _lib
+    gen = torch.Generator().manual_seed(L)
+    K, valid = 4224, [L, L - 1, 131072, 98305, 65536, 32769, 32768, 4225, 4224, 1]
+    rows, stride = len(valid), (L + 15) // 8 * 8
+    sc = torch.full((rows, stride), float("inf"), dtype=torch.float16)       # nothing past a row's length may enter
+    tiny = torch.randint(0, 200, (rows, L), generator=gen).to(torch.int16)   # bit patterns: multiples of 2^-24
+    tiny[3] = torch.randint(0, 3, (L,), generator=gen).to(torch.int16)       # the threshold lies among +0 or beside it
+    tiny[4] = 7                                                              # one value everywhere
+    sc[:, offset:offset + L] = tiny.view(torch.float16)
+    for r, n in enumerate(valid):
+        sc[r, offset + n:] = float("inf")
+    nsel = torch.tensor([4224, 4223, 1, 4224, 4224, 128, 4224, 4224, 4224, 4224], dtype=torch.int32).to(cuda)
+    d, dvalid = sc.to(cuda)[:, offset:offset + L], torch.tensor(valid, dtype=torch.int32).to(cuda)
+    got = kernels.topk_indices(d, K, valid_len=dvalid, n_sel=nsel, fill_value=-1)
+    lib = _lib.init()
+    assert lib.kascade_topk_workspace_bytes(rows, L) > 0
+    want = torch.empty(rows, K, dtype=torch.int32, device=cuda)
+    _lib.check(lib.kascade_topk_call(d.data_ptr(), want.data_ptr(), rows, stride, L, dvalid.data_ptr(), nsel.data_ptr(), rows,
+                                     K, -1, None, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want.cpu())
+    _check(sc[:, offset:offset + L], got.cpu(), lambda r: nsel[r], lambda r: valid[r], K, -1)
