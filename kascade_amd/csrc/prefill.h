@@ -43,7 +43,7 @@ struct PrefillParams {
     int elem;                 // kElemF16 or kElemBF16
     int gs;                   // query heads per KV head: 1 to 16 (0 = 4)
     int key_parts, part_tiles;   // pooling kernel: parts of part_tiles key tiles a query tile's keys are cut into
-    int vsub, accumulate;     // pooling kernel: sub-group of this launch; add to what agg holds
+    int vsub;                 // pooling kernel: sub-group of this launch; those after the first add to what agg holds
 };
 
 // Query heads per KV head and the sub-groups of four head slots they take.

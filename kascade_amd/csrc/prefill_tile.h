@@ -84,9 +84,11 @@ __device__ __forceinline__ void unit_of_workgroup(int B, int G, int nblocks, int
 __device__ __forceinline__ void chunk_of_sequence(const PrefillParams& p, int b, int& q_start, int& rows) {
     q_start = p.q_start;
     rows = p.Lq;
-    if (p.q_start_rows) {
-        q_start = max(0, min(p.q_start_rows[b], p.q_start)) & ~(kTile - 1);
-        if (p.q_len_rows) rows = max(0, min(p.q_len_rows[b], p.Lq));
+    if (p.q_start_rows) {   // scalar loads: as vector loads they would make every position and address that follows per lane
+        typedef const __attribute__((address_space(4))) int* ConstantPtr;
+        b = __builtin_amdgcn_readfirstlane(b);
+        q_start = max(0, min(((ConstantPtr)p.q_start_rows)[b], p.q_start)) & ~(kTile - 1);
+        if (p.q_len_rows) rows = max(0, min(((ConstantPtr)p.q_len_rows)[b], p.Lq));
     }
 }
 

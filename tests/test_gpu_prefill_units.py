@@ -267,3 +267,33 @@ def test_spare_head_slots_change_no_head(cuda, gs, G, D, L):
     hm = torch.arange(G, dtype=torch.int32, device=cuda).flip(0)
     assert torch.equal(kernels.prefill_reuse(q, k, v, idx, hm, 10.0, True),
                        real(kernels.prefill_reuse(qf, k, v, idx, hm, 10.0, True)))
+
+
+@pytest.mark.parametrize("gs", [5, 8, 11, 16])
+@pytest.mark.parametrize("G,D,L", [(8, 128, 161), (4, 64, 417), (3, 128, 1030), (1, 64, 129)])
+def test_pooled_scores_add_up_over_the_sub_groups(cuda, gs, G, D, L):
+    """Query heads are pooled four at a time and later launches add to the scores of the earlier ones.  Against launches
+    over each sub-group alone: rounded to fp16 once per sub-group in either form, so half a step of a part, of the sum up
+    to it and of the whole for every sub-group after the first (a step: 2^-10 of the value, 2^-24 at least)."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(gs + L)
+    q = torch.randn(2, L, G, gs, D, generator=gen).half().to(cuda)
+    k, v = (torch.randn(2, L, G, D, generator=gen).half().to(cuda) for _ in range(2))
+    ls, _ = kernels.prefill_recompute0(q.flatten(2, 3).contiguous(), k, v)
+    parts = ls.unflatten(2, (G, gs))
+    T = (L + 31) // 32
+
+    def pooled(h0, h1):
+        sc = torch.full((2, G, T, L), 7.0, device=cuda, dtype=torch.float16)   # what a buffer holds before does not count
+        kernels.prefill_aggregate(q[:, :, :, h0:h1].flatten(2, 3).contiguous(), k,
+                                  parts[:, :, :, h0:h1].flatten(2, 3).contiguous(), sc, fill_invalid=True)
+        return sc.double()
+    got = pooled(0, gs)
+    want, slack = torch.zeros_like(got), torch.zeros_like(got)
+    for h0 in range(0, gs, 4):
+        part = pooled(h0, min(h0 + 4, gs))
+        want = want + part
+        slack = slack + (part.abs() + want.abs() + got.abs()) * 2.0 ** -11 + 2.0 ** -24
+    inside = torch.isfinite(got)
+    assert torch.equal(inside, torch.isfinite(want)) and bool(inside.any())
+    assert bool(((got - want).abs()[inside] <= slack[inside]).all())
