@@ -955,14 +955,6 @@ void prefill_attn_kernel_q32(PrefillParams p) {
     else prefill_dense_body<1, WITH_V, PAGED, D, T, SPARE>(p, sK, sV);
 }
 
-// The same for log-sums alone with head slots that no query head fills.
-template <bool PAGED, int D, typename T>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
-void prefill_attn_kernel_q32_spare_log_sums(PrefillParams p) {
-    __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
-    prefill_dense_body<1, false, PAGED, D, T, true>(p, sK, static_cast<T*>(nullptr));
-}
-
 // 64 queries per wavefront for the K-only log-sum pass, whose state fits 256 registers: two
 // workgroups per compute unit, and the MFMA results stay in ordinary registers (with the full
 // 512-register budget the compiler parks them in accumulation registers and copies each one out
@@ -1254,10 +1246,8 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         } else if (with_v) {
             hipLaunchKernelGGL((prefill_attn_kernel_q32<false, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
-        } else if constexpr (kSpare) {
-            hipLaunchKernelGGL((prefill_attn_kernel_q32_spare_log_sums<kPaged, D, T>), grid, block, 0, stream, p);
         } else {
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, kPaged, D, T, false>), grid, block, 0, stream, p);
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<false, false, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         }
         return hipSuccess;
     };
