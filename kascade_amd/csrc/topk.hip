@@ -277,8 +277,9 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(
 //  * The selected positions are staged in LDS in their final order, so that the list leaves as
 //    full-width stores.
 // Causal prompt tiles (8 heads x L/32 rows, ragged), against one size of workgroup with a scan over all
-// (chunk, wavefront) pairs: L = 4096 18.6 -> 9.4 us, 8192 34.6 -> 20.5, 16384 73.6 -> 48.8, 32768 179 -> 150,
-// 65536 907 -> 587 us; 2048 full rows of 65536: 175 -> 143 us = 1.9 TB/s.
+// (chunk, wavefront) pairs: L = 4096 18.6 -> 9.4 us, 8192 34.6 -> 20.5, 16384 73.6 -> 48.1, 32768 179 -> 142,
+// 65536 907 -> 546 us; 2048 full rows of 65536: 175 -> 130 us = 2.1 TB/s, of 131072 341 us (145 and 369 while 16 chunks
+// spilled nine registers where the keys are formed).
 // One row on one compute unit (decode anchors, pooling included, 16384 tokens of 4 heads): 13.4 -> 12.3 us with the log-sums'
 // parts requested before the length is known, the histograms cleared under the row's loads, counters addressed by the key's
 // bits in place, and the codes kept.
@@ -616,6 +617,7 @@ void topk_select_reg_kernel(
                 uint32_t key = pk_max_u16(raw ^ (pk_sign_mask_i16(raw) | 0x80008000u), kOne);
                 key = s0 < tail ? key : (at_tail && s0 == tail) ? end_w[1][j] : 0u;
                 if (c == 0) key = at_front ? end_w[0][j] : key;
+                asm volatile("" : "+v"(key));   // chosen here: sunk below the later chunks' branches, both sides of the choices would stay live
                 data[c][j] = key;
             }
         }
