@@ -812,7 +812,8 @@ void decode_pool_select_kernel(DecodePoolParams p, int k, int fill, int* __restr
 // kernels of their own.
 // Bound by dependent trips to memory and the counters' turns in LDS, not by bytes.  32 rows of 131072 to 524288 entries:
 // coarse pass 26.2 -> 19.9 us with the row's loads in front of its length and behind no branch and a bin's copies side by
-// side, fine pass 21.8 -> 18.2 with the same loads, four copies and the scan's sums by DPP instead of LDS exchanges.
+// side, fine pass 21.8 -> 18.2 with the same loads and four copies.  Its scan with a lane per bin, instead of every bin's
+// sum over 64 lanes, spills nothing (12 bytes of scratch before): the whole selection 53.7 -> 51.5 us.
 // --------------------------------------------------------------------------
 constexpr int kSplitU = 4;
 constexpr int kSplitChunk = kSplitU * kChunk;   // 32768 entries per workgroup
@@ -992,36 +993,27 @@ __global__ __launch_bounds__(kThreads) void topk_split_scan1_kernel(
 }
 
 // From the chunks' fine histograms of a row: the threshold key T, the number r of entries equal
-// to T that still fit, and every chunk's offsets into the output.  One wavefront, lane c for
-// chunk c (64 chunks per round).
+// to T that still fit, and every chunk's offsets into the output.  One wavefront: lane l sums fine bin
+// 31 - l % 32 over every other chunk, then lane c takes chunk c (64 chunks per round).
 __device__ __forceinline__ void split_scan2(uint32_t* sel, const uint32_t* rinfo, uint32_t* off, int nchunks) {
     const int lane = threadIdx.x & 63;
     const uint32_t n = sel[5], b1 = sel[1];
-    uint32_t h[32];
+    const uint32_t* bin = rinfo + (31 - (lane & 31));
+    uint32_t h = 0;
+    for (int c0 = lane >> 5; c0 < nchunks; c0 += 16) {   // eight loads on their way (past the last chunk: that one again)
+        uint32_t v[8];
 #pragma unroll
-    for (int j = 0; j < 32; ++j) h[j] = 0;
-    for (int cb = 0; cb < nchunks; cb += 64) {
-        const int c = cb + lane;
-        if (c < nchunks) {
+        for (int u = 0; u < 8; ++u) v[u] = load_device_u32(bin + min(c0 + 2 * u, nchunks - 1) * kInfoWords);
 #pragma unroll
-            for (int j = 0; j < 32; ++j) h[j] += load_device_u32(rinfo + c * kInfoWords + j);
-        }
+        for (int u = 0; u < 8; ++u) h += c0 + 2 * u < nchunks ? v[u] : 0u;
     }
-#pragma unroll
-    for (int j = 0; j < 32; ++j) h[j] = wave_incl_scan(h[j]);   // the sum in the last lane
+    h += (uint32_t)__shfl_xor((int)h, 32);
     // the fine bin of the n-th largest entry, from the top (bin 0 takes whatever is left)
-    uint32_t above = sel[2];
-    int b2 = 0;
-    bool found = false;
-#pragma unroll
-    for (int j = 31; j >= 1; --j) {
-        const uint32_t hj = (uint32_t)__builtin_amdgcn_readlane((int)h[j], 63);
-        if (!found) {
-            if (above + hj >= n) { found = true; b2 = j; }
-            else above += hj;
-        }
-    }
-    const uint32_t r = n - above;
+    const uint32_t incl = wave_incl_scan(lane < 32 ? h : 0u);
+    const uint32_t base = sel[2];
+    const int first = __ffsll((unsigned long long)__ballot(lane == 31 || (lane < 31 && base + incl >= n))) - 1;
+    const int b2 = 31 - first;
+    const uint32_t r = n - (base + (uint32_t)__builtin_amdgcn_readlane((int)(incl - h), first));
     if (lane == 0) { sel[3] = (b1 << 5) | (uint32_t)b2; sel[4] = r; }
     // per-chunk counts of entries above T and equal to T, and their exclusive prefixes
     uint32_t gt_run = 0, eq_run = 0;

@@ -232,3 +232,26 @@ def test_rows_over_several_workgroups_at_the_edges_of_chunks(cuda, L, offset):
     torch.cuda.synchronize()
     assert torch.equal(got.cpu(), want.cpu())
     _check(sc[:, offset:offset + L], got.cpu(), lambda r: nsel[r], lambda r: valid[r], K, -1)
+
+
+@pytest.mark.parametrize("rows,chunks", [(3, 5), (3, 15), (3, 16), (2, 17), (2, 18), (2, 33), (1, 66), (130, 17)])
+def test_threshold_over_the_chunks_of_a_row(cuda, rows, chunks):
+    """The threshold's fine bin is summed over a row's chunks of 32768 entries, sixteen at a time by two lanes a bin: rows
+    around one and two such turns and beyond 64 chunks, in one pass with the scan and (130 rows) with a launch of its own.
+    The same lists as the streaming kernel's."""
+    from kascade_amd import kernels, _lib
+    L = chunks * 32768 - 5
+    gen = torch.Generator(device="cuda").manual_seed(chunks)
+    sc = torch.rand(rows, L, device=cuda, generator=gen).pow_(8).half()
+    sc[0] = torch.randint(0, 40, (L,), device=cuda, generator=gen).to(torch.int16).view(torch.float16)   # subnormals, many ties
+    k = 4224 if rows > 3 else L // 10 // 128 * 128
+    got = kernels.topk_indices(sc, k)
+    lib = _lib.init()
+    assert lib.kascade_topk_workspace_bytes(rows, L) > 0
+    want = torch.empty(rows, k, dtype=torch.int32, device=cuda)
+    _lib.check(lib.kascade_topk_call(sc.data_ptr(), want.data_ptr(), rows, L, L, None, None, 1, k, -1, None,
+                                     torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(got, want)
+    largest = sc[0].float().sort(descending=True).values[:k]
+    assert torch.equal(sc[0][got[0].long()].float().sort(descending=True).values, largest)
+    assert bool((got[:, 1:] > got[:, :-1]).all())

@@ -16,9 +16,9 @@ def selection(tmp_path_factory):
     return re.findall(r"\.name: +(_Z\S+)\n.*?\.private_segment_fixed_size: (\d+)", out.read_text(), re.S)
 
 
-@pytest.mark.parametrize("kernel,instances", [("topk_select_reg_kernel", 9), ("decode_pool_select_kernel", 5)])
+@pytest.mark.parametrize("kernel,instances", [("topk_select_reg_kernel", 9), ("decode_pool_select_kernel", 5), ("topk_split_", 7)])
 def test_selection_keeps_its_row_in_registers(selection, kernel, instances):
-    """None of them uses scratch, up to 16 chunks of 8 entries a thread."""
+    """None of them uses scratch, up to 16 chunks of 8 entries a thread; nor do the passes over long rows' chunks."""
     found = [(name, scratch) for name, scratch in selection if kernel in name]
     assert len(found) == instances
     assert all(scratch == "0" for _, scratch in found), found
