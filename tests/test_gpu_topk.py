@@ -255,3 +255,30 @@ def test_threshold_over_the_chunks_of_a_row(cuda, rows, chunks):
     largest = sc[0].float().sort(descending=True).values[:k]
     assert torch.equal(sc[0][got[0].long()].float().sort(descending=True).values, largest)
     assert bool((got[:, 1:] > got[:, :-1]).all())
+
+
+@pytest.mark.parametrize("L", [131073, 163840, 163848])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_many_short_rows_in_wide_tensors(cuda, L, offset):
+    """The first tiles of a long prompt: thousands of workgroups, whose coarse pass reads only what a row holds.  Lengths at
+    the edges of pieces of 8 entries and chunks of 32768, aligned rows and not, infinities behind every row's end: the same
+    lists as the streaming kernel's."""
+    from kascade_amd import kernels, _lib
+    lens, K, copies = [0, 1, 7, 8, 9, 255, 4097, 32767, 32768, 32769, 65535, L - 1, L], 256, 32
+    rows, stride = len(lens) * copies, (L + 15) // 8 * 8
+    gen = torch.Generator(device="cuda").manual_seed(L)
+    base = torch.full((rows, stride), float("inf"), dtype=torch.float16, device=cuda)
+    d = base[:, offset:offset + L]
+    for r in range(rows):
+        n = lens[r % len(lens)]
+        d[r, :n] = torch.rand(n, device=cuda, generator=gen).pow_(8).half()
+    valid = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    nsel = torch.tensor([4, 1, 3, 0, 9, 32, 256, 256, 1, 255, 256, 17, 256], dtype=torch.int32, device=cuda)
+    got = kernels.topk_indices(d, K, valid_len=valid, n_sel=nsel, fill_value=-1)
+    lib = _lib.init()
+    assert lib.kascade_topk_workspace_bytes(rows, L) > 0 and rows * (-(-L // 32768)) > 2048   # passes and scans apart
+    want = torch.empty(rows, K, dtype=torch.int32, device=cuda)
+    _lib.check(lib.kascade_topk_call(d.data_ptr(), want.data_ptr(), rows, stride, L, valid.data_ptr(), nsel.data_ptr(),
+                                     len(lens), K, -1, None, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(got, want)
+    _check(d.cpu()[:len(lens)], got.cpu()[:len(lens)], lambda r: nsel[r], lambda r: valid[r], K, -1)
