@@ -80,7 +80,8 @@ template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
 // SPARE: the KV head's last sub-group may have fewer than four query heads (gs no multiple of four).  Its wavefronts
 // without a head only stage their rows of every tile, which leaves the matrix unit and the power to the others: 28/4
 // heads bf16, two prompts of 3001 tokens, eight layers with pooling over the heads there are 780 -> 737 us.  A variant of its own, because
-// the second loop costs the allocation of the first (32/8 heads, 517 tokens 119.2 -> 120.4 us).  Rotating the slots over
+// the second loop costs the allocation of the first (32/8 heads, 517 tokens 119.2 -> 120.4 us; with log-sums, 32768
+// tokens, 945 against 958 us).  Rotating the slots over
 // the wavefronts, so that the idle one is not always the same SIMD's, gave nothing.
 // EXACT_SUM: the softmax denominators are summed in fp32 from the unrounded exponentials (the
 // passes whose log-sum is an output); otherwise units sum them as they enter the second product.
@@ -1240,8 +1241,8 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
         if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
             if constexpr (D == 128) hipLaunchKernelGGL((prefill_attn_kernel_q64<kPaged, D, T, kSpare>), grid, block, 0, stream, p);
             else return hipErrorInvalidValue;
-        } else if (reuse && p.log_sum) {   // a reuse pass that also reports its log-sums: fp32 sums, any group
-            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, true, true>), grid, block, 0, stream, p);
+        } else if (reuse && p.log_sum) {   // a reuse pass that also reports its log-sums: fp32 sums
+            hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare, true>), grid, block, 0, stream, p);
         } else if (reuse) {
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         } else if (with_v) {

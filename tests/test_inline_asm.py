@@ -56,3 +56,11 @@ def test_log_sum_units_of_32_queries_fit_four_to_a_compute_unit(assembly):
                          r".*?\.vgpr_count: +(\d+)", assembly, re.S)
     assert len(kernels) == 16
     assert all(int(vgprs) <= 128 and scratch == "0" for _, scratch, vgprs in kernels), kernels
+
+
+def test_whole_groups_run_no_kernel_for_spare_head_slots(assembly):
+    """Every attention kernel is there with and without head slots that no query head fills: the second loop of the
+    former costs groups that fill whole four slots its registers, in passes that report log-sums too."""
+    found = re.findall(r"\.name: +\S+prefill_attn_kernel_q(32ILb\dELb\dE|64I)Lb(\d)ELi(\d+)E(DF16_|DF16b)Lb(\d)E(Lb\dE)?E", assembly)
+    whole, spare = ({(a, b, c, d, f) for a, b, c, d, s, f in found if s == slot} for slot in "01")
+    assert whole == spare and len(whole) == 36
