@@ -569,32 +569,37 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
 // counter and the way back, the more the more query heads and workgroups there are.  Us per launch in a
 // captured graph, one split / as many as kascade_decode_num_split gives, 8 KV heads:
 //   rows   batch    1 head      2           4           5           7           8           16 heads per KV head
-//   256    1        6.0/7.2     6.1/7.2     6.2/7.7     6.5/8.8     6.6/9.2     6.8/9.3     7.8/13.1
-//   384    1        7.3/7.2     7.5/7.4     7.7/7.8     7.9/8.8     8.1/9.2     8.2/9.5     9.2/13.2
-//   384    4        7.8/7.6     7.9/7.7     8.1/8.2     8.3/9.4     8.6/10.0    8.6/10.1    9.6/13.9
-//   384    8        8.2/8.3     8.3/8.4     8.4/8.8     8.7/10.1    8.8/10.5    8.9/10.7    9.8/14.5
-//   512    1                                            9.2/9.0     9.5/9.5     9.5/9.6     10.5/13.4
-//   512    2                                            9.3/9.7     9.7/10.1    9.7/10.2    10.7/14.0
-//   512    8                                            10.1/10.5   10.3/11.0   10.4/11.0   11.4/15.0
-// (4 heads, 512 rows: 9.5/8.5 at batch 1, 11.0/10.5 at 8; with 2 or 4 KV heads one split of 384 rows is up to
-// 6 % behind for 1 and 2 heads, one of 512 up to 5 % for 5 to 7, from 64 and 16 lists on level.)
+//   256    1        5.5/6.7     5.5/6.7     5.6/6.9     6.0/7.8     6.1/8.1     6.1/8.1     7.3/11.2
+//   384    1        6.8/6.6     6.9/6.8     7.0/7.1     7.4/7.9     7.5/8.1     7.6/8.3     8.6/11.4
+//   384    4        7.0/7.1     7.1/7.2     7.3/7.4     7.6/8.2     7.7/8.5     7.8/8.6     8.7/11.8
+//   384    8        7.5/7.5     7.5/7.5     7.7/7.7     7.9/8.7     8.1/9.0     8.1/9.0     9.1/12.2
+//   512    1        7.9/6.9     8.1/6.7     8.2/6.9     8.5/7.9     8.6/8.2     8.8/8.4     9.8/11.5
+//   512    2        8.0/7.1     8.2/7.2     8.3/7.2     8.6/8.4     8.8/8.6     8.8/8.7     9.8/11.8
+//   512    8        9.1/8.0     9.2/8.0     9.3/8.2     9.6/9.2     9.7/9.5     9.7/9.6     10.7/12.8
+// (At 512 rows one split is up to 5 % behind for 5 to 8 heads; the lists' sums would be split otherwise for that.)
 int kascade_gather_lone_rows(int group_size, int lists) {
     if (group_size <= 2) return lists >= 64 ? 384 : 256;
     return group_size >= 8 || (group_size >= 5 && lists >= 16) ? 512 : 384;
 }
 
 // One workgroup pools a row's tokens for all query heads of its KV head, four heads at a time, where a
-// launch of its own spreads them over the chip: the saved launch (2 to 4 us) stops paying as tokens
-// and heads grow, sooner for groups that fill no whole four heads.  Us of an anchor pass without
-// output, one launch / two, 8 KV heads, batch 1:
+// launch of its own spreads them over the chip: the saved launch stops paying as tokens and heads grow.  Us of an anchor
+// pass without output in a captured graph, where a launch costs the host nothing, one launch / two, 8 KV heads, batch 1:
 //   tokens   1 head    2          4          5          8          12         16 heads per KV head
-//   8192     13.6/15.3 14.3/16.7  15.0/18.6  17.5/20.6  18.0/23.5  21.0/27.4  23.5/31.8
-//   18432    23.4/24.9 23.4/25.6  24.4/27.8  29.2/29.3  29.3/32.3  34.4/36.2  39.3/40.6
-//   20480    25.7/25.5 25.4/26.6  26.5/28.4  32.3/29.4  32.6/33.1  38.4/37.0  44.2/42.1
-//   24576    26.0/26.3 27.4/27.5  27.4/29.5  33.0/31.4  33.7/34.2  39.0/38.0  45.0/42.4
-//   32768    31.0/28.8 32.6/30.7  32.7/32.4  39.4/35.0  40.5/37.8  47.2/40.9  55.0/46.1
-// With many rows the selections fill the chip by themselves: batch 8, 24576 tokens 81.9/85.8 with 2
-// heads, 95.7/98.4 with 8, 118.5/120.6 with 16; 32768 110.6/109.0, 132.3/132.8, 166.3/165.4.
+//   8192     14.4/15.6 14.6/15.8  15.4/16.6  17.7/18.4  18.3/19.4  20.6/21.7  23.4/26.1
+//   10240    18.2/18.6 18.5/19.2  19.0/19.9  22.3/21.5  22.7/23.1  26.1/25.9  29.9/27.9
+//   14336    20.3/20.3 20.7/20.7  21.2/21.5  25.8/22.9  26.1/24.9  30.3/27.3  34.8/30.3
+//   18432    24.5/24.0 24.7/24.6  25.2/25.2  28.9/26.4  31.0/29.4  35.1/32.0  39.9/34.7
+//   20480    26.8/24.9 26.9/25.7  27.4/26.3  32.6/28.0  33.6/30.1  38.4/32.5  44.3/36.1
+//   24576    26.9/25.6 27.1/25.9  27.8/26.9  32.9/28.7  33.9/30.8  39.2/33.7  45.0/36.9
+//   32768    31.4/29.0 31.7/29.2  32.6/30.2  38.6/31.8  39.7/34.2  46.9/37.2  54.2/40.8
+// With many rows the selections fill the chip by themselves: batch 8, 24576 tokens 86.3/87.8 with 2 heads, 98.7/94.9 with 8,
+// 122.6/116.3 with 16; 32768 111.3/112.7, 136.0/129.0, 168.6/159.1.
+// The limits lie above the crossover of captured passes, for more than four heads per KV head by up to 10000 tokens: an
+// eager pass also pays the second launch's way through the host, and one over lists of lengths what makes the rows' budgets
+// for it.  With 8192 for those groups, passes over new buffers / among others: serving steps of 8 x 17000 tokens at 64/8 heads
+// 417 -> 450 us / 329 -> 329, of 4 x 12000 at 28/4 228 -> 265 / 144.5 -> 144.2; transformers cache, 17000 tokens at 64/8
+// heads 340 -> 344 / 136.3 -> 130.2.
 int kascade_pool_select_row(int group_size, int rows) {
     return group_size == 3 || group_size == 4 || rows >= 64 ? 24576 : 18432;
 }
