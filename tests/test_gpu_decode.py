@@ -736,21 +736,22 @@ def test_reuse_from_translated_rows_equals_reuse_from_token_lists(cuda, seqlens,
 @pytest.mark.parametrize("named", [True, False])
 @pytest.mark.parametrize("n,ns", [(1, 1), (128, 1), (256, 1), (257, 1), (512, 1), (513, 1), (513, 2), (2049, 1), (2560, 2)])
 @pytest.mark.parametrize("form", ["tokens", "rows", "strided"])
-def test_gather_lists_of_every_staging_with_and_without_the_newest_token(cuda, form, n, ns, named):
-    """A list is staged from registers (up to two entries per thread), or in sub-chunks of 2048; the newest token's
+@pytest.mark.parametrize("G,H,D,dtype", [(4, 12, 128, torch.float16), (2, 16, 128, torch.bfloat16), (1, 9, 128, torch.float16),
+                                         (2, 6, 64, torch.bfloat16), (2, 10, 64, torch.float16), (1, 16, 64, torch.bfloat16)])
+def test_gather_lists_of_every_staging_with_and_without_the_newest_token(cuda, G, H, D, dtype, form, n, ns, named):
+    """Groups of up to 4, 8 and 16 query heads, both head dims.  A list is staged from registers (up to two entries per thread), or in sub-chunks of 2048; the newest token's
     rows arrive beside the cache.  Against the same call on a cache that holds them: the same bits, and both caches
     are equal afterwards, whether or not the list names that token."""
     from kascade_amd import kernels
-    G, H, D, page = 4, 12, 128, 16
-    L = 2 * n + 40
+    page, L = 16, 2 * n + 40
     gen = torch.Generator().manual_seed(n)
-    q = torch.randn(1, H, D, generator=gen).half().to(cuda)
-    k, v = (torch.randn(1, L, G, D, generator=gen).half().to(cuda) for _ in range(2))
+    q = torch.randn(1, H, D, generator=gen).to(dtype).to(cuda)
+    k, v = (torch.randn(1, L, G, D, generator=gen).to(dtype).to(cuda) for _ in range(2))
     idx = torch.stack([torch.randperm(L - 1, generator=gen)[:n].sort().values for _ in range(G)])
     if named:
         idx[:, -1] = L - 1
     idx = idx[None].to(torch.int32).contiguous().to(cuda)
-    hm = torch.tensor([2, 0, 3, 1], dtype=torch.int32, device=cuda)
+    hm = torch.tensor([2, 0, 3, 1] if G == 4 else list(range(G))[::-1], dtype=torch.int32, device=cuda)
     lens = torch.tensor([L], dtype=torch.int32, device=cuda)
     table = None
     kn, vn = k[:, L - 1].contiguous(), v[:, L - 1].contiguous()
