@@ -44,15 +44,27 @@ struct PrefillParams {
     int gs;                   // query heads per KV head: 1 to 16 (0 = 4)
     int key_parts, part_tiles;   // pooling kernel: parts of part_tiles key tiles a query tile's keys are cut into
     int vsub;                 // pooling kernel: sub-group of this launch; those after the first add to what agg holds
+    // set with the grid (UnitGrid)
+    unsigned pair_recip, sub_recip;   // ceil(2^32 / (KV head, sub-group) pairs), ceil(2^32 / sub-groups)
+    int pairs_fill_xcds, all_resident;
 };
 
-// Query heads per KV head and the sub-groups of four head slots they take.
+// Query heads per KV head and the sub-groups of head slots they take.
 struct HeadSlots {
     int gs, subs;
 };
-__host__ __device__ inline HeadSlots head_slots(int gs) {
+__host__ __device__ inline HeadSlots head_slots(int gs, int slots = 4) {
     if (gs <= 0) gs = 4;
-    return HeadSlots{gs, (gs + 3) / 4};
+    return HeadSlots{gs, (gs + slots - 1) / slots};
+}
+// (KV head, sub-group) number -> both
+__device__ __forceinline__ void split_sub_group(const PrefillParams& p, int subs, int& g, int& sub) {
+    sub = 0;
+    if (subs > 1) {
+        const int head = (int)__umulhi((unsigned)g, p.sub_recip);
+        sub = g - head * subs;
+        g = head;
+    }
 }
 
 hipError_t launch_prefill_attn(const PrefillParams& p, bool reuse, bool with_v, int nqb,

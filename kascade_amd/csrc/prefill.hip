@@ -72,6 +72,40 @@ template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
     if (MODE == 5) { if (phase == 0) __builtin_amdgcn_s_setprio(1); else if (phase == 1) __builtin_amdgcn_s_setprio(0); }
 }
 
+// Registers that loads are filling are waited for here.  The compiler does not see the waits of the tile loops and would put
+// one in front of each use in there, behind the next tile's loads.
+template <int N, typename X> __device__ __forceinline__ void arrived(X (&x)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+}
+
+// A wavefront's ROWS output rows, chunk c of row r at c ^ r in LDS, leave as whole rows.  All of them are read before the first
+// is stored and a row's address is the first one's and a scalar: one after another, each read, its address by a 64-bit
+// product and its store took a unit 1.3 us.  out: row 0; row_elems: elements from a row to the next; rows up to last_row.
+template <int D, int ROWS, typename T>
+__device__ __forceinline__ void store_rows(T* out, unsigned row_elems, const T* so, int lrow, int lchunk, int last_row) {
+    constexpr int kChunks = AttnTile<D>::kChunks, kRPL = AttnTile<D>::kRowsPerLoad, kStores = ROWS / kRPL;
+    uint4_t row[kStores];
+#pragma unroll
+    for (int j = 0; j < kStores; ++j) {
+        const int r = j * kRPL + lrow;
+        row[j] = *reinterpret_cast<const uint4_t*>(&so[r * D + (lchunk ^ (r & (kChunks - 1))) * 8]);
+    }
+    T* mine = out + ((unsigned)lrow * (unsigned long long)row_elems + lchunk * 8);
+    // the output is not read again by these kernels: keep it out of the caches
+    auto store = [&](int j) {
+        __builtin_nontemporal_store(row[j], reinterpret_cast<uint4_t*>(mine + (unsigned long long)row_elems * (j * kRPL)));
+    };
+    if (last_row >= ROWS - 1) {   // uniform
+#pragma unroll
+        for (int j = 0; j < kStores; ++j) store(j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kStores; ++j)
+            if (j * kRPL + lrow <= last_row) store(j);
+    }
+}
+
 // Queries are rows [0, Lq) of Q at global positions q_start + row (q_start a multiple of 32);
 // keys are positions [0, L) with L = q_start + Lq.  PAGED: K/V are pages [P, page, G, D]
 // addressed through the block table, and gathered index rows hold physical row numbers.
@@ -85,7 +119,9 @@ template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
 // the wavefronts, so that the idle one is not always the same SIMD's, gave nothing.
 // EXACT_SUM: the softmax denominators are summed in fp32 from the unrounded exponentials (the
 // passes whose log-sum is an output); otherwise units sum them as they enter the second product.
-template <bool PAGED, int D, typename T, bool SPARE, bool EXACT_SUM>
+// NQ: blocks of 16 queries a wavefront takes.  With two, wavefront w has head slot w; with one, four wavefronts are two head
+// slots x two blocks and a unit's four slots take two workgroups.
+template <bool PAGED, int D, typename T, bool SPARE, bool EXACT_SUM, int NQ>
 __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
@@ -95,26 +131,27 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     // products 16x16x32: contraction steps of S^T, 16-row blocks of O^T, 16-key blocks of a tile
     constexpr int kKS = D / 32, kDB = D / 16, kKB = kKT / 16;
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
-    const HeadSlots hs = head_slots(p.gs);
+    constexpr int kSlots = 2 * NQ;       // head slots of a workgroup
+    const HeadSlots hs = head_slots(p.gs, kSlots);
     const int kvh = p.G, nheads = p.G * hs.gs;
     const T* Qp = (const T*)p.Q;
     const T* Kp = (const T*)p.K;
     const T* Vp = (const T*)p.V;
 
-    constexpr int QT = 32, NQ = 2;   // blocks of 16 queries
+    // What the first loads need comes in one trip to memory (the compiler would take one for each branch on the way)
+    asm volatile("" :: "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.head_map), "s"(p.q_start_rows), "s"(p.q_len_rows), "s"(p.q_sb), "s"(p.q_sl),
+                 "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_sl), "s"(p.k_sh), "s"(p.Lq), "s"(p.q_start), "s"(p.max_topk), "s"(p.topk_percent),
+                 "s"(p.gs), "s"(p.pair_recip), "s"(p.pairs_fill_xcds), "s"(p.all_resident));
+    constexpr int QT = 32;
     const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
-    // two workgroups are resident on a compute unit (64 KB of LDS, 256 registers)
-    unit_of_workgroup(p.B, p.G * hs.subs, nqt, 2, blk, g, b);   // g: KV head and sub-group
+    unit_of_workgroup(p, p.G * hs.subs, nqt, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
     const int L = q_start + Lqv;    // keys of this sequence
-    int sub = 0;
-    if (hs.subs > 1) {
-        sub = g % hs.subs;
-        g /= hs.subs;               // the KV head
-    }
+    int sub;
+    split_sub_group(p, hs.subs, g, sub);   // g: the KV head
     // Whose lists a sparse unit reads: a scalar load, on its way while the first rows' addresses are formed (as a vector
     // load every sparse unit waited for it before it requested anything: 3001 tokens 24.3 -> 23.9 us, head_dim 64
     // at 4096 12.4 -> 12.2)
@@ -129,27 +166,26 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     const int q0l = tq * QT;            // first query row of this block
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
-    const int head = g * hs.gs + min(4 * sub + wave, hs.gs - 1);
-    const bool has_head = !SPARE || 4 * sub + __builtin_amdgcn_readfirstlane(wave) < hs.gs;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int slot = kSlots * sub + (NQ == 2 ? wave_u : wave_u >> 1);
+    const int q_off = NQ == 2 ? 0 : 16 * (wave_u & 1);   // this wavefront's first query of the block's
+    const int head = g * hs.gs + min(slot, hs.gs - 1);
+    const bool has_head = !SPARE || slot < hs.gs;
 
     // ---- key regime of this block ----
-    bool sparse = false;
-    int ng = 0;
     const int* idx_row = nullptr;
     // a sequence of a mixed batch keeps the budget it has on its own (the rows are as wide as
     // the longest sequence needs)
     const int width = p.q_start_rows ? min(p.max_topk, topk_width_of(p.topk_percent, L)) : p.max_topk;
-    const int n = min((p.rolling && L > 128) ? rolling_budget(p.topk_percent, q0) : width, width);
-    if (q0 > n) {
-        sparse = true;
-        ng = (n + kKT - 1) / kKT;
-    }
-    const int ntiles = sparse ? ng + 1 : (min(q0 + QT, L) + kKT - 1) / kKT;
+    // (a block behind the widest list is sparse whatever its budget, which is worked out under its first loads)
+    const bool rolls = p.rolling && L > 128;
+    int n = width;
+    if (rolls && q0 <= width) n = min(rolling_budget(p.topk_percent, q0), width);
+    const bool sparse = q0 > n;
     const bool idx_vec = (p.max_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(p.idx) & 15) == 0;
 
     // ---- tile staging: wavefront w fills rows [4w R, 4(w+1) R) of a tile with four loads of R rows
     // each (R = 4 at D = 128, 8 at D = 64); lane = (row within the load, chunk position) ----
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int lrow = lane / kChunks;
     const int lchunk = lane % kChunks;
     // This lane's four rows sit at LDS rows slot0 + j R (j = load) and hold the four consecutive
@@ -168,10 +204,10 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     const uint32_t lds_k = lds_address(sK) + wave_u * 4096;   // this wavefront's 4 KB of a K buffer
     const uint32_t lds_v = lds_address(sV) + wave_u * 4096;
 
-    // key position `pos` of tile `ti` -> key id (contiguous and diagonal tiles)
-    auto tile_key = [&](int ti, int pos) {
-        return min((sparse ? q0 : ti * kKT) + pos, L - 1);
-    };
+    // tiles: gathered ones [0, ng) and the diagonal one behind them in a sparse unit, else consecutive ones
+    int ng = 0, ntiles = 1;
+    // first key of a tile of consecutive keys (the only ones of a sparse unit are the diagonal tile's)
+    auto tile_start = [&](int ti) { return sparse ? q0 : ti * kKT; };
     // ids[j]: what the loads of row j of the next tile need, fetched a tile ahead so that the
     // loads never wait on it.  Gathered tiles: the key id (physical row when PAGED).
     // Consecutive keys, PAGED: the block-table entry of the key's page.  Consecutive keys,
@@ -191,7 +227,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 for (int j = 0; j < 4; ++j) ids[j] = idx_row[min(ti * kKT + pos0 + j, n - 1)];
             }
         } else if (PAGED) {   // four consecutive keys from a multiple of four on: one page
-            ids[0] = bt_row[tile_key(ti, pos0) >> p.page_shift];
+            ids[0] = bt_row[min(tile_start(ti) + pos0, L - 1) >> p.page_shift];
         }
     };
     // K row addresses of the tile whose ids are held; V's are a scalar offset away.  The
@@ -205,6 +241,14 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz16<D>(slot0 + j * kRPL)) * 8);
     }
     const char* row_ptr[4];
+    auto consecutive_rows = [&](int key0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int key = min(key0 + pos0 + j, L - 1);
+            const int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
+            row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
+        }
+    };
     auto next_rows = [&]() {
         if (sparse && pend_ti < ng) {
 #pragma unroll
@@ -213,12 +257,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
             }
         } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int key = tile_key(pend_ti, pos0 + j);
-                const int row = PAGED ? (ids[0] << p.page_shift) + (key & page_mask) : key;
-                row_ptr[j] = lane_ptr[j] + (unsigned long long)row_bytes * (unsigned)row;
-            }
+            consecutive_rows(tile_start(pend_ti));
         }
     };
     constexpr int kNumLoads = 8;
@@ -266,33 +305,45 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     // memory less before the first product of every unit, and units are short (28 tiles on
     // average under rolling budgets).  Softmax is accumulated online, so the order is free.
     auto tile_at = [&](int s) { return sparse ? (s == 0 ? ng : s - 1) : s; };
-    fetch_ids(tile_at(0));
-    next_rows();
+    if (PAGED) ids[0] = bt_row[min(tile_start(0) + pos0, L - 1) >> p.page_shift];
+    consecutive_rows(tile_start(0));
     static_for<0, kNumLoads>([&](auto i) { issue_load(i, 0); });
 
     // ---- Q fragments (B operand of S^T): query col (+ 16 q), d chunk 32*ks + 8*dq; requested after
     // the first tile's rows, which the first barrier waits for ----
     x8_t qf[NQ][kKS];
+    const int last_q = min(QT, Lqv - q0l) - 1;   // of this block
+    const T* q_base = Qp + (long long)b * p.q_sb + (long long)q0l * p.q_sl + (long long)head * p.q_sh;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int ql = q0l + 16 * q + col;
-        const bool ok = ql < Lqv;
-        const T* qp = Qp + (long long)b * p.q_sb + (long long)min(ql, Lqv - 1) * p.q_sl +
-                      (long long)head * p.q_sh + dq * 8;
+        const T* qp = q_base + (unsigned long long)(unsigned)min(q_off + 16 * q + col, last_q) * (unsigned long long)p.q_sl + dq * 8;
 #pragma unroll
         for (int ks = 0; ks < kKS; ++ks) {
             PackT<T> t;
             t.u = ld_global_16(qp + ks * 32);
-            if (!ok) t.u = uint4_t{0, 0, 0, 0};
             qf[q][ks] = t.v8;
         }
     }
 
     if (sparse) {
+        if (rolls && q0 > width) n = min(rolling_budget(p.topk_percent, q0), width);
+        ng = (n + kKT - 1) / kKT;
+        ntiles = ng + 1;
         const int src = max(0, min(mapped, kvh - 1));   // a map built for another head count must not leave the tensor
         idx_row = p.idx + (((long long)b * kvh + src) * p.T + tq) * p.max_topk;
+    } else {
+        ntiles = (min(q0 + QT, L) + kKT - 1) / kKT;
     }
     if (ntiles > 1) fetch_ids(tile_at(1));
+    if (last_q < QT - 1) {   // uniform: rows past the sequence's end are zeros
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int ks = 0; ks < kKS; ++ks)
+                if (q_off + 16 * q + col > last_q) qf[q][ks] = x8_t{};
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) arrived<kKS>(qf[q]);
 
     // One tile: registers -> LDS, next tile's loads, both products, softmax.  Three copies of
     // the code, each straight-line: tiles that need no mask (all but one or two of a unit), tiles
@@ -354,6 +405,11 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         // ---- masks: accumulator v of key block kb is LDS row 16 kb + 4 dq + v of the tile ----
         if (MODE != kFull) {
             const bool diag_here = MODE == kDiag || (sparse && ti == ng);
+            // not known to be the same in every tile: the compiler would form the masks of all rows in front of the loop and
+            // keep them in scalar registers, which the loop of the tiles without masks then spills
+            // (28/4 heads, two prompts of 3001 tokens 42.8 -> 41.2 us)
+            int list_end = n, last_key = L - 1, first_q = q0 + q_off;
+            asm volatile("" : "+s"(list_end), "+s"(last_key), "+s"(first_q));
             if (sparse && !diag_here) {   // a selection that ends inside this tile
 #pragma unroll
                 for (int kb = 0; kb < nkb; ++kb)
@@ -362,7 +418,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                         const int pos = ti * kKT + pos_of_slot(16 * kb + 4 * dq + v);
 #pragma unroll
                         for (int q = 0; q < NQ; ++q)
-                            if (pos >= n) sT[q][kb][v] = -INFINITY;
+                            if (pos >= list_end) sT[q][kb][v] = -INFINITY;
                     }
             } else {                           // the causal edge and the end of the sequence
                 const int kstart = diag_here ? q0 : ti * kKT;
@@ -372,8 +428,8 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                     for (int v = 0; v < 4; ++v) {
                         const int key = kstart + pos_of_slot(16 * kb + 4 * dq + v);
 #pragma unroll
-                        for (int q = 0; q < NQ; ++q)   // q0 + 16 q + col: the query's global position
-                            if (key > q0 + 16 * q + col || key >= L) sT[q][kb][v] = -INFINITY;
+                        for (int q = 0; q < NQ; ++q)   // first_q + 16 q + col: the query's global position
+                            if (key > first_q + 16 * q + col || key > last_key) sT[q][kb][v] = -INFINITY;
                     }
             }
         }
@@ -388,11 +444,19 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 for (int v = 0; v < 4; ++v) mx = fmaxf(mx, sT[q][kb][v]);
             return mx * kScaleLog2;
         };
-        const float ms[NQ] = {maximum(0), maximum(1)};
-        if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) {   // wavefront-uniform
+        // A column's reference moves for its own scores alone, so that its sums do not depend on which columns share a wavefront.
+        float ms[NQ];
+        bool above = false;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            ms[q] = maximum(q);
+            above |= ms[q] > m[q] + kRefSlack;
+        }
+        if (__any(above)) {   // wavefront-uniform
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const float mnew = fmaxf(m[q], max_over_quarters(ms[q]));   // the same in the four lanes of a column
+                const float top = max_over_quarters(ms[q]);   // the same in the four lanes of a column
+                const float mnew = top > m[q] + kRefSlack ? top : m[q];
                 const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
                 m[q] = mnew;
                 l[q] *= corr;
@@ -507,7 +571,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
     T* so = sK + wave * (32 * D);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int ql = q0l + 16 * q + col;
+        const int ql = q0l + q_off + 16 * q + col;
         const float lt = sum_over_quarters(l[q]);
         if (p.log_sum && dq == 0 && ql < Lqv)
             p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[q];
@@ -520,15 +584,8 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
         }
     }
     __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
-#pragma unroll
-    for (int j = 0; j < 32 / kRPL; ++j) {
-        const int r = j * kRPL + lrow;
-        const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
-        const int qr = q0l + r;
-        if (qr < Lqv)   // the output is not read again by these kernels: keep it out of the caches
-            __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
-                (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
-    }
+    store_rows<D, 16 * NQ>((T*)p.O + ((long long)b * Lq + q0l + q_off) * nheads * D + (long long)head * D, (unsigned)(nheads * D),
+                           so, lrow, lchunk, last_q - q_off);
 }
 
 // Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
@@ -556,22 +613,18 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     // (with 16x16x32 products: log-sums alone, 1024 tokens 15.9 -> 15.7 us; dense 2048 45.1 -> 44.5).  Sparse units have
     // more arguments than registers to keep them in: 4096 tokens 31.2 -> 31.8.
     asm volatile("" :: "s"(p.q_start_rows), "s"(p.q_len_rows), "s"(p.q_sb), "s"(p.q_sl), "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_sl),
-                 "s"(p.k_sh), "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.L), "s"(p.gs));
+                 "s"(p.k_sh), "s"(p.Q), "s"(p.K), "s"(p.V), "s"(p.L), "s"(p.gs), "s"(p.pair_recip), "s"(p.pairs_fill_xcds),
+                 "s"(p.all_resident));
     constexpr int QT = 32 * NQB;
     const int Lq = p.Lq;            // rows of Q and of the outputs per sequence
     const int nqt = (Lq + QT - 1) / QT;
     int blk, g, b;
-    // resident per compute unit: two with V (64 KB of LDS, 256 registers), four with K only (32 KB, 128 registers)
-    constexpr int kPerCu = (WITH_V || NQB == 2) ? 2 : 4;
-    unit_of_workgroup(p.B, p.G * hs.subs, nqt, kPerCu, blk, g, b);   // g: KV head and sub-group
+    unit_of_workgroup(p, p.G * hs.subs, nqt, blk, g, b);   // g: KV head and sub-group
     int q_start, Lqv;               // this sequence's first position and how many of the rows are its own
     chunk_of_sequence(p, b, q_start, Lqv);
     const int L = q_start + Lqv;    // keys of this sequence
-    int sub = 0;
-    if (hs.subs > 1) {
-        sub = g % hs.subs;
-        g /= hs.subs;               // the KV head
-    }
+    int sub;
+    split_sub_group(p, hs.subs, g, sub);   // g: the KV head
     const int tq = nqt - 1 - blk;   // long (late) query blocks first
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
@@ -581,14 +634,14 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     const int q0l = tq * QT;            // first query row of this block
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
-    const int head = g * hs.gs + min(4 * sub + wave, hs.gs - 1);
-    const bool has_head = !SPARE || 4 * sub + __builtin_amdgcn_readfirstlane(wave) < hs.gs;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int head = g * hs.gs + min(4 * sub + wave_u, hs.gs - 1);
+    const bool has_head = !SPARE || 4 * sub + wave_u < hs.gs;
 
     const int ntiles = (min(q0 + QT, L) + kKT - 1) / kKT;
 
     // ---- tile staging: wavefront w fills rows [4w R, 4(w+1) R) of a tile with four loads of R rows
     // each (R = 4 at D = 128, 8 at D = 64); lane = (row within the load, chunk position) ----
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int lrow = lane / kChunks;
     const int lchunk = lane % kChunks;
     // This lane's four rows sit at LDS rows slot0 + j R (j = load) and hold the four consecutive
@@ -689,20 +742,27 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     // ---- Q fragments (B operand of S^T): query li (+32 qb), d chunk 16*ks + 8*lg; requested after
     // the first tile's rows, which the first barrier waits for ----
     x8_t qf[NQB][kKS];
+    const int last_q = min(QT, Lqv - q0l) - 1;   // of this block
+    const T* q_base = Qp + (long long)b * p.q_sb + (long long)q0l * p.q_sl + (long long)head * p.q_sh;
 #pragma unroll
     for (int qb = 0; qb < NQB; ++qb) {
-        const int ql = q0l + 32 * qb + li;
-        const bool ok = ql < Lqv;
-        const T* qp = Qp + (long long)b * p.q_sb + (long long)min(ql, Lqv - 1) * p.q_sl +
-                      (long long)head * p.q_sh + lg * 8;
+        const T* qp = q_base + (unsigned long long)(unsigned)min(32 * qb + li, last_q) * (unsigned long long)p.q_sl + lg * 8;
 #pragma unroll
         for (int ks = 0; ks < kKS; ++ks) {
             PackT<T> t;
             t.u = ld_global_16(qp + ks * 16);
-            if (!ok) t.u = uint4_t{0, 0, 0, 0};
             qf[qb][ks] = t.v8;
         }
     }
+    if (last_q < QT - 1) {   // uniform: rows past the sequence's end are zeros
+#pragma unroll
+        for (int qb = 0; qb < NQB; ++qb)
+#pragma unroll
+            for (int ks = 0; ks < kKS; ++ks)
+                if (32 * qb + li > last_q) qf[qb][ks] = x8_t{};
+    }
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) arrived<kKS>(qf[qb]);
 
     // One tile: next tile's loads, both products, softmax.  Two copies of
     // the code, each straight-line: tiles that need no mask (all but one or two of a unit) and tiles
@@ -931,15 +991,8 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
                     *reinterpret_cast<x4_t*>(&so[li * D + (((4 * db + v4) ^ (li & (kChunks - 1))) * 8) + 4 * lg]) = o;
                 }
             __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
-#pragma unroll
-            for (int j = 0; j < 32 / kRPL; ++j) {
-                const int r = j * kRPL + lrow;
-                const uint4_t row = *reinterpret_cast<const uint4_t*>(&so[r * D + lchunk * 8]);
-                const int qr = q0l + r;
-                if (qr < Lqv)   // the output is not read again by these kernels: keep it out of the caches
-                    __builtin_nontemporal_store(row, reinterpret_cast<uint4_t*>(
-                        (T*)p.O + (((long long)b * Lq + qr) * nheads + head) * D + ((lchunk ^ (r & (kChunks - 1))) * 8)));
-            }
+            store_rows<D, 32>((T*)p.O + ((long long)b * Lq + q0l) * nheads * D + (long long)head * D, (unsigned)(nheads * D), so, lrow,
+                          lchunk, last_q);
         }
     }
 }
@@ -952,8 +1005,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(REUSE 
 void prefill_attn_kernel_q32(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
     __shared__ __attribute__((aligned(1024))) T sV[WITH_V ? 2 * AttnTile<D>::kTileElems : 8];
-    if constexpr (REUSE) prefill_reuse_body<PAGED, D, T, SPARE, EXACT_SUM>(p, sK, sV);
+    if constexpr (REUSE) prefill_reuse_body<PAGED, D, T, SPARE, EXACT_SUM, 2>(p, sK, sV);
     else prefill_dense_body<1, WITH_V, PAGED, D, T, SPARE>(p, sK, sV);
+}
+
+// Sparse units in halves of two head slots, 16 queries per wavefront (see kSplitUnits).
+template <bool PAGED, int D, typename T, bool SPARE>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void prefill_sparse_halves_kernel(PrefillParams p) {
+    __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
+    __shared__ __attribute__((aligned(1024))) T sV[2 * AttnTile<D>::kTileElems];
+    prefill_reuse_body<PAGED, D, T, SPARE, false, 1>(p, sK, sV);
 }
 
 // 64 queries per wavefront for the K-only log-sum pass, whose state fits 256 registers: two
@@ -1009,11 +1071,11 @@ void prefill_aggregate_kernel(PrefillParams p) {
     // bf16 4096 tokens 81.2 -> 79.6; two prompts of 3001 tokens at 28/4 heads 50.8 -> 48.6 and, adding, 45.4 -> 41.2)
     asm volatile("" :: "s"(p.Q), "s"(p.K), "s"(p.log_sum_in), "s"(p.agg), "s"(p.q_start_rows), "s"(p.q_len_rows), "s"(p.q_sb),
                  "s"(p.q_sl), "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_sl), "s"(p.k_sh), "s"(p.L), "s"(p.gs), "s"(p.part_tiles),
-                 "s"(p.vsub), "s"(p.fill_invalid));
+                 "s"(p.vsub), "s"(p.fill_invalid), "s"(p.pair_recip), "s"(p.pairs_fill_xcds), "s"(p.all_resident));
     const int Ls = p.L;                  // width of a row of pooled scores
     const int Lq = p.Lq;
     int blk, g, b;
-    unit_of_workgroup(p.B, p.G, p.T * p.key_parts, 2, blk, g, b);
+    unit_of_workgroup(p, p.G, p.T * p.key_parts, blk, g, b);
     const int part = blk / p.T;          // part 0 of every tile first, long tiles first within a part
     blk -= part * p.T;
     int q_start, Lqv;                    // this sequence's first position and how many of the rows are its own
@@ -1226,18 +1288,29 @@ void prefill_aggregate_kernel(PrefillParams p) {
 
 namespace {
 
+// Sparse units (a query tile and four head slots) up to which they are cut in two, one block of 16 queries to a wavefront:
+// where the halves are resident at once, two on each of 256 compute units.  A unit alone on its compute unit is a
+// chain of a wavefront's own instructions; half of them take (32/8 heads, 517 tokens) 9.3 -> 7.4 us, 28/4 517 9.2 -> 7.1,
+// 8/2 heads of 64, 2048 9.6 -> 7.4, 32/8 1024 (256 units) 9.9 -> 9.0.  With more the rows that both halves
+// stage cost more than that: 32/8, 1300 tokens (328 units) 12.4 -> 13.7 us, 2048 14.1 -> 16.9.
+constexpr long long kSplitUnits = 256;
+
 template <int D, typename T>
-hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nqb, hipStream_t stream) {
+hipError_t launch_attn_t(PrefillParams p, bool reuse, bool with_v, int nqb, hipStream_t stream) {
     const int qt = 32 * nqb;
     const bool paged = p.block_table != nullptr;
     const int nqt = (p.Lq + qt - 1) / qt;
-    const int gv = p.G * head_slots(p.gs).subs;   // (KV head, sub-group of four query heads) pairs
-    dim3 grid(nqt, gv, p.B), block(kThreads);
-    if (pairs_fill_xcds(p.B, gv)) {
-        const long long total = (long long)nqt * gv * p.B;
-        if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-        grid = dim3((unsigned)total);
-    }
+    const bool split = reuse && !p.log_sum && (long long)nqt * p.G * head_slots(p.gs).subs * p.B <= kSplitUnits;
+    const HeadSlots hs = head_slots(p.gs, split ? 2 : 4);
+    const int gv = p.G * hs.subs;   // (KV head, sub-group of four or two query heads) pairs
+    p.sub_recip = hs.subs > 1 ? 0xffffffffu / (unsigned)hs.subs + 1u : 0u;
+    // resident per compute unit: two with V (64 KB of LDS, 256 registers), four with K only (32 KB, 128 registers)
+    UnitGrid units;
+    if (!unit_grid(p.B, gv, nqt, reuse || with_v || nqb == 2 ? 2 : 4, units)) return hipErrorInvalidConfiguration;
+    const dim3 grid = units.grid, block(kThreads);
+    p.pair_recip = units.recip;
+    p.pairs_fill_xcds = units.pairs_fill_xcds;
+    p.all_resident = units.all_resident;
     auto launch = [&](auto paged_c, auto spare_c) -> hipError_t {
         constexpr bool kPaged = decltype(paged_c)::value, kSpare = decltype(spare_c)::value;
         if (nqb == 2) {   // K-only log-sum pass, D = 128 (at 64 the state of 64 queries spills)
@@ -1245,6 +1318,8 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
             else return hipErrorInvalidValue;
         } else if (reuse && p.log_sum) {   // a reuse pass that also reports its log-sums: fp32 sums
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare, true>), grid, block, 0, stream, p);
+        } else if (split) {
+            hipLaunchKernelGGL((prefill_sparse_halves_kernel<kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         } else if (reuse) {
             hipLaunchKernelGGL((prefill_attn_kernel_q32<true, true, kPaged, D, T, kSpare>), grid, block, 0, stream, p);
         } else if (with_v) {
@@ -1254,7 +1329,7 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
         }
         return hipSuccess;
     };
-    const bool spare = head_slots(p.gs).gs % 4 != 0;
+    const bool spare = hs.gs % (split ? 2 : 4) != 0;
     const hipError_t e = paged ? (spare ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{}))
                                : (spare ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{}));
     if (e != hipSuccess) return e;
@@ -1262,13 +1337,13 @@ hipError_t launch_attn_t(const PrefillParams& p, bool reuse, bool with_v, int nq
 }
 
 template <int D, typename T>
-hipError_t launch_aggregate_t(const PrefillParams& p, hipStream_t stream) {
-    dim3 grid(p.T * p.key_parts, p.G, p.B), block(kThreads);
-    if (pairs_fill_xcds(p.B, p.G)) {
-        const long long total = (long long)p.T * p.key_parts * p.G * p.B;
-        if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-        grid = dim3((unsigned)total);
-    }
+hipError_t launch_aggregate_t(PrefillParams p, hipStream_t stream) {
+    UnitGrid units;
+    if (!unit_grid(p.B, p.G, (long long)p.T * p.key_parts, 2, units)) return hipErrorInvalidConfiguration;
+    const dim3 grid = units.grid, block(kThreads);
+    p.pair_recip = units.recip;
+    p.pairs_fill_xcds = units.pairs_fill_xcds;
+    p.all_resident = units.all_resident;
     auto launch_as = [&](auto heads, auto later) {
         constexpr int kHeads = decltype(heads)::value;
         constexpr bool kLater = decltype(later)::value;

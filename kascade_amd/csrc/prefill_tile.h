@@ -52,27 +52,44 @@ template <typename P> __device__ __forceinline__ uint32_t lds_address(P* ptr) {
 
 // Workgroup -> (query block, KV head, sequence).  Workgroups go to the eight XCDs round-robin in
 // launch order and each XCD has an L2 of its own.  When the number of (sequence, KV head) pairs
-// is a multiple of eight the launch is one-dimensional and consecutive workgroups take eight
-// different pairs: all units of a pair, which read the same K/V rows, run on one XCD.
-__host__ __device__ inline bool pairs_fill_xcds(int B, int G) { return (B * G) % 8 == 0; }
+// is a multiple of eight, consecutive workgroups take eight different pairs: all units of a pair, which read the same
+// K/V rows, run on one XCD.  The launch is (8 pairs, blocks, pairs / 8) then, in that order of dispatch, and
+// the pair's sequence is a product with a reciprocal from the host: with a one-dimensional launch every workgroup
+// began with two divisions, a hundred dependent instructions in front of its first load.
+struct UnitGrid {
+    dim3 grid;
+    unsigned recip;   // ceil(2^32 / G), G > 1
+    int pairs_fill_xcds, all_resident;
+};
+inline bool unit_grid(int B, int G, long long nblocks, int per_cu, UnitGrid& u) {
+    const long long pairs = (long long)B * G;
+    // exact quotients below 2^32 / G; grid dimensions behind the first are 16 bits
+    u.pairs_fill_xcds = pairs % 8 == 0 && nblocks <= 65535 && pairs / 8 <= 65535 && pairs * G < (1ll << 32);
+    u.recip = G > 1 ? (unsigned)(0xffffffffu / (unsigned)G + 1u) : 0u;
+    u.all_resident = nblocks * pairs <= (long long)per_cu * 256;
+    if (u.pairs_fill_xcds) {
+        u.grid = dim3(8, (unsigned)nblocks, (unsigned)(pairs / 8));
+        return nblocks * pairs <= 0x7fffffffLL;
+    }
+    u.grid = dim3((unsigned)nblocks, G, B);
+    return nblocks <= 0x7fffffffLL;
+}
 // Blocks go out long ones first.  Where all workgroups are resident at once (`per_cu` on each of 256
 // compute units) nothing evens out their lengths later, and every second round of 32 workgroups of an
 // XCD -- one per compute unit -- is taken in reverse, so that a compute unit's workgroups add up to about
 // the same work: 32/8 heads, 2048 tokens dense 52 -> 48.5 us, log-sum pass 4096 tokens 97 -> 83.  With more
 // workgroups than that the plain order is the better one (dense, 4096 tokens: 142 against 149 us).
-__device__ __forceinline__ void unit_of_workgroup(int B, int G, int nblocks, int per_cu, int& blk, int& g, int& b) {
-    if (pairs_fill_xcds(B, G)) {
-        const int i = blockIdx.x;
-        const int r = i >> 3;
-        const int pair = (r / nblocks) * 8 + (i & 7);
-        blk = r % nblocks;
-        constexpr int kCus = 256, kXcdCus = 32;
-        if ((blk & kXcdCus) && (long long)nblocks * B * G <= per_cu * kCus) {
+__device__ __forceinline__ void unit_of_workgroup(const PrefillParams& p, int G, int nblocks, int& blk, int& g, int& b) {
+    if (p.pairs_fill_xcds) {
+        const int pair = blockIdx.z * 8 + blockIdx.x;
+        blk = blockIdx.y;
+        constexpr int kXcdCus = 32;
+        if ((blk & kXcdCus) && p.all_resident) {
             const int base = blk & ~(kXcdCus - 1);
             blk = base + min(kXcdCus, nblocks - base) - 1 - (blk - base);
         }
-        g = pair % G;
-        b = pair / G;
+        b = G > 1 ? (int)__umulhi((unsigned)pair, p.pair_recip) : pair;
+        g = pair - b * G;
     } else {
         blk = blockIdx.x;
         g = blockIdx.y;

@@ -297,3 +297,41 @@ def test_pooled_scores_add_up_over_the_sub_groups(cuda, gs, G, D, L):
     inside = torch.isfinite(got)
     assert torch.equal(inside, torch.isfinite(want)) and bool(inside.any())
     assert bool(((got - want).abs()[inside] <= slack[inside]).all())
+
+
+# 256 units are cut in halves, 264 (or more) are not: copies of a prompt, and the same prompt over the paged cache
+@pytest.mark.parametrize("heads,G,D,L,copies,dtype", [
+    (32, 8, 128, 1024, 2, torch.float16), (32, 8, 128, 517, 2, torch.bfloat16), (28, 4, 128, 300, 7, torch.float16),
+    (14, 2, 64, 2000, 2, torch.bfloat16), (8, 8, 128, 700, 2, torch.float16), (24, 8, 64, 129, 7, torch.float16),
+    (5, 1, 128, 200, 19, torch.float16), (32, 2, 128, 161, 6, torch.bfloat16)])
+def test_sparse_rows_do_not_depend_on_the_cut_of_a_unit(cuda, heads, G, D, L, copies, dtype):
+    """Sparse units in halves (16 queries per wavefront, two head slots per workgroup) and whole ones: the same bits,
+    with empty slots in one half or in both and blocks that end inside either 16 queries."""
+    from kascade_amd import budgets, kernels
+    p = 10
+    gen = torch.Generator().manual_seed(L + heads)
+    q = torch.randn(1, L, heads, D, generator=gen).to(dtype).to(cuda) * 2   # references that move behind the first tile
+    k, v = (torch.randn(1, L, G, D, generator=gen).to(dtype) for _ in range(2))
+    kp, table = _paged_copies(k, 16, gen, 1, cuda)
+    rows = torch.zeros(kp.shape[0] * 16, G, D, dtype=dtype)
+    rows[:L] = v[0]
+    vp = torch.empty_like(kp)
+    vp[table[0].long()] = rows.view(-1, 16, G, D).to(cuda)
+    T, W = (L + 31) // 32, budgets.topk_width(L, p)
+    idx = torch.zeros(1, G, T, W, dtype=torch.int32)
+    for t in range(1, T):
+        n = min(32 * t, W)
+        for g in range(G):
+            idx[0, g, t, :n] = torch.randperm(32 * t, generator=gen)[:n].sort().values
+    maps = torch.arange(G - 1, -1, -1, dtype=torch.int32, device=cuda)
+    units = T * G * -(-heads // G // 4)
+    assert units <= 256 < units * copies
+    kd, vd, idx = k.to(cuda), v.to(cuda), idx.to(cuda)
+    one = kernels.prefill_reuse(q, kd, vd, idx, maps, float(p), True)
+    many = kernels.prefill_reuse(*(x.repeat(copies, 1, 1, 1) for x in (q, kd, vd, idx)), maps, float(p), True)
+    assert all(torch.equal(one[0], m) for m in many)
+    lists = kernels.translate_indices(idx.contiguous(), table, L, 16)
+    assert torch.equal(kernels.prefill_chunk_reuse(q, kp, vp, lists, maps, float(p), True, table, 0, 16), one)
+    want = orc.reuse_prefill(q.cpu(), k, v, idx.cpu(), maps.tolist(), 32, True, float(p))
+    atol, rtol = (2e-3, 1e-2) if dtype == torch.float16 else (1.6e-2, 2e-2)   # one rounding of P and of the output
+    assert_close(one, want, "sparse rows", atol=atol, rtol=rtol)
