@@ -326,6 +326,20 @@ int kascade_topk_rows_call(const kascade_half* scores, int32_t* out_idx, int row
                            const int32_t* block_table, int max_pages, int page_size,
                            int rows_per_sequence, void* stream);
 
+/* Pooled tile scores and their selection in one call: what kascade_prefill_aggregate_range_shaped_call (strided K:
+ * kv_strides, no block table) or kascade_prefill_chunk_aggregate_shaped_call (pages) followed by kascade_topk_rows_call
+ * gives, for rows [batch, kv_heads, tiles] of the queries' 32-row tiles; in one launch where rows are short.
+ *   scores: scratch [batch, kv_heads, tiles, q_start + q_len] fp16, left with unspecified contents
+ *   valid_len / n_sel [period], both required: keys row r looks at (at most those in front of its tile) and takes
+ *   out_idx [rows, k]; out_rows [rows, k] or NULL: the same as cache rows (with a block table)
+ *   workspace: as for kascade_topk_call, kascade_topk_workspace_bytes(rows, q_start + q_len) bytes or NULL. */
+int kascade_prefill_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K, const float* log_sum,
+                                     kascade_half* scores, int32_t* out_idx, int32_t* out_rows, int batch, int q_start, int q_len,
+                                     kascade_strides q_strides, const kascade_strides* kv_strides, const int32_t* block_table,
+                                     int max_pages, int page_size, int num_pages, const int32_t* q_start_rows,
+                                     const int32_t* q_len_rows, const int32_t* valid_len, const int32_t* n_sel, int period, int k,
+                                     int fill_value, void* workspace, void* stream);
+
 /* The selection in the form torch.topk(scores[..., :uniform_len], k).indices has
  * (EfficientKascadeStrategy.py:82, 90, 111): full-width rows ordered by descending score, for a
  * consumer that slices its own prefix of a row.

@@ -171,7 +171,7 @@ int set_append(DecodeParams& p, const kascade_half* k_new, const kascade_half* v
 
 extern "C" {
 
-int kascade_abi_version(void) { return 12; }
+int kascade_abi_version(void) { return 13; }
 
 const char* kascade_get_last_error(void) { return g_err; }
 
@@ -791,7 +791,7 @@ int prefill_aggregate_impl(const Shape& sh, const kascade_half* Q, const kascade
     p.q_sb = q_strides.b; p.q_sl = q_strides.l; p.q_sh = q_strides.h;
     p.k_sb = kv_strides.b; p.k_sl = kv_strides.l; p.k_sh = kv_strides.h;
     p.B = batch; p.L = seq_len; p.Lq = seq_len; p.T = (seq_len + kTile - 1) / kTile; p.fill_invalid = fill_invalid;
-    return check_hip(launch_prefill_aggregate(p, static_cast<hipStream_t>(stream)),
+    return check_hip(launch_prefill_aggregate(p, nullptr, static_cast<hipStream_t>(stream)),
                      "prefill_aggregate");
 }
 }  // namespace
@@ -815,25 +815,32 @@ int kascade_prefill_aggregate_shaped_call(const kascade_shape* shape, const kasc
 
 }  // extern "C"
 namespace {
-int prefill_aggregate_range_impl(const Shape& sh, const kascade_half* Q, const kascade_half* K,
-                                         const float* log_sum, kascade_half* aggregate_scores,
-                                         int batch, int q_start, int q_len,
-                                         kascade_strides q_strides, kascade_strides kv_strides,
-                                         int fill_invalid, void* stream) {
+int range_params(PrefillParams& p, const Shape& sh, const kascade_half* Q, const kascade_half* K, const float* log_sum,
+                 kascade_half* aggregate_scores, int batch, int q_start, int q_len, kascade_strides q_strides,
+                 kascade_strides kv_strides, int fill_invalid) {
     REQUIRE(Q && K && log_sum && aggregate_scores, "prefill_aggregate_range: null pointer argument");
     REQUIRE(batch > 0 && q_len > 0 && batch <= 65535, "prefill_aggregate_range: bad batch/q_len");
     REQUIRE(q_start >= 0 && q_start % kTile == 0, "prefill_aggregate_range: q_start must be a multiple of 32");
     REQUIRE((long long)q_start + q_len < (1LL << 31), "prefill_aggregate_range: q_start + q_len out of range");
     REQUIRE(aligned16(Q) && aligned16(K), "prefill_aggregate_range: Q/K must be 16-byte aligned");
     if (check_strides(q_strides, "Q") || check_strides(kv_strides, "K")) return -1;
-    PrefillParams p{};
     p.G = sh.G; p.head_dim = sh.D; p.elem = sh.elem; p.gs = sh.gs;
     p.Q = H(Q); p.K = H(K); p.V = H(K); p.log_sum_in = log_sum; p.agg = H(aggregate_scores);
     p.q_sb = q_strides.b; p.q_sl = q_strides.l; p.q_sh = q_strides.h;
     p.k_sb = kv_strides.b; p.k_sl = kv_strides.l; p.k_sh = kv_strides.h;
     p.B = batch; p.L = q_start + q_len; p.Lq = q_len; p.q_start = q_start;
     p.T = (q_len + kTile - 1) / kTile; p.fill_invalid = fill_invalid;
-    return check_hip(launch_prefill_aggregate(p, static_cast<hipStream_t>(stream)),
+    return 0;
+}
+
+int prefill_aggregate_range_impl(const Shape& sh, const kascade_half* Q, const kascade_half* K,
+                                         const float* log_sum, kascade_half* aggregate_scores,
+                                         int batch, int q_start, int q_len,
+                                         kascade_strides q_strides, kascade_strides kv_strides,
+                                         int fill_invalid, void* stream) {
+    PrefillParams p{};
+    if (range_params(p, sh, Q, K, log_sum, aggregate_scores, batch, q_start, q_len, q_strides, kv_strides, fill_invalid)) return -1;
+    return check_hip(launch_prefill_aggregate(p, nullptr, static_cast<hipStream_t>(stream)),
                      "prefill_aggregate_range");
 }
 }  // namespace
@@ -1106,7 +1113,7 @@ int prefill_chunk_aggregate_impl(const Shape& sh, const kascade_half* Q, const k
         return -1;
     p.K = E(K_pages); p.V = E(K_pages); p.log_sum_in = log_sum; p.agg = H(aggregate_scores);
     p.fill_invalid = fill_invalid;
-    return check_hip(launch_prefill_aggregate(p, static_cast<hipStream_t>(stream)),
+    return check_hip(launch_prefill_aggregate(p, nullptr, static_cast<hipStream_t>(stream)),
                      "prefill_chunk_aggregate");
 }
 
@@ -1136,6 +1143,45 @@ int prefill_chunk_reuse_impl(const Shape& sh, const kascade_half* Q, const kasca
 }
 }  // namespace
 extern "C" {
+
+int kascade_prefill_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K, const float* log_sum,
+                                     kascade_half* scores, int32_t* out_idx, int32_t* out_rows, int batch, int q_start, int q_len,
+                                     kascade_strides q_strides, const kascade_strides* kv_strides, const int32_t* block_table,
+                                     int max_pages, int page_size, int num_pages, const int32_t* q_start_rows,
+                                     const int32_t* q_len_rows, const int32_t* valid_len, const int32_t* n_sel, int period, int k,
+                                     int fill_value, void* workspace, void* stream) {
+    Shape sh;
+    if (get_shape(shape, &sh)) return -1;
+    REQUIRE(Q && K && log_sum && scores && out_idx && valid_len && n_sel, "prefill_anchor_topk: null pointer argument");
+    REQUIRE(block_table || kv_strides, "prefill_anchor_topk: K is strided or behind a block table");
+    REQUIRE(!out_rows || block_table, "prefill_anchor_topk: out_rows needs a block table");
+    REQUIRE(k > 0 && period > 0, "prefill_anchor_topk: k and period must be > 0");
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    PrefillParams p{};
+    if (block_table) {
+        REQUIRE(aligned16(K), "prefill_anchor_topk: K must be 16-byte aligned");
+        if (chunk_params(p, sh, Q, batch, q_start, q_len, q_strides, block_table, max_pages, page_size, num_pages, q_start_rows,
+                         q_len_rows))
+            return -1;
+        p.K = E(K); p.V = E(K); p.log_sum_in = log_sum; p.agg = H(scores);
+    } else {
+        REQUIRE(!q_start_rows && !q_len_rows, "prefill_anchor_topk: rows of their own come with a block table");
+        if (range_params(p, sh, Q, K, log_sum, scores, batch, q_start, q_len, q_strides, *kv_strides, 0)) return -1;
+    }
+    const long long rows = (long long)p.B * p.G * p.T;
+    REQUIRE(rows < (1LL << 31), "prefill_anchor_topk: too many rows");
+    TopkRows tr{};
+    if (out_rows) {
+        tr.out_rows = out_rows; tr.block_table = block_table; tr.max_pages = max_pages; tr.page_shift = p.page_shift;
+        tr.rows_per_seq = p.G * p.T;
+    }
+    if (prefill_pool_selects(p)) {
+        SelectParams sel{valid_len, n_sel, out_idx, tr, period, k, fill_value};
+        return check_hip(launch_prefill_aggregate(p, &sel, s), "prefill_anchor_topk");
+    }
+    if (check_hip(launch_prefill_aggregate(p, nullptr, s), "prefill_anchor_topk")) return -1;
+    return select_rows(p.agg, out_idx, (int)rows, p.L, p.L, valid_len, n_sel, period, k, fill_value, workspace, tr, s);
+}
 
 int kascade_prefill_chunk_dense_call(const kascade_half* Q, const kascade_half* K_pages,
                                      const kascade_half* V_pages, float* log_sum,

@@ -359,10 +359,10 @@ PyObject* hf_prefill_anchor(PyObject* const* a) {
         check(kascade_prefill_dense_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), with_output ? half_ptr(h.v) : nullptr,
                                                 float_ptr(log_sum), with_output ? half_ptr(out) : nullptr, (int)h.B, (int)h.L,
                                                 qs, ks, with_output, stream));
-        check(kascade_prefill_aggregate_shaped_call(&h.shape, half_ptr(h.q), half_ptr(h.k), float_ptr(log_sum), half_ptr(scores),
-                                                    (int)h.B, (int)h.L, qs, ks, 0, stream));
-        check(kascade_topk_call(half_ptr(scores), int_ptr(idx), (int)(h.B * h.G * T), h.L, (int)h.L, int_ptr(valid),
-                                int_ptr(nsel), (int)T, (int)width, (int)h.L - 1, nullptr, stream));
+        check(kascade_prefill_anchor_topk_call(&h.shape, half_ptr(h.q), half_ptr(h.k), float_ptr(log_sum), half_ptr(scores),
+                                               int_ptr(idx), nullptr, (int)h.B, 0, (int)h.L, qs, &ks, nullptr, 0, 1, 0, nullptr,
+                                               nullptr, int_ptr(valid), int_ptr(nsel), (int)T, (int)width, (int)h.L - 1, nullptr,
+                                               stream));
         if (!with_output) prompt_reuse(h, idx, hm, percent, rolling, out, stream);
     }
     return pair(out, idx);

@@ -1,6 +1,7 @@
 // Host-visible launchers of the prefill kernels (prefill.hip).
 #pragma once
 #include "common.h"
+#include "topk.h"
 
 namespace kascade {
 
@@ -43,6 +44,7 @@ struct PrefillParams {
     int elem;                 // kElemF16 or kElemBF16
     int gs;                   // query heads per KV head: 1 to 16 (0 = 4)
     int key_parts, part_tiles;   // pooling kernel: parts of part_tiles key tiles a query tile's keys are cut into
+    int pool_waves;           // pooling with selection: wavefronts of a workgroup
     int vsub;                 // pooling kernel: sub-group of this launch; those after the first add to what agg holds
     // set with the grid (UnitGrid)
     unsigned pair_recip, sub_recip;   // ceil(2^32 / (KV head, sub-group) pairs), ceil(2^32 / sub-groups)
@@ -69,7 +71,18 @@ __device__ __forceinline__ void split_sub_group(const PrefillParams& p, int subs
 
 hipError_t launch_prefill_attn(const PrefillParams& p, bool reuse, bool with_v, int nqb,
                                hipStream_t stream);
-hipError_t launch_prefill_aggregate(const PrefillParams& p, hipStream_t stream);
+// Selection from the pooled scores by the launch that forms them: what launch_topk takes, for the tiles' rows [B, G, T].
+struct SelectParams {
+    const int* valid_len;     // per row modulo period
+    const int* n_sel;
+    int* out_idx;             // [B*G*T, k]
+    TopkRows rows;
+    int period, k, fill;
+};
+constexpr int kPoolSelectKeys = 4096;   // longest pooled row that fits beside the tiles
+// select (or null): needs q_start + 32 (T - 1) <= kPoolSelectKeys; agg then holds nothing but the scores of earlier sub-groups.
+bool prefill_pool_selects(const PrefillParams& p);   // whether that pays against a launch of its own for the selection
+hipError_t launch_prefill_aggregate(const PrefillParams& p, const SelectParams* select, hipStream_t stream);
 // out[b,i] = physical cache row of token idx[b,i] (clamped to [0, L)); out may alias idx.
 hipError_t launch_translate_indices(const int* idx, int* out, const int* block_table, int B,
                                     long long per_seq, int max_pages, int page_shift, int L,

@@ -35,6 +35,7 @@
 //   rows is an in-lane sum over accumulator registers.
 #include "prefill.h"
 #include "prefill_tile.h"
+#include "topk_row.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -62,7 +63,6 @@ namespace kascade {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kAggKT = 128;        // keys per tile (aggregate kernel)
 
 // phase: 0 = first product begins, 1 = softmax begins, 2 = second product begins (or the tile ends)
 template <int MODE> __device__ __forceinline__ void tile_phase(int phase) {
@@ -1049,9 +1049,13 @@ void prefill_attn_kernel_q64(PrefillParams p) {
 // ACC: adds to the scores of the KV head's earlier sub-groups, which are requested with the tile's products ahead of them.
 // A uniform branch instead of the template: 40/8 heads, 517 tokens 12.9 -> 14.3 us, 28/4 heads, two prompts of 3001 tokens
 // 83.6 -> 87.3 (both launches each).
-template <bool PAGED, int D, typename T, int NH, bool ACC>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-void prefill_aggregate_kernel(PrefillParams p) {
+// WAVES: wavefronts of the workgroup, a tile is 32 keys for each.
+// MAXC > 0: the workgroup has all keys of its tile, keeps the pooled row in LDS and selects from it (see
+// prefill_pool_select_kernel).
+template <bool PAGED, int D, typename T, int NH, bool ACC, int WAVES, int MAXC>
+__device__ __forceinline__ void prefill_pool_body(const PrefillParams& p, const SelectParams& sel) {
+    constexpr int kThreads = WAVES * 64, kAggKT = WAVES * 32;
+    constexpr bool SELECT = MAXC > 0;
     typedef typename Elem<T>::x8 x8_t;
     constexpr int kKS = D / 16;
     constexpr int kChunks = D / 8;
@@ -1063,8 +1067,12 @@ void prefill_aggregate_kernel(PrefillParams p) {
     const int kvh = p.G, nheads = p.G * hs.gs;
     const T* Qp = (const T*)p.Q;
     const T* Kp = (const T*)p.K;
-    __shared__ __attribute__((aligned(1024))) T sK[2 * 4 * kWaveElems];
+    typedef SelectLds<kThreads, false> Histograms;   // in the tiles' place
+    constexpr size_t kTileBytes = 2 * WAVES * kWaveElems * sizeof(T);
+    __shared__ __attribute__((aligned(1024))) char s_tiles[SELECT && sizeof(Histograms) > kTileBytes ? sizeof(Histograms) : kTileBytes];
+    T* sK = reinterpret_cast<T*>(s_tiles);
     __shared__ __attribute__((aligned(16))) float s_lse[128];
+    __shared__ __attribute__((aligned(16))) uint16_t s_row[SELECT ? kThreads * 8 * MAXC : 8];   // pooled scores as fp16
 
     // All arguments in one trip to memory, and the log-sums, which the first exponentials need, not waited for before the
     // first rows are requested (with the scores of earlier sub-groups ahead of a tile's products: 517 tokens 8.8 -> 7.9 us,
@@ -1110,7 +1118,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
         // heads: 512 queries at 2048 12.5 -> 12.1) ----
         constexpr bool kLanePages = PAGED && D == 64;
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-        const int n = min(ti1 - ti0, (ts / 32 - (4 * ti0 + wave_u) + 3) / 4);
+        const int n = min(ti1 - ti0, (ts / 32 - (WAVES * ti0 + wave_u) + WAVES - 1) / WAVES);
         auto key_of_tile = [&](int ti) { return n > 0 ? min(ti, ti0 + n - 1) * kAggKT + 32 * wave_u : 0; };
         const int lrow = lane / kChunks;
         const int lchunk = lane % kChunks;
@@ -1124,7 +1132,8 @@ void prefill_aggregate_kernel(PrefillParams p) {
                                         (lchunk ^ swz<D>(j * kRPL + lrow)) * 8);
         const int* bt_row = PAGED ? p.block_table + (long long)b * p.max_pages : nullptr;
         const int page_mask = (1 << p.page_shift) - 1;
-        const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * 4 * kWaveElems * 2
+        constexpr int kBufElems = WAVES * kWaveElems;
+        const uint32_t lds_w = lds_address(sK) + wave_u * (kWaveElems * 2);   // + buf * kBufElems * 2
         const T* my_k = sK + wave * kWaveElems;
         // Block-table entries of 64 pages, one per lane (pages are at least four tokens, 64 of them two tiles),
         // and of the 64 behind them; with kLanePages the entries of the slice's 32 keys and of the next slice's
@@ -1168,7 +1177,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
             }
         };
         auto issue_load = [&](int j, int buf) {   // loads of a tile in order
-            const uint32_t lds = lds_w + buf * (4 * kWaveElems * 2) + j * 1024;
+            const uint32_t lds = lds_w + buf * (kBufElems * 2) + j * 1024;
             unsigned long long off = row_off;
             if (PAGED) {
                 const int key = key0 + j * kRPL;
@@ -1188,12 +1197,15 @@ void prefill_aggregate_kernel(PrefillParams p) {
         // other buffer, chunks permuted like the keys' (fragments read from memory directly, every
         // wavefront all four heads, 16 bytes of 32 rows per instruction, held every workgroup up at its start:
         // 32/8 heads, 512 tokens 13.1 -> 10.4 us, 1024 18.9 -> 16.2, 2048 35.5 -> 28.9, 4096 87 -> 84).
+        constexpr int kQLoads = kLoads * 4 / WAVES;   // a slot's rows by one wavefront, or half of them by each of two
+        const int q_slot = wave_u & 3, q_first = (wave_u >> 2) * kQLoads;
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const int row = j * kRPL + lrow;
+        for (int j = 0; j < kQLoads; ++j) {
+            const int row = (q_first + j) * kRPL + lrow;
             const T* qp = Qp + (long long)b * p.q_sb + (long long)min(tl + row, Lqv - 1) * p.q_sl +
-                          (long long)min(head0 + wave_u, g * hs.gs + hs.gs - 1) * p.q_sh;
-            load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_w + ((ti0 + 1) & 1) * (4 * kWaveElems * 2) + j * 1024);
+                          (long long)min(head0 + q_slot, g * hs.gs + hs.gs - 1) * p.q_sh;
+            load_to_lds_16(qp + (lchunk ^ swz<D>(row)) * 8, lds_address(sK) + ((ti0 + 1) & 1) * (kBufElems * 2) +
+                                                            q_slot * (kWaveElems * 2) + (q_first + j) * 1024);
         }
         enter_tile(ti0);
 #pragma unroll
@@ -1205,7 +1217,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
         __syncthreads();                                   // everybody's, and s_lse
         // A operands: row block rb = head slot rb, row li = query tl + li
         x8_t qa[NH][kKS];
-        const T* sQ = sK + ((ti0 + 1) & 1) * (4 * kWaveElems);
+        const T* sQ = sK + ((ti0 + 1) & 1) * kBufElems;
 #pragma unroll
         for (int rb = 0; rb < NH; ++rb)
 #pragma unroll
@@ -1220,7 +1232,7 @@ void prefill_aggregate_kernel(PrefillParams p) {
         for (int ti = ti0; ti < ti1; ++ti) {
             // this tile's rows have landed (and the next tile's block-table entries arrived)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            const T* bK = my_k + (ti & 1) * (4 * kWaveElems);
+            const T* bK = my_k + (ti & 1) * kBufElems;
             const int tn = min(ti + 1, ti1 - 1);   // after the last tile: its rows once more, unused
             const int nbuf = (ti + 1) & 1;
             const int key = ti * kAggKT + 32 * wave + li;
@@ -1269,7 +1281,9 @@ void prefill_aggregate_kernel(PrefillParams p) {
             exponentials(acc[(NH - 1) & 1], 0, 16);
             sum = sum_with_other_half(sum);
             tile_phase<KASCADE_PRIO_AGG>(2);
-            if (lg == 0 && key < Ls) {
+            if (SELECT) {
+                if (lg == 0 && key < ts) s_row[key] = __builtin_bit_cast(uint16_t, (half_t)(ACC ? sum + (float)earlier : sum));
+            } else if (lg == 0 && key < Ls) {
                 if (key < ts)
                     out[key] = (half_t)(ACC ? sum + (float)earlier : sum);
                 else if (p.fill_invalid)
@@ -1278,10 +1292,58 @@ void prefill_aggregate_kernel(PrefillParams p) {
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS after the workgroup has left
     }
-    if (p.fill_invalid) {
+    if constexpr (SELECT) {
+        Histograms& lds = *reinterpret_cast<Histograms*>(s_tiles);
+        const long long row = ((long long)b * kvh + g) * p.T + t;
+        const int pr = (int)(row % sel.period);
+        const int len = min(sel.valid_len[pr], ts);
+        const int count = max(0, min(sel.n_sel[pr], sel.k));
+        const RowsOut ro{sel.rows.out_rows, sel.rows.block_table, sel.rows.max_pages, sel.rows.page_shift, sel.rows.rows_per_seq};
+        if (len <= count || count == 0) {   // uniform
+            list_head<kThreads>(count, sel.k, sel.fill, sel.out_idx, row, ro);
+            return;
+        }
+        __syncthreads();   // the row is complete, the tiles are done with
+        lds.clear();
+        const int nch = (len + kThreads * 8 - 1) / (kThreads * 8);   // <= MAXC (host)
+        const int first = wave * nch * 512 + lane * 8;
+        const uint32_t one = pk_hidden(0x00010001u);
+        uint4_t data[MAXC];
+        static_for<0, MAXC>([&](auto c_c) {   // order keys, at least 1; 0 past the row's end
+            constexpr int c = decltype(c_c)::value;
+            data[c] = uint4_t{0, 0, 0, 0};
+            const int j0 = first + c * 512;
+            if (c < nch && j0 < len) {
+                const uint4_t raw = *reinterpret_cast<const uint4_t*>(&s_row[j0]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t key = pk_max_u16(raw[j] ^ (pk_sign_mask_i16(raw[j]) | 0x80008000u), one);
+                    if (j0 + 2 * j + 1 >= len) key = j0 + 2 * j < len ? key & 0xFFFFu : 0u;
+                    data[c][j] = key;
+                }
+            }
+        });
+        __syncthreads();   // cleared histograms
+        select_row<kThreads, MAXC, false>(lds, data, nch, 0, len, count, sel.k, sel.fill, sel.out_idx, row, ro);
+    } else if (p.fill_invalid) {
         const int end = part == p.key_parts - 1 ? Ls : min(Ls, (ti0 + p.part_tiles) * kAggKT);
         for (int key = max(ntiles, ti0) * kAggKT + tid; key < end; key += kThreads) out[key] = neg_inf;
     }
+}
+
+template <bool PAGED, int D, typename T, int NH, bool ACC>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void prefill_aggregate_kernel(PrefillParams p) {
+    prefill_pool_body<PAGED, D, T, NH, ACC, 4, 0>(p, SelectParams{});
+}
+
+// Pooling and selection of a query tile in one workgroup: the pooled row, rounded to fp16 as it would be in memory, goes from the
+// products to the selection through LDS (8 KB beside the tiles, whose place the histograms take afterwards), and one
+// workgroup's selection runs under the products of the other one on its compute unit.  See prefill_pool_selects.
+template <bool PAGED, int D, typename T, int NH, bool ACC, int WAVES, int MAXC>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void prefill_pool_select_kernel(PrefillParams p, SelectParams sel) {
+    prefill_pool_body<PAGED, D, T, NH, ACC, WAVES, MAXC>(p, sel);
 }
 
 }  // namespace
@@ -1337,7 +1399,7 @@ hipError_t launch_attn_t(PrefillParams p, bool reuse, bool with_v, int nqb, hipS
 }
 
 template <int D, typename T>
-hipError_t launch_aggregate_t(PrefillParams p, hipStream_t stream) {
+hipError_t launch_aggregate_t(PrefillParams p, const SelectParams* sel, hipStream_t stream) {
     UnitGrid units;
     if (!unit_grid(p.B, p.G, (long long)p.T * p.key_parts, 2, units)) return hipErrorInvalidConfiguration;
     const dim3 grid = units.grid, block(kThreads);
@@ -1347,7 +1409,18 @@ hipError_t launch_aggregate_t(PrefillParams p, hipStream_t stream) {
     auto launch_as = [&](auto heads, auto later) {
         constexpr int kHeads = decltype(heads)::value;
         constexpr bool kLater = decltype(later)::value;
-        if (p.block_table)
+        auto select = [&](auto paged, auto waves, auto chunks) {
+            constexpr int kWaves = decltype(waves)::value;
+            hipLaunchKernelGGL((prefill_pool_select_kernel<decltype(paged)::value, D, T, kHeads, kLater, kWaves, decltype(chunks)::value>),
+                               grid, dim3(kWaves * 64), 0, stream, p, *sel);
+        };
+        if (sel && p.pool_waves == 8)
+            p.block_table ? select(std::true_type{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{})
+                          : select(std::false_type{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+        else if (sel)
+            p.block_table ? select(std::true_type{}, std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{})
+                          : select(std::false_type{}, std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+        else if (p.block_table)
             hipLaunchKernelGGL((prefill_aggregate_kernel<true, D, T, kHeads, kLater>), grid, block, 0, stream, p);
         else
             hipLaunchKernelGGL((prefill_aggregate_kernel<false, D, T, kHeads, kLater>), grid, block, 0, stream, p);
@@ -1364,6 +1437,10 @@ hipError_t launch_aggregate_t(PrefillParams p, hipStream_t stream) {
 
 }  // namespace
 
+// Pooling that selects: units up to which a workgroup has eight wavefronts, one workgroup on each compute unit (pooling and
+// selection with four / eight: 32/8 heads, 517 tokens 11.7/11.3 us, 1024 16.5/15.3, 28/4 2048 40.4/36.2; with 328 units 19.8/21.5).
+constexpr long long kWidePoolUnits = 256;
+
 // p.head_dim in {64, 128}, p.elem in {kElemF16, kElemBF16}: checked by the callers
 hipError_t launch_prefill_attn(const PrefillParams& p, bool reuse, bool with_v, int nqb,
                                hipStream_t stream) {
@@ -1374,7 +1451,22 @@ hipError_t launch_prefill_attn(const PrefillParams& p, bool reuse, bool with_v, 
                                : launch_attn_t<64, half_t>(p, reuse, with_v, nqb, stream);
 }
 
-hipError_t launch_prefill_aggregate(const PrefillParams& p0, hipStream_t stream) {
+// Pooling that selects saves a launch, its first trip to memory and the pooled scores' way there and back (pooling and
+// selection, 32/8 heads: 517 tokens 15.3 -> 11.3 us, 2048 32.7 -> 27.9, 3001 56.1 -> 52.6, 4096 90.3 -> 88.3; three prompts of
+// 2048 82.6 -> 76.3), but a tile's keys are not cut into parts then, which small calls need: where workgroups of eight
+// wavefronts do not make up for it they keep two launches.  Us with two launches / as the rule would have it:
+//   units up to 192, more than 6 tiles of 128 keys: 512 queries at 512 15.8/17.1, at 3584 32.2/38.5, 8/2 heads of 64, 2048 tokens
+//   13.8/15.9 (6 tiles: 32/8, 768 tokens 14.0/13.2);  193 to 256: 28/4, 2048 tokens 40.8/36.2, 1024 queries at 3072 47.8/43.7, but
+//   at head_dim 64, where products take half the time, 8/2 heads, 4096 tokens 24.6/26.2;  257 to 448: 32/8, 1536 tokens
+//   24.9/22.1, but 28/4, 3001 tokens (24 tiles) 68.4/69.8;  512: 2048 queries at 2048 74.0/66.3, 28/4, 4096 tokens 108.7/106.5.
+bool prefill_pool_selects(const PrefillParams& p) {
+    const int keys = p.q_start + kTile * (p.T - 1), tiles = (keys + 127) / 128;
+    const long long units = (long long)p.B * p.G * p.T;
+    if (keys > kPoolSelectKeys) return false;
+    return units > 448 || tiles <= (units > 256 ? 16 : units <= 192 ? 6 : p.head_dim == 64 ? 8 : 32);
+}
+
+hipError_t launch_prefill_aggregate(const PrefillParams& p0, const SelectParams* select, hipStream_t stream) {
     // one launch per sub-group of four query heads; the launches after the first add to the
     // pooled scores (launches on a stream run in order)
     PrefillParams p = p0;
@@ -1386,18 +1478,25 @@ hipError_t launch_prefill_aggregate(const PrefillParams& p0, hipStream_t stream)
     // LDS, first rows) costs as much as two or three.  32/8 heads: 1024 tokens 16.2 -> 11.9 us,
     // 2048 28.9 -> 26.0, chunks at position 12288 of 512 queries 159 -> 70, of 1024 168 -> 127, of 2048
     // 250 -> 251; with 752 units (3001 tokens) two parts 48.6 -> 50.2.
+    constexpr int kKT = 128;   // keys per tile
     const long long units = (long long)p.B * p.G * p.T;
-    const int max_tiles = std::max(1, (p.q_start + kTile * (p.T - 1) + kAggKT - 1) / kAggKT);
+    const int max_tiles = std::max(1, (p.q_start + kTile * (p.T - 1) + kKT - 1) / kKT);
     const int want = units <= 512 ? (int)((1024 + units - 1) / units) : 1;
     p.part_tiles = std::max((max_tiles + want - 1) / want, std::min(4, max_tiles));
     p.key_parts = (max_tiles + p.part_tiles - 1) / p.part_tiles;
     for (int v = 0; v < subs; ++v) {
         p.vsub = v;
+        const SelectParams* sel = v == subs - 1 ? select : nullptr;
+        if (sel) {
+            p.key_parts = 1;
+            p.pool_waves = units <= kWidePoolUnits ? 8 : 4;
+            p.part_tiles = max_tiles;
+        }
         hipError_t e;
         if (p.head_dim == 128)
-            e = p.elem == kElemBF16 ? launch_aggregate_t<128, bf16_t>(p, stream) : launch_aggregate_t<128, half_t>(p, stream);
+            e = p.elem == kElemBF16 ? launch_aggregate_t<128, bf16_t>(p, sel, stream) : launch_aggregate_t<128, half_t>(p, sel, stream);
         else
-            e = p.elem == kElemBF16 ? launch_aggregate_t<64, bf16_t>(p, stream) : launch_aggregate_t<64, half_t>(p, stream);
+            e = p.elem == kElemBF16 ? launch_aggregate_t<64, bf16_t>(p, sel, stream) : launch_aggregate_t<64, half_t>(p, sel, stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -813,6 +813,45 @@ def prefill_chunk_aggregate(Q, K_pages, log_sum, scores, block_table, q_start: i
         _ptr(q_lens), _stream()))
 
 
+def prefill_anchor_topk(Q, K, log_sum, scores, k: int, valid_len, n_sel, fill_value: Optional[int] = None,
+                        block_table: Optional[torch.Tensor] = None, q_start: int = 0, page_size: int = 16,
+                        q_starts=None, q_lens=None):
+    """``aggregate_kernel`` and ``torch.topk`` of a prompt or chunk in one call (EfficientKascadeStrategy.py:81-82):
+    ``prefill_aggregate_range`` or, with a block table, ``prefill_chunk_aggregate``, then ``topk_indices`` -- one launch
+    where the rows are short.  ``scores`` [B,G,ceil(Lq/32),q_start+Lq] is scratch.  Returns the indices or, with a
+    block table, (indices, cache_rows)."""
+    lib = _lib.init()
+    if block_table is not None:
+        B, Lq, qs, shape = _chunk_args(Q, K, block_table, q_start, page_size, q_starts, q_lens)
+        ks, pages = None, (_ptr(block_table), block_table.shape[1], page_size, K.shape[0], _ptr(q_starts), _ptr(q_lens))
+    else:
+        shape = _shape(Q, K)
+        _req(Q, shape[3], "Q", False); _req(K, shape[3], "K", False)
+        B, Lq = Q.shape[:2]
+        qs, ks, pages = _blhd_strides(Q, "Q"), ctypes.byref(_blhd_strides(K, "K")), (None, 0, 1, 0, None, None)
+        if K.shape[1] < q_start + Lq:
+            raise KascadeError("K must hold the positions up to q_start + rows of Q")
+    Hq, Gk, Dh, dt = shape
+    _req(log_sum, torch.float32, "log_sum"); _req(scores, torch.float16, "scores")
+    _req(valid_len, torch.int32, "valid_len"); _req(n_sel, torch.int32, "n_sel")
+    T, Lk = (Lq + TILE - 1) // TILE, q_start + Lq
+    if tuple(scores.shape) != (B, Gk, T, Lk):
+        raise KascadeError("scores must be [B,G,ceil(Lq/32),q_start+Lq]")
+    if log_sum.dim() != 3 or log_sum.shape[0] != B or log_sum.shape[2] != Hq or log_sum.shape[1] != Lq:
+        raise KascadeError("log_sum must be [B,Lq,H]")
+    if valid_len.numel() != n_sel.numel() or valid_len.numel() == 0:
+        raise KascadeError("valid_len and n_sel must have the same length")
+    idx = torch.empty(B, Gk, T, k, device=Q.device, dtype=torch.int32)
+    rows = torch.empty_like(idx) if block_table is not None else None
+    ws_bytes = lib.kascade_topk_workspace_bytes(B * Gk * T, Lk)
+    ws = _topk_workspace(ws_bytes, Q.device) if ws_bytes > 0 else None
+    _lib.check(lib.kascade_prefill_anchor_topk_call(
+        ctypes.byref(_lib.Shape(Gk, Dh, _ELEM[dt], Hq // Gk)), _ptr(Q), _ptr(K), _ptr(log_sum), _ptr(scores), _ptr(idx), _ptr(rows), B, q_start, Lq, qs, ks, *pages[:4],
+        *pages[4:], _ptr(valid_len), _ptr(n_sel), valid_len.numel(), k, Lk - 1 if fill_value is None else fill_value, _ptr(ws),
+        _stream()))
+    return idx if block_table is None else (idx, rows)
+
+
 def translate_indices(token_idx, block_table, kv_len: int, page_size: int = 16, out=None):
     """Token positions [B, ...] -> rows of the paged cache (block_table[b, t // page] * page +
     t % page), what the chunked reuse kernel gathers from."""

@@ -540,14 +540,13 @@ class PagedKascadePrefill:
                                                  self.page_size, with_output=(layer == 0),
                                                  q_starts=qs_dev, q_lens=ql_dev)
         scores = self._score_buffer(B, T, Lk)
-        kernels.prefill_chunk_aggregate(q, k_pages, log_sum, scores, block_table, qs_max, self.page_size,
-                                        q_starts=qs_dev, q_lens=ql_dev)
         if qs_dev is None:
             valid, nsel = self._tile_budgets(qs_max, Lq, width)
         else:
             valid, nsel = self._ragged_budgets(starts, lens, Lq, width)
-        self._topk_to_reuse, self._rows_to_reuse = kernels.topk_indices(
-            scores, width, valid_len=valid, n_sel=nsel, block_table=block_table, page_size=self.page_size)
+        self._topk_to_reuse, self._rows_to_reuse = kernels.prefill_anchor_topk(
+            q, k_pages, log_sum, scores, width, valid, nsel, block_table=block_table, q_start=qs_max, page_size=self.page_size,
+            q_starts=qs_dev, q_lens=ql_dev)
         if layer != 0:
             o = self._reuse(q, k_pages, v_pages, block_table, qs_max, self._hm[None], qs_dev, ql_dev)
         return o

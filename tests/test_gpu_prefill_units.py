@@ -335,3 +335,92 @@ def test_sparse_rows_do_not_depend_on_the_cut_of_a_unit(cuda, heads, G, D, L, co
     want = orc.reuse_prefill(q.cpu(), k, v, idx.cpu(), maps.tolist(), 32, True, float(p))
     atol, rtol = (2e-3, 1e-2) if dtype == torch.float16 else (1.6e-2, 2e-2)   # one rounding of P and of the output
     assert_close(one, want, "sparse rows", atol=atol, rtol=rtol)
+
+
+def _anchor_inputs(cuda, gen, heads, G, D, L, B, dtype):
+    q = torch.randn(B, L, heads, D, generator=gen).to(dtype).to(cuda)
+    k = torch.randn(B, L, G, D, generator=gen).to(dtype)
+    k[:, 0] += 1.0
+    k[:, 5:40] = k[:, 4:5]   # equal keys: ties
+    return q, k
+
+
+# units and key tiles on both sides of each line of the rule: 192 units with 6 tiles and with 7, 216 and 256 units, head_dim 64
+# with 8 and 9 tiles, 264 and 448 units, 16 and 17 tiles, 456 units, rows of up to 4096 keys and longer ones; tails of every kind
+@pytest.mark.parametrize("heads,G,D,L,B,dtype", [
+    (32, 8, 128, 1, 1, torch.float16), (32, 8, 128, 33, 1, torch.bfloat16), (32, 8, 128, 768, 1, torch.float16),
+    (28, 4, 128, 897, 1, torch.bfloat16), (32, 8, 128, 843, 1, torch.float16), (32, 8, 128, 1024, 1, torch.float16),
+    (32, 8, 64, 1024, 1, torch.float16), (32, 8, 64, 1025, 1, torch.float16), (8, 2, 64, 2049, 2, torch.bfloat16),
+    (40, 8, 128, 1050, 1, torch.float16), (32, 8, 128, 1791, 1, torch.float16), (28, 4, 128, 2081, 1, torch.float16),
+    (28, 4, 128, 2050, 1, torch.bfloat16), (24, 8, 128, 1801, 1, torch.float16), (14, 2, 64, 4128, 2, torch.float16),
+    (4, 4, 128, 4128, 1, torch.float16), (4, 4, 128, 4129, 1, torch.float16), (16, 1, 64, 517, 3, torch.float16)])
+def test_pooling_that_selects_gives_the_lists_of_two_launches(cuda, heads, G, D, L, B, dtype):
+    """Prompts, strided and over shuffled pages: the lists of pooling and selection by calls of their own."""
+    from kascade_amd import budgets, kernels
+    gen = torch.Generator().manual_seed(L + heads)
+    q, k = _anchor_inputs(cuda, gen, heads, G, D, L, B, dtype)
+    kp, table = _paged_copies(k[:1], 16, gen, 1, cuda)
+    k = k.to(cuda)
+    log_sum = kernels.prefill_recompute1(q, k)
+    T = (L + 31) // 32
+    for p, rolling in ((10, True), (5, False)):
+        W = budgets.topk_width(L, p)
+        valid, nsel = (torch.tensor(x, dtype=torch.int32, device=cuda)
+                       for x in budgets.prefill_tile_budgets(L, 32, p, rolling, W))
+        scores = torch.full((B, G, T, L), float("nan"), device=cuda, dtype=torch.float16)
+        kernels.prefill_aggregate(q, k, log_sum, scores)
+        want = kernels.topk_indices(scores, W, valid_len=valid, n_sel=nsel, fill_value=L - 1)
+        got = kernels.prefill_anchor_topk(q, k, log_sum, torch.empty_like(scores), W, valid, nsel)
+        assert torch.equal(got, want)
+        own, rows = kernels.prefill_anchor_topk(q[:1], kp, log_sum[:1].contiguous(), torch.empty_like(scores[:1]), W, valid, nsel,
+                                                block_table=table)
+        assert torch.equal(own, want[:1]) and torch.equal(rows, kernels.translate_indices(own.contiguous(), table, L, 16))
+
+
+@pytest.mark.parametrize("heads,G,D,start,n,B", [(32, 8, 128, 0, 512, 1), (32, 8, 128, 1024, 1024, 1), (32, 8, 128, 2048, 2048, 1),
+                                                 (28, 4, 128, 2048, 2017, 1), (8, 2, 64, 256, 300, 4), (64, 8, 128, 64, 500, 3)])
+def test_pooling_that_selects_over_chunks(cuda, heads, G, D, start, n, B):
+    """Chunks at one position and, with starts and row counts of their own (none and remainders among them), mixed ones:
+    the lists and cache rows of two launches."""
+    from kascade_amd import kernels
+    from kascade_amd.strategy import PagedKascadePrefill
+    gen = torch.Generator().manual_seed(start + n)
+    L, T = start + n, (n + 31) // 32
+    q, k = _anchor_inputs(cuda, gen, heads, G, D, L, B, torch.float16)
+    kp, table = _paged_copies(k[:1], 8, gen, B, cuda)
+    q = q[:, start:].contiguous()
+    rule = PagedKascadePrefill(10, [list(range(G))], [0], page_size=8, device=cuda, kv_heads=G)
+    starts = [(32 * b) % (start + 32) // 32 * 32 for b in range(B)]
+    lens = [(n, 0, n - 17, 1)[b % 4] for b in range(B)]
+    for mixed in (False, True):
+        at, rows_of = (starts, lens) if mixed else (start, None)
+        qs, qs_dev, ql_dev, s, c = rule._geometry(at, rows_of, n)
+        Lk = qs + n
+        W = 128 * -(-max(128, Lk // 10) // 128)
+        valid, nsel = rule._ragged_budgets(s, c, n, W) if mixed else rule._tile_budgets(qs, n, W)
+        log_sum, _ = kernels.prefill_chunk_dense(q, kp, kp, table, qs, 8, with_output=False, q_starts=qs_dev, q_lens=ql_dev)
+        scores = torch.zeros(B, G, T, Lk, device=cuda, dtype=torch.float16)
+        kernels.prefill_chunk_aggregate(q, kp, log_sum, scores, table, qs, 8, q_starts=qs_dev, q_lens=ql_dev)
+        want = kernels.topk_indices(scores, W, valid_len=valid, n_sel=nsel, block_table=table, page_size=8)
+        got = kernels.prefill_anchor_topk(q, kp, log_sum, torch.empty_like(scores), W, valid, nsel, block_table=table, q_start=qs,
+                                          page_size=8, q_starts=qs_dev, q_lens=ql_dev)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), f"mixed {mixed}"
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 60000.0])
+def test_pooling_that_selects_takes_keys_of_every_value(cuda, value):
+    """Keys that make scores infinite or no number, one and a whole tile of them: the lists of two launches."""
+    from kascade_amd import budgets, kernels
+    L, G = 700, 8
+    gen = torch.Generator().manual_seed(3)
+    q, k = _anchor_inputs(cuda, gen, 32, G, 128, L, 1, torch.float16)
+    k[0, 200:340, 1] = value
+    k[0, 50, 2, 3] = value
+    k = k.to(cuda)
+    log_sum = kernels.prefill_recompute1(q, k)
+    T, W = (L + 31) // 32, budgets.topk_width(L, 10)
+    valid, nsel = (torch.tensor(x, dtype=torch.int32, device=cuda) for x in budgets.prefill_tile_budgets(L, 32, 10, True, W))
+    scores = torch.empty(1, G, T, L, device=cuda, dtype=torch.float16)
+    kernels.prefill_aggregate(q, k, log_sum, scores)
+    want = kernels.topk_indices(scores, W, valid_len=valid, n_sel=nsel, fill_value=L - 1)
+    assert torch.equal(kernels.prefill_anchor_topk(q, k, log_sum, torch.empty_like(scores), W, valid, nsel), want)
