@@ -10,11 +10,11 @@
 //   registers, no LDS store instructions) into one of two buffers, so a tile costs one
 //   barrier: wait for the own loads, barrier, start the next tile's loads into the other
 //   buffer, compute.  Rows lie in LDS as they lie in memory; the 16-byte chunk c of row R
-//   sits at chunk c ^ swz(R) (swz16 in sparse units), chosen by the lane that fetches it (each lane picks the global
+//   sits at chunk c ^ swz(R) (swz16 and swz_pairs for 16x16x32 products), chosen by the lane that fetches it (each lane picks the global
 //   chunk that belongs at its LDS position), which makes both read patterns below free of
 //   bank conflicts without padding.
 //
-//   The kernel works on S^T = K Q^T so that two lanes (four in sparse units) own one query column:
+//   The kernel works on S^T = K Q^T so that two lanes (four of 16x16x32 products) own one query column:
 //   row max / row sum are in-lane reductions plus one or two exchanges, and
 //   the exponentiated scores are already in the B-operand layout of the second
 //   product O^T = V^T P^T -- P never leaves registers.  The A operand of that product,
@@ -24,7 +24,7 @@
 //   What bounds long calls is the chip's power, and per product 16x16x32 takes less of it than 32x32x16 (1.84
 //   against 1.59 PFLOP/s on random operands in registers): sparse units use it (32/8 heads: 3001 tokens 23.8 -> 23.1 us,
 //   4096 31.6 -> 30.4, 16384 277 -> 262, 32768 982 -> 933; no gain at 2048 tokens, 12.8 both and in bf16 12.6 -> 12.8, nor
-//   below).  Dense passes and pooling keep 32x32x16 (see there).  Against row addresses formed by a
+//   below), and dense passes with an output at head_dim 128; the others keep 32x32x16 (see there).  Against row addresses formed by a
 //   64-bit product per tensor and row and block-table entries requested behind the tile's loads: dense 517 tokens
 //   14.6 -> 13.5 us, 2048 49.4 -> 46.9, chunks at position 14336 of 512 queries 326 -> 247 us, of 2048 532 -> 520;
 //   log-sums alone 517 10.2 -> 9.6 us, 32768 4.39 -> 4.24 ms, chunks of 512 205 -> 173 us, of 2048 310 -> 301.
@@ -588,20 +588,31 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                            so, lrow, lchunk, last_q - q_off);
 }
 
-// Dense passes, with an output or for log-sums alone: products 32x32x16.  16x16x32 products were 6 % faster here (32768
-// tokens 8.1 -> 7.6 ms, log-sums alone 4.2 -> 3.9), but a row's sum is then spread over four lanes instead of two, and
-// the last bits of the log-sums decide between tokens whose pooled scores lie within one step at a selection's
-// threshold: single output rows of a 32768-token prompt moved by up to 0.27 of the outputs' root mean square.  The order
-// of the additions is all that differs: four chained 16x16x32 products and eight 32x32x16 ones gave the same bits in
-// all of 524288 dot products of 128 elements.
+// Dense passes, with an output or for log-sums alone.
+// A row's exponentials are added up in two lanes, as 32x32x16 products leave them, whatever the products: spread over the
+// four lanes of 16x16x32 ones the last bits of the log-sums differ, and they decide between tokens whose pooled scores lie
+// within one step at a selection's threshold (single output rows of a 32768-token prompt moved by up to 0.27 of the outputs'
+// root mean square).  The products' own bits are the same: four chained 16x16x32 products and eight 32x32x16 ones agreed
+// in all of 524288 dot products of 128 elements.
+// With an output at head_dim 128 (PAIRS): products 16x16x32, and half an instruction per score (swap_pairs) brings the
+// exponentials where they are added up.  Against 32x32x16 products, 32/8 heads: 32768 tokens 8.43 -> 7.75 ms, chunks of 2048
+// queries at up to 14336 284 -> 268 us, 2300 tokens 62.6 -> 59.7; 517, 1500 and 4096 the same.
+// Log-sums alone and pooling have half the products per score and wait for vector instructions: with
+// the swaps 32768 tokens 4.30 -> 4.34 ms and 4.71 -> 4.85; head_dim 64 with an output, 16000 tokens of 8/2 heads in bf16, 299 ->
+// 362 us, 4096 48.4 -> 51.7.  These keep 32x32x16.
 template <int NQB, bool WITH_V, bool PAGED, int D, typename T, bool SPARE>
 __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK, T* sV) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
+    // Products 16x16x32 (see above)
+    constexpr bool PAIRS = WITH_V && D == 128;
+    typedef typename std::conditional<PAIRS, float4_t, float16_t>::type Acc;
     typedef AttnTile<D> G_;
     constexpr int kKT = G_::kKT, kChunks = G_::kChunks, kRPL = G_::kRowsPerLoad, kTileElems = G_::kTileElems;
-    // products 32x32x16: contraction steps of S^T, 32-row blocks of O^T, 32-key blocks of a tile
-    constexpr int kKS = D / 16, kDB = D / 32, kKB = kKT / 32;
+    // rows and columns of a product; contraction steps of S^T, row blocks of O^T, key blocks of a tile, blocks of queries
+    constexpr int kOp = PAIRS ? 16 : 32;
+    constexpr int kKS = D * kOp / 512, kDB = D / kOp, kKB = kKT / kOp, kQB = NQB * 32 / kOp;
+    constexpr int kAcc = kOp * kOp / 64;   // elements of a result per lane
     constexpr float kScaleLog2 = ScaleLog2<D>::value;
     const HeadSlots hs = head_slots(p.gs);
     const int kvh = p.G, nheads = p.G * hs.gs;
@@ -631,6 +642,8 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     const int lane = tid & 63;
     const int li = lane & 31;
     const int lg = lane >> 5;
+    const int col = lane & (kOp - 1);   // of an operand or result
+    const int dq = lane / kOp;          // which 8 elements of a contraction step, which 4 rows of a result
     const int q0l = tq * QT;            // first query row of this block
     if (q0l >= Lqv) return;             // a block past this sequence's rows (uniform over the workgroup)
     const int q0 = q_start + q0l;       // its global position
@@ -677,7 +690,7 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     const char* lane_ptr[kPtrs];
 #pragma unroll
     for (int j = 0; j < kPtrs; ++j)
-        lane_ptr[j] = (const char*)(kbase + (lchunk ^ swz<D>(slot0 + j * kRPL)) * 8) +
+        lane_ptr[j] = (const char*)(kbase + (lchunk ^ (PAIRS ? swz_pairs<D>(slot0 + j * kRPL) : swz<D>(slot0 + j * kRPL))) * 8) +
                       (unsigned long long)row_bytes * (unsigned)(PAGED ? (pos0 + j) & page_mask : pos0 + j);
     const char* row_ptr[4];
     auto next_rows = [&](int ti) {
@@ -703,15 +716,18 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
         if constexpr (i < 4) load_to_lds_16<i * 1024>(row_ptr[i], lds_k + buf * (kTileElems * 2));
         else load_to_lds_16<(i - 4) * 1024>(row_ptr[i - 4] + v_from_k, lds_v + buf * (kTileElems * 2));
     };
-    // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 32 kb + li,
-    // chunk 2 ks + lg.  A operand of O^T (two transposing reads h = 0, 1 of four keys each):
-    // the 16 lanes of a group address rows 16 s + 8 h + 4 lg + (0..3) of a key block, 16 columns
-    // of V from column 32 db + 16 (group & 1) on, and receive one column of the four rows each.
-    const int kx = lg ^ swz<D>(li);
-    const int krd = li * D;
+    // LDS read positions (elements, within a tile buffer).  A operand of S^T: row 16 kb + pair_row(col), chunk 4 ks + dq; of
+    // 32x32x16 products row 32 kb + col, chunk 2 ks + dq.  A operand of O^T (two transposing reads h = 0, 1 of four
+    // keys each): the 16 lanes of a quarter address rows 32 s + 16 h + pair_row(4 dq) + (0..3), 16 columns of V from
+    // column 16 db on, and receive one column of the four rows each; of 32x32x16 products rows 16 s + 8 h + 4 lg + (0..3)
+    // of a key block, 16 columns from column 32 db + 16 (quarter & 1) on.
+    const int a_row = PAIRS ? pair_row(col) : col;
+    const int kx = dq ^ (PAIRS ? swz_pairs<D>(a_row) : swz<D>(a_row));
+    const int krd = a_row * D;
     const int vcol = lane & 15;
-    const int vrow = 4 * lg + (vcol >> 2);                          // + 32 kb + 16 s + 8 h
-    const int vchunk = 2 * ((lane >> 4) & 1) + ((vcol >> 1) & 1);    // + 4 db
+    const int vrow = (PAIRS ? pair_row(4 * dq) : 4 * lg) + (vcol >> 2);
+    const int vchunk = PAIRS ? ((vcol >> 1) & 1) ^ swz_pairs<D>(vrow)                  // ^ 2 db
+                             : 2 * ((lane >> 4) & 1) + ((vcol >> 1) & 1);               // + 4 db
     const int vrd = vrow * D + 4 * (vcol & 1);
 
     // Softmax state.  m[] is the reference the exponentials are taken against, in log2 units of
@@ -722,47 +738,48 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     // never.  The quotient is the same: numerator and denominator carry the same factor.
     constexpr int kPrio = WITH_V ? KASCADE_PRIO_V : KASCADE_PRIO_K;
     constexpr float kRefSlack = 8.f;
-    float m[NQB], l[NQB];
-    float16_t oT[NQB][kDB];
+    float m[kQB], l[NQB];    // m: of the queries kOp q + col; l: of the queries 32 qb + li
+    Acc oT[kQB][kDB];        // query block, kOp output columns
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        m[qb] = -INFINITY;
-        l[qb] = 0.f;
+    for (int q = 0; q < kQB; ++q) {
+        m[q] = -INFINITY;
 #pragma unroll
         for (int db = 0; db < kDB; ++db)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) oT[qb][db][v] = 0.f;
+            for (int v = 0; v < kAcc; ++v) oT[q][db][v] = 0.f;
     }
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) l[qb] = 0.f;
 
     fetch_page(0);
     next_rows(0);
     static_for<0, kNumLoads>([&](auto i) { issue_load(i, 0); });
     if (ntiles > 1) fetch_page(1);
 
-    // ---- Q fragments (B operand of S^T): query li (+32 qb), d chunk 16*ks + 8*lg; requested after
+    // ---- Q fragments (B operand of S^T): query kOp q + col, d chunk dq of step ks; requested after
     // the first tile's rows, which the first barrier waits for ----
-    x8_t qf[NQB][kKS];
+    x8_t qf[kQB][kKS];
     const int last_q = min(QT, Lqv - q0l) - 1;   // of this block
     const T* q_base = Qp + (long long)b * p.q_sb + (long long)q0l * p.q_sl + (long long)head * p.q_sh;
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        const T* qp = q_base + (unsigned long long)(unsigned)min(32 * qb + li, last_q) * (unsigned long long)p.q_sl + lg * 8;
+    for (int q = 0; q < kQB; ++q) {
+        const T* qp = q_base + (unsigned long long)(unsigned)min(kOp * q + col, last_q) * (unsigned long long)p.q_sl + dq * 8;
 #pragma unroll
         for (int ks = 0; ks < kKS; ++ks) {
             PackT<T> t;
-            t.u = ld_global_16(qp + ks * 16);
-            qf[qb][ks] = t.v8;
+            t.u = ld_global_16(qp + ks * (512 / kOp));
+            qf[q][ks] = t.v8;
         }
     }
     if (last_q < QT - 1) {   // uniform: rows past the sequence's end are zeros
 #pragma unroll
-        for (int qb = 0; qb < NQB; ++qb)
+        for (int q = 0; q < kQB; ++q)
 #pragma unroll
             for (int ks = 0; ks < kKS; ++ks)
-                if (32 * qb + li > last_q) qf[qb][ks] = x8_t{};
+                if (kOp * q + col > last_q) qf[q][ks] = x8_t{};
     }
 #pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) arrived<kKS>(qf[qb]);
+    for (int q = 0; q < kQB; ++q) arrived<kKS>(qf[q]);
 
     // One tile: next tile's loads, both products, softmax.  Two copies of
     // the code, each straight-line: tiles that need no mask (all but one or two of a unit) and tiles
@@ -787,18 +804,20 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
         const int nbuf = (sq + 1) & 1;
 
         tile_phase<kPrio>(0);
-        // ---- S^T = K_tile Q^T.  Step c = (key block c / kKS, contraction step c % kKS); operands are
+        // ---- S^T = K_tile Q^T.  Step c = (key block, contraction step), with an output two key blocks in turn; operands are
         // read from LDS two windows (four steps) ahead of the products that use them, in program
         // order, because LDS reads do not move across the load statements ----
         constexpr int kSteps = nkb * kKS;
-        float16_t sT[NQB][nkb];
-        float16_t zero16;
+        Acc sT[kQB][nkb];
+        Acc zero;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) zero16[v] = 0.f;
+        for (int v = 0; v < kAcc; ++v) zero[v] = 0.f;
+        auto key_block = [](int c) { return PAIRS ? 2 * (c / (2 * kKS)) + (c & 1) : c / kKS; };
+        auto k_step = [](int c) { return PAIRS ? (c % (2 * kKS)) >> 1 : c % kKS; };
         auto read_a = [&](int c) {
-            return *reinterpret_cast<const x8_t*>(&bK[32 * (c / kKS) * D + krd + ((2 * (c % kKS)) ^ kx) * 8]);
+            return *reinterpret_cast<const x8_t*>(&bK[kOp * key_block(c) * D + krd + ((64 / kOp * k_step(c)) ^ kx) * 8]);
         };
-        constexpr int kAhead = (kKB <= 2) ? 2 : 1;   // windows read ahead (registers are scarcer at D = 64)
+        constexpr int kAhead = (D == 128) ? 2 : 1;   // windows read ahead (registers are scarcer at D = 64)
         x8_t aw[kAhead + 1][2];
 #pragma unroll
         for (int c = 0; c < 2 * kAhead && c < kSteps; ++c) aw[c >> 1][c & 1] = read_a(c);
@@ -811,119 +830,121 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
             __builtin_amdgcn_sched_barrier(0);   // the scheduler would sink the reads to their use
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int kb = (2 * w + i) / kKS, ks = (2 * w + i) % kKS;
+                const int kb = key_block(2 * w + i), ks = k_step(2 * w + i);
 #pragma unroll
-                for (int qb = 0; qb < NQB; ++qb)   // the first product starts from a constant zero
-                    sT[qb][kb] = Elem<T>::mma_32x32x16(aw[w % (kAhead + 1)][i], qf[qb][ks], ks == 0 ? zero16 : sT[qb][kb]);
+                for (int q = 0; q < kQB; ++q) {   // the first product starts from a constant zero
+                    const Acc c = ks == 0 ? zero : sT[q][kb];
+                    if constexpr (PAIRS) sT[q][kb] = Elem<T>::mma_16x16x32(aw[w % (kAhead + 1)][i], qf[q][ks], c);
+                    else sT[q][kb] = Elem<T>::mma_32x32x16(aw[w % (kAhead + 1)][i], qf[q][ks], c);
+                }
             }
             if constexpr (w < kNumLoads) issue_load(w_c, nbuf);
         });
         static_for<kSteps / 2, kNumLoads>([&](auto i) { issue_load(i, nbuf); });
-        // ---- masks: accumulator v of key block kb is LDS row 32kb + 8(v/4) + 4lg + v%4 of the tile ----
+        // ---- masks: accumulator v of key block kb is LDS row 16 kb + pair_row(4 dq) + v of the tile
+        // (32x32x16: 32 kb + 8 (v/4) + 4 dq + v%4) ----
         if (MASKED) {   // the causal edge and the end of the sequence
 #pragma unroll
-            for (int qb = 0; qb < NQB; ++qb) {
-                const int q = q0 + 32 * qb + li;   // global position
+            for (int qb = 0; qb < kQB; ++qb) {
+                const int q = q0 + kOp * qb + col;   // global position
 #pragma unroll
                 for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int key = sq * kKT + pos_of_slot(32 * kb + 8 * (v >> 2) + 4 * lg + (v & 3));
+                    for (int v = 0; v < kAcc; ++v) {
+                        const int row = PAIRS ? pair_row(4 * dq) + v : 8 * (v >> 2) + 4 * dq + (v & 3);
+                        const int key = sq * kKT + pos_of_slot(kOp * kb + row);
                         if (key > q || key >= L) sT[qb][kb][v] = -INFINITY;
                     }
             }
         }
-        // ---- online softmax (one query column per lane pair: lanes li and li + 32) ----
+        // ---- online softmax (a query's scores lie in the four lanes of equal col; of 32x32x16 products in two) ----
         tile_phase<kPrio>(1);
-        x8_t pf[NQB][2 * nkb];
+        if constexpr (PAIRS) {
+            x8_t pf[2][nkb / 2];
+            float ms[2];
 #pragma unroll
-        for (int qb = 0; qb < NQB; ++qb) {
-            float sum;
-            auto exponentials = [&](float mu) {
-                sum = 0.f;
-                float e[nkb][16];
-                // At head_dim 64 a tile's 64 additions stand behind all of its exponentials: mixed with them, as at 128,
-                // their chain holds these up (14/2 heads, 4096 tokens: log-sums alone 48.6 -> 45.6 us, dense 66.7 ->
-                // 60.6; 32/8 heads: 53.2 -> 51.7 and 88.7 -> 84.0; a chunk of 2048 queries at 14336 196 -> 181 and 293
-                // -> 277; slower at 3001 tokens of 32/8 heads, log-sums alone 32.7 -> 33.7, and 8192 of 14/2, dense 188
-                // -> 193).  The order of addition is the same.
-                constexpr bool kSumsBehind = D == 64;
-#pragma unroll
-                for (int kb = 0; kb < nkb; ++kb)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        e[kb][v] = fast_exp2(__builtin_fmaf(sT[qb][kb][v], kScaleLog2, -mu));
-                        if (!kSumsBehind) sum += e[kb][v];
-                    }
-                if (WITH_V) {
-#pragma unroll
-                    for (int s = 0; s < 2 * nkb; ++s) {
-                        x8_t t;
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) t[i] = (T)e[s >> 1][8 * (s & 1) + i];
-                        pf[qb][s] = t;
-                    }
-                }
-                if (kSumsBehind) {
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int kb = 0; kb < nkb; ++kb)
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) sum += e[kb][v];
-                }
-            };
-            // Log-sums alone: the maximum is only formed on a unit's first tiles, which move the reference often (16 of 64
-            // keys, all of 128), and where a lane's sum says that a score may lie kRefSlack above the reference (its
-            // exponential alone is 2^kRefSlack then), or is no number (the reference still is -inf); then the
-            // exponentials are formed anew.  The rule is the same: the log-sums have the bits of the pass with an output.
-            constexpr float kSumLimit = 250.f;
-            bool look = WITH_V || D == 64 || sq < 16;   // wavefront-uniform
-            if (!look) {
-                exponentials(m[qb]);
-                look = __any(!(sum <= kSumLimit));
-            }
-            if (look) {
+            for (int q = 0; q < 2; ++q) {
                 float mx = -INFINITY;
 #pragma unroll
                 for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sT[qb][kb][v]);
-                const float ms = mx * kScaleLog2;
-                if (__any(ms > m[qb] + kRefSlack)) {   // wavefront-uniform
-                    const float mnew = fmaxf(m[qb], max_with_other_half(ms));   // the same in both lanes of a column
-                    const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[qb] - mnew);
-                    m[qb] = mnew;
-                    l[qb] *= corr;
-                    if (WITH_V) {
-#pragma unroll
-                        for (int db = 0; db < kDB; ++db)
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) oT[qb][db][v] *= corr;
-                    }
-                }
-                exponentials((m[qb] == -INFINITY) ? 0.f : m[qb]);
+                    for (int v = 0; v < 4; ++v) mx = fmaxf(mx, sT[q][kb][v]);
+                ms[q] = mx * kScaleLog2;
             }
-            l[qb] += sum;   // per-lane partial sum (own key positions)
-        }
-        tile_phase<kPrio>(2);
-        // ---- O^T += V^T P^T: step s covers the keys of accumulators 8(s&1) .. 8(s&1)+7 of key block
-        // s/2, i.e. rows 16 s + 8 h + 4 lg + (0..3), h = 0, 1, of the tile.  The operands of a block
-        // of 32 output rows are read while the block before it is multiplied ----
-        if (WITH_V) {
-            constexpr int kPS = 2 * nkb;
+            if (__any(ms[0] > m[0] + kRefSlack || ms[1] > m[1] + kRefSlack)) {   // wavefront-uniform
+                float corr[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const float mnew = fmaxf(m[q], max_over_quarters(ms[q]));   // the same in the four lanes of a column
+                    corr[q] = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
+                    m[q] = mnew;
+#pragma unroll
+                    for (int db = 0; db < kDB; ++db) oT[q][db] *= corr[q];
+                }
+                l[0] *= lane & 16 ? corr[1] : corr[0];
+            }
+            const float mu[2] = {m[0] == -INFINITY ? 0.f : m[0], m[1] == -INFINITY ? 0.f : m[1]};
+            float sum = 0.f;
+            float4_t e[2][nkb];
+            // The sums are formed where and as those of the pass for log-sums alone: in two lanes per query, by the same
+            // additions (lane & 16 picks a lane's query of the two whose reference it holds).  Behind the conversions: the
+            // swap is made in place then, in front of them the compiler copied every exponential first (32768
+            // tokens 7.74 ms both, 4096 156 -> 149 us, 517 17.0 -> 15.9).
+            auto add = [&](int kb) {
+                float4_t first, second;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float x, y;
+                    swap_pairs(e[0][kb][v], e[1][kb][v], x, y);
+                    first[v] = x;
+                    second[v] = y;
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sum += first[v];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sum += second[v];
+            };
+#pragma unroll
+            for (int st = 0; st < nkb / 2; ++st) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    x8_t t;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const int kb = 2 * st + (i >> 2), v = i & 3;
+                        e[q][kb][v] = fast_exp2(__builtin_fmaf(sT[q][kb][v], kScaleLog2, -mu[q]));
+                        t[i] = (T)e[q][kb][v];
+                    }
+                    pf[q][st] = t;
+                }
+                if (st > 0) {
+                    add(2 * st - 2);
+                    add(2 * st - 1);
+                }
+            }
+            add(nkb - 2);
+            add(nkb - 1);
+            l[0] += sum;   // per-lane partial sum (own key positions)
+            tile_phase<kPrio>(2);
+            // ---- O^T += V^T P^T: step s covers the keys of blocks 2 s and 2 s + 1, whose scores lane dq holds: rows
+            // 32 s + 16 h + pair_row(4 dq) + (0..3), h = 0, 1, of the tile.  The operands of a group of steps are read
+            // while the group before it is multiplied ----
+            constexpr int kPS = nkb / 2;
             auto read_v = [&](int db, int s, int h) {
-                const int row = 16 * s + 8 * h;   // + vrow; only its low four bits enter swz
-                const T* vp = bV + row * D + vrd + ((4 * db + vchunk) ^ swz<D>(row + vrow)) * 8;
+                const T* vp = bV + (32 * s + 16 * h) * D + vrd + ((2 * db) ^ vchunk) * 8;
                 return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
             };
-            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block)
-            constexpr int kGrp = (kKB <= 2) ? 4 : 2;
+            // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block),
+            // two column blocks in turn
+            constexpr int kGrp = (D == 128) ? 4 : 2;
             constexpr int kGroupsPV = kDB * kPS / kGrp;
+            auto out_block = [](int t) { return 2 * (t / (2 * kPS)) + (t & 1); };
+            auto p_step = [](int t) { return (t % (2 * kPS)) >> 1; };
             short4_t av[2][kGrp][2];
 #pragma unroll
             for (int i = 0; i < kGrp; ++i)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(i / kPS, i % kPS, h);
+                for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(out_block(i), p_step(i), h);
 #pragma unroll
             for (int gq = 0; gq < kGroupsPV; ++gq) {
                 if (gq + 1 < kGroupsPV) {
@@ -931,17 +952,127 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
                     for (int i = 0; i < kGrp; ++i)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
-                            av[(gq + 1) & 1][i][h] = read_v((kGrp * (gq + 1) + i) / kPS, (kGrp * (gq + 1) + i) % kPS, h);
+                            av[(gq + 1) & 1][i][h] = read_v(out_block(kGrp * (gq + 1) + i), p_step(kGrp * (gq + 1) + i), h);
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int i = 0; i < kGrp; ++i) {
-                    const int db = (kGrp * gq + i) / kPS, s = (kGrp * gq + i) % kPS;
+                    const int db = out_block(kGrp * gq + i), s = p_step(kGrp * gq + i);
                     const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
                     const x8_t a = __builtin_bit_cast(x8_t, both);
 #pragma unroll
-                    for (int qb = 0; qb < NQB; ++qb)
-                        oT[qb][db] = Elem<T>::mma_32x32x16(a, pf[qb][s], oT[qb][db]);
+                    for (int q = 0; q < 2; ++q) oT[q][db] = Elem<T>::mma_16x16x32(a, pf[q][s], oT[q][db]);
+                }
+            }
+        } else {
+            x8_t pf[NQB][2 * nkb];
+#pragma unroll
+            for (int qb = 0; qb < NQB; ++qb) {
+                float sum;
+                auto exponentials = [&](float mu) {
+                    sum = 0.f;
+                    float e[nkb][16];
+                    // At head_dim 64 a tile's 64 additions stand behind all of its exponentials: mixed with them, as at 128,
+                    // their chain holds these up (14/2 heads, 4096 tokens: log-sums alone 48.6 -> 45.6 us, dense 66.7 ->
+                    // 60.6; 32/8 heads: 53.2 -> 51.7 and 88.7 -> 84.0; a chunk of 2048 queries at 14336 196 -> 181 and 293
+                    // -> 277; slower at 3001 tokens of 32/8 heads, log-sums alone 32.7 -> 33.7, and 8192 of 14/2, dense 188
+                    // -> 193).  The order of addition is the same.
+                    constexpr bool kSumsBehind = D == 64;
+#pragma unroll
+                    for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            e[kb][v] = fast_exp2(__builtin_fmaf(sT[qb][kb][v], kScaleLog2, -mu));
+                            if (!kSumsBehind) sum += e[kb][v];
+                        }
+                    if (WITH_V) {
+#pragma unroll
+                        for (int s = 0; s < 2 * nkb; ++s) {
+                            x8_t t;
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) t[i] = (T)e[s >> 1][8 * (s & 1) + i];
+                            pf[qb][s] = t;
+                        }
+                    }
+                    if (kSumsBehind) {
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) sum += e[kb][v];
+                    }
+                };
+                // Log-sums alone: the maximum is only formed on a unit's first tiles, which move the reference often (16 of 64
+                // keys, all of 128), and where a lane's sum says that a score may lie kRefSlack above the reference (its
+                // exponential alone is 2^kRefSlack then), or is no number (the reference still is -inf); then the
+                // exponentials are formed anew.  The rule is the same: the log-sums have the bits of the pass with an output.
+                constexpr float kSumLimit = 250.f;
+                bool look = WITH_V || D == 64 || sq < 16;   // wavefront-uniform
+                if (!look) {
+                    exponentials(m[qb]);
+                    look = __any(!(sum <= kSumLimit));
+                }
+                if (look) {
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int kb = 0; kb < nkb; ++kb)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sT[qb][kb][v]);
+                    const float ms = mx * kScaleLog2;
+                    if (__any(ms > m[qb] + kRefSlack)) {   // wavefront-uniform
+                        const float mnew = fmaxf(m[qb], max_with_other_half(ms));   // the same in both lanes of a column
+                        const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[qb] - mnew);
+                        m[qb] = mnew;
+                        l[qb] *= corr;
+                        if (WITH_V) {
+#pragma unroll
+                            for (int db = 0; db < kDB; ++db)
+#pragma unroll
+                                for (int v = 0; v < 16; ++v) oT[qb][db][v] *= corr;
+                        }
+                    }
+                    exponentials((m[qb] == -INFINITY) ? 0.f : m[qb]);
+                }
+                l[qb] += sum;   // per-lane partial sum (own key positions)
+            }
+            tile_phase<kPrio>(2);
+            // ---- O^T += V^T P^T: step s covers the keys of accumulators 8(s&1) .. 8(s&1)+7 of key block
+            // s/2, i.e. rows 16 s + 8 h + 4 lg + (0..3), h = 0, 1, of the tile.  The operands of a block
+            // of 32 output rows are read while the block before it is multiplied ----
+            if (WITH_V) {
+                constexpr int kPS = 2 * nkb;
+                auto read_v = [&](int db, int s, int h) {
+                    const int row = 16 * s + 8 * h;   // + vrow; only its low four bits enter swz
+                    const T* vp = bV + row * D + vrd + ((4 * db + vchunk) ^ swz<D>(row + vrow)) * 8;
+                    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)vp);
+                };
+                // steps in groups of kGrp (a group = 2 kGrp transposing reads, kGrp products per query block)
+                constexpr int kGrp = (kKB <= 2) ? 4 : 2;
+                constexpr int kGroupsPV = kDB * kPS / kGrp;
+                short4_t av[2][kGrp][2];
+#pragma unroll
+                for (int i = 0; i < kGrp; ++i)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) av[0][i][h] = read_v(i / kPS, i % kPS, h);
+#pragma unroll
+                for (int gq = 0; gq < kGroupsPV; ++gq) {
+                    if (gq + 1 < kGroupsPV) {
+#pragma unroll
+                        for (int i = 0; i < kGrp; ++i)
+#pragma unroll
+                            for (int h = 0; h < 2; ++h)
+                                av[(gq + 1) & 1][i][h] = read_v((kGrp * (gq + 1) + i) / kPS, (kGrp * (gq + 1) + i) % kPS, h);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < kGrp; ++i) {
+                        const int db = (kGrp * gq + i) / kPS, s = (kGrp * gq + i) % kPS;
+                        const short8_t both = __builtin_shufflevector(av[gq & 1][i][0], av[gq & 1][i][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        const x8_t a = __builtin_bit_cast(x8_t, both);
+#pragma unroll
+                        for (int qb = 0; qb < NQB; ++qb)
+                            oT[qb][db] = Elem<T>::mma_32x32x16(a, pf[qb][s], oT[qb][db]);
+                    }
                 }
             }
         }
@@ -977,10 +1108,31 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
     for (int qb = 0; qb < NQB; ++qb) {
         const int ql = q0l + 32 * qb + li;
         const float lt = sum_with_other_half(l[qb]);
+        const float ref = !PAIRS ? m[qb] : lane & 16 ? m[kQB - 1] : m[0];
         if (p.log_sum && lg == 0 && ql < Lqv)
-            p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + m[qb];
-        if (WITH_V) {
-            T* so = sK + wave * (32 * D);
+            p.log_sum[((long long)b * Lq + ql) * nheads + head] = fast_log2(lt) + ref;
+        T* so = sK + wave * (32 * D);
+        auto store = [&]() {
+            __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
+            store_rows<D, 32>((T*)p.O + ((long long)b * Lq + q0l) * nheads * D + (long long)head * D, (unsigned)(nheads * D), so, lrow,
+                              lchunk, last_q);
+        };
+        if constexpr (PAIRS) {
+            const float inv_li = 1.f / lt;
+            float inv[2];   // of the queries 16 q + col
+            swap_pairs(inv_li, inv_li, inv[0], inv[1]);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int row = 16 * q + col;
+#pragma unroll
+                for (int db = 0; db < kDB; ++db) {   // d = 16 db + 4 dq .. +3: half of chunk 2 db + dq / 2
+                    const x4_t o = {(T)(oT[q][db][0] * inv[q]), (T)(oT[q][db][1] * inv[q]), (T)(oT[q][db][2] * inv[q]),
+                                    (T)(oT[q][db][3] * inv[q])};
+                    *reinterpret_cast<x4_t*>(&so[row * D + (((2 * db + (dq >> 1)) ^ (row & (kChunks - 1))) * 8) + 4 * (dq & 1)]) = o;
+                }
+            }
+            store();
+        } else if constexpr (WITH_V) {
             const float inv = 1.f / lt;
 #pragma unroll
             for (int db = 0; db < kDB; ++db)
@@ -990,9 +1142,7 @@ __device__ __forceinline__ void prefill_dense_body(const PrefillParams& p, T* sK
                               (T)(oT[qb][db][4 * v4 + 2] * inv), (T)(oT[qb][db][4 * v4 + 3] * inv)};
                     *reinterpret_cast<x4_t*>(&so[li * D + (((4 * db + v4) ^ (li & (kChunks - 1))) * 8) + 4 * lg]) = o;
                 }
-            __builtin_amdgcn_wave_barrier();   // the reads below are other lanes' writes (same wavefront: in order)
-            store_rows<D, 32>((T*)p.O + ((long long)b * Lq + q0l) * nheads * D + (long long)head * D, (unsigned)(nheads * D), so, lrow,
-                          lchunk, last_q);
+            store();
         }
     }
 }

@@ -34,6 +34,19 @@ template <int D> __device__ __forceinline__ int swz(int row);
 template <> __device__ __forceinline__ int swz<128>(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 template <> __device__ __forceinline__ int swz<64>(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 
+// Exponentials of 16x16x32 products in the places they have after 32x32x16 ones.  A result of 16 columns has a column
+// in four lanes, of 32 columns in two; v_permlane16_swap of two results of 16 columns each gives lane (lg, li) rows
+// 0 .. 3 of quarter 2 lg (first) and 2 lg + 1 (second) of column li.  With operand row r taken from row pair_row(r) of
+// the 16 that is rows 4 lg + (0..3) and 8 + 4 lg + (0..3), as a 32x32x16 product has them.
+__device__ __forceinline__ int pair_row(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
+__device__ __forceinline__ void swap_pairs(float x, float y, float& first, float& second) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y), false, false);
+    first = __builtin_bit_cast(float, (uint32_t)r[0]);
+    second = __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+// swz16 for operands whose rows are taken in that order
+template <int D> __device__ __forceinline__ int swz_pairs(int row) { return swz16<D>(pair_row(row)); }
+
 // One wavefront-wide load of 16 bytes per lane from global memory into LDS: lane i's bytes
 // land at lds_base + OFF + 16 i (lds_base wavefront-uniform).  Counted by vmcnt like any load; the
 // compiler does not know that it writes LDS, so whoever reads the bytes waits for vmcnt and

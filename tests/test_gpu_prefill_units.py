@@ -203,6 +203,26 @@ def test_attention_over_pages_of_every_size(cuda, page, heads, G, D, dtype):
         assert torch.equal(o, sparse_alone[:, start:end]), f"sparse rows {start}..{end}, no log-sums"
 
 
+@pytest.mark.parametrize("L", [1, 15, 16, 17, 33, 47, 64, 65, 95, 129, 260])
+@pytest.mark.parametrize("heads,G,dtype", [(32, 8, torch.float16), (7, 1, torch.bfloat16)])
+def test_dense_rows_at_the_edges_of_query_and_key_blocks(cuda, L, heads, G, dtype):
+    """Products of 16 queries whose exponentials are added up as those of 32: the log-sums have the bits of the pass
+    for log-sums alone, outputs and log-sums are the oracle's (outputs to a rounding of the probabilities and one of the
+    result)."""
+    from kascade_amd import kernels
+    gen = torch.Generator().manual_seed(L)
+    q = torch.randn(2, L, heads, 128, generator=gen).to(dtype)
+    k, v = (torch.randn(2, L, G, 128, generator=gen).to(dtype) for _ in range(2))
+    k[:, 0] *= 3   # a reference that later tiles lie below, and above
+    k[:, L // 2] *= 5
+    want, want_sums = orc.dense_prefill(q, k, v)
+    log_sum, out = kernels.prefill_recompute0(q.to(cuda), k.to(cuda), v.to(cuda))
+    assert torch.equal(log_sum, kernels.prefill_recompute1(q.to(cuda), k.to(cuda)))
+    assert_close(log_sum, want_sums, f"log-sums L={L}", atol=2e-3, rtol=1e-4)
+    step = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7   # |v| reaches 4.5: two half steps of it
+    assert_close(out, want, f"outputs L={L}", atol=4.5 * step, rtol=step)
+
+
 @pytest.mark.parametrize("heads,G,D,dtype", [(32, 8, 128, torch.float16), (32, 8, 128, torch.bfloat16), (14, 2, 64, torch.float16)])
 @pytest.mark.parametrize("batch", [1, 9])
 def test_log_sums_alone_follow_late_maxima(cuda, batch, heads, G, D, dtype):
