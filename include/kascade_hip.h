@@ -254,7 +254,8 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
 /* Split counts for the decode calls (num_split), as the callers in this repository choose them.
  * kascade_decode_num_split: for lists or caches of up to max_rows rows per (sequence, KV head),
  *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
- *   least min_rows rows each, at most cap_rows (0: no cap); 1 to 256.
+ *   least min_rows rows each, at most cap_rows (0: no cap); 1 to 256.  Counts between one workgroup per unit
+ *   and two become whole ones.
  * kascade_gather_lone_rows: the longest list a gather call takes in one split, for so many query heads per
  *   KV head and so many lists (batch times KV heads).
  * KASCADE_GATHER_ROWS_PER_SPLIT: cap_rows of gather calls.

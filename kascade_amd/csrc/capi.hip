@@ -560,9 +560,28 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     // small launch (short lists, small batch): latency, not set-up, is what counts, so spread down to
     // 128 rows per workgroup to put one workgroup on every compute unit
     if (total_rows / per < compute_units) per = fmax(fmin(128, min_rows), total_rows / compute_units);
+    if (per <= 0) return 1;
+    const double ns = fmax(1, fmin(256, nearbyint(max_rows / per)));
+    // Between one workgroup per compute unit and two, the units with two finish last and the others wait: splits for one
+    // on (almost) every unit instead, or for two where those fill the chip better by more than an eighth.  Us per launch (anchor
+    // pass with output / without, pooling launch included; gathers of 10 %) by splits, the nearest count first:
+    //   8 x 3000 tokens, 64/8 heads    6: 37.7/35.3   4: 34.3/33.2   8: 35.7/34.4
+    //   2 x 9000, 64/8                18: 41.9/39.6  16: 37.0/37.2  32: 39.2/37.7
+    //   9 x 2500, 32/8                 5: 35.5/31.4   3: 31.9/29.2   7: 31.5/29.1
+    //   12 x 1200, 32/8                3: 28.7/25.5   2: 25.7/23.8   5: 24.3/23.0
+    //   36 x 5000, 8/2 heads of 64     4: 37.2/36.2   3: 35.5/34.8   7: 32.4/31.9
+    //   gather of 12 x 896 rows        3: 17.7        2: 15.1        5: 15.4
+    //   gather of 9 x 1664 rows        4: 22.4        3: 18.3        7: 17.3
+    //   gather of 7 x 1664, 64/8       5: 21.1        4: 16.9        9: 17.7
+    const double lists = total_rows / max_rows, wgs = lists * ns;
+    if (wgs > compute_units && wgs < 0.9 * 2 * compute_units) {
+        const double one = floor(compute_units / lists), two = floor(2 * compute_units / lists);
+        const double pick = one >= 1 && one * lists / compute_units >= two * lists / (2 * compute_units) - 0.125 ? one : two;
+        return (int)fmax(1, fmin(256, pick));
+    }
     // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
     // of workgroups on a few units, one fewer costs nothing
-    return per > 0 ? (int)fmax(1, fmin(256, nearbyint(max_rows / per))) : 1;
+    return (int)ns;
 }
 
 // A lone split writes its result itself; merging several costs a trip through device-coherent memory, a

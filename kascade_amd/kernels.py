@@ -134,6 +134,9 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
                 wgs, rps = count(ns)
                 if wgs <= rounds * target_wgs and rps >= min(min_rows, max_rows):
                     best = ns
+            # equal lengths between one workgroup per compute unit and two: kascade_decode_num_split knows better
+            if len(set(row_counts)) == 1 and cus < count(best)[0] < 0.9 * 2 * cus:
+                break
             if not cap_rows or count(best)[1] <= 4096 or rounds >= 8:
                 return best
             rounds += 1

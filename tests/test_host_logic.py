@@ -169,6 +169,25 @@ def test_split_count_of_a_ragged_batch_with_known_lengths(monkeypatch):
     assert kernels.default_num_split(8 * 600, 300, row_counts=[300, 300]) == kernels.default_num_split(8 * 600, 300)
 
 
+@pytest.mark.parametrize("batch,heads,rows,want", [(8, 8, 3064, 4), (16, 8, 1564, 2), (2, 8, 9064, 16), (9, 8, 2564, 7), (12, 8, 1264, 5),
+                                                   (36, 2, 5064, 7), (33, 8, 600, 1), (1, 8, 16384, 32), (4, 8, 3064, 8)])
+def test_splits_of_equal_lists_fill_whole_rounds(monkeypatch, batch, heads, rows, want):
+    """No count between one workgroup per compute unit and nearly two, with the lengths known or not; counts outside
+    stay those of the nearest number of rows."""
+    from kascade_amd import kernels, _lib
+
+    class FakeLib:
+        def kascade_device_cu_count(self):
+            return 256
+    monkeypatch.setattr(_lib, "init", lambda: FakeLib())
+    lists = batch * heads
+    assert kernels.default_num_split(lists * rows, rows, heads=heads) == want
+    for hint in (None, [rows] * batch):
+        for n in (rows, rows + 1, rows + 777, 3 * rows):
+            ns = kernels.default_num_split(lists * n, n, heads=heads, row_counts=hint and [n] * batch)
+            assert not 256 < lists * ns < 461 or lists > 256, (n, ns)
+
+
 def test_workloads_are_seeded_and_shaped():
     a = workloads.prefill_inputs(1, 256, seed=3)
     b = workloads.prefill_inputs(1, 256, seed=3)
