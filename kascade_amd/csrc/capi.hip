@@ -559,12 +559,29 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     if (cap_rows > 0) per = fmin(per, cap_rows);
     // small launch (short lists, small batch): latency, not set-up, is what counts, so spread down to
     // 128 rows per workgroup to put one workgroup on every compute unit
-    if (total_rows / per < compute_units) per = fmax(fmin(128, min_rows), total_rows / compute_units);
+    const bool small = total_rows / per < compute_units;
+    if (small) per = fmax(fmin(128, min_rows), total_rows / compute_units);
     if (per <= 0) return 1;
-    const double ns = fmax(1, fmin(256, nearbyint(max_rows / per)));
-    // Between one workgroup per compute unit and two, the units with two finish last and the others wait: splits for one
-    // on (almost) every unit instead, or for two where those fill the chip better by more than an eighth.  Us per launch (anchor
-    // pass with output / without, pooling launch included; gathers of 10 %) by splits, the nearest count first:
+    double ns = fmax(1, fmin(256, nearbyint(max_rows / per)));
+    // Small gathers: the merge requests 16 splits' results in one trip to memory and pays another for more, which lists of up
+    // to about 384 rows a split don't make good; longer ones stop at 64.  Us, batch 1, by splits (the last: 128 rows each):
+    //   3328 rows   32/8 heads 16: 10.2  26: 11.2    64/8 11.9  13.4    28/4 11.1  11.5    8/2 heads of 64 8.1  8.3
+    //   6016 rows   28/4 16: 12.7  47: 13.2          8/2 heads of 64 16: 9.2  47: 10.9     64/8 16: 14.5  32: 15.8
+    //   8064 rows   32/8 16: 14.7  32: 14.1          11008, 28/4 32: 14.9  64: 14.1        12032, 8/2 64: 10.7  94: 12.7
+    if (small && cap_rows > 0) ns = fmin(ns, max_rows <= 16 * 384 ? 16 : 64);
+    // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
+    // of workgroups on a few units, one fewer costs nothing
+    return (int)ns;
+}
+
+int kascade_decode_num_split_equal(int lists, double rows, int compute_units, double wgs_per_cu, double min_rows, double cap_rows) {
+    const int ns = kascade_decode_num_split((double)lists * rows, rows, compute_units, wgs_per_cu, min_rows, cap_rows);
+    if (lists <= 0) return ns;
+    // Lists of different lengths fill in behind each other (a gather of 17 sequences' lists of 512 to 896 rows by this rule: its
+    // step 1.5 % slower); equal ones do not.  Between one workgroup per compute unit and two, the units with two finish last
+    // and the others wait: splits for one on (almost) every unit instead, or for two where those fill the chip better by more
+    // than an eighth.  Us per launch (anchor pass with output / without, pooling launch included; gathers of 10 %) by
+    // splits, the nearest count first:
     //   8 x 3000 tokens, 64/8 heads    6: 37.7/35.3   4: 34.3/33.2   8: 35.7/34.4
     //   2 x 9000, 64/8                18: 41.9/39.6  16: 37.0/37.2  32: 39.2/37.7
     //   9 x 2500, 32/8                 5: 35.5/31.4   3: 31.9/29.2   7: 31.5/29.1
@@ -573,15 +590,17 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     //   gather of 12 x 896 rows        3: 17.7        2: 15.1        5: 15.4
     //   gather of 9 x 1664 rows        4: 22.4        3: 18.3        7: 17.3
     //   gather of 7 x 1664, 64/8       5: 21.1        4: 16.9        9: 17.7
-    const double lists = total_rows / max_rows, wgs = lists * ns;
-    if (wgs > compute_units && wgs < 0.9 * 2 * compute_units) {
-        const double one = floor(compute_units / lists), two = floor(2 * compute_units / lists);
-        const double pick = one >= 1 && one * lists / compute_units >= two * lists / (2 * compute_units) - 0.125 ? one : two;
+    const double wgs = (double)lists * ns;
+    // Few lists, streamed: one is the better number also where two fill the chip, as far as measured (to 4100
+    // rows a unit; batch 1, 32/8 heads: 40000 tokens 54.6/48.9 -> 52.1/48.7 us, 65536 79.7/66.4 -> 76.0/65.6, 131072
+    // 137.8/107.1 -> 131.2/104.9; 28/4: 40000 46.2/45.6 -> 43.1/44.4; four sequences of 16000 62.8/50.9 -> 60.9/50.7).
+    const bool few = cap_rows <= 0 && lists <= 64 && lists * rows <= 4160. * compute_units;
+    if (wgs > compute_units && (wgs < 0.9 * 2 * compute_units || (few && wgs <= 2 * compute_units))) {
+        const double one = floor((double)compute_units / lists), two = floor(2. * compute_units / lists);
+        const double pick = one >= 1 && one * lists / compute_units >= two * lists / (2. * compute_units) - 0.125 ? one : two;
         return (int)fmax(1, fmin(256, pick));
     }
-    // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
-    // of workgroups on a few units, one fewer costs nothing
-    return (int)ns;
+    return ns;
 }
 
 // A lone split writes its result itself; merging several costs a trip through device-coherent memory, a

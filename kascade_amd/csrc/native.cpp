@@ -117,9 +117,9 @@ at::Tensor empty_like_type(at::IntArrayRef size, const at::Tensor& like, at::Sca
 }
 
 // What kernels.default_num_split takes by default: two workgroups per compute unit, 512 rows each.
-int num_split(double total_rows, double max_rows, double cap_rows) {
+int num_split(int64_t lists, double rows, double cap_rows) {
     const int cus = kascade_device_cu_count();
-    return kascade_decode_num_split(total_rows, max_rows, cus > 0 ? cus : 256, 2, 512, cap_rows);
+    return kascade_decode_num_split_equal((int)lists, rows, cus > 0 ? cus : 256, 2, 512, cap_rows);
 }
 
 // Arrival counters of the fused split merge: zero when made, and zero again after every launch, so
@@ -215,7 +215,7 @@ struct Gather {
 Gather plan_gather(const HfTensors& h, int64_t topk, PyObject* counters, void* stream) {
     Gather g{topk, 1, {}};
     if (topk > kascade_gather_lone_rows(h.shape.group_size, (int)(h.B * h.G)))
-        g.ns = num_split((double)h.B * h.G * topk, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
+        g.ns = num_split(h.B * h.G, (double)topk, KASCADE_GATHER_ROWS_PER_SPLIT);
     if (g.ns <= KASCADE_FUSED_MERGE_MAX_SPLITS) g.sync = counters_for(counters, stream, h.B * h.G, h.q);
     return g;
 }
@@ -266,7 +266,7 @@ PyObject* hf_decode_anchor(PyObject* const* a) {
     const at::Tensor& hm = head_map(a[6], h.G);
     need(width > 0, "the selection takes at least one token");
     void* stream = stream_of(device_of_caller());
-    const int ns = num_split((double)h.B * h.G * h.L, (double)h.L, 0);
+    const int ns = num_split(h.B * h.G, (double)h.L, 0);
     const int64_t stride = (h.L + 7) / 8 * 8, heads = h.B * h.H;
     auto pad = [](int64_t x) { return (x + 63) / 64 * 64; };
     const int64_t n_lse = pad(heads * ns), n_part = with_output ? pad(heads * ns * h.D) : 0, n_sums = pad(heads);

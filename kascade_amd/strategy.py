@@ -318,8 +318,10 @@ class PagedKascadeDecoder:
         # 76.9 us with 256 workgroups against 78.6 with 512; 8 x 65536: 44.0 against 45.0); ragged
         # batches want two, so that the short sequences' workgroups fill in behind the long ones.
         uniform = seqlens_hint is not None and len(set(int(n) for n in seqlens_hint)) == 1
+        gathered = (max_batch * self.max_topk if seqlens_hint is None and total_tokens is None
+                    else budgets.decode_budget(total, k))
         self.ns_reuse = num_split_reuse or kernels.default_num_split(
-            G * budgets.decode_budget(total, k), self.max_topk, wgs_per_cu=1 if uniform else 2,
+            G * gathered, self.max_topk, wgs_per_cu=1 if uniform else 2,
             cap_rows=kernels.GATHER_ROWS_PER_SPLIT, row_counts=reuse_rows, heads=G,
             lone_rows=kernels.gather_lone_rows(group_size, max_batch * G))
         # The anchor passes (which also write their score codes) run 2 % faster with twice the
