@@ -122,7 +122,7 @@ __device__ __forceinline__ void store_rows(T* out, unsigned row_elems, const T* 
 // NQ: blocks of 16 queries a wavefront takes.  With two, wavefront w has head slot w; with one, four wavefronts are two head
 // slots x two blocks and a unit's four slots take two workgroups.
 template <bool PAGED, int D, typename T, bool SPARE, bool EXACT_SUM, int NQ>
-__device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK, T* sV) {
+__device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK, T* sV, int* s_move = nullptr) {
     typedef typename Elem<T>::x8 x8_t;
     typedef typename Elem<T>::x4 x4_t;
     typedef typename Elem<T>::x2 x2_t;
@@ -345,6 +345,20 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
 #pragma unroll
     for (int q = 0; q < NQ; ++q) arrived<kKS>(qf[q]);
 
+    // Of two wavefronts with a head slot's two blocks of 16 queries: whether either says so.  Every wavefront comes here once a
+    // tile behind the first; the tile's own barrier keeps this read from the next tile's write.  Rows on their way into LDS are
+    // not waited for.
+    auto lds_barrier = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto either_half = [&](bool mine) -> bool {
+        if (lane == 0) s_move[wave_u] = mine;
+        lds_barrier();
+        return mine || __builtin_amdgcn_readfirstlane(s_move[wave_u ^ 1]) != 0;
+    };
+
     // One tile: registers -> LDS, next tile's loads, both products, softmax.  Three copies of
     // the code, each straight-line: tiles that need no mask (all but one or two of a unit), tiles
     // that do (the causal edge, the end of the sequence, a selection that ends inside a tile), and
@@ -444,7 +458,6 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 for (int v = 0; v < 4; ++v) mx = fmaxf(mx, sT[q][kb][v]);
             return mx * kScaleLog2;
         };
-        // A column's reference moves for its own scores alone, so that its sums do not depend on which columns share a wavefront.
         float ms[NQ];
         bool above = false;
 #pragma unroll
@@ -452,11 +465,16 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
             ms[q] = maximum(q);
             above |= ms[q] > m[q] + kRefSlack;
         }
-        if (__any(above)) {   // wavefront-uniform
+        // The references of a block's 32 queries move together: most rows then have their largest probability as an exact 1
+        // (each query's for its own scores alone: 1.5 to 2.5 % further from 64-bit outputs).  In halves the other
+        // wavefront's queries count too.  (On a first tile the references are -inf and a wavefront in which nothing lies
+        // above them has nothing to move.)
+        bool move = __any(above);   // wavefront-uniform
+        if (NQ == 1 && sq > 0) move = either_half(move);
+        if (move) {
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const float top = max_over_quarters(ms[q]);   // the same in the four lanes of a column
-                const float mnew = top > m[q] + kRefSlack ? top : m[q];
+                const float mnew = fmaxf(m[q], max_over_quarters(ms[q]));   // the same in the four lanes of a column
                 const float corr = (mnew == -INFINITY) ? 1.f : fast_exp2(m[q] - mnew);
                 m[q] = mnew;
                 l[q] *= corr;
@@ -548,6 +566,7 @@ __device__ __forceinline__ void prefill_reuse_body(const PrefillParams& p, T* sK
                 if (s + 2 < ntiles) fetch_ids(tile_at(s + 2));
                 static_for<0, kNumLoads>([&](auto i) { issue_load(i, (s + 1) & 1); });
             }
+            if (NQ == 1 && s > 0) lds_barrier();   // the one in either_half
         }
         __syncthreads();   // the one behind the last tile
         return;
@@ -1165,7 +1184,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_sparse_halves_kernel(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) T sK[2 * AttnTile<D>::kTileElems];
     __shared__ __attribute__((aligned(1024))) T sV[2 * AttnTile<D>::kTileElems];
-    prefill_reuse_body<PAGED, D, T, SPARE, false, 1>(p, sK, sV);
+    __shared__ int s_move[kThreads / 64];   // either_half
+    prefill_reuse_body<PAGED, D, T, SPARE, false, 1>(p, sK, sV, s_move);
 }
 
 // 64 queries per wavefront for the K-only log-sum pass, whose state fits 256 registers: two
@@ -1502,9 +1522,10 @@ namespace {
 
 // Sparse units (a query tile and four head slots) up to which they are cut in two, one block of 16 queries to a wavefront:
 // where the halves are resident at once, two on each of 256 compute units.  A unit alone on its compute unit is a
-// chain of a wavefront's own instructions; half of them take (32/8 heads, 517 tokens) 9.3 -> 7.4 us, 28/4 517 9.2 -> 7.1,
-// 8/2 heads of 64, 2048 9.6 -> 7.4, 32/8 1024 (256 units) 9.9 -> 9.0.  With more the rows that both halves
-// stage cost more than that: 32/8, 1300 tokens (328 units) 12.4 -> 13.7 us, 2048 14.1 -> 16.9.
+// chain of a wavefront's own instructions; half of them, and a barrier a tile for the common references, take, us whole / in
+// halves: 32/8 heads, 300 tokens 8.4/6.6, 517 8.6/7.5, 1024 (256 units) 10.3/10.0, 28/4 517 8.7/7.3, 8/2 heads of 64, 2048 8.7/6.7,
+// 4096 13.1/12.3.  With more the rows that both halves stage cost more than that: 32/8, 1300 tokens (328 units) 12.4/13.7,
+// 2048 14.1/16.9 (without the barrier).
 constexpr long long kSplitUnits = 256;
 
 template <int D, typename T>
