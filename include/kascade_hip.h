@@ -256,8 +256,10 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
  *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
  *   least min_rows rows each, at most cap_rows (0: no cap, a streaming call; else a gather); 1 to 256.  Small
  *   gathers take up to 16 or 64 splits.
- * kascade_decode_num_split_equal: the same for `lists` lists (batch times KV heads) of `rows` rows each; counts
- *   between one workgroup per unit and two become whole ones.
+ * kascade_decode_num_split_equal: the same for `lists` lists (batch times KV heads) of `rows` rows each, in whole rounds.
+ * kascade_decode_whole_rounds: for such lists and num_split splits of each, whose workgroups are more than one per unit
+ *   and less than two, the splits that make whole rounds of them; other counts are returned as they are.
+ *   A gather's splits (cap_rows > 0) stay within cap_rows, or what num_split makes them.
  * kascade_gather_lone_rows: the longest list a gather call takes in one split, for so many query heads per
  *   KV head and so many lists (batch times KV heads).
  * KASCADE_GATHER_ROWS_PER_SPLIT: cap_rows of gather calls.
@@ -269,6 +271,7 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
                              double cap_rows);
 int kascade_decode_num_split_equal(int lists, double rows, int compute_units, double wgs_per_cu, double min_rows,
                                    double cap_rows);
+int kascade_decode_whole_rounds(int lists, double rows, int num_split, int compute_units, double cap_rows);
 int kascade_gather_lone_rows(int group_size, int lists);
 
 /* An anchor pass and the selection over its pooled scores in one call: what

@@ -50,6 +50,7 @@ SIGNATURES = {
     "kascade_pool_select_row": (_I, [_I, _I]),
     "kascade_decode_num_split": (_I, [C.c_double, C.c_double, _I, C.c_double, C.c_double, C.c_double]),
     "kascade_decode_num_split_equal": (_I, [_I, C.c_double, _I, C.c_double, C.c_double, C.c_double]),
+    "kascade_decode_whole_rounds": (_I, [_I, C.c_double, _I, _I, C.c_double]),
     "kascade_gather_lone_rows": (_I, [_I, _I]),
     "kascade_topk_workspace_bytes": (_L, [_I, _L]),
     "kascade_topk_call": (_I, [_P, _P, _I, _L, _I, _P, _P, _I, _I, _I, _P, _P]),

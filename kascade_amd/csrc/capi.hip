@@ -574,33 +574,57 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     return (int)ns;
 }
 
+}  // extern "C"
+namespace {
+// Splits per list that make whole rounds of workgroups: one on (almost) every unit, or two where those fill the chip better by
+// more than an eighth.  A gather whose splits would in one round be longer than cap_rows, and than num_split makes them, takes
+// two, or three on the same terms (8 KV heads, 22 sequences' lists of 6656 rows, us by splits: 2 124, 3 127, 4 107; 17: 3
+// 88.2, 4 94.5, 5 85.3; 25: 2 130, 3 135, 4 134).
+int whole_rounds(int lists, double rows, int num_split, int compute_units, double cap_rows) {
+    const auto splits = [&](int rounds) { return fmax(1, floor((double)rounds * compute_units / lists)); };
+    const auto fill = [&](int rounds) { return splits(rounds) * lists / ((double)rounds * compute_units); };
+    const bool too_long = cap_rows > 0 && rows / splits(1) > fmax(cap_rows, rows / num_split);
+    int rounds = lists <= compute_units && !too_long && fill(1) >= fill(2) - 0.125 ? 1 : 2;
+    if (too_long && fill(3) > fill(2) + 0.125) rounds = 3;
+    return (int)fmin(256, splits(rounds));
+}
+}  // namespace
+extern "C" {
+
+// Lists of different lengths fill in behind each other (a gather of 17 sequences' lists of 512 to 896 rows by this rule: its
+// step 1.5 % slower); equal ones do not.  Between one workgroup per compute unit and two, the units with two finish last
+// and the others wait.  Us per launch (anchor pass with output / without, pooling launch included; gathers of 10 %) by
+// splits, the nearest count first:
+//   8 x 3000 tokens, 64/8 heads    6: 37.7/35.3   4: 34.3/33.2   8: 35.7/34.4
+//   2 x 9000, 64/8                18: 41.9/39.6  16: 37.0/37.2  32: 39.2/37.7
+//   9 x 2500, 32/8                 5: 35.5/31.4   3: 31.9/29.2   7: 31.5/29.1
+//   12 x 1200, 32/8                3: 28.7/25.5   2: 25.7/23.8   5: 24.3/23.0
+//   36 x 5000, 8/2 heads of 64     4: 37.2/36.2   3: 35.5/34.8   7: 32.4/31.9
+//   gather of 12 x 896 rows        3: 17.7        2: 15.1        5: 15.4
+//   gather of 9 x 1664 rows        4: 22.4        3: 18.3        7: 17.3
+//   gather of 7 x 1664, 64/8       5: 21.1        4: 16.9        9: 17.7
+// and with many lists, where one round leaves up to a third of the units without a workgroup (32/8 heads; by splits):
+//   17 x 3000    1: 58.1/36.7   2: 63.6/39.0   3: 52.8/32.6      17 x 16384   1: 275/150   2: 292/160   3: 234/130
+//   22 x 3000    1: 64.2/39.6   2: 70.5/41.6   3: 71.6/43.7      22 x 16384   1: 302/162   2: 316/172   3: 325/176
+//   26 x 3000    1: 69.6/42.2   2: 74.6/43.9                     26 x 32768   1: 674/349   2: 695/374
+//   28 x 1000    1: 31.6/22.2   2: 34.8/23.0                     28 x 32768   1: 702/377   2: 722/389
+//   gather of 26 x 896 rows 1: 20.7  2: 25.2    of 26 x 1664 1: 34.4  2: 39.1    of 17 x 6656 1: 103.6  2: 113.3  3: 88.2  4: 94.5
+int kascade_decode_whole_rounds(int lists, double rows, int num_split, int compute_units, double cap_rows) {
+    if (lists <= 0 || num_split <= 0) return num_split > 0 ? num_split : 1;
+    const double wgs = (double)lists * num_split;
+    return wgs > compute_units && wgs < 0.9 * 2 * compute_units ? whole_rounds(lists, rows, num_split, compute_units, cap_rows) : num_split;
+}
+
 int kascade_decode_num_split_equal(int lists, double rows, int compute_units, double wgs_per_cu, double min_rows, double cap_rows) {
     const int ns = kascade_decode_num_split((double)lists * rows, rows, compute_units, wgs_per_cu, min_rows, cap_rows);
     if (lists <= 0) return ns;
-    // Lists of different lengths fill in behind each other (a gather of 17 sequences' lists of 512 to 896 rows by this rule: its
-    // step 1.5 % slower); equal ones do not.  Between one workgroup per compute unit and two, the units with two finish last
-    // and the others wait: splits for one on (almost) every unit instead, or for two where those fill the chip better by more
-    // than an eighth.  Us per launch (anchor pass with output / without, pooling launch included; gathers of 10 %) by
-    // splits, the nearest count first:
-    //   8 x 3000 tokens, 64/8 heads    6: 37.7/35.3   4: 34.3/33.2   8: 35.7/34.4
-    //   2 x 9000, 64/8                18: 41.9/39.6  16: 37.0/37.2  32: 39.2/37.7
-    //   9 x 2500, 32/8                 5: 35.5/31.4   3: 31.9/29.2   7: 31.5/29.1
-    //   12 x 1200, 32/8                3: 28.7/25.5   2: 25.7/23.8   5: 24.3/23.0
-    //   36 x 5000, 8/2 heads of 64     4: 37.2/36.2   3: 35.5/34.8   7: 32.4/31.9
-    //   gather of 12 x 896 rows        3: 17.7        2: 15.1        5: 15.4
-    //   gather of 9 x 1664 rows        4: 22.4        3: 18.3        7: 17.3
-    //   gather of 7 x 1664, 64/8       5: 21.1        4: 16.9        9: 17.7
-    const double wgs = (double)lists * ns;
     // Few lists, streamed: one is the better number also where two fill the chip, as far as measured (to 4100
     // rows a unit; batch 1, 32/8 heads: 40000 tokens 54.6/48.9 -> 52.1/48.7 us, 65536 79.7/66.4 -> 76.0/65.6, 131072
     // 137.8/107.1 -> 131.2/104.9; 28/4: 40000 46.2/45.6 -> 43.1/44.4; four sequences of 16000 62.8/50.9 -> 60.9/50.7).
+    const double wgs = (double)lists * ns;
     const bool few = cap_rows <= 0 && lists <= 64 && lists * rows <= 4160. * compute_units;
-    if (wgs > compute_units && (wgs < 0.9 * 2 * compute_units || (few && wgs <= 2 * compute_units))) {
-        const double one = floor((double)compute_units / lists), two = floor(2. * compute_units / lists);
-        const double pick = one >= 1 && one * lists / compute_units >= two * lists / (2. * compute_units) - 0.125 ? one : two;
-        return (int)fmax(1, fmin(256, pick));
-    }
-    return ns;
+    if (few && wgs > compute_units && wgs <= 2 * compute_units) return whole_rounds(lists, rows, ns, compute_units, 0);
+    return kascade_decode_whole_rounds(lists, rows, ns, compute_units, cap_rows);
 }
 
 // A lone split writes its result itself; merging several costs a trip through device-coherent memory, a

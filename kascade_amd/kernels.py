@@ -134,12 +134,14 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
                 wgs, rps = count(ns)
                 if wgs <= rounds * target_wgs and rps >= min(min_rows, max_rows):
                     best = ns
-            # equal lengths between one workgroup per compute unit and two: kascade_decode_num_split_equal knows better
-            if len(set(row_counts)) == 1 and cus < count(best)[0] < 0.9 * 2 * cus:
-                break
             if not cap_rows or count(best)[1] <= 4096 or rounds >= 8:
-                return best
+                break
             rounds += 1
+        if len(set(row_counts)) == 1:   # whole rounds of equal lists
+            lists = heads * len(row_counts)
+            whole = _lib.load().kascade_decode_whole_rounds(lists, max_rows, count(best)[0] // lists, cus, cap_rows or 0)
+            return best if whole * lists == count(best)[0] else whole
+        return best
     if row_counts is not None and len(set(row_counts)) == 1:
         total_rows = heads * len(row_counts) * max_rows
     elif row_counts is not None or max_rows <= 0 or total_rows % max_rows:   # lists of different lengths

@@ -82,6 +82,20 @@ def test_split_rules_have_one_home(lib):
         assert lib.kascade_decode_num_split(total, longest, cus, per_cu, least, cap) == want
 
 
+@pytest.mark.parametrize("lists,rows,splits,cap,want", [
+    (64, 3064, 6, 0, 4), (72, 2564, 5, 0, 7), (42, 1664, 8, 1664, 6),            # one round, two, a gather's one
+    (64, 3064, 4, 0, 4), (64, 3064, 8, 0, 8), (58, 3064, 8, 0, 8),                # whole rounds, and 464 of 512: as they are
+    (208, 5000, 2, 0, 1), (208, 4000, 2, 1664, 2), (208, 1600, 2, 1664, 1),       # one round only where a gather's splits allow it
+    (136, 6656, 3, 1664, 3), (176, 6656, 2, 1664, 4), (200, 6656, 2, 1664, 2),    # two rounds or three then
+    (264, 896, 1, 1664, 1), (300, 9000, 1, 1664, 1), (300, 9000, 1, 0, 1),        # more lists than units
+    (0, 100, 3, 0, 3), (8, 100, 0, 0, 1)])
+def test_whole_rounds_of_workgroups(lib, lists, rows, splits, cap, want):
+    got = lib.kascade_decode_whole_rounds(lists, rows, splits, 256, cap)
+    assert got == want
+    if cap and lists and splits:
+        assert rows / got <= max(cap, rows / splits)
+
+
 def _err(lib):
     return lib.kascade_get_last_error().decode()
 
