@@ -254,8 +254,8 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
 /* Split counts for the decode calls (num_split), as the callers in this repository choose them.
  * kascade_decode_num_split: for lists or caches of up to max_rows rows per (sequence, KV head),
  *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
- *   least min_rows rows each, at most cap_rows (0: no cap, a streaming call; else a gather); 1 to 256.  Small
- *   gathers take up to 16 or 64 splits.
+ *   least min_rows rows each and about cap_rows at most (0: no cap, a streaming call; else a gather); 1 to 256.
+ *   Small gathers take up to 16 or 64 splits, unless cap_rows asks for more.
  * kascade_decode_num_split_equal: the same for `lists` lists (batch times KV heads) of `rows` rows each, in whole rounds.
  * kascade_decode_whole_rounds: for such lists and num_split splits of each, whose workgroups are more than one per unit
  *   and less than two, the splits that make whole rounds of them; other counts are returned as they are.

@@ -564,11 +564,12 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     if (per <= 0) return 1;
     double ns = fmax(1, fmin(256, nearbyint(max_rows / per)));
     // Small gathers: the merge requests 16 splits' results in one trip to memory and pays another for more, which lists of up
-    // to about 384 rows a split don't make good; longer ones stop at 64.  Us, batch 1, by splits (the last: 128 rows each):
+    // to about 384 rows a split don't make good; longer ones stop at 64, or what cap_rows asks for.  Us, batch 1, by splits
+    // (the last: 128 rows each):
     //   3328 rows   32/8 heads 16: 10.2  26: 11.2    64/8 11.9  13.4    28/4 11.1  11.5    8/2 heads of 64 8.1  8.3
     //   6016 rows   28/4 16: 12.7  47: 13.2          8/2 heads of 64 16: 9.2  47: 10.9     64/8 16: 14.5  32: 15.8
     //   8064 rows   32/8 16: 14.7  32: 14.1          11008, 28/4 32: 14.9  64: 14.1        12032, 8/2 64: 10.7  94: 12.7
-    if (small && cap_rows > 0) ns = fmin(ns, max_rows <= 16 * 384 ? 16 : 64);
+    if (small && cap_rows > 0) ns = fmin(ns, fmax(max_rows <= 16 * 384 ? 16 : 64, ceil(max_rows / cap_rows)));
     // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
     // of workgroups on a few units, one fewer costs nothing
     return (int)ns;

@@ -1,6 +1,7 @@
 """CPU-only checks of the C ABI: the library loads, exports every symbol the header declares,
 and rejects bad arguments before touching a GPU (return code -1 + message)."""
 import ctypes as C
+import math
 import os
 import re
 
@@ -70,15 +71,21 @@ def test_split_rules_have_one_home(lib):
     assert strategy.FUSED_MERGE_MAX_SPLITS == int(constants["KASCADE_FUSED_MERGE_MAX_SPLITS"])
     source = open(os.path.join(ROOT, "kascade_amd", "csrc", "native.cpp")).read()
     assert not re.search(r"\b(1664|384|nearbyint)\b", source)
-    # the rule as the wrappers always had it
+    # the rule in Python; gathers (cap > 0) among the small launches with short and long lists, and one whose cap asks for more
     for total, longest, cus, per_cu, least, cap in ((128 * 6656, 6656, 256, 2, 512, 0), (8 * 1664, 1664, 256, 2, 512, 1664),
                                                     (8 * 100, 100, 256, 2, 512, 0), (128 * 13184, 13184, 256, 2, 512, 1664),
-                                                    (3, 1, 256, 1, 1, 0), (8 * 524288, 524288, 256, 1, 64, 0), (0, 0, 256, 2, 0, 0)):
+                                                    (3, 1, 256, 1, 1, 0), (8 * 524288, 524288, 256, 1, 64, 0), (0, 0, 256, 2, 0, 0),
+                                                    (8 * 3328, 3328, 256, 2, 512, 1664), (8 * 3328, 3328, 256, 2, 512, 0),
+                                                    (8 * 6144, 6144, 256, 2, 512, 1664), (2 * 12032, 12032, 256, 2, 512, 1664),
+                                                    (200000, 200000, 256, 2, 512, 1664)):
         per = max(least, total / (per_cu * cus))
         per = min(per, cap) if cap else per
-        if per and total / per < cus:
+        small = bool(per) and total / per < cus
+        if small:
             per = max(min(128, least), total / cus)
         want = max(1, min(256, round(longest / per))) if per else 1
+        if small and cap:
+            want = min(want, max(16 if longest <= 6144 else 64, math.ceil(longest / cap)))
         assert lib.kascade_decode_num_split(total, longest, cus, per_cu, least, cap) == want
 
 
