@@ -91,6 +91,7 @@ def _blhd_strides(t: torch.Tensor, name: str) -> Strides:
 
 
 GATHER_ROWS_PER_SPLIT = 1664   # KASCADE_GATHER_ROWS_PER_SPLIT of the header
+FUSED_MERGE_MAX_SPLITS = 32    # KASCADE_FUSED_MERGE_MAX_SPLITS
 
 
 def gather_lone_rows(group_size: int, lists: int = 1 << 30) -> int:
@@ -111,12 +112,44 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
     GATHER_ROWS_PER_SPLIT rows: twice that is 1-3 % faster on uniform batches (batch 16 x 26240
     rows: 307 us against 316 us) but 6 % slower on the ragged batch of four long sequences
     (109 us against 103 us); the streaming kernels do not care.
-    row_counts: the rows of every sequence (per KV head), when the caller knows them.
+    row_counts: the rows of every sequence (per KV head), when the caller knows them; max_rows may be more, what the lists
+    can grow to (room for 131072 tokens, 8 sequences of 3000 at 64/8 heads: splits of 768 rows, not a whole list each).
     lone_rows: lists of up to that many rows are one split (gather launches: gather_lone_rows)."""
     if max_rows <= lone_rows:
         return 1
     cus = _lib.init().kascade_device_cu_count() or 256
+    lib, cap = _lib.load(), cap_rows or 0
     target_wgs = wgs_per_cu * cus
+
+    def rows_per_split(ns):
+        return ((-(-max_rows // ns) + 63) // 64) * 64
+
+    def of_list(ns):
+        """Splits that each of the equal lists has with num_split ns: fewer where they are shorter than max_rows."""
+        return max(1, -(-rows // rows_per_split(ns)))
+
+    def with_splits(want):
+        """num_split for lists that fill less than three quarters of the room: `want` splits of each, as near as the 64-row steps
+        allow and without a few workgroups more than one per compute unit.  Of the numbers that give as many the one with the
+        shortest splits: the last one is not much shorter then, and lists that grow get more.
+        Two things limit num_split.  The room that is not filled is workgroups that only look at their length, about 2 ns
+        each, and a launch merges up to 32 splits itself, 3 us less than one behind it.  Anchor pass with output, room for
+        131072 tokens, us by num_split: 64 lists of 4096 rows 32 80.7, 64 64.4, 128 63.9, 256 88.2; 32 of 8000 32 79.0, 64 59.7,
+        128 52.6, 256 69.9; 8 of 4096 32 65.8, 128 36.4, 256 33.5; room for 32768, 96 of 1000 32 32.7, 43 35.3, 64 36.9, 128 53.7.
+        Gathers, room for 131072: 64 lists of 384 rows 32 10.2, 64 16.6, 128 29.3; 32 of 896 32 12.7, 64 11.7, 86 14.5.  Lone
+        splits have nothing to set against them: gathers of 208 lists of 256 rows 1 9.3, 4 10.1, 26 16.8, of 136 lists of 128
+        rows 3 5.5, 8 6.6, 26 10.6; anchor pass without output, 208 lists of 2000 rows 4 52.7, 32 56.9."""
+        most = min(64, 2048 // lists) if cap else min(256, 4096 // lists)
+        most = most if most >= 64 else FUSED_MERGE_MAX_SPLITS
+        near = min((of_list(ns) for ns in range(1, most + 1) if of_list(ns) <= max(want, cus // lists)),
+                   key=lambda n: (abs(n - want), n), default=1)
+        last = most if near > 1 else max(1, min(FUSED_MERGE_MAX_SPLITS, 1024 // lists))
+        return min(((rows_per_split(ns), ns) for ns in range(1, last + 1) if of_list(ns) == near), default=(0, 1))[1]
+
+    equal = row_counts is not None and len(set(row_counts)) == 1
+    if equal:   # hints of nearly all the room stand for all of it, which the lists soon fill
+        rows, lists = min(int(row_counts[0]), max_rows), heads * len(row_counts)
+        rows = max_rows if 4 * rows >= 3 * max_rows else rows
     if row_counts is not None and len(row_counts) > 1 and total_rows / max(min_rows, 1) >= cus:
         # Ragged batch with known lengths: count the workgroups exactly.  Each sequence rounds its
         # split count up, and a few workgroups beyond what is resident at once run when almost
@@ -125,7 +158,7 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
         # take the largest split count whose workgroups still fit `rounds` residencies, more
         # than one only when a split would otherwise exceed about 4096 rows.
         def count(ns):
-            rps = ((-(-max_rows // ns) + 63) // 64) * 64
+            rps = rows_per_split(ns)
             return heads * sum(max(1, -(-int(n) // rps)) for n in row_counts), rps
         rounds = 1
         while True:
@@ -137,17 +170,19 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
             if not cap_rows or count(best)[1] <= 4096 or rounds >= 8:
                 break
             rounds += 1
-        if len(set(row_counts)) == 1:   # whole rounds of equal lists
-            lists = heads * len(row_counts)
-            whole = _lib.load().kascade_decode_whole_rounds(lists, max_rows, count(best)[0] // lists, cus, cap_rows or 0)
-            return best if whole * lists == count(best)[0] else whole
-        return best
-    if row_counts is not None and len(set(row_counts)) == 1:
-        total_rows = heads * len(row_counts) * max_rows
-    elif row_counts is not None or max_rows <= 0 or total_rows % max_rows:   # lists of different lengths
-        return _lib.load().kascade_decode_num_split(total_rows, max_rows, cus, wgs_per_cu, min_rows, cap_rows or 0)
-    return _lib.load().kascade_decode_num_split_equal(int(total_rows // max_rows), max_rows, cus, wgs_per_cu, min_rows,
-                                                      cap_rows or 0)
+        if not equal:
+            return best
+        of_best = count(best)[0] // lists
+        want = 1 if rows <= lone_rows else lib.kascade_decode_whole_rounds(lists, rows, of_best, cus, cap)
+        if rows < max_rows:
+            return with_splits(want)
+        return best if want == of_best else want
+    if row_counts is None and max_rows > 0 and total_rows % max_rows == 0:
+        return lib.kascade_decode_num_split_equal(int(total_rows // max_rows), max_rows, cus, wgs_per_cu, min_rows, cap)
+    if not equal or rows <= 0:
+        return lib.kascade_decode_num_split(total_rows, max_rows, cus, wgs_per_cu, min_rows, cap)
+    want = 1 if rows <= lone_rows else lib.kascade_decode_num_split_equal(lists, rows, cus, wgs_per_cu, min_rows, cap)
+    return want if rows == max_rows else with_splits(want)
 
 
 # ---------------------------------------------------------------- decode

@@ -34,7 +34,7 @@ from . import _lib, budgets, kernels
 from ._lib import KascadeError
 
 H, G, D, TILE = 32, 8, 128, 32
-FUSED_MERGE_MAX_SPLITS = 32   # KASCADE_FUSED_MERGE_MAX_SPLITS of the header
+FUSED_MERGE_MAX_SPLITS = kernels.FUSED_MERGE_MAX_SPLITS
 ANCHOR_ROWS_PER_SPLIT = 8192
 
 

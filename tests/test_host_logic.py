@@ -219,6 +219,30 @@ def test_gathers_of_equal_lists_counted_exactly(monkeypatch, rows, want):
     assert got == want
 
 
+@pytest.mark.parametrize("batch,hint,room,dense,gather", [
+    (1, 4096, 131072, 8, 2), (8, 3000, 131072, 2, 1), (8, 4096, 131072, 2, 2), (4, 8000, 131072, 8, 4), (2, 9000, 32768, 16, 8),
+    (16, 1500, 32768, 2, 1), (16, 8192, 32768, 4, 2), (17, 8192, 32768, 3, 3), (26, 1024, 32768, 1, 1), (1, 32768, 131072, 32, 13),
+    (1, 3000, 3064, 24, 1), (8, 3000, 3064, 4, 1), (16, 65536, 65600, 4, 2)])
+def test_splits_of_hints_below_the_room(monkeypatch, batch, hint, room, dense, gather):
+    """Equal hints of 1/4 and 1/32 of the room, and of all of it: the splits that each list has are those of lists of that
+    length, as near as the limits on num_split and splits in steps of 64 rows come, not those of full ones."""
+    from kascade_amd import kernels, _lib
+
+    class FakeLib:
+        def kascade_device_cu_count(self):
+            return 256
+    monkeypatch.setattr(_lib, "init", lambda: FakeLib())
+
+    def splits(ns, rows, longest):
+        return max(1, -(-rows // (((-(-longest // ns) + 63) // 64) * 64)))
+    ns = kernels.default_num_split(8 * batch * hint, room, row_counts=[hint] * batch)
+    assert splits(ns, hint, room) == dense
+    rows, longest = budgets.decode_budget(hint, 10), budgets.decode_budget(room, 10)
+    ns = kernels.default_num_split(8 * batch * rows, longest, wgs_per_cu=1, cap_rows=kernels.GATHER_ROWS_PER_SPLIT,
+                                   row_counts=[rows] * batch, lone_rows=kernels.gather_lone_rows(4, 8 * batch))
+    assert splits(ns, rows, longest) == gather
+
+
 def test_workloads_are_seeded_and_shaped():
     a = workloads.prefill_inputs(1, 256, seed=3)
     b = workloads.prefill_inputs(1, 256, seed=3)
