@@ -255,8 +255,9 @@ int kascade_decode_recompute_paged_shaped_call(const kascade_shape* shape, const
  * kascade_decode_num_split: for lists or caches of up to max_rows rows per (sequence, KV head),
  *   total_rows over all of them: about wgs_per_cu workgroups on each of compute_units units with at
  *   least min_rows rows each and about cap_rows at most (0: no cap, a streaming call; else a gather); 1 to 256.
- *   Small gathers take up to 16 or 64 splits, unless cap_rows asks for more.
- * kascade_decode_num_split_equal: the same for `lists` lists (batch times KV heads) of `rows` rows each, in whole rounds.
+ *   Small gathers take up to 64 splits, unless cap_rows asks for more.
+ * kascade_decode_num_split_equal: the same for `lists` lists (batch times KV heads) known to have `rows` rows each, which
+ *   fill the launch's room: in whole rounds, few streamed lists in one, gathers of up to 6144 rows in up to 16 splits.
  * kascade_decode_whole_rounds: for such lists and num_split splits of each, whose workgroups are more than one per unit
  *   and less than two, the splits that make whole rounds of them; other counts are returned as they are.
  *   A gather's splits (cap_rows > 0) stay within cap_rows, or what num_split makes them.

@@ -563,13 +563,10 @@ int kascade_decode_num_split(double total_rows, double max_rows, int compute_uni
     if (small) per = fmax(fmin(128, min_rows), total_rows / compute_units);
     if (per <= 0) return 1;
     double ns = fmax(1, fmin(256, nearbyint(max_rows / per)));
-    // Small gathers: the merge requests 16 splits' results in one trip to memory and pays another for more, which lists of up
-    // to about 384 rows a split don't make good; longer ones stop at 64, or what cap_rows asks for.  Us, batch 1, by splits
-    // (the last: 128 rows each):
-    //   3328 rows   32/8 heads 16: 10.2  26: 11.2    64/8 11.9  13.4    28/4 11.1  11.5    8/2 heads of 64 8.1  8.3
-    //   6016 rows   28/4 16: 12.7  47: 13.2          8/2 heads of 64 16: 9.2  47: 10.9     64/8 16: 14.5  32: 15.8
-    //   8064 rows   32/8 16: 14.7  32: 14.1          11008, 28/4 32: 14.9  64: 14.1        12032, 8/2 64: 10.7  94: 12.7
-    if (small && cap_rows > 0) ns = fmin(ns, fmax(max_rows <= 16 * 384 ? 16 : 64, ceil(max_rows / cap_rows)));
+    // Small gathers stop at 64 splits, or what cap_rows asks for, whatever part of max_rows is filled.  Us, batch 1, 32/8 heads,
+    // room for 13184 rows, with 64 / 103 splits (128 rows each): 512 rows 10.3/10.8, 1664 10.9/11.5, 3328 11.6/12.3, 6656
+    // 13.0/15.6, 13184 18.8/24.8; 12032 rows at 8/2 heads of 64 with 64 / 94: 10.7/12.7.
+    if (small && cap_rows > 0) ns = fmin(ns, fmax(64, ceil(max_rows / cap_rows)));
     // to the nearest: one workgroup more than a whole number per compute unit costs a full extra wave
     // of workgroups on a few units, one fewer costs nothing
     return (int)ns;
@@ -617,11 +614,21 @@ int kascade_decode_whole_rounds(int lists, double rows, int num_split, int compu
 }
 
 int kascade_decode_num_split_equal(int lists, double rows, int compute_units, double wgs_per_cu, double min_rows, double cap_rows) {
-    const int ns = kascade_decode_num_split((double)lists * rows, rows, compute_units, wgs_per_cu, min_rows, cap_rows);
+    int ns = kascade_decode_num_split((double)lists * rows, rows, compute_units, wgs_per_cu, min_rows, cap_rows);
     if (lists <= 0) return ns;
+    // Gathers (only small ones come to more than 12): the merge requests 16 splits' results in one trip to memory and pays
+    // another for more, which lists of up to about 384 rows a split don't make good.  Us, batch 1, by splits (the last: 128
+    // rows each):
+    //   3328 rows   32/8 heads 16: 10.2  26: 11.2    64/8 11.9  13.4    28/4 11.1  11.5    8/2 heads of 64 8.1  8.3
+    //   6016 rows   28/4 16: 12.7  47: 13.2          8/2 heads of 64 16: 9.2  47: 10.9     64/8 16: 14.5  32: 15.8
+    //   8064 rows   32/8 16: 14.7  32: 14.1          11008, 28/4 32: 14.9  64: 14.1
+    // Not where the lists may be shorter than the launch has room for: room for 3328 rows, 512 8.7 against 7.5 with 26, 1664 9.5/8.5.
+    if (cap_rows > 0 && rows <= 16 * 384 && min_rows >= 384) ns = (int)fmin(ns, 16);
     // Few lists, streamed: one is the better number also where two fill the chip, as far as measured (to 4100
     // rows a unit; batch 1, 32/8 heads: 40000 tokens 54.6/48.9 -> 52.1/48.7 us, 65536 79.7/66.4 -> 76.0/65.6, 131072
     // 137.8/107.1 -> 131.2/104.9; 28/4: 40000 46.2/45.6 -> 43.1/44.4; four sequences of 16000 62.8/50.9 -> 60.9/50.7).
+    // Not where they may be shorter than the launch has room for: room for 131072, 32768 tokens 100.3/72.9 against 80.7/59.7
+    // with two.
     const double wgs = (double)lists * ns;
     const bool few = cap_rows <= 0 && lists <= 64 && lists * rows <= 4160. * compute_units;
     if (few && wgs > compute_units && wgs <= 2 * compute_units) return whole_rounds(lists, rows, ns, compute_units, 0);

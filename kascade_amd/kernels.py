@@ -102,7 +102,7 @@ def gather_lone_rows(group_size: int, lists: int = 1 << 30) -> int:
 
 def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_rows: int = 512,
                       cap_rows: Optional[int] = None, row_counts=None, heads: int = G,
-                      lone_rows: int = 0) -> int:
+                      lone_rows: int = 0, lengths: str = "equal") -> int:
     """Split count for a decode launch.  Every split covers the same number of rows
     (ceil(max_rows/num_split)), so the number of non-empty workgroups is about
     total_rows / rows_per_split; aim at wgs_per_cu of them per compute unit without
@@ -113,7 +113,8 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
     rows: 307 us against 316 us) but 6 % slower on the ragged batch of four long sequences
     (109 us against 103 us); the streaming kernels do not care.
     row_counts: the rows of every sequence (per KV head), when the caller knows them; max_rows may be more, what the lists
-    can grow to (room for 131072 tokens, 8 sequences of 3000 at 64/8 heads: splits of 768 rows, not a whole list each).
+    can grow to.  Without them `lengths` says what total_rows stands for: "equal", lists of max_rows each; "capacity",
+    lists that may all grow to max_rows, but may be shorter; "mixed", lists of different lengths.
     lone_rows: lists of up to that many rows are one split (gather launches: gather_lone_rows)."""
     if max_rows <= lone_rows:
         return 1
@@ -146,7 +147,7 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
         last = most if near > 1 else max(1, min(FUSED_MERGE_MAX_SPLITS, 1024 // lists))
         return min(((rows_per_split(ns), ns) for ns in range(1, last + 1) if of_list(ns) == near), default=(0, 1))[1]
 
-    equal = row_counts is not None and len(set(row_counts)) == 1
+    rows, equal = 0, row_counts is not None and len(set(row_counts)) == 1
     if equal:   # hints of nearly all the room stand for all of it, which the lists soon fill
         rows, lists = min(int(row_counts[0]), max_rows), heads * len(row_counts)
         rows = max_rows if 4 * rows >= 3 * max_rows else rows
@@ -177,10 +178,18 @@ def default_num_split(total_rows: int, max_rows: int, wgs_per_cu: int = 2, min_r
         if rows < max_rows:
             return with_splits(want)
         return best if want == of_best else want
-    if row_counts is None and max_rows > 0 and total_rows % max_rows == 0:
-        return lib.kascade_decode_num_split_equal(int(total_rows // max_rows), max_rows, cus, wgs_per_cu, min_rows, cap)
+    if row_counts is None and lengths != "mixed" and max_rows > 0 and total_rows % max_rows == 0:
+        equal, rows, lists = lengths == "equal", max_rows, int(total_rows // max_rows)
+    plain = lib.kascade_decode_num_split(total_rows, max_rows, cus, wgs_per_cu, min_rows, cap)
+    if row_counts is None and lengths == "capacity" and rows > 0:
+        # Whole rounds of full lists, unless that takes more than a third of the splits from shorter ones.  Anchor pass with output,
+        # us with the nearest count / whole rounds: 8 sequences at 64/8 heads, room for 3064 tokens, 6 / 4 splits: 700 24.5/24.1,
+        # 1000 25.4/28.1, 1500 32.9/29.4, 3000 38.5/35.2; at 32/8, room for 3564, 7 / 4: 700 21.8/22.6, 1500 23.8/29.1, 3500
+        # 36.2/35.4; 9 sequences, 2564, 5 / 7: 600 24.2/21.5, 2500 36.2/31.8.
+        whole = lib.kascade_decode_whole_rounds(lists, rows, plain, cus, cap)
+        return whole if 3 * whole >= 2 * plain else plain
     if not equal or rows <= 0:
-        return lib.kascade_decode_num_split(total_rows, max_rows, cus, wgs_per_cu, min_rows, cap)
+        return plain
     want = 1 if rows <= lone_rows else lib.kascade_decode_num_split_equal(lists, rows, cus, wgs_per_cu, min_rows, cap)
     return want if rows == max_rows else with_splits(want)
 

@@ -312,8 +312,9 @@ class PagedKascadeDecoder:
         total = total_tokens if total_tokens is not None else max_batch * max_seqlen
         dense_rows = list(seqlens_hint) if seqlens_hint is not None else None
         reuse_rows = [budgets.decode_budget(n, k) for n in seqlens_hint] if seqlens_hint is not None else None
+        lengths = "capacity" if total_tokens is None else "mixed"   # what is known of them without a hint
         self.ns_dense = num_split_dense or kernels.default_num_split(G * total, max_seqlen, row_counts=dense_rows,
-                                                                         heads=G)
+                                                                     heads=G, lengths=lengths)
         # A batch of equal lengths gathers fastest with one workgroup per compute unit (16 x 65536:
         # 76.9 us with 256 workgroups against 78.6 with 512; 8 x 65536: 44.0 against 45.0); ragged
         # batches want two, so that the short sequences' workgroups fill in behind the long ones.
@@ -323,7 +324,7 @@ class PagedKascadeDecoder:
         self.ns_reuse = num_split_reuse or kernels.default_num_split(
             G * gathered, self.max_topk, wgs_per_cu=1 if uniform else 2,
             cap_rows=kernels.GATHER_ROWS_PER_SPLIT, row_counts=reuse_rows, heads=G,
-            lone_rows=kernels.gather_lone_rows(group_size, max_batch * G))
+            lone_rows=kernels.gather_lone_rows(group_size, max_batch * G), lengths=lengths)
         # The anchor passes (which also write their score codes) run 2 % faster with twice the
         # splits where two workgroups per compute unit leave a split more than 8192 rows
         # (16 x 65536: 795 / 508 us with 8 splits against 815 / 521 with 4); dense decode does not

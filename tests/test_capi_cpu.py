@@ -71,7 +71,7 @@ def test_split_rules_have_one_home(lib):
     assert strategy.FUSED_MERGE_MAX_SPLITS == int(constants["KASCADE_FUSED_MERGE_MAX_SPLITS"])
     source = open(os.path.join(ROOT, "kascade_amd", "csrc", "native.cpp")).read()
     assert not re.search(r"\b(1664|384|nearbyint)\b", source)
-    # the rule in Python; gathers (cap > 0) among the small launches with short and long lists, and one whose cap asks for more
+    # the rule in Python; gathers (cap > 0) among the small launches, up to 64 splits and more, and one whose cap asks for more
     for total, longest, cus, per_cu, least, cap in ((128 * 6656, 6656, 256, 2, 512, 0), (8 * 1664, 1664, 256, 2, 512, 1664),
                                                     (8 * 100, 100, 256, 2, 512, 0), (128 * 13184, 13184, 256, 2, 512, 1664),
                                                     (3, 1, 256, 1, 1, 0), (8 * 524288, 524288, 256, 1, 64, 0), (0, 0, 256, 2, 0, 0),
@@ -85,8 +85,16 @@ def test_split_rules_have_one_home(lib):
             per = max(min(128, least), total / cus)
         want = max(1, min(256, round(longest / per))) if per else 1
         if small and cap:
-            want = min(want, max(16 if longest <= 6144 else 64, math.ceil(longest / cap)))
+            want = min(want, max(64, math.ceil(longest / cap)))
         assert lib.kascade_decode_num_split(total, longest, cus, per_cu, least, cap) == want
+
+
+def test_known_equal_lists_share_the_rule(lib):
+    """Lists known to fill the launch: gathers of up to 6144 rows within 16 splits, few streamed lists one workgroup per unit."""
+    for lists, rows, cap, plain, equal in ((8, 3328, 1664, 26, 16), (8, 6144, 1664, 32, 16), (8, 6272, 1664, 32, 32), (8, 1664, 1664, 13, 13),
+                                           (8, 65536, 0, 64, 32), (64, 3064, 0, 6, 4), (128, 13184, 1664, 8, 8)):
+        assert lib.kascade_decode_num_split(lists * rows, rows, 256, 2, 512, cap) == plain
+        assert lib.kascade_decode_num_split_equal(lists, rows, 256, 2, 512, cap) == equal
 
 
 @pytest.mark.parametrize("lists,rows,splits,cap,want", [

@@ -243,6 +243,44 @@ def test_splits_of_hints_below_the_room(monkeypatch, batch, hint, room, dense, g
     assert splits(ns, rows, longest) == gather
 
 
+@pytest.mark.parametrize("total,want", [(8 * 65536, 64), (16 * 32768, 64), (8 * 65536 + 8, 64)])
+def test_splits_of_a_batch_of_different_lengths(monkeypatch, total, want):
+    """A total that happens to be a multiple of the longest list does not make the lists equal ones."""
+    from kascade_amd import kernels, _lib
+
+    class FakeLib:
+        def kascade_device_cu_count(self):
+            return 256
+    monkeypatch.setattr(_lib, "init", lambda: FakeLib())
+    assert kernels.default_num_split(total, 65536, lengths="mixed") == want
+    assert kernels.default_num_split(24 * 3064, 3064, lengths="mixed") == kernels.default_num_split(24 * 3064 + 1, 3064, lengths="mixed")
+
+
+@pytest.mark.parametrize("batch,room,heads,group,dense,reuse", [
+    (1, 131136, 8, 4, 64, 32), (1, 32832, 8, 4, 64, 26), (8, 3064, 8, 8, 4, 1), (8, 3564, 8, 4, 7, 1), (9, 2564, 8, 4, 7, 1),
+    (4, 16064, 8, 4, 16, 8), (12, 8960, 8, 4, 5, 5), (8, 16448, 8, 4, 8, 4), (36, 5064, 2, 4, 7, 7)])
+def test_splits_of_a_decoder_without_hints(monkeypatch, batch, room, heads, group, dense, reuse):
+    """Its lists may be shorter than the room: no counts that pay for full ones alone (one round for few streamed lists, 16 splits
+    of short gathers), and whole rounds only where they keep two thirds of the splits.  The gathers are planned as max_batch
+    lists of max_topk, which is more than the budget of all tokens together."""
+    from kascade_amd import _lib, kernels
+    from kascade_amd.strategy import PagedKascadeDecoder
+
+    class FakeLib:
+        def kascade_device_cu_count(self):
+            return 256
+    monkeypatch.setattr(_lib, "init", lambda: FakeLib())
+    dec = PagedKascadeDecoder(10, [list(range(heads))], [0], batch, room, device="cpu", kv_heads=heads, group_size=group)
+    assert (dec.ns_dense, dec.ns_reuse) == (dense, reuse)
+    plans = []
+    monkeypatch.setattr(kernels, "default_num_split", lambda *a, **k: plans.append((*a[:2], k["lengths"])) or 1)
+    PagedKascadeDecoder(10, [list(range(heads))], [0], batch, room, device="cpu", kv_heads=heads, group_size=group)
+    PagedKascadeDecoder(10, [list(range(heads))], [0], batch, room, device="cpu", kv_heads=heads, group_size=group,
+                        total_tokens=batch * room // 2)
+    assert plans[:2] == [(heads * batch * room, room, "capacity"), (heads * batch * dec.max_topk, dec.max_topk, "capacity")]
+    assert [p[2] for p in plans[2:]] == ["mixed", "mixed"]
+
+
 def test_workloads_are_seeded_and_shaped():
     a = workloads.prefill_inputs(1, 256, seed=3)
     b = workloads.prefill_inputs(1, 256, seed=3)
