@@ -624,13 +624,15 @@ int kascade_decode_num_split_equal(int lists, double rows, int compute_units, do
     //   8064 rows   32/8 16: 14.7  32: 14.1          11008, 28/4 32: 14.9  64: 14.1
     // Not where the lists may be shorter than the launch has room for: room for 3328 rows, 512 8.7 against 7.5 with 26, 1664 9.5/8.5.
     if (cap_rows > 0 && rows <= 16 * 384 && min_rows >= 384) ns = (int)fmin(ns, 16);
-    // Few lists, streamed: one is the better number also where two fill the chip, as far as measured (to 4100
-    // rows a unit; batch 1, 32/8 heads: 40000 tokens 54.6/48.9 -> 52.1/48.7 us, 65536 79.7/66.4 -> 76.0/65.6, 131072
-    // 137.8/107.1 -> 131.2/104.9; 28/4: 40000 46.2/45.6 -> 43.1/44.4; four sequences of 16000 62.8/50.9 -> 60.9/50.7).
+    // Few lists, streamed: one is the better number also where two fill the chip.  Up to 32 lists at any length (batch 1, 32/8
+    // heads, two / one: 40000 tokens 54.6/48.9 -> 52.1/48.7 us, 131072 148.7/100.0 -> 142.3/97.7, 180000 174.4/107.6 -> 172.3/104.5,
+    // 524288 415.1/233.7 -> 409.8/230.7; 28/4, 262144 144.0/91.9 -> 140.4/91.7; four sequences of 16000 64.8/41.0 -> 63.6/40.8, of
+    // 65536 209.0/123.1 -> 209.6/121.3, of 131072 426.3/248.9 -> 421.6/242.3), up to 64 to 4160 rows a unit: eight of 16000
+    // 109.9/63.6 -> 106.8/62.5, of 24000 (6000 rows a unit) 155.6/89.5 -> 156.0/87.4, of 32768 200.4/114.3 -> 205.6/114.0.
     // Not where they may be shorter than the launch has room for: room for 131072, 32768 tokens 100.3/72.9 against 80.7/59.7
     // with two.
     const double wgs = (double)lists * ns;
-    const bool few = cap_rows <= 0 && lists <= 64 && lists * rows <= 4160. * compute_units;
+    const bool few = cap_rows <= 0 && (lists <= 32 || (lists <= 64 && lists * rows <= 4160. * compute_units));
     if (few && wgs > compute_units && wgs <= 2 * compute_units) return whole_rounds(lists, rows, ns, compute_units, 0);
     return kascade_decode_whole_rounds(lists, rows, ns, compute_units, cap_rows);
 }

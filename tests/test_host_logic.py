@@ -188,12 +188,12 @@ def test_splits_of_equal_lists_fill_whole_rounds(monkeypatch, batch, heads, rows
             assert not 256 < lists * ns < 461 or lists > 256, (n, ns)
 
 
-@pytest.mark.parametrize("lists,rows,cap,want", [(8, 40064, 0, 32), (8, 131136, 0, 32), (8, 134000, 0, 64), (4, 40064, 0, 64), (32, 16064, 0, 8),
+@pytest.mark.parametrize("lists,rows,cap,want", [(8, 40064, 0, 32), (8, 524352, 0, 32), (32, 131136, 0, 8), (64, 16448, 0, 4), (64, 32832, 0, 8), (8, 131136, 0, 32), (8, 134000, 0, 32), (4, 40064, 0, 64), (32, 16064, 0, 8),
                                                  (128, 3064, 0, 4), (8, 1664, 1664, 13), (8, 2176, 1664, 16), (8, 6144, 1664, 16),
                                                  (8, 6272, 1664, 32), (2, 12032, 1664, 64), (4, 11008, 1664, 64)])
 def test_splits_of_few_lists(monkeypatch, lists, rows, cap, want):
-    """Few streamed lists are one workgroup per compute unit up to about 4100 rows of it; small gathers stay within what their
-    merge requests in one trip."""
+    """Few streamed lists are one workgroup per compute unit, at any length measured up to 32 lists; small gathers stay within
+    what their merge requests in one trip."""
     from kascade_amd import kernels, _lib
 
     class FakeLib:
