@@ -328,9 +328,12 @@ class PagedKascadeDecoder:
         # The anchor passes (which also write their score codes) run 2 % faster with twice the
         # splits where two workgroups per compute unit leave a split more than 8192 rows
         # (16 x 65536: 795 / 508 us with 8 splits against 815 / 521 with 4); dense decode does not
-        # care, and beyond 32 splits the merge inside the launch would be lost.
+        # care, and beyond 32 splits the merge inside the launch would be lost.  One round of workgroups
+        # is one round for them too (26 x 16384: 333 / 182 us, with two splits 345 / 187; 26 x 32768:
+        # 674 / 349 and 695 / 374).
         self.ns_anchor = self.ns_dense
         if (not num_split_dense and -(-max_seqlen // self.ns_dense) > ANCHOR_ROWS_PER_SPLIT
+                and max_batch * G * self.ns_dense > (_lib.init().kascade_device_cu_count() or 256)
                 and 2 * self.ns_dense <= FUSED_MERGE_MAX_SPLITS):
             self.ns_anchor = 2 * self.ns_dense
         ns = max(self.ns_dense, self.ns_reuse, self.ns_anchor)

@@ -281,6 +281,20 @@ def test_splits_of_a_decoder_without_hints(monkeypatch, batch, room, heads, grou
     assert [p[2] for p in plans[2:]] == ["mixed", "mixed"]
 
 
+@pytest.mark.parametrize("batch,tokens,dense,anchor", [(26, 16384, 1, 1), (22, 32768, 1, 1), (16, 65536, 4, 8), (33, 32768, 1, 2), (8, 8192, 8, 8)])
+def test_anchor_passes_take_twice_the_splits_of_two_rounds(monkeypatch, batch, tokens, dense, anchor):
+    """Of more than 8192 rows, and only where there are two: one round of workgroups stays one."""
+    from kascade_amd import _lib
+    from kascade_amd.strategy import PagedKascadeDecoder
+
+    class FakeLib:
+        def kascade_device_cu_count(self):
+            return 256
+    monkeypatch.setattr(_lib, "init", lambda: FakeLib())
+    dec = PagedKascadeDecoder(10, [list(range(8))], [0], batch, tokens + 64, device="cpu", seqlens_hint=[tokens] * batch)
+    assert (dec.ns_dense, dec.ns_anchor) == (dense, anchor)
+
+
 def test_workloads_are_seeded_and_shaped():
     a = workloads.prefill_inputs(1, 256, seed=3)
     b = workloads.prefill_inputs(1, 256, seed=3)
