@@ -341,7 +341,9 @@ int kascade_topk_rows_call(const kascade_half* scores, int32_t* out_idx, int row
  *   scores: scratch [batch, kv_heads, tiles, q_start + q_len] fp16, left with unspecified contents
  *   valid_len / n_sel [period], both required: keys row r looks at (at most those in front of its tile) and takes
  *   out_idx [rows, k]; out_rows [rows, k] or NULL: the same as cache rows (with a block table)
- *   workspace: as for kascade_topk_call, kascade_topk_workspace_bytes(rows, q_start + q_len) bytes or NULL. */
+ *   workspace: as for kascade_topk_call, kascade_topk_workspace_bytes(rows, q_start + q_len) bytes or NULL.
+ * kascade_prefill_pool_selects: 1 where one launch pools and selects, 0 where two do; the lists are the same. */
+int kascade_prefill_pool_selects(int kv_heads, int head_dim, int batch, int q_start, int q_len);
 int kascade_prefill_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K, const float* log_sum,
                                      kascade_half* scores, int32_t* out_idx, int32_t* out_rows, int batch, int q_start, int q_len,
                                      kascade_strides q_strides, const kascade_strides* kv_strides, const int32_t* block_table,

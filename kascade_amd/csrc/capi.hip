@@ -1216,6 +1216,13 @@ int prefill_chunk_reuse_impl(const Shape& sh, const kascade_half* Q, const kasca
 }  // namespace
 extern "C" {
 
+int kascade_prefill_pool_selects(int kv_heads, int head_dim, int batch, int q_start, int q_len) {
+    if (kv_heads < 1 || batch < 1 || q_start < 0 || q_len < 1 || (long long)q_start + q_len >= (1LL << 31)) return 0;
+    PrefillParams p{};
+    p.G = kv_heads; p.head_dim = head_dim; p.B = batch; p.q_start = q_start; p.T = (q_len + kTile - 1) / kTile;
+    return prefill_pool_selects(p) ? 1 : 0;
+}
+
 int kascade_prefill_anchor_topk_call(const kascade_shape* shape, const kascade_half* Q, const kascade_half* K, const float* log_sum,
                                      kascade_half* scores, int32_t* out_idx, int32_t* out_rows, int batch, int q_start, int q_len,
                                      kascade_strides q_strides, const kascade_strides* kv_strides, const int32_t* block_table,

@@ -1628,13 +1628,24 @@ hipError_t launch_prefill_attn(const PrefillParams& p, bool reuse, bool with_v, 
 // wavefronts do not make up for it they keep two launches.  Us with two launches / as the rule would have it:
 //   units up to 192, more than 6 tiles of 128 keys: 512 queries at 512 15.8/17.1, at 3584 32.2/38.5, 8/2 heads of 64, 2048 tokens
 //   13.8/15.9 (6 tiles: 32/8, 768 tokens 14.0/13.2);  193 to 256: 28/4, 2048 tokens 40.8/36.2, 1024 queries at 3072 47.8/43.7, but
-//   at head_dim 64, where products take half the time, 8/2 heads, 4096 tokens 24.6/26.2;  257 to 448: 32/8, 1536 tokens
-//   24.9/22.1, but 28/4, 3001 tokens (24 tiles) 68.4/69.8;  512: 2048 queries at 2048 74.0/66.3, 28/4, 4096 tokens 108.7/106.5.
+//   at head_dim 64, where products take half the time, 8/2 heads, 4096 tokens 24.6/26.2.
+// Up to 512 units all are resident at once, where short and long ones only meet on a compute unit if the (KV head, sequence)
+// pairs fill the XCDs (unit_of_workgroup):
+//   257 to 448, pairs that do: 32/8, 1100 tokens 19.3/17.9, 1536 24.9/22.1, 1780 31.0/24.8, two prompts of 1600 at 28/4 42.0/40.1;
+//   others: two of 1300 at 28/4 34.1/31.3, five of 1300 at 8/2 heads of 64 21.1/18.9 (10 tiles), but 20/5, 2040 tokens 27.5/33.7,
+//   two of 2400 at 8/2 heads of 64 21.2/27.1, 28/4, 3001 68.4/69.8;
+//   449 to 512, pairs that do: 2048 queries at 2048 74.0/66.3; others: two of 2450 at 12/3 heads of 64 30.0/29.2 (19 tiles), but 8/2
+//   heads of 64, two of 3620 35.5/38.8, two of 4000 38.5/44.4, 28/4, 3800 85.9/87.9.
+// Beyond, two launches do not cut keys either: two of 2800 at 12/3 heads of 64 (528 units) 39.1/35.5, 3001 tokens 55.8/52.5.
 bool prefill_pool_selects(const PrefillParams& p) {
     const int keys = p.q_start + kTile * (p.T - 1), tiles = (keys + 127) / 128;
-    const long long units = (long long)p.B * p.G * p.T;
+    const long long pairs = (long long)p.B * p.G, units = pairs * p.T;
+    const bool fill_xcds = pairs % 8 == 0;
     if (keys > kPoolSelectKeys) return false;
-    return units > 448 || tiles <= (units > 256 ? 16 : units <= 192 ? 6 : p.head_dim == 64 ? 8 : 32);
+    if (units > 512) return true;
+    if (units > 448) return fill_xcds || tiles <= 20;
+    if (units > 256) return tiles <= (fill_xcds ? 16 : 10);
+    return tiles <= (units <= 192 ? 6 : p.head_dim == 64 ? 8 : 32);
 }
 
 hipError_t launch_prefill_aggregate(const PrefillParams& p0, const SelectParams* select, hipStream_t stream) {

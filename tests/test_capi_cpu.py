@@ -111,6 +111,18 @@ def test_whole_rounds_of_workgroups(lib, lists, rows, splits, cap, want):
         assert rows / got <= max(cap, rows / splits)
 
 
+def test_pooling_selects_where_the_rule_says(lib):
+    """Prompt pooling: one launch or two, on both sides of each line."""
+    from tests.test_gpu_prefill_units import POOLING_CASES, POOLING_CHUNKS
+    calls = [(G, D, B, 0, L, want) for _, G, D, L, B, _, want in POOLING_CASES]
+    calls += [(G, D, B, start, n, want) for _, G, D, start, n, B, want in POOLING_CHUNKS]
+    assert {want for *_, want in calls} == {0, 1}
+    for *call, want in calls:
+        assert lib.kascade_prefill_pool_selects(*call) == want, call
+    for none in ((0, 128, 1, 0, 32), (8, 128, 0, 0, 32), (8, 128, 1, 0, 0), (8, 128, 1, -32, 32), (8, 128, 1, 2 ** 31 - 32, 32)):
+        assert lib.kascade_prefill_pool_selects(*none) == 0
+
+
 def _err(lib):
     return lib.kascade_get_last_error().decode()
 

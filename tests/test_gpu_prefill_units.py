@@ -367,18 +367,32 @@ def _anchor_inputs(cuda, gen, heads, G, D, L, B, dtype):
     return q, k
 
 
-# units and key tiles on both sides of each line of the rule: 192 units with 6 tiles and with 7, 216 and 256 units, head_dim 64
-# with 8 and 9 tiles, 264 and 448 units, 16 and 17 tiles, 456 units, rows of up to 4096 keys and longer ones; tails of every kind
-@pytest.mark.parametrize("heads,G,D,L,B,dtype", [
-    (32, 8, 128, 1, 1, torch.float16), (32, 8, 128, 33, 1, torch.bfloat16), (32, 8, 128, 768, 1, torch.float16),
-    (28, 4, 128, 897, 1, torch.bfloat16), (32, 8, 128, 843, 1, torch.float16), (32, 8, 128, 1024, 1, torch.float16),
-    (32, 8, 64, 1024, 1, torch.float16), (32, 8, 64, 1025, 1, torch.float16), (8, 2, 64, 2049, 2, torch.bfloat16),
-    (40, 8, 128, 1050, 1, torch.float16), (32, 8, 128, 1791, 1, torch.float16), (28, 4, 128, 2081, 1, torch.float16),
-    (28, 4, 128, 2050, 1, torch.bfloat16), (24, 8, 128, 1801, 1, torch.float16), (14, 2, 64, 4128, 2, torch.float16),
-    (4, 4, 128, 4128, 1, torch.float16), (4, 4, 128, 4129, 1, torch.float16), (16, 1, 64, 517, 3, torch.float16)])
-def test_pooling_that_selects_gives_the_lists_of_two_launches(cuda, heads, G, D, L, B, dtype):
+# Units and key tiles on both sides of each line of the rule (kascade_prefill_pool_selects, the last column), with tails of every
+# kind: up to 192 units with 6 tiles and with 7, 216 and 256 units, head_dim 64 with 8 and 9 tiles; up to 448 units with 16 and 17
+# tiles (the latter among the chunks), 10 and 11 where the (KV head, sequence) pairs are no multiple of eight; up to 512 units with
+# 18, 20 and 29 tiles; 516 and 528 units; rows of up to 4096 keys and longer ones.
+POOLING_CASES = [
+    (32, 8, 128, 1, 1, torch.float16, 1), (32, 8, 128, 33, 1, torch.bfloat16, 1), (32, 8, 128, 768, 1, torch.float16, 1),
+    (28, 4, 128, 897, 1, torch.bfloat16, 0), (32, 8, 128, 843, 1, torch.float16, 1), (32, 8, 128, 1024, 1, torch.float16, 1),
+    (32, 8, 64, 1024, 1, torch.float16, 1), (32, 8, 64, 1025, 1, torch.float16, 1), (8, 2, 64, 2049, 2, torch.bfloat16, 0),
+    (40, 8, 128, 1050, 1, torch.float16, 1), (32, 8, 128, 1791, 1, torch.float16, 1), (28, 4, 128, 2081, 1, torch.float16, 0),
+    (28, 4, 128, 2050, 1, torch.bfloat16, 0), (24, 8, 128, 1801, 1, torch.float16, 1), (14, 2, 64, 4128, 2, torch.float16, 1),
+    (4, 4, 128, 4128, 1, torch.float16, 1), (4, 4, 128, 4129, 1, torch.float16, 0), (16, 1, 64, 517, 3, torch.float16, 1),
+    (8, 2, 64, 1100, 3, torch.float16, 0), (14, 2, 128, 1300, 4, torch.bfloat16, 1), (36, 9, 64, 1281, 1, torch.float16, 1),
+    (36, 9, 128, 1313, 1, torch.bfloat16, 0), (28, 4, 128, 1300, 2, torch.float16, 1), (28, 7, 64, 2300, 1, torch.float16, 1),
+    (12, 3, 64, 2592, 2, torch.bfloat16, 1), (8, 2, 128, 3620, 2, torch.float16, 0), (12, 3, 64, 2800, 2, torch.float16, 1)]
+
+
+def assert_pooling_route(G, D, B, q_start, rows, one_launch):
+    from kascade_amd import _lib
+    assert _lib.load().kascade_prefill_pool_selects(G, D, B, q_start, rows) == one_launch
+
+
+@pytest.mark.parametrize("heads,G,D,L,B,dtype,one_launch", POOLING_CASES)
+def test_pooling_that_selects_gives_the_lists_of_two_launches(cuda, heads, G, D, L, B, dtype, one_launch):
     """Prompts, strided and over shuffled pages: the lists of pooling and selection by calls of their own."""
     from kascade_amd import budgets, kernels
+    assert_pooling_route(G, D, B, 0, L, one_launch)
     gen = torch.Generator().manual_seed(L + heads)
     q, k = _anchor_inputs(cuda, gen, heads, G, D, L, B, dtype)
     kp, table = _paged_copies(k[:1], 16, gen, 1, cuda)
@@ -399,12 +413,16 @@ def test_pooling_that_selects_gives_the_lists_of_two_launches(cuda, heads, G, D,
         assert torch.equal(own, want[:1]) and torch.equal(rows, kernels.translate_indices(own.contiguous(), table, L, 16))
 
 
-@pytest.mark.parametrize("heads,G,D,start,n,B", [(32, 8, 128, 0, 512, 1), (32, 8, 128, 1024, 1024, 1), (32, 8, 128, 2048, 2048, 1),
-                                                 (28, 4, 128, 2048, 2017, 1), (8, 2, 64, 256, 300, 4), (64, 8, 128, 64, 500, 3)])
-def test_pooling_that_selects_over_chunks(cuda, heads, G, D, start, n, B):
+POOLING_CHUNKS = [(32, 8, 128, 0, 512, 1, 1), (32, 8, 128, 1024, 1024, 1, 1), (32, 8, 128, 2048, 2048, 1, 1), (28, 4, 128, 2048, 2017, 1, 1),
+                  (8, 2, 64, 256, 300, 4, 1), (64, 8, 128, 64, 500, 3, 1), (32, 8, 128, 800, 1280, 1, 1), (32, 8, 128, 832, 1280, 1, 0)]
+
+
+@pytest.mark.parametrize("heads,G,D,start,n,B,one_launch", POOLING_CHUNKS)
+def test_pooling_that_selects_over_chunks(cuda, heads, G, D, start, n, B, one_launch):
     """Chunks at one position and, with starts and row counts of their own (none and remainders among them), mixed ones:
     the lists and cache rows of two launches."""
     from kascade_amd import kernels
+    assert_pooling_route(G, D, B, start, n, one_launch)
     from kascade_amd.strategy import PagedKascadePrefill
     gen = torch.Generator().manual_seed(start + n)
     L, T = start + n, (n + 31) // 32
@@ -434,6 +452,7 @@ def test_pooling_that_selects_takes_keys_of_every_value(cuda, value):
     """Keys that make scores infinite or no number, one and a whole tile of them: the lists of two launches."""
     from kascade_amd import budgets, kernels
     L, G = 700, 8
+    assert_pooling_route(G, 128, 1, 0, L, 1)
     gen = torch.Generator().manual_seed(3)
     q, k = _anchor_inputs(cuda, gen, 32, G, 128, L, 1, torch.float16)
     k[0, 200:340, 1] = value
