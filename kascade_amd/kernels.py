@@ -883,8 +883,8 @@ def prefill_anchor_topk(Q, K, log_sum, scores, k: int, valid_len, n_sel, fill_va
         _req(Q, shape[3], "Q", False); _req(K, shape[3], "K", False)
         B, Lq = Q.shape[:2]
         qs, ks, pages = _blhd_strides(Q, "Q"), ctypes.byref(_blhd_strides(K, "K")), (None, 0, 1, 0, None, None)
-        if K.shape[1] < q_start + Lq:
-            raise KascadeError("K must hold the positions up to q_start + rows of Q")
+        if K.shape[0] != B or K.shape[1] < q_start + Lq:
+            raise KascadeError("K must hold Q's sequences and the positions up to q_start + rows of Q")
     Hq, Gk, Dh, dt = shape
     _req(log_sum, torch.float32, "log_sum"); _req(scores, torch.float16, "scores")
     _req(valid_len, torch.int32, "valid_len"); _req(n_sel, torch.int32, "n_sel")

@@ -467,6 +467,21 @@ def test_pooling_that_selects_takes_keys_of_every_value(cuda, value):
     assert torch.equal(kernels.prefill_anchor_topk(q, k, log_sum, torch.empty_like(scores), W, valid, nsel), want)
 
 
+def test_pooling_that_selects_refuses_keys_of_other_sequences(cuda):
+    """K of fewer sequences than Q, or of fewer positions, is refused before anything is launched."""
+    from kascade_amd import kernels
+    from kascade_amd._lib import KascadeError
+    L, G = 64, 8
+    q = torch.zeros(2, L, 32, 128, device=cuda, dtype=torch.float16)
+    counts = torch.zeros(2, device=cuda, dtype=torch.int32)
+    scores, log_sum = torch.zeros(2, G, 2, L, device=cuda, dtype=torch.float16), torch.zeros(2, L, 32, device=cuda)
+    for k in (q[:1, :, :G], q[:, :L - 1, :G], torch.zeros(3, L, G, 128, device=cuda, dtype=torch.float16)):
+        with pytest.raises(KascadeError, match="Q's sequences"):
+            kernels.prefill_anchor_topk(q, k, log_sum, scores, 128, counts, counts)
+    idx = kernels.prefill_anchor_topk(q, q[:1, :, :G].expand(2, -1, -1, -1), log_sum, scores, 128, counts, counts)
+    assert idx.shape == (2, G, 2, 128) and bool((idx == L - 1).all())   # nothing selected: the filling
+
+
 def _sparse_rows_as_documented(q, k, v, idx, p):
     """Rows of sparse units [L,H,D] with everything in 64 bits but the probabilities, which are rounded to the element type
     against references that the 32 queries of a block move together: when a score of any lies more than 2^8 above its own.
