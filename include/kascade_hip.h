@@ -339,7 +339,9 @@ int kascade_topk_rows_call(const kascade_half* scores, int32_t* out_idx, int row
  * kv_strides, no block table) or kascade_prefill_chunk_aggregate_shaped_call (pages) followed by kascade_topk_rows_call
  * gives, for rows [batch, kv_heads, tiles] of the queries' 32-row tiles; in one launch where rows are short.
  *   scores: scratch [batch, kv_heads, tiles, q_start + q_len] fp16, left with unspecified contents
- *   valid_len / n_sel [period], both required: keys row r looks at (at most those in front of its tile) and takes
+ *   valid_len / n_sel [period], both required: keys row r looks at and takes.  More keys than lie in front of the row's
+ *     tile are the caller's mistake, which is not looked for: that row's list is unspecified then (positions below
+ *     valid_len, but taken by whatever scores the scratch held), the others are not touched by it
  *   out_idx [rows, k]; out_rows [rows, k] or NULL: the same as cache rows (with a block table)
  *   workspace: as for kascade_topk_call, kascade_topk_workspace_bytes(rows, q_start + q_len) bytes or NULL.
  * kascade_prefill_pool_selects: 1 where one launch pools and selects, 0 where two do; the lists are the same. */

@@ -872,8 +872,9 @@ def prefill_anchor_topk(Q, K, log_sum, scores, k: int, valid_len, n_sel, fill_va
                         q_starts=None, q_lens=None):
     """``aggregate_kernel`` and ``torch.topk`` of a prompt or chunk in one call (EfficientKascadeStrategy.py:81-82):
     ``prefill_aggregate_range`` or, with a block table, ``prefill_chunk_aggregate``, then ``topk_indices`` -- one launch
-    where the rows are short.  ``scores`` [B,G,ceil(Lq/32),q_start+Lq] is scratch.  Returns the indices or, with a
-    block table, (indices, cache_rows)."""
+    where the rows are short.  ``scores`` [B,G,ceil(Lq/32),q_start+Lq] is scratch.  ``valid_len`` of a row must not be more
+    than the keys in front of its tile: its list is unspecified then.  Returns the indices or, with a block table,
+    (indices, cache_rows)."""
     lib = _lib.init()
     if block_table is not None:
         B, Lq, qs, shape = _chunk_args(Q, K, block_table, q_start, page_size, q_starts, q_lens)

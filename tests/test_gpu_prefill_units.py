@@ -482,6 +482,28 @@ def test_pooling_that_selects_refuses_keys_of_other_sequences(cuda):
     assert idx.shape == (2, G, 2, 128) and bool((idx == L - 1).all())   # nothing selected: the filling
 
 
+@pytest.mark.parametrize("heads,G,L,one_launch", [(32, 8, 700, 1), (28, 4, 897, 0)])
+def test_pooling_that_selects_keeps_a_wrong_length_to_its_row(cuda, heads, G, L, one_launch):
+    """A valid_len beyond the keys in front of its tile is the caller's mistake: that row's positions are unspecified below it,
+    every other row's are as they were."""
+    from kascade_amd import budgets, kernels
+    assert_pooling_route(G, 128, 1, 0, L, one_launch)
+    gen = torch.Generator().manual_seed(L)
+    q, k = _anchor_inputs(cuda, gen, heads, G, 128, L, 1, torch.float16)
+    k = k.to(cuda)
+    log_sum = kernels.prefill_recompute1(q, k)
+    T, W = (L + 31) // 32, budgets.topk_width(L, 10)
+    valid, nsel = (torch.tensor(x, dtype=torch.int32, device=cuda) for x in budgets.prefill_tile_budgets(L, 32, 10, True, W))
+    scores = torch.zeros(1, G, T, L, device=cuda, dtype=torch.float16)
+    want = kernels.prefill_anchor_topk(q, k, log_sum, scores.clone(), W, valid, nsel)
+    valid[T // 2] += 70
+    got = kernels.prefill_anchor_topk(q, k, log_sum, scores, W, valid, nsel)
+    rows = torch.arange(T, device=cuda) != T // 2
+    assert torch.equal(got[:, :, rows], want[:, :, rows])
+    taken = got[:, :, T // 2, :int(nsel[T // 2])]
+    assert bool(((taken >= 0) & (taken < valid[T // 2])).all())
+
+
 def _sparse_rows_as_documented(q, k, v, idx, p):
     """Rows of sparse units [L,H,D] with everything in 64 bits but the probabilities, which are rounded to the element type
     against references that the 32 queries of a block move together: when a score of any lies more than 2^8 above its own.
